@@ -36,7 +36,7 @@ enum { CV_SUCCESS = 0, CV_TOO_MUCH_WORK = -1, CV_TOO_MUCH_ACC = -2, CV_ERR_FAILU
        CV_FIRST_RHSFUNC_ERR = -9, CV_REPTD_RHSFUNC_ERR = -10, CV_UNREC_RHSFUNC_ERR = -11,
        CV_ILL_INPUT = -22 };
 enum { FIRST_CALL = 1, PREV_CONV_FAIL, PREV_ERR_FAIL };
-enum { DO_ERROR_TEST = 2, PREDICT_AGAIN, CONV_FAIL, TRY_AGAIN, RHSFUNC_RECVR };
+enum { DO_ERROR_TEST = 2, PREDICT_AGAIN, CONV_FAIL, TRY_AGAIN, RHSFUNC_RECVR, NEWTON_F, ERR_TEST_F };
 enum { CV_NO_FAILURES = 0, CV_FAIL_BAD_J = 1, CV_FAIL_OTHER = 2 };
 
 __device__ __forceinline__ double rpowerr(double b, double e) { return b <= 0.0 ? 0.0 : pow(b, e); }
@@ -45,6 +45,13 @@ __device__ __forceinline__ double rpoweri(double b, int e) {
   for (int i = 1; i <= (e < 0 ? -e : e); ++i) p *= b;
   return e < 0 ? 1.0 / p : p;
 }
+
+// A condition on wave-uniform values as a scalar: every lane of the wavefront
+// is active and agrees, but the compiler cannot see that of values that come
+// through LDS or calls, and one branch it takes for divergent makes every
+// control variable set under it per-lane (the whole integrator then ran under
+// execution masks, with its control state copied between vector registers).
+__device__ __forceinline__ bool uc(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
 
 // A wave-uniform double kept in scalar registers: every assignment reads the
 // first active lane's value (all lanes hold the same one), so the value
@@ -71,16 +78,25 @@ struct UDouble {
 };
 
 // MP selects the multi-phase instantiation: gas-phase programs run a kernel
-// without the aerosol code (smaller code and register footprint).
-template <bool MP>
+// without the aerosol code (smaller code and register footprint).  KG: the
+// rate constants are read in place in global memory (s_k) and, for the f
+// terms, held by the lanes (kt).
+template <bool MP, bool KG>
 struct CellCv {
-  // the kernel argument's program (kernarg memory: uniform, read-only, so
-  // its fields are reloaded with scalar loads rather than kept in registers)
-  const DevProgram& P;
-  __device__ explicit CellCv(const DevProgram& prog) : P(prog) {}
+  // The kernel argument's program, read from kernarg memory anew where a phase
+  // begins: the pointer is opaque to the compiler there, so the phase's fields
+  // come with a few scalar loads.  Loaded once at the kernel's start, as the
+  // compiler would otherwise, the ~90 pointers overflow the scalar registers
+  // into lanes of vector registers, and each use costs a v_readlane pair (24
+  // cycles each).
+  __device__ __forceinline__ static const DevProgram& program() {
+    auto k = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(k));
+    return *(const DevProgram*)(const __attribute__((address_space(4))) DevProgram*)k;
+  }
   int lane, nv;
-  double *s_state, *s_k, *s_rate, *znb, *ewt, *acor, *y, *tempv, *ftemp, *last, *acinit, *gh1, *gh2,
-      *w, *lu, *s_fb;
+  double *s_state, *s_k, *s_rate, *z01, *z2, *ewt, *acor, *y, *tempv, *ftemp, *last, *acinit,
+      *w, *lu, *slu, *s_fb;
   double *Js, *Jy, *Jf;
   MpLds mpl;   // multi-phase extras (LDS); unused for gas-phase programs
   double* Jr;  // reaction Jacobian scratch (global) of multi-phase programs
@@ -89,12 +105,34 @@ struct CellCv {
   UDouble rl1, gamma, gammap, gamrat, crate, acnrm, saved_tq5;
   int q, qprime, L, qwait, jcur, use_acinit, guess_on, maxcf, max_steps, projected;
   int nst, nfe, nsetups, nni, ncfn, netf, nje, nstlp, nstlj;
+  // the rate constants of the lane's first kTermRegs terms
+  double kt[kTermRegs];
+  __device__ __forceinline__ void load_term_constants() {
+    const DevProgram& P = program();
+#pragma unroll
+    for (int g = 0; g < kTermRegs; ++g) {
+      int t = lane + g * kWave;
+      kt[g] = t < P.n_terms ? s_k[P.t_rec[t].x & 0x0FFFFFFF] : 0.0;
+    }
+  }
   // optional shader-clock counters (cycles in f, Jac, LU factor, LU solve)
   bool prof;
   long long c_f, c_j, c_lu, c_sol, c_fr, c_fg;
   __device__ __forceinline__ long long tick() const { return prof ? clock64() : 0; }
 
-  __device__ __forceinline__ double* zn(int j) const { return znb + (size_t)j * nv; }
+  // Nordsieck vectors 0 and 1 (read in every Newton iteration) and 2 to 5,
+  // which may live apart
+  __device__ __forceinline__ double* zn0() const { return z01; }
+  __device__ __forceinline__ double* zn1() const { return z01 + nv; }
+  __device__ __forceinline__ double* znh(int j) const { return z2 + (size_t)(j - 2) * nv; }
+  __device__ __forceinline__ double zget(int j, int i) const {
+    return j == 0 ? zn0()[i] : j == 1 ? zn1()[i] : znh(j)[i];
+  }
+  __device__ __forceinline__ void zset(int j, int i, double v) const {
+    if (j == 0) zn0()[i] = v;
+    else if (j == 1) zn1()[i] = v;
+    else znh(j)[i] = v;
+  }
 
   __device__ __forceinline__ double wrms(const double* x) {
     double s = 0.0;
@@ -106,61 +144,69 @@ struct CellCv {
     return sqrt(s / nv);
   }
 
-  __device__ __forceinline__ void ewt_set(const double* ycur) {
-    for (int i = lane; i < nv; i += kWave)
-      ewt[i] = 1.0 / (rtol * fabs(ycur[i]) + P.abs_tol_dep[i]);
-    wsync();
-  }
-
-  // CAMP f(): camp_solver.c:843-958 for one cell (use_deriv_est = 1)
-  __device__ __forceinline__ int f(const double* yv, double* out) {
-    nfe++;
-    long long t0 = tick();
-    double ts = next_h > 0.0 ? next_h : init_h;
-    int bad = cell_set_state(P, lane, yv, s_state);
-    if (!bad) {
-      if (MP) mp_f_prologue(P, lane, s_state, s_k, mpl);
-      cell_rates(P, lane, s_state, s_k, s_rate);
-      wsync();
-      long long t1 = tick();
-      if (prof) c_fr += t1 - t0;
-      cell_deriv(P, lane, s_state, s_rate, yv, Js, Jy, Jf, true, ts, out, s_fb, mpl.slot);
-      wsync();
-      if (prof) c_fg += clock64() - t1;
+  // the error weights of zn[0], and zn[0]'s WRMS norm under them
+  __device__ __forceinline__ double ewt_set() {
+    const DevProgram& P = program();
+    double s = 0.0;
+    for (int i = lane; i < nv; i += kWave) {
+      double z = zn0()[i], wt = 1.0 / (rtol * fabs(z) + P.abs_tol_dep[i]);
+      ewt[i] = wt;
+      double p = z * wt;
+      s += p * p;
     }
     wsync();
-    if (prof) c_f += clock64() - t0;
+    return sqrt(wave_sum(s) / nv);
+  }
+
+  // CAMP f(): camp_solver.c:843-958 for one cell; est = false is the pure f
+  // that Jac() runs first (camp_solver.c:1052-1063).  y -> ftemp always: fixed
+  // arguments keep their address spaces known to the compiler.
+  __device__ __forceinline__ int f(bool est) {
+    const DevProgram& P = program();
+    long long t0 = tick();
+    double ts = next_h > 0.0 ? next_h : init_h;
+    int bad = cell_set_state(P, lane, y, s_state);
+    if (!bad) {
+      if (MP) mp_f_prologue(P, lane, s_state, s_k, mpl);
+      cell_rates<KG>(P, lane, s_state, s_k, s_rate, kt);
+      wsync();
+      long long t1 = tick();
+      if (prof && est) c_fr += t1 - t0;
+      cell_deriv(P, lane, s_state, s_rate, y, Js, Jy, Jf, est, ts, ftemp, s_fb, mpl.slot);
+      wsync();
+      if (prof && est) c_fg += clock64() - t1;
+    }
+    wsync();
+    if (prof) (est ? c_f : c_j) += clock64() - t0;
     return bad;
   }
 
-  // CAMP Jac(): pure f into fy, J into the cell's J_solver, save history
-  __device__ __forceinline__ int jac(const double* yv, double* fy) {
+  // CAMP Jac() after its pure f: J into the cell's J_solver, save history
+  __device__ __forceinline__ void jac() {
+    const DevProgram& P = program();
     long long t0 = tick();
     double ts = next_h > 0.0 ? next_h : init_h;
-    if (cell_set_state(P, lane, yv, s_state)) return 1;
     if (MP) {
-      mp_f_prologue(P, lane, s_state, s_k, mpl);
-      cell_rates(P, lane, s_state, s_k, s_rate);
-      wsync();
-      cell_deriv(P, lane, s_state, s_rate, yv, Js, Jy, Jf, false, ts, fy, s_fb, mpl.slot);
-      wsync();
       mp_refresh(P, lane, s_state, mpl);
       mp_j_prologue(P, lane, s_state, s_k, mpl);
       cell_jac_mp(P, lane, s_state, s_k, ts, mpl, Jr, Js);
     } else {
-      cell_rates(P, lane, s_state, s_k, s_rate);
-      wsync();
-      cell_deriv(P, lane, s_state, s_rate, yv, Js, Jy, Jf, false, ts, fy, s_fb);
-      cell_jac(P, lane, s_state, s_k, ts, Js);
+      const double* k = s_k;
+      if (KG) {
+        // J reads its constants at random: staged where the LU goes next
+        for (int i = lane; i < P.n_env; i += kWave) lu[i] = s_k[i];
+        wsync();
+        k = lu;
+      }
+      cell_jac(P, lane, s_state, k, ts, Js);
     }
     for (int i = lane; i < nv; i += kWave) {
-      Jy[i] = yv[i];
-      Jf[i] = fy[i];
+      Jy[i] = y[i];
+      Jf[i] = ftemp[i];
     }
     __threadfence_block();
     wsync();
     if (prof) c_j += clock64() - t0;
-    return 0;
   }
 
   // The history updates below work on one row of the Nordsieck array at a
@@ -172,7 +218,7 @@ struct CellCv {
   __device__ __forceinline__ void hist_load(int i, double* z) const {
 #pragma unroll
     for (int j = 0; j <= QMAX; ++j)
-      if (j <= q) z[j] = zn(j)[i];
+      if (j <= q) z[j] = zget(j, i);
   }
 
   __device__ __forceinline__ void rescale() {
@@ -188,7 +234,7 @@ struct CellCv {
       hist_load(i, z);
 #pragma unroll
       for (int j = 1; j <= QMAX; ++j)
-        if (j <= q) zn(j)[i] = z[j] * fac[j];
+        if (j <= q) zset(j, i, z[j] * fac[j]);
     }
     h = hscale * eta;
     next_h = h;
@@ -196,9 +242,11 @@ struct CellCv {
     wsync();
   }
 
-  // zn[j-1] += zn[j] (SIGN 1) or -= (SIGN -1), k = 1..q, j = q..k
+  // zn[j-1] += zn[j] (SIGN 1) or -= (SIGN -1), k = 1..q, j = q..k; a
+  // prediction also goes to y, and its minimum is returned
   template <int SIGN>
-  __device__ __forceinline__ void pascal() {
+  __device__ __forceinline__ double pascal() {
+    double mn = 1.0e308;
     for (int i = lane; i < nv; i += kWave) {
       double z[QMAX + 1];
       hist_load(i, z);
@@ -209,14 +257,19 @@ struct CellCv {
           if (j <= q) z[j - 1] = SIGN > 0 ? z[j - 1] + z[j] : z[j - 1] - z[j];
 #pragma unroll
       for (int j = 0; j < QMAX; ++j)
-        if (j < q) zn(j)[i] = z[j];
+        if (j < q) zset(j, i, z[j]);
+      if (SIGN > 0) {
+        y[i] = z[0];
+        mn = fmin(mn, z[0]);
+      }
     }
     wsync();
+    return mn;
   }
 
-  __device__ __forceinline__ void predict() {
+  __device__ __forceinline__ double predict() {
     tn += h;
-    pascal<1>();
+    return wave_min(pascal<1>());
   }
 
   __device__ __forceinline__ void restore(double saved_t) {
@@ -224,54 +277,76 @@ struct CellCv {
     pascal<-1>();
   }
 
-  __device__ __forceinline__ void set_tq(double hsum, double alpha0, double alpha0_hat, double xi_inv,
-                         double xistar_inv) {
+  // cvSet and cvSetTqBDF.  All step-size quotients h / (h + tau_1 + ... +
+  // tau_(j-1)) are formed at once (their divisions overlap; those past the
+  // order are not used), and l is built in registers and stored once: loops
+  // over the LDS arrays were a chain of LDS round trips and divisions.
+  __device__ __forceinline__ void set() {
+    double hs = h, x[QMAX + 2], L_[QMAX + 1];
+#pragma unroll
+    for (int j = 2; j <= QMAX + 1; ++j) {
+      hs += tau[j - 1];
+      x[j] = h / hs;
+    }
+    L_[0] = L_[1] = 1.0;
+#pragma unroll
+    for (int j = 2; j <= QMAX; ++j) L_[j] = 0.0;
+    double alpha0 = -1.0, alpha0_hat = -1.0, xi_inv = 1.0, xistar_inv = 1.0, lq = 1.0, rq = 1.0;
+    double xi_next = x[2];
+    if (q > 1) {
+#pragma unroll
+      for (int j = 2; j < QMAX; ++j)
+        if (j < q) {
+          alpha0 -= 1.0 / j;
+#pragma unroll
+          for (int i = QMAX; i >= 1; --i)
+            if (i <= j) L_[i] += L_[i - 1] * x[j];
+        }
+#pragma unroll
+      for (int j = 2; j <= QMAX; ++j)
+        if (j == q) {
+          rq = 1.0 / j;
+          xi_inv = x[j];
+          xi_next = x[j + 1];
+        }
+      alpha0 -= rq;
+      xistar_inv = -L_[1] - alpha0;
+      alpha0_hat = -L_[1] - xi_inv;
+#pragma unroll
+      for (int i = QMAX; i >= 1; --i)
+        if (i <= q) L_[i] += L_[i - 1] * xistar_inv;
+#pragma unroll
+      for (int j = 2; j <= QMAX; ++j)
+        if (j == q) lq = L_[j];
+    } else {
+      lq = L_[1];
+    }
     double A1 = 1.0 - alpha0_hat + alpha0;
     double A2 = 1.0 + q * A1;
-    tq[2] = fabs(A1 / (alpha0 * A2));
-    tq[5] = fabs(A2 * xistar_inv / (l[q] * xi_inv));
+    double tq2 = fabs(A1 / (alpha0 * A2));
+    double tq5 = fabs(A2 * xistar_inv / (lq * xi_inv));
+    tq[2] = tq2;
+    tq[5] = tq5;
     if (qwait == 1) {
       if (q > 1) {
-        double C = xistar_inv / l[q];
-        double A3 = alpha0 + 1.0 / q;
+        double C = xistar_inv / lq;
+        double A3 = alpha0 + rq;
         double A4 = alpha0_hat + xi_inv;
         double Cpinv = (1.0 - A4 + A3) / A3;
         tq[1] = fabs(C * Cpinv);
       } else {
         tq[1] = 1.0;
       }
-      hsum += tau[q];
-      xi_inv = h / hsum;
       double A5 = alpha0 - (1.0 / (q + 1));
-      double A6 = alpha0_hat - xi_inv;
+      double A6 = alpha0_hat - xi_next;
       double Cppinv = (1.0 - A6 + A5) / A2;
-      tq[3] = fabs(Cppinv / (xi_inv * (q + 2) * A5));
+      tq[3] = fabs(Cppinv / (xi_next * (q + 2) * A5));
     }
-    tq[4] = NLSCOEF / tq[2];
-  }
-
-  __device__ __forceinline__ void set() {
-    double alpha0, alpha0_hat, xi_inv, xistar_inv, hsum;
-    l[0] = l[1] = xi_inv = xistar_inv = 1.0;
-    for (int z = 2; z <= q; ++z) l[z] = 0.0;
-    alpha0 = alpha0_hat = -1.0;
-    hsum = h;
-    if (q > 1) {
-      for (int j = 2; j < q; ++j) {
-        hsum += tau[j - 1];
-        xi_inv = h / hsum;
-        alpha0 -= 1.0 / j;
-        for (int i = j; i >= 1; --i) l[i] += l[i - 1] * xi_inv;
-      }
-      alpha0 -= 1.0 / q;
-      xistar_inv = -l[1] - alpha0;
-      hsum += tau[q - 1];
-      xi_inv = h / hsum;
-      alpha0_hat = -l[1] - xi_inv;
-      for (int i = q; i >= 1; --i) l[i] += l[i - 1] * xistar_inv;
-    }
-    set_tq(hsum, alpha0, alpha0_hat, xi_inv, xistar_inv);
-    rl1 = 1.0 / l[1];
+    tq[4] = NLSCOEF / tq2;
+#pragma unroll
+    for (int j = 0; j <= QMAX; ++j)
+      if (j <= q) l[j] = L_[j];
+    rl1 = 1.0 / L_[1];
     gamma = h * rl1;
     if (nst == 0) gammap = gamma;
     gamrat = (nst > 0) ? gamma / gammap : 1.0;
@@ -296,9 +371,9 @@ struct CellCv {
     }
     A1 = (-alpha0 - alpha1) / prod;
     for (int i = lane; i < nv; i += kWave) {
-      double v = A1 * zn(QMAX)[i];
-      zn(L)[i] = v;
-      for (int j = 2; j <= q; ++j) zn(j)[i] += l[j] * v;
+      double v = A1 * znh(QMAX)[i];
+      znh(L)[i] = v;
+      for (int j = 2; j <= q; ++j) znh(j)[i] += l[j] * v;
     }
     wsync();
   }
@@ -314,7 +389,7 @@ struct CellCv {
       for (int i = j + 2; i >= 2; --i) l[i] = l[i] * xi + l[i - 1];
     }
     for (int i = lane; i < nv; i += kWave)
-      for (int j = 2; j < q; ++j) zn(j)[i] += (-l[j]) * zn(q)[i];
+      for (int j = 2; j < q; ++j) znh(j)[i] += (-l[j]) * znh(q)[i];
     wsync();
   }
 
@@ -330,69 +405,52 @@ struct CellCv {
     rescale();
   }
 
-  // guess_helper, camp_solver.c:1321-1408 (called with h_n = h > 0)
-  // y_n_min: the minimum of y_n, which the caller has computed
-  __device__ __forceinline__ int guess_helper(double t_n, double h_n, const double* y_n, const double* y_n1,
-                              const double* hf, double* tmp1, double* corr, double y_n_min) {
-    if (y_n_min > -1.0e-30) return 0;
-    double c = 1.0 / h_n;
+  // The jump of one guess_helper iteration (camp_solver.c:1321-1408, called
+  // with h_n = h > 0): y moved along ftemp by the longest step that keeps it
+  // non-negative; returns the step.
+  __device__ __forceinline__ double guess_jump(int iter, double t_n, double t_0, double t_j) {
+    double h_j = t_n - (t_0 + t_j);
+    double best = h_j;
+    int found = 0;
     for (int i = lane; i < nv; i += kWave) {
-      tmp1[i] = y_n1[i];
-      corr[i] = c * hf[i];
-    }
-    wsync();
-    double t_0 = t_n - h_n;
-    double t_j = 0.0;
-    for (int iter = 0; iter < GUESS_MAX_ITER && t_0 + t_j < t_n; iter++) {
-      double h_j = t_n - (t_0 + t_j);
-      double best = h_j;
-      int found = 0;
-      for (int i = lane; i < nv; i += kWave) {
-        double t_star = -tmp1[i] / corr[i];
-        if ((t_star > 0.0 || (t_star == 0.0 && corr[i] < 0.0)) && t_star < best) {
-          best = t_star;
-          found = 1;
-        }
+      double c = ftemp[i], t_star = -y[i] / c;
+      if ((t_star > 0.0 || (t_star == 0.0 && c < 0.0)) && t_star < best) {
+        best = t_star;
+        found = 1;
       }
-      best = wave_min(best);
-      found = wave_or(found);
-      h_j = best;
-      if (found) h_j *= 0.95 + 0.1 * iter / (double)GUESS_MAX_ITER;
-      h_j = t_n < t_0 + t_j + h_j ? t_n - (t_0 + t_j) : h_j;
-      for (int i = lane; i < nv; i += kWave) tmp1[i] += h_j * corr[i];
-      wsync();
-      t_j += h_j;
-      if (f(tmp1, corr)) return -1;
     }
-    for (int i = lane; i < nv; i += kWave) corr[i] = (tmp1[i] - y_n[i]) * 0.999;
+    best = wave_min(best);
+    found = wave_or(found);
+    h_j = best;
+    if (uc(found != 0)) h_j *= 0.95 + 0.1 * iter / (double)GUESS_MAX_ITER;
+    h_j = t_n < t_0 + t_j + h_j ? t_n - (t_0 + t_j) : h_j;
+    for (int i = lane; i < nv; i += kWave) y[i] += h_j * ftemp[i];
     wsync();
-    return 1;
+    return h_j;
   }
 
-  __device__ __forceinline__ int lsetup(int convfail, const double* ypred, double* fpred) {
+  // whether the linear setup needs a new Jacobian (cvLsSetup)
+  __device__ __forceinline__ bool jac_bad(int convfail) {
     double dgamma = fabs(gamma / gammap - 1.0);
-    int jbad = (nst == 0) || (nst > nstlj + MSBJ) ||
-               ((convfail == CV_FAIL_BAD_J) && (dgamma < DGMAX_JBAD)) ||
-               (convfail == CV_FAIL_OTHER);
-    if (!jbad) {
-      jcur = 0;
-    } else {
-      nje++;
-      nstlj = nst;
-      jcur = 1;
-      if (jac(ypred, fpred)) return 1;
-    }
+    return (nst == 0) || (nst > nstlj + MSBJ) ||
+           ((convfail == CV_FAIL_BAD_J) && uc(dgamma < DGMAX_JBAD)) || (convfail == CV_FAIL_OTHER);
+  }
+
+  __device__ __forceinline__ int factor() {
+    const DevProgram& P = program();
     long long t0 = tick();
     int rc = cell_lu_factor(P, lane, Js, gamma, lu);
+    if (MP) cell_lu_order(P, lane, lu, slu);
     if (prof) c_lu += clock64() - t0;
     return rc;
   }
 
   __device__ __forceinline__ void lsolve(double* b) {
+    const DevProgram& P = program();
     long long t0 = tick();
-    cell_lu_solve(P, lane, lu, b, w);
+    cell_lu_solve<MP>(P, lane, MP ? slu : lu, b, w);
     if (prof) c_sol += clock64() - t0;
-    if (gamrat != 1.0) {
+    if (uc(gamrat != 1.0)) {
       double s = 2.0 / (1.0 + gamrat);
       for (int i = lane; i < nv; i += kWave) b[i] *= s;
       wsync();
@@ -412,113 +470,62 @@ struct CellCv {
     for (int i = lane; i < nv; i += kWave)
       if (y[i] < -1.0e-30) worst = fmax(worst, -y[i] * ewt[i]);
     worst = -wave_min(-worst);
-    if (worst > 1.0) return 1;
-    if (worst < 0.0) return -1;
+    if (uc(worst > 1.0)) return 1;
+    if (uc(worst < 0.0)) return -1;
     for (int i = lane; i < nv; i += kWave)
       if (y[i] < -1.0e-30) {
-        corr[i] = 1.0e-60 - zn(0)[i];
+        corr[i] = 1.0e-60 - zn0()[i];
         y[i] = 1.0e-60;
       }
     wsync();
     return 0;
   }
 
-  __device__ __forceinline__ int newton_iteration() {
-    int m = 0;
-    double del = 0.0, delp = 0.0;
-    for (;;) {
-      for (int i = lane; i < nv; i += kWave) {
-        double t = rl1 * zn(1)[i] + acor[i];
-        tempv[i] = gamma * ftemp[i] - t;
-      }
-      wsync();
-      lsolve(tempv);
-      nni++;
-      // the correction's WRMS norm, the corrected state and the per-lane sum
-      // of the new correction's norm in one pass over the rows (one round
-      // trip for the error weights and zn[0] instead of two)
-      double s_del = 0.0, s_acor = 0.0;
-      for (int i = lane; i < nv; i += kWave) {
-        double t = tempv[i], wt = ewt[i];
-        double p = t * wt;
-        s_del += p * p;
-        double a = acor[i] + t;
-        acor[i] = a;
-        y[i] = zn(0)[i] + a;
-        double pa = a * wt;
-        s_acor += pa * pa;
-      }
-      del = sqrt(wave_sum(s_del) / nv);
-      wsync();
-      if (m > 0) crate = fmax(CRDOWN * crate, del / delp);
-      double dcon = del * fmin(1.0, crate) / tq[4];
-      if (dcon <= 1.0) {
-        int pr = project(acor);
-        if (pr > 0) return jcur ? RHSFUNC_RECVR : TRY_AGAIN;
-        projected = pr == 0;
-        // (without a projection acor is the one summed above)
-        acnrm = pr < 0 ? (m == 0 ? del : sqrt(wave_sum(s_acor) / nv)) : wrms(acor);
-        jcur = 0;
-        return CV_SUCCESS;
-      }
+  // One Newton iteration up to the next f(y): NEWTON_F where it needs one
+  // (y holds the iterate), else the nonlinear solve's outcome.  m, del and
+  // delp carry the iteration count and the last two correction norms.
+  __device__ __forceinline__ int newton_pass(int& m, UDouble& delp) {
+    for (int i = lane; i < nv; i += kWave) {
+      double t = rl1 * zn1()[i] + acor[i];
+      tempv[i] = gamma * ftemp[i] - t;
+    }
+    wsync();
+    lsolve(tempv);
+    nni++;
+    // the correction's WRMS norm, the corrected state and the per-lane sum
+    // of the new correction's norm in one pass over the rows (one round
+    // trip for the error weights and zn[0] instead of two)
+    double s_del = 0.0, s_acor = 0.0;
+    for (int i = lane; i < nv; i += kWave) {
+      double t = tempv[i], wt = ewt[i];
+      double p = t * wt;
+      s_del += p * p;
+      double a = acor[i] + t;
+      acor[i] = a;
+      y[i] = zn0()[i] + a;
+      double pa = a * wt;
+      s_acor += pa * pa;
+    }
+    double del = sqrt(wave_sum(s_del) / nv);
+    wsync();
+    if (m > 0) crate = fmax(CRDOWN * crate, del / delp);
+    double dcon = del * fmin(1.0, crate) / tq[4];
+    const bool ok = uc(dcon <= 1.0);
+    if (!ok) {
       m++;
-      if ((m == MAXCOR) || ((m >= 2) && (del > RDIV * delp))) return jcur ? CONV_FAIL : TRY_AGAIN;
+      if ((m == MAXCOR) || ((m >= 2) && uc(del > RDIV * delp))) return jcur ? CONV_FAIL : TRY_AGAIN;
+    }
+    int pr = project(acor);
+    if (pr > 0) return jcur ? RHSFUNC_RECVR : TRY_AGAIN;
+    if (!ok) {
       delp = del;
-      if (project(acor) > 0) return jcur ? RHSFUNC_RECVR : TRY_AGAIN;
-      if (f(y, ftemp)) return jcur ? RHSFUNC_RECVR : TRY_AGAIN;
+      return NEWTON_F;
     }
-  }
-
-  __device__ __forceinline__ int nls(int nflag) {
-    int convfail = ((nflag == FIRST_CALL) || (nflag == PREV_ERR_FAIL)) ? CV_NO_FAILURES : CV_FAIL_OTHER;
-    int callSetup = (nflag == PREV_CONV_FAIL) || (nflag == PREV_ERR_FAIL) || (nst == 0) ||
-                    (nst >= nstlp + MSBP) || (fabs(gamrat - 1.0) > DGMAX);
-    use_acinit = 0;
-    if (guess_on) {
-      double mn = 1.0e308;
-      for (int i = lane; i < nv; i += kWave) {
-        double z = zn(0)[i];
-        acinit[i] = z - last[i];
-        mn = fmin(mn, z);
-      }
-      wsync();
-      int gh = guess_helper(tn, h, zn(0), last, acinit, gh1, gh2, wave_min(mn));
-      if (gh == 1) {
-        for (int i = lane; i < nv; i += kWave) acinit[i] = gh2[i];
-        wsync();
-        use_acinit = 1;
-      }
-    }
-    for (;;) {
-      for (int i = lane; i < nv; i += kWave) y[i] = use_acinit ? zn(0)[i] + acinit[i] : zn(0)[i];
-      wsync();
-      double mn = 1.0e308;
-      for (int i = lane; i < nv; i += kWave) mn = fmin(mn, y[i]);
-      if (wave_min(mn) < -1.0e-30) {
-        if (!use_acinit) {
-          for (int i = lane; i < nv; i += kWave) acinit[i] = 0.0;
-          wsync();
-          use_acinit = 1;
-        }
-        project(acinit);
-      }
-      if (f(y, ftemp)) return RHSFUNC_RECVR;
-      if (callSetup) {
-        int ier = lsetup(convfail, y, ftemp);
-        nsetups++;
-        callSetup = 0;
-        gamrat = crate = 1.0;
-        gammap = gamma;
-        nstlp = nst;
-        if (ier > 0) return CONV_FAIL;
-      }
-      for (int i = lane; i < nv; i += kWave) acor[i] = use_acinit ? acinit[i] : 0.0;
-      wsync();
-      int ier = newton_iteration();
-      if (ier != TRY_AGAIN) return ier;
-      callSetup = 1;
-      convfail = CV_FAIL_BAD_J;
-    }
+    projected = pr == 0;
+    // (without a projection acor is the one summed above)
+    acnrm = pr < 0 ? (m == 0 ? del : sqrt(wave_sum(s_acor) / nv)) : wrms(acor);
+    jcur = 0;
+    return CV_SUCCESS;
   }
 
   __device__ __forceinline__ int handle_nflag(int* nflagPtr, double saved_t, int* ncfPtr) {
@@ -542,7 +549,7 @@ struct CellCv {
   __device__ __forceinline__ int do_error_test(int* nflagPtr, double saved_t, int* nefPtr, double* dsmPtr) {
     double dsm = acnrm * tq[2];
     *dsmPtr = dsm;
-    if (dsm <= 1.0) return CV_SUCCESS;
+    if (uc(dsm <= 1.0)) return CV_SUCCESS;
     (*nefPtr)++;
     netf++;
     *nflagPtr = PREV_ERR_FAIL;
@@ -570,17 +577,18 @@ struct CellCv {
     next_h = h;
     hscale = h;
     qwait = LONG_WAIT;
-    if (f(zn(0), tempv)) return CV_UNREC_RHSFUNC_ERR;
-    for (int i = lane; i < nv; i += kWave) zn(1)[i] = h * tempv[i];
-    wsync();
-    return TRY_AGAIN;
+    return ERR_TEST_F;  // zn[1] restarts from f(zn[0])
   }
 
   __device__ __forceinline__ void complete_step() {
     nst++;
     hu = h;
-    for (int i = q; i >= 2; --i) tau[i] = tau[i - 1];
-    if ((q == 1) && (nst > 1)) tau[2] = tau[1];
+    double ta[QMAX + 1];
+#pragma unroll
+    for (int i = 1; i <= QMAX; ++i) ta[i] = tau[i];
+#pragma unroll
+    for (int i = QMAX; i >= 2; --i)
+      if (i <= q || (i == 2 && nst > 1)) tau[i] = ta[i - 1];
     tau[1] = h;
     qwait--;
     bool save = (qwait == 1) && (q != QMAX);
@@ -602,8 +610,8 @@ struct CellCv {
       }
 #pragma unroll
       for (int j = 0; j <= QMAX; ++j)
-        if (j <= q) zn(j)[i] = z[j];
-      if (save) zn(QMAX)[i] = a;
+        if (j <= q) zset(j, i, z[j]);
+      if (save) znh(QMAX)[i] = a;
       last[i] = z[0];
     }
     if (save) saved_tq5 = tq[5];
@@ -611,7 +619,7 @@ struct CellCv {
   }
 
   __device__ __forceinline__ void set_eta() {
-    if (eta < THRESH) {
+    if (uc(eta < THRESH)) {
       eta = 1.0;
       hprime = h;
     } else {
@@ -621,14 +629,45 @@ struct CellCv {
   }
 
   __device__ __forceinline__ void prepare_next_step(double dsm) {
-    if (etamax == 1.0) {
+    if (uc(etamax == 1.0)) {
       qwait = qwait > 2 ? qwait : 2;
       qprime = q;
       hprime = h;
       eta = 1.0;
       return;
     }
-    etaq = 1.0 / (rpowerr(BIAS2 * dsm, 1.0 / L) + ADDON);
+    double ddn = -1.0, dup = -1.0;
+    if (qwait == 0) {
+      if (q > 1) {
+        ddn = wrms(znh(q)) * tq[1];
+      }
+      if (q != QMAX && uc(saved_tq5 != 0.0)) {
+        double cquot = (tq[5] / saved_tq5) * rpoweri(h / tau[2], L);
+        for (int i = lane; i < nv; i += kWave) tempv[i] = -cquot * znh(QMAX)[i] + acor[i];
+        wsync();
+        dup = wrms(tempv) * tq[3];
+      }
+    }
+    // The candidate ratios eta = 1 / (b^(1/n) + ADDON): one per lane, so that
+    // up to three powers (about 1000 cycles each) cost one, and none when all
+    // lie under THRESH for certain -- b >= (2/3)^n, rounded up, puts eta
+    // below 1.4999935 -- for then their values decide nothing.
+    const int w = lane % 3;
+    const int n = w == 0 ? L : w == 1 ? q : L + 1;
+    const bool on = w == 0 || (w == 1 ? ddn >= 0.0 : dup >= 0.0);
+    const double b = w == 0 ? BIAS2 * dsm : w == 1 ? BIAS1 * ddn : BIAS3 * dup;
+    double lim = 1.0;
+    for (int j = 0; j < n; ++j) lim *= 0.66667;
+    const bool small = !on || b >= lim;
+    if (__builtin_amdgcn_ballot_w64(!small) == 0) {
+      if (qwait == 0) qwait = 2;
+      eta = 1.0;
+      qprime = q;
+      hprime = h;
+      return;
+    }
+    const double r = on ? 1.0 / (rpowerr(b, 1.0 / n) + ADDON) : 0.0;
+    etaq = readlane_d(r, 0);
     if (qwait != 0) {
       eta = etaq;
       qprime = q;
@@ -636,78 +675,46 @@ struct CellCv {
       return;
     }
     qwait = 2;
-    etaqm1 = 0.0;
-    if (q > 1) {
-      double ddn = wrms(zn(q)) * tq[1];
-      etaqm1 = 1.0 / (rpowerr(BIAS1 * ddn, 1.0 / q) + ADDON);
-    }
-    etaqp1 = 0.0;
-    if (q != QMAX && saved_tq5 != 0.0) {
-      double cquot = (tq[5] / saved_tq5) * rpoweri(h / tau[2], L);
-      for (int i = lane; i < nv; i += kWave) tempv[i] = -cquot * zn(QMAX)[i] + acor[i];
-      wsync();
-      double dup = wrms(tempv) * tq[3];
-      etaqp1 = 1.0 / (rpowerr(BIAS3 * dup, 1.0 / (L + 1)) + ADDON);
-    }
+    etaqm1 = readlane_d(r, 1);
+    etaqp1 = readlane_d(r, 2);
     double etam = fmax(etaqm1, fmax(etaq, etaqp1));
-    if (etam < THRESH) {
+    if (uc(etam < THRESH)) {
       eta = 1.0;
       qprime = q;
-    } else if (etam == etaq) {
+    } else if (uc(etam == etaq)) {
       eta = etaq;
       qprime = q;
-    } else if (etam == etaqm1) {
+    } else if (uc(etam == etaqm1)) {
       eta = etaqm1;
       qprime = q - 1;
     } else {
       eta = etaqp1;
       qprime = q + 1;
-      for (int i = lane; i < nv; i += kWave) zn(QMAX)[i] = acor[i];
+      for (int i = lane; i < nv; i += kWave) znh(QMAX)[i] = acor[i];
       wsync();
     }
     set_eta();
-  }
-
-  __device__ __forceinline__ int step() {
-    double saved_t = tn, dsm = 0.0;
-    int ncf = 0, nef = 0, nflag = FIRST_CALL;
-    if ((nst > 0) && (hprime != h)) adjust_params();
-    for (;;) {
-      predict();
-      set();
-      nflag = nls(nflag);
-      int kflag = handle_nflag(&nflag, saved_t, &ncf);
-      if (kflag == PREDICT_AGAIN) continue;
-      if (kflag != DO_ERROR_TEST) return kflag;
-      int eflag = do_error_test(&nflag, saved_t, &nef, &dsm);
-      if (eflag == TRY_AGAIN) continue;
-      if (eflag != CV_SUCCESS) return eflag;
-      break;
-    }
-    complete_step();
-    prepare_next_step(dsm);
-    etamax = (nst <= SMALL_NST) ? ETAMX2 : ETAMX3;
-    for (int i = lane; i < nv; i += kWave) acor[i] *= tq[2];
-    wsync();
-    return CV_SUCCESS;
   }
 
   // Measurement: the cycles of f(y), J(y), the LU factorisation (gamma =
   // 10) and one triangular solve at the cell's staged state, averaged over
   // reps repetitions, into pr[0..3].  Integrates nothing.
   __device__ int bench_phases(int reps, double* pr) {
-    for (int i = lane; i < nv; i += kWave) y[i] = zn(0)[i];
+    for (int i = lane; i < nv; i += kWave) y[i] = zn0()[i];
     wsync();
     next_h = init_h = 1.0;
-    if (jac(y, ftemp)) return -101;
+    if (f(false)) return -101;
+    jac();
     long long cf = 0, cj = 0, clu = 0, cs = 0;
     for (int r = 0; r < reps; ++r) {
       long long t0 = clock64();
-      f(y, ftemp);
+      f(true);
       long long t1 = clock64();
-      jac(y, ftemp);
+      f(false);
+      jac();
       long long t2 = clock64();
-      if (cell_lu_factor(P, lane, Js, 10.0, lu)) return -102;
+      gamma = 10.0;
+      if (factor()) return -102;
       long long t3 = clock64();
       for (int i = lane; i < nv; i += kWave) tempv[i] = ftemp[i];
       wsync();
@@ -731,7 +738,7 @@ struct CellCv {
   // CVodeReInit + CVodeSetInitStep + CVode(tout, CV_NORMAL); zn(0) holds y0
   // on entry, y holds y(tout) on successful exit.
   __device__ __forceinline__ int solve(double t0, double tout) {
-    for (int i = lane; i < nv; i += kWave) last[i] = zn(0)[i];
+    for (int i = lane; i < nv; i += kWave) last[i] = zn0()[i];
     tn = t0;
     q = 1;
     L = 2;
@@ -752,33 +759,236 @@ struct CellCv {
     init_h = tout - t0;
     next_h = 0.0;
     wsync();
-    ewt_set(zn(0));
-    if (f(zn(0), zn(1))) return CV_FIRST_RHSFUNC_ERR;
-    h = init_h;
-    for (int i = lane; i < nv; i += kWave) zn(1)[i] *= h;
+    ewt_set();
+    // The integrator as one loop over actions, so that f(y) -- which the
+    // start, the guess helper, the predictor, Jac(), every Newton iteration
+    // and the error test's restart call -- and the other phases each appear
+    // once in the kernel: inlined at every call they made 130 KB of code (263
+    // KB with aerosol), several times the instruction cache.  An action that
+    // needs f puts its argument into y, sets where to go on (then) and hands
+    // over to ACT_F; bad is f's outcome.
+    enum { ACT_F, ACT_START, ACT_MAIN, ACT_PREDICT, ACT_GUESS, ACT_GUESS_F, ACT_NLS, ACT_NLS_F,
+           ACT_JAC, ACT_FACTOR, ACT_NEWTON, ACT_NEWTON_F, ACT_NLS_END, ACT_RESTART };
+    int act = ACT_F, then = ACT_START, bad = 0;
+    bool f_est = true;
+    auto call_f = [&](int next) {
+      f_est = true;
+      act = ACT_F;
+      then = next;
+    };
+    for (int i = lane; i < nv; i += kWave) y[i] = zn0()[i];
     wsync();
-    hscale = h;
-    hprime = h;
-    int nstloc = 0;
+    int nstloc = 0, ncf = 0, nef = 0, nflag = FIRST_CALL, convfail = 0, call_setup = 0, m = 0,
+        iter = 0, rc = 0;
+    double dsm = 0.0;
+    UDouble saved_t = tn, delp = 0.0, t_j = 0.0;
     for (;;) {
-      next_h = h;
-      if (nst > 0) ewt_set(zn(0));
-      if (nstloc >= max_steps) return CV_TOO_MUCH_WORK;
-      double nrm = wrms(zn(0));
-      if (2.220446049250313e-16 * nrm > 1.0) return CV_TOO_MUCH_ACC;
-      int kflag = step();
-      if (kflag != CV_SUCCESS) return kflag;
-      nstloc++;
-      if ((tn - tout) * h >= 0.0) {
-        double s = (tout - tn) / h;
-        for (int i = lane; i < nv; i += kWave) {
-          double v = zn(q)[i];
-          for (int j = q - 1; j >= 0; --j) v = zn(j)[i] + s * v;
-          y[i] = v;
+      // (addresses derived from these are computed in the action that uses
+      // them, not kept through all of them)
+      nv = phase_uniform(nv);
+      lane = phase_lane(lane);
+      switch (act) {
+        case ACT_F:
+          if (f_est) nfe++;
+          bad = f(f_est);
+          act = then;
+          break;
+        case ACT_START:
+          if (bad) return CV_FIRST_RHSFUNC_ERR;
+          h = init_h;
+          for (int i = lane; i < nv; i += kWave) zn1()[i] = ftemp[i] * h;
+          wsync();
+          hscale = h;
+          hprime = h;
+          act = ACT_MAIN;
+          break;
+        case ACT_MAIN: {  // CVode's loop, then the start of cvStep
+          next_h = h;
+          if (nstloc >= max_steps) return CV_TOO_MUCH_WORK;
+          double nrm = ewt_set();  // (before the first step: as it is)
+          if (uc(2.220446049250313e-16 * nrm > 1.0)) return CV_TOO_MUCH_ACC;
+          saved_t = tn;
+          dsm = 0.0;
+          ncf = nef = 0;
+          nflag = FIRST_CALL;
+          if ((nst > 0) && uc(hprime != h)) adjust_params();
+          act = ACT_PREDICT;
+          break;
         }
-        wsync();
-        next_h = hprime;
-        return CV_SUCCESS;
+        case ACT_PREDICT: {  // then the start of the nonlinear solve
+          double mn = predict();
+          set();
+          convfail = ((nflag == FIRST_CALL) || (nflag == PREV_ERR_FAIL)) ? CV_NO_FAILURES
+                                                                         : CV_FAIL_OTHER;
+          call_setup = (nflag == PREV_CONV_FAIL) || (nflag == PREV_ERR_FAIL) || (nst == 0) ||
+                       (nst >= nstlp + MSBP) || uc(fabs(gamrat - 1.0) > DGMAX);
+          use_acinit = 0;
+          if (uc(mn > -1.0e-30)) {
+            call_f(ACT_NLS_F);  // y is the prediction
+            break;
+          }
+          act = ACT_NLS;
+          // the guess helper acts on a negative prediction only
+          if (guess_on) {
+            double c = 1.0 / h;
+            for (int i = lane; i < nv; i += kWave) {
+              double la = last[i];
+              y[i] = la;
+              ftemp[i] = c * (zn0()[i] - la);
+            }
+            wsync();
+            t_j = 0.0;
+            iter = 0;
+            act = ACT_GUESS;
+          }
+          break;
+        }
+        case ACT_GUESS: {
+          double t_n = tn, t_0 = t_n - h;
+          if (iter < GUESS_MAX_ITER && uc(t_0 + t_j < t_n)) {
+            t_j += guess_jump(iter, t_n, t_0, t_j);
+            call_f(ACT_GUESS_F);
+            break;
+          }
+          for (int i = lane; i < nv; i += kWave) acinit[i] = (y[i] - zn0()[i]) * 0.999;
+          wsync();
+          use_acinit = 1;
+          act = ACT_NLS;
+          break;
+        }
+        case ACT_GUESS_F:
+          iter++;
+          act = bad ? ACT_NLS : ACT_GUESS;
+          break;
+        case ACT_NLS: {
+          double mn = 1.0e308;
+          for (int i = lane; i < nv; i += kWave) {
+            double v = use_acinit ? zn0()[i] + acinit[i] : zn0()[i];
+            y[i] = v;
+            mn = fmin(mn, v);
+          }
+          wsync();
+          if (uc(wave_min(mn) < -1.0e-30)) {
+            if (!use_acinit) {
+              for (int i = lane; i < nv; i += kWave) acinit[i] = 0.0;
+              wsync();
+              use_acinit = 1;
+            }
+            project(acinit);
+          }
+          call_f(ACT_NLS_F);
+          break;
+        }
+        case ACT_NLS_F:
+          if (bad) {
+            nflag = RHSFUNC_RECVR;
+            act = ACT_NLS_END;
+          } else if (!call_setup) {
+            m = -1;
+            act = ACT_NEWTON;
+          } else if (jac_bad(convfail)) {
+            nje++;
+            nstlj = nst;
+            jcur = 1;
+            call_f(ACT_JAC);
+            f_est = false;
+          } else {
+            jcur = 0;
+            bad = 0;
+            act = ACT_FACTOR;
+          }
+          break;
+        case ACT_JAC:
+          if (!bad) jac();
+          act = ACT_FACTOR;
+          break;
+        case ACT_FACTOR:
+          if (!bad) bad = uc(factor() != 0);
+          nsetups++;
+          call_setup = 0;
+          gamrat = crate = 1.0;
+          gammap = gamma;
+          nstlp = nst;
+          m = -1;
+          act = ACT_NEWTON;
+          if (bad) {
+            nflag = CONV_FAIL;
+            act = ACT_NLS_END;
+          }
+          break;
+        case ACT_NEWTON:
+          if (m < 0) {
+            for (int i = lane; i < nv; i += kWave) acor[i] = use_acinit ? acinit[i] : 0.0;
+            wsync();
+            m = 0;
+            delp = 0.0;
+          }
+          rc = newton_pass(m, delp);
+          if (rc == NEWTON_F) {
+            call_f(ACT_NEWTON_F);
+          } else if (rc == TRY_AGAIN) {
+            call_setup = 1;
+            convfail = CV_FAIL_BAD_J;
+            act = ACT_NLS;
+          } else {
+            nflag = rc;
+            act = ACT_NLS_END;
+          }
+          break;
+        case ACT_NEWTON_F:
+          act = ACT_NEWTON;
+          if (bad && jcur) {
+            nflag = RHSFUNC_RECVR;
+            act = ACT_NLS_END;
+          } else if (bad) {
+            call_setup = 1;
+            convfail = CV_FAIL_BAD_J;
+            act = ACT_NLS;
+          }
+          break;
+        case ACT_NLS_END: {
+          int kflag = handle_nflag(&nflag, saved_t, &ncf);
+          act = ACT_PREDICT;
+          if (kflag == PREDICT_AGAIN) break;
+          if (kflag != DO_ERROR_TEST) return kflag;
+          int eflag = do_error_test(&nflag, saved_t, &nef, &dsm);
+          if (eflag == TRY_AGAIN) break;
+          if (eflag == ERR_TEST_F) {
+            for (int i = lane; i < nv; i += kWave) y[i] = zn0()[i];
+            wsync();
+            call_f(ACT_RESTART);
+            break;
+          }
+          if (eflag != CV_SUCCESS) return eflag;
+          complete_step();
+          prepare_next_step(dsm);
+          etamax = (nst <= SMALL_NST) ? ETAMX2 : ETAMX3;
+          for (int i = lane; i < nv; i += kWave) acor[i] *= tq[2];
+          wsync();
+          nstloc++;
+          act = ACT_MAIN;
+          if (uc((tn - tout) * h >= 0.0)) {
+            double s = (tout - tn) / h;
+            for (int i = lane; i < nv; i += kWave) {
+              double z[QMAX + 1], v = 0.0;
+              hist_load(i, z);
+#pragma unroll
+              for (int j = QMAX; j >= 0; --j)
+                if (j <= q) v = j == q ? z[j] : z[j] + s * v;
+              y[i] = v;
+            }
+            wsync();
+            next_h = hprime;
+            return CV_SUCCESS;
+          }
+          break;
+        }
+        case ACT_RESTART:
+          if (bad) return CV_UNREC_RHSFUNC_ERR;
+          for (int i = lane; i < nv; i += kWave) zn1()[i] = h * ftemp[i];
+          wsync();
+          act = ACT_PREDICT;
+          break;
       }
     }
   }
@@ -787,7 +997,7 @@ struct CellCv {
 }  // namespace
 
 // MP: multi-phase program; PL: the placement (kPlaceLds, kPlaceGlobal:
-// the Nordsieck history, 7 of the 10 work vectors and the J history in
+// the Nordsieck history, 5 of the 8 work vectors and the J history in
 // global memory, kPlaceGlobalLu: the LU factors as well; multi-phase
 // programs run kPlaceGlobal with global LU factors).  Each variant is
 // compiled for the wavefronts per SIMD its LDS footprint lets onto a CU
@@ -811,40 +1021,47 @@ __global__ void __launch_bounds__(256)
   double* scratch = GH ? a.wave_scratch + ((size_t)blockIdx.x * (blockDim.x / kWave) + wv) *
                                               cell_bdf_wave_scratch(P, kPlace)
                        : nullptr;
-  CellCv<MP> cv(P);
+  CellCv<MP, !MP && PL == kPlaceGlobal> cv;
   cv.lane = lane;
   cv.nv = nv;
   cv.s_state = base;
-  cv.s_k = cv.s_state + P.ns;
-  cv.mpl = mp_lds(P, cv.s_k + P.n_env,
-                  MP ? scratch + P.lu_nnz + kWave + 1 + P.rnnz : nullptr);
-  cv.s_rate = cv.s_k + P.n_env + mp_lds_doubles(P);
+  constexpr bool kNewtonLds = !MP && PL == kPlaceGlobal;
+  // (kNewtonLds: no rate constants in LDS, see CellCv::kt)
+  double* sk_end = cv.s_state + P.ns;
+  if (!kNewtonLds) {
+    cv.s_k = sk_end;
+    sk_end += P.n_env;
+  }
+  cv.mpl = mp_lds(P, sk_end,
+                  MP ? scratch + 2 * (P.lu_nnz + kWave + 1) + P.rnnz : nullptr);
+  cv.s_rate = sk_end + mp_lds_doubles(P);
   double* v = cv.s_rate + 2 * (size_t)P.n_terms;
   // With GH the Nordsieck history and the work vectors other than y, acor
   // and w live in the wavefront's global scratch (after the LU where it is
   // global, and for multi-phase programs the J_rxn and Jacobian scalars);
   // else all in LDS.
-  double* g = MP   ? scratch + P.lu_nnz + kWave + 1 + P.rnnz + mp_jsc_doubles(P)
+  double* g = MP   ? scratch + 2 * (P.lu_nnz + kWave + 1) + P.rnnz + mp_jsc_doubles(P)
               : GL ? scratch + P.lu_nnz + kWave + 1
                    : scratch;
   double*& vh = GH ? g : v;
-  constexpr bool kNewtonLds = !MP && PL == kPlaceGlobal;
-  cv.znb = vh;
-  vh += 6 * (size_t)nv;
-  cv.last = vh; vh += nv;
-  cv.acinit = vh; vh += nv;
-  cv.ewt = vh; vh += nv;
-  // gas-phase cells with the history in global memory keep the Newton
-  // iteration's two work vectors in LDS as well (six cells still fit a CU)
+  // gas-phase cells with the history in global memory keep what every Newton
+  // iteration and step reads in LDS: zn[0], zn[1], the error weights and the
+  // iteration's two work vectors (six cells still fit a CU, as the rate
+  // constants stay in global memory and the lanes' registers)
   if (kNewtonLds) {
+    cv.z01 = v; v += 2 * (size_t)nv;
+    cv.ewt = v; v += nv;
     cv.tempv = v; v += nv;
     cv.ftemp = v; v += nv;
   } else {
+    cv.z01 = vh; vh += 2 * (size_t)nv;
+    cv.ewt = vh; vh += nv;
     cv.tempv = vh; vh += nv;
     cv.ftemp = vh; vh += nv;
   }
-  cv.gh1 = vh; vh += nv;
-  cv.gh2 = vh; vh += nv;
+  cv.z2 = vh; vh += 4 * (size_t)nv;
+  cv.last = vh; vh += nv;
+  cv.acinit = vh; vh += nv;
   cv.acor = v; v += nv;
   cv.y = v; v += nv;
   // the column solve's scratch w (nv > 128 only: smaller programs solve in
@@ -861,7 +1078,8 @@ __global__ void __launch_bounds__(256)
   // the f gather's scratch follows the LU values (gas: also the LU's sinks)
   if (MP) {
     cv.lu = scratch;
-    cv.Jr = scratch + P.lu_nnz + kWave + 1;
+    cv.slu = scratch + P.lu_nnz + kWave + 1;
+    cv.Jr = cv.slu + P.lu_nnz + kWave + 1;
     cv.s_fb = v; v += fb_sink_doubles(P);
   } else {
     cv.Jr = nullptr;
@@ -869,7 +1087,7 @@ __global__ void __launch_bounds__(256)
       cv.lu = scratch;
     } else {
       cv.lu = v;
-      v += P.lu_nnz;
+      v += kNewtonLds ? cell_lu_lds(P) : P.lu_nnz;
     }
     cv.s_fb = v; v += fb_sink_doubles(P);
     if (!GH) {
@@ -888,6 +1106,7 @@ __global__ void __launch_bounds__(256)
   cv.prof = !BENCH && a.prof != nullptr;
 
   for (;;) {
+    const DevProgram& P = cv.program();
     int q = 0;
     if (lane == 0) q = atomicAdd(a.counter, 1);
     q = __builtin_amdgcn_readfirstlane(q);  // lane 0's ticket, as a scalar
@@ -933,17 +1152,25 @@ __global__ void __launch_bounds__(256)
           state_c[i] = s;
         }
       }
-      for (int i = lane; i < P.n_env; i += kWave) cv.s_k[i] = renv_c[i];
+      if (kNewtonLds)
+        cv.s_k = renv_c;
+      else
+        for (int i = lane; i < P.n_env; i += kWave) cv.s_k[i] = renv_c[i];
       wsync();
       // rate constants for the cell's environment (rxn_update_env_state)
       double T = a.env[2 * cell], Pa = a.env[2 * cell + 1];
       cell_rate_constants(P, lane, T, Pa, cv.s_k);
       wsync();
       if (MP) mp_cell_env(P, lane, T, Pa, cv.mpl);
-      for (int i = lane; i < P.n_env; i += kWave) renv_c[i] = cv.s_k[i];
+      if (kNewtonLds) {
+        __threadfence_block();
+        cv.load_term_constants();
+      } else {
+        for (int i = lane; i < P.n_env; i += kWave) renv_c[i] = cv.s_k[i];
+      }
       for (int i = lane; i < nv; i += kWave) {
         double s = cv.s_state[P.dep_state[i]];
-        cv.zn(0)[i] = s > 1.0e-60 ? s : 1.0e-60;
+        cv.zn0()[i] = s > 1.0e-60 ? s : 1.0e-60;
       }
       wsync();
       cv.c_f = cv.c_j = cv.c_lu = cv.c_sol = cv.c_fr = cv.c_fg = 0;

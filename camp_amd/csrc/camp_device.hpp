@@ -37,14 +37,15 @@ struct DevProgram {
   int n_cs;                            // state variables that are not solver variables
   const int* cs_ids;
   const int *perm, *m_to_lu, *diag_pos, *e_diag;
-  const int *l_pos, *l_row, *u_pos, *u_row;  // column solve: padded columns (Program::cs_*)
   const uint64_t* up_rec;  // LU update records: dst | l << 16 | u << 32, rows of 64
-  const int4* lu_hdr;       // per pivot: {l range, update range}, {diag position, u range}
   const int* lf_pos;        // L positions the factorisation scales, rows of 64
   const int4* lf_hdr;       // per pivot: {lf_pos row start, up_rec row start,
                             //  L rows | update rows << 16, diag position}
-  const int4* ts_tbl;        // register solve: per block of 8 pivots and lane, 2 int4
-                             //  of pos(row t) | pos(row t + 64) << 16; nullptr when nv > 128
+  // triangular solves (Program::tri_e and following)
+  int tri_s, tri_d, tri_nf, tri_nb, tt_nf, tt_nb;
+  const int4 *tri_e, *tt;
+  const int2* tri_r;
+  const int *tri_diag, *tri_src;
   const int4* je_a;  // packed J records (see Program in camp_model.hpp)
   const int* je_b;
   const double* je_c;
@@ -113,6 +114,14 @@ __host__ __device__ __forceinline__ int phase_lane(int lane) {
   asm volatile("" : "+v"(lane));
 #endif
   return lane;
+}
+// A wave-uniform value made opaque the same way, in its scalar register.
+__host__ __device__ __forceinline__ int phase_uniform(int v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  v = __builtin_amdgcn_readfirstlane(v);
+  asm volatile("" : "+s"(v));
+#endif
+  return v;
 }
 // Read-only program data at a wave-uniform index through the scalar cache
 // (the program is never written while a kernel runs): the value lands in
@@ -278,11 +287,16 @@ __device__ __forceinline__ void cell_rate_constants(const DevProgram& P, int lan
 // (n_terms double-doubles): k * prod(reactants) as the per-type
 // calc_deriv_contrib computes it (rxn_arrhenius.c:143-147 and alike);
 // first-order loss rounds k * y to double (rxn_first_order_loss.c:150).
+// KT: the constants of a lane's first kTermRegs terms are in its registers
+// (kt), the others' in global memory.
+constexpr int kTermRegs = 4;
+template <bool KT = false>
 __host__ __device__ __forceinline__ void cell_rates(const DevProgram& P, int lane, const double* s_state,
-                                           const double* s_k, double* s_rate) {
+                                           const double* s_k, double* s_rate,
+                                           const double* kt = nullptr) {
   lane = phase_lane(lane);
   // a lane's terms in groups of four whose program loads are issued together
-  constexpr int TG = 4;
+  constexpr int TG = kTermRegs;
   for (int t0 = lane; t0 < P.n_terms; t0 += TG * kWave) {
     int4 tr[TG];
 #pragma unroll
@@ -295,7 +309,7 @@ __host__ __device__ __forceinline__ void cell_rates(const DevProgram& P, int lan
       int t = t0 + g * kWave;
       if (t >= P.n_terms) break;
       int fl = tr[g].x >> 28;
-      double k = s_k[tr[g].x & 0x0FFFFFFF];
+      double k = KT && t0 == lane ? kt[g] : s_k[tr[g].x & 0x0FFFFFFF];
       double y0 = s_state[tr[g].y >= 0 ? tr[g].y : 0], y1 = s_state[tr[g].z >= 0 ? tr[g].z : 0],
              y2 = s_state[tr[g].w >= 0 ? tr[g].w : 0];
       dd rate = {k, 0.0};
@@ -735,208 +749,219 @@ __device__ __forceinline__ double readlane_d(double v, int l) {
   return __hiloint2double(hi, lo);
 }
 
-// One block of 8 pivots of a triangular sweep whose pivot values sit in
-// register X of their owner lanes (lane k - k_base, k_base = 64 when X1).
-// The lane's two program words per pivot give the LU positions of its rows'
-// entries in the pivot's column (the zero slot where a row has none or the
-// pivot is outside the sweep), so the block's 16 weights are LDS loads that
-// depend on nothing but the program; then the chain, one readlane pair and
-// one FMA per row and pivot.  DIR is +1 (forward, L) or -1 (backward, U,
-// weights pre-scaled by the row's inverse diagonal).
-template <int DIR, bool X1>
-__device__ __forceinline__ void tri_block(int kb, int k_base, int4 t0, int4 t1, const double* lu,
-                                          double s0, double s1, double& x0, double& x1) {
-  constexpr int B = 8;
-  const int tw[B] = {t0.x, t0.y, t0.z, t0.w, t1.x, t1.y, t1.z, t1.w};
-  double w0[B], w1[B];
-#pragma unroll
-  for (int u = 0; u < B; ++u) {
-    w0[u] = lu[tw[u] & 0xFFFF] * s0;
-    w1[u] = lu[(unsigned)tw[u] >> 16] * s1;
-  }
-#pragma unroll
-  for (int u = 0; u < B; ++u) {
-    int k = kb + DIR * u;
-    double xk = readlane_d(X1 ? x1 : x0, (k - k_base) & (kWave - 1));
-    x0 = fma(-w0[u], xk, x0);
-    x1 = fma(-w1[u], xk, x1);
-  }
-}
+// ---------------------------------------------------------------------
+// Triangular solves (LU) x = b.
+//
+// A sweep is a chain: unknown k needs every earlier unknown of its row.  Taken
+// pivot by pivot (a column of L or U at a time) the CB05-scale mechanism with
+// its aerosol is 608 dependent steps of about 1000 cycles, though its
+// elimination order has only 63 (forward) and 58 (backward) levels.  So the
+// pivots are split (Program::tri_e):
+//  * the tail, the last min(64, nv) pivots, where the fill makes nearly every
+//    pivot wait on the one before it: one unknown per lane in a register, the
+//    pivot's value broadcast with v_readlane, one multiply-add per pivot;
+//  * the head before it, in batches of rows whose unknowns are ready: a lane
+//    takes up to 8 entries of one row, in the row's order, with the unknowns
+//    in LDS, so that a batch costs one LDS round trip and independent rows
+//    (the aerosol's size bins) run side by side.
+// Every row adds its entries in elimination order, one product at a time, so
+// the results are those of the pivot-by-pivot sweeps bit for bit.  All LU
+// values and positions are known before the sweep and are loaded ahead of it
+// (AH batches; the program NS ahead), so a batch waits on the unknowns only.
+// Cycles per solve: 1024 multi-phase cells 557k -> 84k, one cell 381k -> 54k;
+// 2000 CB05-scale gas cells 18.9k -> 10.9k, one cell 17.3k -> 10.0k.
+//
+// FMA (nv <= kTriInPlace): fused multiply-adds, the backward sweep on
+// D^-1 U x = D^-1 y (weights and right-hand side times the reciprocal
+// diagonal); otherwise separate products and a division by the diagonal.
+// ---------------------------------------------------------------------
+// AH: batches whose LU values are loaded ahead; NS: register sets of the
+// pipelines, the look-ahead of the program (AH + 1 < NS <= kTriPad)
 
-// Triangular solves with the solution vector in registers (nv <= 128):
-// lane t owns permuted rows t and t+64.  Pivot k's value is broadcast with
-// v_readlane (no LDS round trip, no barrier), so the dependency chain per
-// pivot is one readlane pair and one FMA.  The LU values each lane needs
-// come from the program's position table (the next block's words are
-// fetched while a block runs), so they are LDS loads issued ahead of the
-// chain; every block runs its 8 steps, pivots outside the sweep having
-// zero weights.  The sweeps are split at pivot 64 so each loop reads one
-// register, and the backward sweep solves D^-1 U x = D^-1 y, so no division
-// sits on the chain.
-__device__ __forceinline__ void cell_lu_solve_reg(const DevProgram& P, int lane, double* lu,
-                                                  double* b) {
-  lane = phase_lane(lane);
-  const int nv = P.nv;
-  const int r0 = lane, r1 = lane + kWave;
-  const bool has0 = r0 < nv, has1 = r1 < nv;
-  double x0 = has0 ? b[P.perm[r0]] : 0.0;
-  double x1 = has1 ? b[P.perm[r1]] : 0.0;
-  // the zero slot, after the LU values and the factorisation's sinks
-  if (lane == 0) lu[P.lu_nnz + kWave] = 0.0;
-  wsync();
-  constexpr int B = 8;
-  const int4* tb = P.ts_tbl + 2 * lane;
-  int blk = 0;
-  int4 t0 = tb[0], t1 = tb[1];
-  int4 u0 = tb[2 * kWave], u1 = tb[2 * kWave + 1];
-  const int kf = nv - 1;  // forward pivots 0 .. nv-2
-  const int split = kf < kWave ? kf : kWave;
-  // blocks are fetched two ahead (a block's work is shorter than the
-  // memory latency); the table has two blocks of padding past the last, so
-  // the look-ahead loads never leave it
-  for (int kb = 0; kb < split; kb += B) {
-    int4 n0 = tb[2 * kWave * (blk + 2)], n1 = tb[2 * kWave * (blk + 2) + 1];
-    tri_block<1, false>(kb, 0, t0, t1, lu, 1.0, 1.0, x0, x1);
-    t0 = u0; t1 = u1; u0 = n0; u1 = n1; ++blk;
-  }
-  for (int kb = split; kb < kf; kb += B) {
-    int4 n0 = tb[2 * kWave * (blk + 2)], n1 = tb[2 * kWave * (blk + 2) + 1];
-    tri_block<1, true>(kb, kWave, t0, t1, lu, 1.0, 1.0, x0, x1);
-    t0 = u0; t1 = u1; u0 = n0; u1 = n1; ++blk;
-  }
-  double d0 = has0 ? 1.0 / lu[P.diag_pos[r0]] : 0.0;
-  double d1 = has1 ? 1.0 / lu[P.diag_pos[r1]] : 0.0;
-  x0 *= d0;
-  x1 *= d1;
-  for (int kb = nv - 1; kb >= kWave; kb -= B) {
-    int4 n0 = tb[2 * kWave * (blk + 2)], n1 = tb[2 * kWave * (blk + 2) + 1];
-    tri_block<-1, true>(kb, kWave, t0, t1, lu, d0, d1, x0, x1);
-    t0 = u0; t1 = u1; u0 = n0; u1 = n1; ++blk;
-  }
-  for (int kb = (nv - 1 < kWave - 1 ? nv - 1 : kWave - 1); kb >= 0; kb -= B) {
-    int4 n0 = tb[2 * kWave * (blk + 2)], n1 = tb[2 * kWave * (blk + 2) + 1];
-    tri_block<-1, false>(kb, 0, t0, t1, lu, d0, d1, x0, x1);
-    t0 = u0; t1 = u1; u0 = n0; u1 = n1; ++blk;
-  }
-  wsync();
-  if (has0) b[P.perm[r0]] = x0;
-  if (has1) b[P.perm[r1]] = x1;
-  wsync();
-}
-
-// Column sweeps of the triangular solves (nv > 128): one stage per pivot k
-// -- its column range, the rows and LU positions of its first 64 entries
-// (one per lane), their LU values and, backward, the pivot's diagonal -- and
-// the range of the pivot the stage takes next (rn).
-struct ColStage {
-  int4 r, rn;
-  int row, pos;
-  double val, dg;
+struct TriBatch {
+  int4 a, b;
+  int2 r;
+  double w[8], dg;
 };
-// {column start, column end, diagonal position} of pivot k; zero outside
-// 0..nv-1
-template <bool FWD>
-__device__ __forceinline__ int4 col_range(const DevProgram& P, int k) {
-  if (k < 0 || k >= P.nv) return int4{0, 0, 0, 0};
-  int4 h = ld_uniform(P.lu_hdr, 2 * k);
-  int4 h2 = ld_uniform(P.lu_hdr, 2 * k + 1);
-  return FWD ? int4{h.x, h.y, h2.x, 0} : int4{h2.y, h2.z, h2.x, 0};
-}
-// the stage's next pivot: its range (fetched a step earlier, in rn), rows
-// and positions
-template <bool FWD>
-__device__ __forceinline__ void col_fetch_rows(const DevProgram& P, int lane, ColStage& S) {
-  const int* pos_a = FWD ? P.l_pos : P.u_pos;
-  const int* row_a = FWD ? P.l_row : P.u_row;
-  S.r = S.rn;
-  // (columns are padded to whole rows of 64 with row -1, position 0)
-  const int q = S.r.x + lane;
-  S.row = row_a[q];
-  S.pos = pos_a[q];
+__device__ __forceinline__ void tri_prog(const DevProgram& P, int lane, int n, TriBatch& S) {
+  S.a = P.tri_e[(size_t)(2 * n) * kWave + lane];
+  S.b = P.tri_e[(size_t)(2 * n + 1) * kWave + lane];
+  S.r = P.tri_r[(size_t)n * kWave + lane];
 }
 template <bool FWD>
-__device__ __forceinline__ void col_fetch_vals(const DevProgram& P, int k, const double* lu,
-                                               ColStage& S) {
-  S.val = lu[S.pos];  // (position 0 for padding: read, never used)
-  S.dg = (!FWD && k >= 0 && k < P.nv) ? lu[S.r.z] : 1.0;
+__device__ __forceinline__ void tri_vals(const double* lu, TriBatch& S) {
+  const int e[8] = {S.a.x, S.a.y, S.a.z, S.a.w, S.b.x, S.b.y, S.b.z, S.b.w};
+#pragma unroll
+  for (int u = 0; u < 8; ++u) S.w[u] = lu[e[u] & 0xFFFF];
+  S.dg = FWD ? 1.0 : lu[S.r.y];
 }
-// Pivot k of a sweep: x_k (divided by the diagonal, backward) updates the
-// rows of its column.
-template <bool FWD>
-__device__ __forceinline__ void col_pivot(const DevProgram& P, int lane, int k, const ColStage& S,
-                                          const double* lu, double* w) {
-  const int* pos_a = FWD ? P.l_pos : P.u_pos;
-  const int* row_a = FWD ? P.l_row : P.u_row;
-  double xk = w[k];
-  if (!FWD) {
-    xk = xk / S.dg;
-    wsync();
-    if (lane == 0) w[k] = xk;
+template <bool FWD, bool FMA>
+__device__ __forceinline__ void tri_run(const TriBatch& S, double* X) {
+  const int e[8] = {S.a.x, S.a.y, S.a.z, S.a.w, S.b.x, S.b.y, S.b.z, S.b.w};
+  const int row = S.r.x & 0xFFFF;
+  const bool idle = row == 0xFFFF;
+  double x[8];
+  double acc = X[idle ? 0 : row];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) x[u] = X[(unsigned)e[u] >> 16];
+  __builtin_amdgcn_sched_barrier(0);  // (all nine reads in flight)
+  double d = 1.0;
+  if (!FWD && FMA) {
+    d = 1.0 / S.dg;
+    acc = (S.r.x & (1 << 16)) ? acc * d : acc;
   }
-  if (S.row >= 0) w[S.row] = w[S.row] - S.val * xk;
-  for (int q = S.r.x + kWave + lane; q < S.r.y; q += kWave) {
-    int i = row_a[q];
-    w[i] = w[i] - lu[pos_a[q]] * xk;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    if (FMA) acc = fma(-(FWD ? S.w[u] : S.w[u] * d), x[u], acc);
+    else acc = acc - S.w[u] * x[u];
   }
+  if (!FWD && !FMA) acc = (S.r.x & (1 << 17)) ? acc / S.dg : acc;
+  if (!idle) X[row] = acc;
   wsync();
 }
-// One step of the pipelined sweep: the LU values of pivot k + 2 (stage C,
-// whose rows were fetched a step earlier), pivot k (stage A), the rows of
-// pivot k + 3 into A (its range fetched a step earlier) and the range of
-// pivot k + 4 into B, the stage of the next step.
-template <bool FWD>
-__device__ __forceinline__ void col_step(const DevProgram& P, int lane, int n, const double* lu,
-                                         double* w, ColStage& A, ColStage& B, ColStage& C) {
-  constexpr int st = FWD ? 1 : -1;
-  const int k = FWD ? n : P.nv - 1 - n;
-  col_fetch_vals<FWD>(P, k + 2 * st, lu, C);
-  if (n < P.nv) col_pivot<FWD>(P, lane, k, A, lu, w);
-  col_fetch_rows<FWD>(P, lane, A);
-  B.rn = col_range<FWD>(P, k + 4 * st);
-}
-// The sweep, unrolled by three over three stages so that each stage keeps
-// its registers: LU values are fetched two pivots ahead, rows three ahead
-// and ranges four ahead, with no copy between stages that would wait for
-// the newest load.
-template <bool FWD>
-__device__ __forceinline__ void col_sweep(const DevProgram& P, int lane, const double* lu,
-                                          double* w) {
-  constexpr int st = FWD ? 1 : -1;
-  const int k0 = FWD ? 0 : P.nv - 1;
-  ColStage S0, S1, S2;
-  S0.rn = col_range<FWD>(P, k0);
-  S1.rn = col_range<FWD>(P, k0 + st);
-  S2.rn = col_range<FWD>(P, k0 + 2 * st);
-  col_fetch_rows<FWD>(P, lane, S0);
-  col_fetch_rows<FWD>(P, lane, S1);
-  col_fetch_rows<FWD>(P, lane, S2);
-  S0.rn = col_range<FWD>(P, k0 + 3 * st);
-  col_fetch_vals<FWD>(P, k0, lu, S0);
-  col_fetch_vals<FWD>(P, k0 + st, lu, S1);
-  vm_drain();
-  for (int n = 0; n < P.nv; n += 3) {
-    col_step<FWD>(P, lane, n, lu, w, S0, S1, S2);
-    col_step<FWD>(P, lane, n + 1, lu, w, S1, S2, S0);
-    col_step<FWD>(P, lane, n + 2, lu, w, S2, S0, S1);
+// (both pipelines leave their loops in the middle: a step that was skipped
+// instead would leave the compiler unsure how many loads are in flight, and
+// it would wait for all of them)
+template <bool FWD, bool FMA, int AH, int NS>
+__device__ __forceinline__ void tri_head(const DevProgram& P, int lane, const double* lu,
+                                         double* X) {
+  const int n0 = FWD ? 0 : P.tri_nf + kTriPad, nb = FWD ? P.tri_nf : P.tri_nb;
+  if (nb == 0) return;
+  TriBatch S[NS];
+#pragma unroll
+  for (int u = 0; u < NS; ++u) tri_prog(P, lane, n0 + u, S[u]);
+#pragma unroll
+  for (int u = 0; u < AH; ++u) tri_vals<FWD>(lu, S[u]);
+  for (int n = 0;; n += NS) {
+#pragma unroll
+    for (int u = 0; u < NS; ++u) {
+      if (n + u >= nb) return;
+      tri_vals<FWD>(lu, S[(u + AH) % NS]);
+      __builtin_amdgcn_sched_barrier(0);  // keeps the loads ahead of the chain
+      tri_run<FWD, FMA>(S[u], X);
+      tri_prog(P, lane, n0 + n + u + NS, S[u]);
+    }
   }
 }
 
-// Solve (LU) x = b in place; b in dep order, w a scratch vector (nv).
-__device__ __forceinline__ void cell_lu_solve(const DevProgram& P, int lane, double* lu,
-                                              double* b, double* w) {
-  lane = phase_lane(lane);
-  if (P.ts_tbl) {
-    cell_lu_solve_reg(P, lane, lu, b);
+// The tail: x is the lane's unknown (row tri_s + lane); dg its diagonal and y
+// the diagonal's reciprocal.
+struct TailBlock {
+  int4 t;
+  double w[8];
+};
+__device__ __forceinline__ void tail_vals(const double* lu, TailBlock& S) {
+  const int t[4] = {S.t.x, S.t.y, S.t.z, S.t.w};
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+    S.w[u] = lu[u % 2 ? (unsigned)t[u / 2] >> 16 : t[u / 2] & 0xFFFF];
+}
+// x / dg for every lane: the quotient from the correctly rounded reciprocal y
+// with two residual corrections, which is the correctly rounded quotient (P.
+// Markstein, IBM J. Res. Dev. 34(1), 1990) in a third of the latency of the
+// division, which sits on the chain of every pivot.
+__device__ __forceinline__ double quot(double x, double dg, double y) {
+  double q = x * y;
+  q = fma(fma(-dg, q, x), y, q);
+  return fma(fma(-dg, q, x), y, q);
+}
+// Eight pivots of the tail, k0 onwards (or downwards).
+template <bool FWD, bool FMA>
+__device__ __forceinline__ void tail_run(int k0, const TailBlock& S, double dg, double y,
+                                         double& x) {
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const double v = !FWD && !FMA ? quot(x, dg, y) : x;
+    const double xk = readlane_d(v, (FWD ? k0 + u : k0 - u) & (kWave - 1));
+    if (FMA) x = fma(-(FWD ? S.w[u] : S.w[u] * y), xk, x);
+    else x = x - S.w[u] * xk;
+  }
+}
+// A full tail (64 pivots) is unrolled: a readlane of a fixed lane costs two
+// thirds of one whose lane is a register (28 against 43 cycles with the
+// multiply-add that waits on it).  Shorter tails loop over their blocks.
+template <bool FWD, bool FMA, int AH>
+__device__ __forceinline__ void tri_tail(const DevProgram& P, int lane, const double* lu,
+                                         double dg, double y, double& x) {
+  const int nb = FWD ? P.tt_nf : P.tt_nb;
+  const int4* tb = P.tt + (size_t)(FWD ? 0 : P.tt_nf + kTriPad) * kWave + lane;
+  if (P.tri_d == kWave) {
+    TailBlock S[8];
+#pragma unroll
+    for (int b = 0; b < 8; ++b) S[b].t = tb[b * kWave];
+#pragma unroll
+    for (int b = 0; b < AH; ++b) tail_vals(lu, S[b]);
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      if (b + AH < 8) tail_vals(lu, S[b + AH]);
+      __builtin_amdgcn_sched_barrier(0);
+      tail_run<FWD, FMA>(FWD ? 8 * b : kWave - 1 - 8 * b, S[b], dg, y, x);
+    }
     return;
   }
-  // Column sweeps with the solution in LDS (nv > 128).  Pivot k's L (or U)
-  // column: the first 64 entries go one per lane, the rest inline; the
-  // program and LU reads run ahead of the pivots (col_sweep), so a pivot
-  // waits on LDS only (the LU of multi-phase cells lives in global memory).
+  for (int n = 0; n < nb; ++n) {
+    TailBlock S;
+    S.t = tb[n * kWave];
+    tail_vals(lu, S);
+    tail_run<FWD, FMA>(FWD ? 8 * n : P.tri_d - 1 - 8 * n, S, dg, y, x);
+  }
+}
+
+// x in X (LDS): indexed by solver variable for FMA programs, else by pivot.
+template <bool FMA, int AH, int NS>
+__device__ __forceinline__ void tri_solve(const DevProgram& P, int lane, const double* lu,
+                                          double* X) {
+  vm_drain();
+  const bool on = lane < P.tri_d;
+  const int r = on ? P.tri_s + lane : 0;
+  const int ix = FMA ? P.perm[r] : r;
+  const double dg = on ? lu[P.tri_diag[r]] : 1.0;
+  tri_head<true, FMA, AH, NS>(P, lane, lu, X);
+  double x = on ? X[ix] : 0.0;
+  tri_tail<true, FMA, AH>(P, lane, lu, 1.0, 1.0, x);
+  const double y = 1.0 / dg;
+  if (FMA) x *= y;
+  tri_tail<false, FMA, AH>(P, lane, lu, dg, y, x);
+  if (!FMA) x = quot(x, dg, y);
+  if (on) X[ix] = x;
+  wsync();
+  tri_head<false, FMA, AH, NS>(P, lane, lu, X);
+}
+
+// The factors of multi-phase programs (in global memory) in the order the
+// solve reads them (Program::tri_src), the zero slot after them: a batch's
+// loads of one entry per lane are then consecutive addresses (a row-major
+// gather touches a cache line per lane, and the solves outnumber the
+// factorisations eight to one).
+__device__ __forceinline__ void cell_lu_order(const DevProgram& P, int lane, const double* lu,
+                                              double* out) {
+  lane = phase_lane(lane);
+  for (int p = lane; p < P.lu_nnz; p += kWave) out[p] = lu[P.tri_src[p]];
+  if (lane == 0) out[P.lu_nnz + kWave] = 0.0;
+  __threadfence_block();
+  wsync();
+}
+
+// Solve (LU) x = b in place; b in dep order, w a scratch vector (nv) in LDS,
+// used past kTriInPlace.  FAR: the factors are those of cell_lu_order, in
+// global memory, and are fetched two batches ahead instead of one.
+template <bool FAR>
+__device__ __forceinline__ void cell_lu_solve(const DevProgram& P, int lane, double* lu, double* b,
+                                              double* w) {
+  lane = phase_lane(lane);
+  if (!FAR) {
+    // the zero slot, after the LU values and the factorisation's sinks (the
+    // f gather's scratch shares it)
+    if (lane == 0) lu[P.lu_nnz + kWave] = 0.0;
+    wsync();
+  }
+  if (P.nv <= kTriInPlace) {
+    tri_solve<true, FAR ? 2 : 1, 4>(P, lane, lu, b);
+    return;
+  }
   for (int k = lane; k < P.nv; k += kWave) w[k] = b[P.perm[k]];
   wsync();
-  col_sweep<true>(P, lane, lu, w);
-  col_sweep<false>(P, lane, lu, w);
+  tri_solve<false, FAR ? 2 : 1, 4>(P, lane, lu, w);
   for (int k = lane; k < P.nv; k += kWave) b[P.perm[k]] = w[k];
   wsync();
 }

@@ -424,7 +424,8 @@ __global__ void __launch_bounds__(64) k_lu_factor(DevProgram P, int nc, const do
       continue;
     }
     double* out = LU + (size_t)c * P.lu_nnz;
-    for (int p = lane; p < P.lu_nnz; p += kWave) out[p] = s_lu[p];
+    // (multi-phase programs: in the order the solve reads them)
+    for (int p = lane; p < P.lu_nnz; p += kWave) out[p] = s_lu[P.mp ? P.tri_src[p] : p];
     wsync();
   }
 }
@@ -445,7 +446,7 @@ __global__ void __launch_bounds__(64) k_lu_solve(DevProgram P, int nc, const dou
     double* bc = b + (size_t)c * P.nv;
     for (int i = lane; i < P.nv; i += kWave) s_b[i] = bc[i];
     wsync();
-    cell_lu_solve(P, lane, s_lu, s_b, s_w);
+    cell_lu_solve<false>(P, lane, s_lu, s_b, s_w);
     for (int i = lane; i < P.nv; i += kWave) bc[i] = s != 1.0 ? s_b[i] * s : s_b[i];
     wsync();
   }

@@ -17,19 +17,19 @@ constexpr int kCellProf = 7;
 
 // Where a cell's working set lives in the persistent kernel.
 //  kPlaceLds     everything in LDS: state, rate data, per-term rates,
-//                Nordsieck history (6 vectors), 10 work vectors, the f
+//                Nordsieck history (6 vectors), 8 work vectors, the f
 //                gather's scratch, the LU factors, the J history and 24
 //                slots for the BDF coefficient arrays l, tq and tau (gas
 //                phase only: 4 cells per CU for the CB05-scale mechanism);
 //  kPlaceGlobal  the Nordsieck history and most work vectors in
-//                per-wavefront global scratch (gas phase: all but y, acor,
-//                tempv and ftemp; multi-phase: all but y, acor and w) and
+//                per-wavefront global scratch (gas phase: all but zn[0], zn[1],
+//                the error weights, y, acor, tempv and ftemp; multi-phase: all but y, acor and w) and
 //                the J history used in place in HBM, so that more cells fit
 //                a CU's LDS (6 for the CB05-scale mechanism; compiled for
 //                two wavefronts per SIMD).  Multi-phase programs always run
 //                so, with their LU factors, reaction Jacobian and
 //                per-instance Jacobian scalars in the scratch as well.
-//  kPlaceGlobalLu  the Nordsieck history, 7 of the 10 work vectors and the
+//  kPlaceGlobalLu  the Nordsieck history, 5 of the 8 work vectors and the
 //                LU factors (with the factorisation's sink slots and the
 //                solve's zero slot) in the scratch (gas phase: 12 cells per
 //                CU for the CB05-scale mechanism, compiled for two
@@ -42,30 +42,41 @@ __host__ __device__ inline int cell_placement(const DevProgram& P, int place) {
 __host__ __device__ inline bool cell_lu_global(const DevProgram& P, int place) {
   return P.mp || place == kPlaceGlobalLu;
 }
-// work vectors of a cell in LDS: all 16 with the history in LDS; for
-// gas-phase cells with the history in global memory y, acor and the Newton
-// iteration's tempv and ftemp; otherwise y, acor and the solve's w
+// vectors of a cell in LDS: all 14 with the history in LDS; for
+// gas-phase cells with the history in global memory zn[0], zn[1], the error
+// weights, y, acor, tempv and ftemp; otherwise y, acor and the solve's w
 __host__ __device__ inline int cell_lds_vectors(const DevProgram& P, int place) {
   const int pl = cell_placement(P, place);
-  return pl == kPlaceLds ? 16 : (!P.mp && pl == kPlaceGlobal) ? 4 : 3;
+  return pl == kPlaceLds ? 14 : (!P.mp && pl == kPlaceGlobal) ? 7 : 3;
+}
+// rate constants in LDS (gas-phase kPlaceGlobal reads them in global memory)
+__host__ __device__ inline size_t cell_lds_env(const DevProgram& P, int place) {
+  return !P.mp && cell_placement(P, place) == kPlaceGlobal ? 0 : (size_t)P.n_env;
+}
+// gas-phase kPlaceGlobal: the LU's LDS, where J(y) also stages the rate constants
+__host__ __device__ inline size_t cell_lu_lds(const DevProgram& P) {
+  return P.lu_nnz > P.n_env ? P.lu_nnz : P.n_env;
 }
 __host__ __device__ inline size_t cell_bdf_lds_doubles(const DevProgram& P, int place) {
   const bool g = cell_placement(P, place) != kPlaceLds;
-  return (size_t)P.ns + P.n_env + mp_lds_doubles(P) + 2 * (size_t)P.n_terms +
+  return (size_t)P.ns + cell_lds_env(P, place) + mp_lds_doubles(P) + 2 * (size_t)P.n_terms +
          (size_t)cell_lds_vectors(P, place) * P.nv + fb_sink_doubles(P) +
-         (cell_lu_global(P, place) ? 0 : (size_t)P.lu_nnz) +
+         (cell_lu_global(P, place) ? 0 : cell_placement(P, place) == kPlaceGlobal ? cell_lu_lds(P)
+                                                                       : (size_t)P.lu_nnz) +
          (g ? 0 : (size_t)P.nnz + 2 * (size_t)P.nv) + 24;
 }
 // Global scratch doubles per wavefront: the LU factors where they are global
-// (with the factorisation's 64 sink slots and the solve's zero slot), for
+// (with the factorisation's 64 sink slots and the solve's zero slot; for
+// multi-phase programs a second copy in the solve's order), for
 // multi-phase programs then the reaction Jacobian and the per-instance
 // Jacobian scalars, then (kPlaceGlobal, kPlaceGlobalLu) the Nordsieck
-// history and the work vectors not in LDS (13 vectors; 12 for gas-phase
+// history and the work vectors not in LDS (11 vectors; 7 for gas-phase
 // kPlaceGlobal).
 __host__ __device__ inline size_t cell_bdf_wave_scratch(const DevProgram& P, int place) {
-  if (P.mp) return (size_t)P.lu_nnz + kWave + 1 + P.rnnz + mp_jsc_doubles(P) + 13 * (size_t)P.nv;
-  if (place == kPlaceGlobalLu) return (size_t)P.lu_nnz + kWave + 1 + 13 * (size_t)P.nv;
-  return place == kPlaceGlobal ? 12 * (size_t)P.nv : 0;
+  if (P.mp)
+    return 2 * ((size_t)P.lu_nnz + kWave + 1) + P.rnnz + mp_jsc_doubles(P) + 11 * (size_t)P.nv;
+  if (place == kPlaceGlobalLu) return (size_t)P.lu_nnz + kWave + 1 + 11 * (size_t)P.nv;
+  return place == kPlaceGlobal ? 7 * (size_t)P.nv : 0;
 }
 
 // The no-allocation entry point's scratch (a file-scope device array of

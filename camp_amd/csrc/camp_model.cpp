@@ -431,6 +431,192 @@ static void build_mp_j_order(Program& P) {
   P.mj_rec.resize((size_t)8 * 64 * (rec_rows + 1), 0);  // the look-ahead's padding row
 }
 
+// One chain of the triangular solves' batches: a row's entries {LU position,
+// pivot} in elimination order.
+struct TriRow {
+  int row;
+  std::vector<std::pair<int, int>> ent;
+};
+
+// Packs the rows' chains into batches of 64 lanes (the layout of
+// Program::tri_e / tri_r) and returns their number.  done[k]: pivot k's
+// unknown is final before the first batch; a row that ends makes its own
+// final for the next batch.  Where more than 64 rows can go on, those with
+// the longest way to the end of the sweep go first.
+static int pack_tri_batches(const std::vector<TriRow>& rows, std::vector<char> done,
+                            const std::vector<int>& xi, const std::vector<int>& diag, int zero,
+                            bool empty_rows, std::vector<int>& te, std::vector<int>& tr) {
+  const int n = (int)rows.size();
+  std::vector<int> at(n, 0), left(n, 0);
+  // entries on the longest chain of rows that waits on each row
+  std::vector<long> weight(n, 0);
+  std::vector<int> row_of(done.size(), -1);
+  for (int i = 0; i < n; ++i) row_of[rows[i].row] = i;
+  for (int i = n - 1; i >= 0; --i)  // rows come in an order that respects the chains
+    for (int q = 0; q < (int)rows[i].ent.size(); ++q) {
+      int j = row_of[rows[i].ent[q].second];
+      if (j >= 0)
+        weight[j] = std::max(weight[j], weight[i] + 8 + (long)rows[i].ent.size() - q);
+    }
+  std::vector<char> open(n, 1);
+  int n_open = 0, batches = 0;
+  for (int i = 0; i < n; ++i) {
+    if (rows[i].ent.empty() && !empty_rows) {
+      done[rows[i].row] = 1;
+      open[i] = 0;
+    } else {
+      ++n_open;
+    }
+  }
+  while (n_open) {
+    std::vector<int> cand;
+    for (int i = 0; i < n; ++i) {
+      if (!open[i]) continue;
+      const auto& e = rows[i].ent;
+      int r = 0;
+      while (r < 8 && at[i] + r < (int)e.size() && done[e[at[i] + r].second]) ++r;
+      left[i] = r;
+      if (r > 0 || e.empty()) cand.push_back(i);
+    }
+    if (cand.size() > 64) {
+      std::stable_sort(cand.begin(), cand.end(), [&](int a, int b) {
+        return weight[a] + (long)rows[a].ent.size() - at[a] >
+               weight[b] + (long)rows[b].ent.size() - at[b];
+      });
+      cand.resize(64);
+    }
+    const size_t e0 = te.size(), r0 = tr.size();
+    te.resize(e0 + 2 * 64 * 4, zero);
+    tr.resize(r0 + 2 * 64, 0);
+    for (int l = 0; l < 64; ++l) tr[r0 + 2 * l] = 0xFFFF;
+    std::vector<int> ended;
+    for (int l = 0; l < (int)cand.size(); ++l) {
+      const int i = cand[l];
+      const auto& e = rows[i].ent;
+      const int x = xi[rows[i].row];
+      const bool first = at[i] == 0, last = at[i] + left[i] == (int)e.size();
+      for (int u = 0; u < 8; ++u) {
+        int w = zero | (x << 16);
+        if (u < left[i]) w = e[at[i] + u].first | (xi[e[at[i] + u].second] << 16);
+        te[e0 + ((size_t)(u / 4) * 64 + l) * 4 + u % 4] = w;
+      }
+      at[i] += left[i];
+      tr[r0 + 2 * l] = x | (first << 16) | (last << 17);
+      tr[r0 + 2 * l + 1] = diag[rows[i].row];
+      if (last) ended.push_back(i);
+    }
+    for (int i : ended) {
+      open[i] = 0;
+      --n_open;
+      done[rows[i].row] = 1;
+    }
+    ++batches;
+  }
+  return batches;
+}
+
+// The triangular solves' program (Program::tri_e and following) of the
+// filled pattern F with value positions pos (row-major, nv x nv, pivot
+// order).
+static void build_tri_program(Program& P, const std::vector<char>& F,
+                              const std::vector<int>& pos) {
+  const int nv = P.nv, zero = P.lu_nnz + 64;
+  const int d = P.tri_d = std::min(64, nv), s = P.tri_s = nv - d;
+  std::vector<int> xi(nv);
+  for (int k = 0; k < nv; ++k) xi[k] = nv <= kTriInPlace ? P.perm[k] : k;
+  auto pad = [&](std::vector<int>& e, std::vector<int>& r) {
+    e.resize(e.size() + (size_t)kTriPad * 2 * 64 * 4, zero);
+    for (int q = 0; q < kTriPad * 64; ++q) {
+      r.push_back(0xFFFF);
+      r.push_back(0);
+    }
+  };
+  P.tri_e.clear();
+  P.tri_r.clear();
+  std::vector<TriRow> rows;
+  for (int i = 0; i < nv; ++i) {
+    TriRow t{i, {}};
+    for (int k = 0; k < std::min(i, s); ++k)
+      if (F[(size_t)i * nv + k]) t.ent.push_back({pos[(size_t)i * nv + k], k});
+    rows.push_back(t);
+  }
+  P.tri_nf = pack_tri_batches(rows, std::vector<char>(nv, 0), xi, P.diag_pos, zero, false,
+                              P.tri_e, P.tri_r);
+  pad(P.tri_e, P.tri_r);
+  rows.clear();
+  std::vector<char> done(nv, 0);
+  for (int k = s; k < nv; ++k) done[k] = 1;
+  for (int i = s - 1; i >= 0; --i) {
+    TriRow t{i, {}};
+    for (int k = nv - 1; k > i; --k)
+      if (F[(size_t)i * nv + k]) t.ent.push_back({pos[(size_t)i * nv + k], k});
+    rows.push_back(t);
+  }
+  P.tri_nb = pack_tri_batches(rows, done, xi, P.diag_pos, zero, true, P.tri_e, P.tri_r);
+  pad(P.tri_e, P.tri_r);
+  // the tail: blocks of 8 pivots in the order the sweeps visit them
+  P.tt.clear();
+  auto block = [&](int kb, int dir) {
+    for (int l = 0; l < 64; ++l)
+      for (int u = 0; u < 8; u += 2) {
+        int w = 0;
+        for (int h = 0; h < 2; ++h) {
+          const int k = kb + dir * (u + h), r = l;
+          int p = zero;
+          if (k >= 0 && k < d && r < d && (dir > 0 ? r > k : r < k) &&
+              F[(size_t)(s + r) * nv + s + k])
+            p = pos[(size_t)(s + r) * nv + s + k];
+          w |= p << (16 * h);
+        }
+        P.tt.push_back(w);
+      }
+  };
+  P.tri_diag = P.diag_pos;
+  P.tri_src.clear();
+  P.tt_nf = P.tt_nb = 0;
+  for (int kb = 0; kb < d - 1; kb += 8, ++P.tt_nf) block(kb, 1);
+  for (int q = 0; q < kTriPad; ++q) block(d, 1);
+  for (int kb = d - 1; kb >= 0; kb -= 8, ++P.tt_nb) block(kb, -1);
+  for (int q = 0; q < kTriPad; ++q) block(-1, -1);
+  if (!P.mp) return;
+  // renumber the LU values in the order the batches and blocks read them,
+  // lane after lane for each entry, the diagonals first
+  std::vector<int> to(zero + 1, -1);
+  to[zero] = zero;
+  auto take = [&](int p) {
+    if (to[p] < 0) {
+      to[p] = (int)P.tri_src.size();
+      P.tri_src.push_back(p);
+    }
+    return to[p];
+  };
+  for (int k = 0; k < nv; ++k) P.tri_diag[k] = take(P.diag_pos[k]);
+  auto head = [&](int b0, int nb) {
+    for (int b = b0; b < b0 + nb; ++b)
+      for (int u = 0; u < 8; ++u)
+        for (int l = 0; l < 64; ++l) {
+          int& w = P.tri_e[(((size_t)2 * b + u / 4) * 64 + l) * 4 + u % 4];
+          w = take(w & 0xFFFF) | (int)((unsigned)w & 0xFFFF0000u);
+        }
+  };
+  auto tail = [&](int b0, int nb) {
+    for (int b = b0; b < b0 + nb; ++b)
+      for (int u = 0; u < 8; ++u)
+        for (int l = 0; l < 64; ++l) {
+          int& w = P.tt[((size_t)b * 64 + l) * 4 + u / 2];
+          const int sh = 16 * (u % 2);
+          const int p = take((int)(((unsigned)w >> sh) & 0xFFFF));
+          w = (int)(((unsigned)w & ~(0xFFFFu << sh)) | ((unsigned)p << sh));
+        }
+  };
+  head(0, P.tri_nf);
+  tail(0, P.tt_nf);
+  tail(P.tt_nf + kTriPad, P.tt_nb);
+  head(P.tri_nf + kTriPad, P.tri_nb);
+  for (size_t q = 0; q < P.tri_r.size(); q += 2)
+    if ((P.tri_r[q] & 0xFFFF) != 0xFFFF) P.tri_r[q + 1] = to[P.tri_r[q + 1]];
+}
+
 std::string Model::initialize() {
   if (n_added != n_rxn) return "not all reactions were added before solver_initialize";
   // --- reaction Jacobian pattern: diagonal + per-type used elements -------
@@ -1100,66 +1286,8 @@ std::string Model::initialize() {
     P.u_ptr.push_back((int)P.u_pos.size());
     P.up_ptr.push_back((int)P.up_dst.size());
   }
-  if (P.l_pos.empty()) { P.l_pos.push_back(0); P.l_row.push_back(0); }
-  if (P.u_pos.empty()) { P.u_pos.push_back(0); P.u_row.push_back(0); }
-  if (P.up_dst.empty()) { P.up_dst.push_back(0); P.up_l.push_back(0); P.up_u.push_back(0); }
-  // the column solve's padded columns: {start, start + entries} per pivot
-  P.cs_lpos.clear(); P.cs_lrow.clear(); P.cs_upos.clear(); P.cs_urow.clear();
-  std::vector<int> cl(2 * nv), cu(2 * nv);
-  auto pad_cols = [&](const std::vector<int>& ptr, const std::vector<int>& vpos,
-                      const std::vector<int>& vrow, std::vector<int>& opos, std::vector<int>& orow,
-                      std::vector<int>& rng) {
-    for (int k = 0; k < nv; ++k) {
-      int n = ptr[k + 1] - ptr[k], start = (int)opos.size();
-      rng[2 * k] = start;
-      rng[2 * k + 1] = start + n;
-      for (int q = 0; q < std::max(1, (n + 63) / 64) * 64; ++q) {
-        opos.push_back(q < n ? vpos[ptr[k] + q] : 0);
-        orow.push_back(q < n ? vrow[ptr[k] + q] : -1);
-      }
-    }
-    // entries read for the pivots past the end (header zero): the first row
-    if (opos.size() < 64) { opos.resize(64, 0); orow.resize(64, -1); }
-  };
-  pad_cols(P.l_ptr, P.l_pos, P.l_row, P.cs_lpos, P.cs_lrow, cl);
-  pad_cols(P.u_ptr, P.u_pos, P.u_row, P.cs_upos, P.cs_urow, cu);
-  P.lu_hdr.assign((size_t)8 * (nv + 2), 0);
-  for (int k = 0; k < nv; ++k) {
-    int* h = &P.lu_hdr[(size_t)8 * k];
-    h[0] = cl[2 * k]; h[1] = cl[2 * k + 1]; h[2] = P.up_ptr[k]; h[3] = P.up_ptr[k + 1];
-    h[4] = P.diag_pos[k]; h[5] = cu[2 * k]; h[6] = cu[2 * k + 1];
-  }
-  // The register triangular solve's program (nv <= 128): per block of 8
-  // pivots, in the order the device sweeps visit them, and per lane t, the
-  // LU positions of the entries (row t, pivot) and (row t + 64, pivot) as
-  // pos0 | pos1 << 16 -- the zero slot lu_nnz + 64 where the row has no
-  // entry or the pivot is outside the sweep -- two int4 per lane and block.
-  P.ts_tbl.clear();
-  P.ts_fwd_blocks = P.ts_bwd_blocks = 0;
-  if (nv <= 128) {
-    if (P.lu_nnz + 65 > 65535) return "LU fill too large for the register solve";
-    const int W = 64, zero = P.lu_nnz + 64;
-    auto block = [&](int kb, int dir, int lo, int hi) {  // pivots kb + dir*u in [lo, hi)
-      for (int l = 0; l < W; ++l)
-        for (int u = 0; u < 8; ++u) {
-          int k = kb + dir * u, w = 0;
-          for (int h = 0; h < 2; ++h) {
-            int r = l + h * W, p = zero;
-            bool in_sweep = k >= lo && k < hi && r < nv;
-            if (in_sweep && (dir > 0 ? r > k : r < k) && F[(size_t)r * nv + k])
-              p = pos[(size_t)r * nv + k];
-            w |= p << (16 * h);
-          }
-          P.ts_tbl.push_back(w);
-        }
-    };
-    const int kf = nv - 1, split = std::min(kf, W);
-    for (int kb = 0; kb < split; kb += 8, ++P.ts_fwd_blocks) block(kb, 1, 0, split);
-    for (int kb = split; kb < kf; kb += 8, ++P.ts_fwd_blocks) block(kb, 1, split, kf);
-    for (int kb = nv - 1; kb >= W; kb -= 8, ++P.ts_bwd_blocks) block(kb, -1, W, nv);
-    for (int kb = std::min(nv - 1, W - 1); kb >= 0; kb -= 8, ++P.ts_bwd_blocks) block(kb, -1, 0, W);
-    P.ts_tbl.insert(P.ts_tbl.end(), (size_t)2 * 8 * W, zero | (zero << 16));  // look-ahead padding
-  }
+  if (P.lu_nnz + 64 > 65535) return "LU fill exceeds 65471 entries per cell";
+  build_tri_program(P, F, pos);
   // The factorisation's program: per pivot, the L positions to scale and the
   // update records {dst, l, u}, each padded to whole rows of 64 (at least
   // one row of L positions) with entries that write lane l's sink slot
@@ -1169,7 +1297,6 @@ std::string Model::initialize() {
   // batch with no per-row selection; lf_hdr[k] = {first L position, first
   // update record, L rows | update rows << 16, diagonal position} (two empty
   // pivots past the end).
-  if (P.lu_nnz + 64 > 65535) return "LU fill exceeds 65471 entries per cell";
   P.lf_pos.clear();
   P.up_rec.clear();
   P.lf_hdr.assign((size_t)4 * (nv + 2), 0);

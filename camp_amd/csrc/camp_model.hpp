@@ -22,6 +22,12 @@ namespace camp {
 // together: a pivot's first kLuRowBatch rows, then its further rows in
 // batches of kLuRowBatch (the program pads those to whole batches).
 constexpr int kLuRowBatch = 5;
+// The triangular solves: programs of up to kTriInPlace solver variables solve
+// in the right-hand side with fused multiply-adds and reciprocal diagonals,
+// larger ones in a scratch vector with separate products and divisions; the
+// programs' empty batches past the end, which the look-ahead loads.
+constexpr int kTriInPlace = 128;
+constexpr int kTriPad = 4;
 // Row-view entries of the f estimate's ELL a lane reads per batch.
 constexpr int kEstBatch = 8;
 
@@ -115,23 +121,35 @@ struct Program {
   std::vector<int> l_ptr, l_pos, l_row;             // per pivot k: L(:,k) below k
   std::vector<int> u_ptr, u_pos, u_row;             // per pivot k: U(:,k) above k
   std::vector<int> up_ptr;                          // per pivot k: update range
-  // the column solve's copies of L(:,k) and U(:,k): each column padded to
-  // whole rows of 64 entries with (row -1, position 0), so that a column's
-  // first 64 entries load with no bounds check; lu_hdr's ranges index them
-  std::vector<int> cs_lpos, cs_lrow, cs_upos, cs_urow;
-  std::vector<int> lu_hdr;  // per pivot k: {l_ptr[k], l_ptr[k+1], up_ptr[k], up_ptr[k+1],
-                            //  diag_pos[k], u_ptr[k], u_ptr[k+1], 0} (two 16-byte
-                            //  loads), then 2 empty pivots
   std::vector<uint16_t> up_dst, up_l, up_u;         // LU[dst] -= LU[l] * LU[u]
   // the factorisation's program (built in Model::initialize): per pivot L
   // positions (lf_pos) and update records dst | l << 16 | u << 32 (up_rec),
   // each padded to rows of 64 with writes to the lanes' sink slots past the
   // LU values, and lf_hdr = 4 ints per pivot
   std::vector<int> lf_pos, lf_hdr;
-  // the register triangular solve's program (built in Model::initialize):
-  // per block of 8 pivots and lane, 8 words pos(row t) | pos(row t+64) << 16
-  std::vector<int> ts_tbl;
-  int ts_fwd_blocks = 0, ts_bwd_blocks = 0;
+  // The triangular solves' program (built by build_tri_program).  The last
+  // tri_d = min(64, nv) pivots are the tail, whose unknowns sit one per lane;
+  // the tri_s = nv - tri_d pivots before it are the head.
+  //  * Head entries of both sweeps (and the tail rows' head entries of the
+  //    forward sweep) in batches: a lane of a batch adds up to 8 consecutive
+  //    entries of one row, in the row's elimination order, of unknowns that
+  //    are final before the batch.  tri_e: per batch, quad (2) and lane, four
+  //    words LU position | index of the unknown << 16; tri_r: per batch and
+  //    lane {row index | first batch of the row << 16 | last << 17,
+  //    diagonal position}, row index 0xFFFF where the lane is idle.  tri_nf forward batches, kTriPad empty ones, tri_nb
+  //    backward batches, kTriPad empty ones.
+  //  * tt: the tail's LU positions, per block of 8 pivots and lane eight
+  //    16-bit positions (the zero slot lu_nnz + 64 where the lane's row has
+  //    no entry), tt_nf forward blocks, kTriPad empty ones, tt_nb backward
+  //    blocks, kTriPad empty ones.
+  // Unknowns are indexed by solver variable where the solve works in the
+  // right-hand side itself (nv <= kTriInPlace), else by pivot.  The LU
+  // values are read at the factorisation's positions; by multi-phase programs
+  // from a copy in the solve's own order, position p of it being tri_src[p] of
+  // the factorisation (tri_diag: the diagonals' positions as the solve reads
+  // them).
+  int tri_s = 0, tri_d = 0, tri_nf = 0, tri_nb = 0, tt_nf = 0, tt_nb = 0;
+  std::vector<int> tri_e, tri_r, tt, tri_diag, tri_src;
   std::vector<uint64_t> up_rec;
   long n_updates() const { return (long)up_dst.size(); }
 

@@ -80,12 +80,17 @@ void Solver::setup_device() {
   P.m_to_lu = dev_upload(G.m_to_lu, owned);
   P.diag_pos = dev_upload(G.diag_pos, owned);
   P.e_diag = dev_upload(G.e_diag, owned);
-  // (the column solve's padded copies; the host keeps the plain columns)
-  P.l_pos = dev_upload(G.cs_lpos, owned);
-  P.l_row = dev_upload(G.cs_lrow, owned);
-  P.u_pos = dev_upload(G.cs_upos, owned);
-  P.u_row = dev_upload(G.cs_urow, owned);
-  P.lu_hdr = reinterpret_cast<const int4*>(dev_upload(G.lu_hdr, owned));
+  P.tri_s = G.tri_s;
+  P.tri_d = G.tri_d;
+  P.tri_nf = G.tri_nf;
+  P.tri_nb = G.tri_nb;
+  P.tt_nf = G.tt_nf;
+  P.tt_nb = G.tt_nb;
+  P.tri_e = reinterpret_cast<const int4*>(dev_upload(G.tri_e, owned));
+  P.tri_r = reinterpret_cast<const int2*>(dev_upload(G.tri_r, owned));
+  P.tt = reinterpret_cast<const int4*>(dev_upload(G.tt, owned));
+  P.tri_diag = dev_upload(G.tri_diag, owned);
+  P.tri_src = dev_upload(G.tri_src, owned);
   P.up_rec = dev_upload(G.up_rec, owned);
   P.lf_pos = dev_upload(G.lf_pos, owned);
   P.lf_hdr = reinterpret_cast<const int4*>(dev_upload(G.lf_hdr, owned));
@@ -100,8 +105,6 @@ void Solver::setup_device() {
   P.je_a = reinterpret_cast<const int4*>(dev_upload(G.je_a, owned));
   P.je_b = dev_upload(G.je_b, owned);
   P.je_c = dev_upload(G.je_c, owned);
-  P.ts_tbl = G.ts_tbl.empty() ? nullptr
-                              : reinterpret_cast<const int4*>(dev_upload(G.ts_tbl, owned));
   std::vector<int> rx_type(m.n_rxn), rx_fidx(m.n_rxn), rx_eidx(m.n_rxn), rx_nreact(m.n_rxn);
   for (int r = 0; r < m.n_rxn; ++r) {
     int* id = m.rint(r);
