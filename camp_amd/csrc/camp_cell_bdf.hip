@@ -1190,10 +1190,9 @@ __global__ void __launch_bounds__(256)
           // the post-solve sub_model_calculate (camp_solver.c:685-687) on the
           // final state; the sub models' outputs go back to the state array
           wsync();
-          for (int z = lane; z < P.n_zi; z += kWave) {
-            mp_zsr_water(P, z, cv.mpl.sub_env, cv.s_state);
+          mp_zsr(P, lane, cv.mpl.sub_env, cv.s_state, cv.mpl.slot);
+          for (int z = lane; z < P.n_zi; z += kWave)
             state_c[P.zi_water[z]] = cv.s_state[P.zi_water[z]];
-          }
         }
       }
       if (!GH) {

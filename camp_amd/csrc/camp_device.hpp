@@ -64,8 +64,9 @@ struct DevProgram {
   // camp_model.hpp for their meaning
   int mp, rnnz, pnnz, n_pi, n_zi, n_sp, n_aq, n_slots, n_sub_env;
   double min_mass_hi, min_mass_lo, min_moles_hi, min_moles_lo, min_volume;
-  const int *pi_start, *pi_model, *pm_ptr, *pm_counted;
-  const double *pi_dp, *pm_mw, *pm_dens;
+  int n_it, n_zp;
+  const int *pit_ptr, *pit_state, *pit_pi, *zp_zi;
+  const double *pi_dp, *pit_mw, *pit_dens;
   const int *zi_water, *zi_gw, *zi_sub, *zi_pair_ptr, *zp_cat, *zp_an, *zp_ncat, *zp_nan, *zp_ny,
       *zp_jgw, *zp_jcat, *zp_jan;
   const double *zp_catmw, *zp_anmw, *zp_lowrh, *zp_y;

@@ -1366,6 +1366,18 @@ std::string Model::compile_multiphase(std::vector<std::vector<int>>& f_slots) {
       }
     }
   }
+  P.pit_ptr.assign(1, 0);
+  for (size_t i = 0; i < P.pi_start.size(); ++i) {
+    const int pm = P.pi_model[i];
+    for (int q = P.pm_ptr[pm]; q < P.pm_ptr[pm + 1]; ++q) {
+      if (!P.pm_counted[q]) continue;
+      P.pit_state.push_back(P.pi_start[i] + q - P.pm_ptr[pm]);
+      P.pit_pi.push_back((int)i);
+      P.pit_mw.push_back(P.pm_mw[q]);
+      P.pit_dens.push_back(P.pm_dens[q]);
+    }
+    P.pit_ptr.push_back((int)P.pit_state.size());
+  }
   // ZSR items
   P.zi_pair_ptr.assign(1, 0);
   for (int k = 0; k < n_sub; ++k) {
@@ -1376,6 +1388,7 @@ std::string Model::compile_multiphase(std::vector<std::vector<int>>& f_slots) {
       P.zi_sub.push_back(k);
       for (int x = 0; x < z.npair(); ++x) {
         if (z.ny(x) > 8) return "ZSR molality polynomials of more than 8 terms";
+        P.zp_zi.push_back((int)P.zi_water.size() - 1);
         P.zp_cat.push_back(z.phase(p) + z.cation(x));
         P.zp_an.push_back(z.phase(p) + z.anion(x));
         P.zp_ncat.push_back(z.n_cation(x));
@@ -1441,8 +1454,8 @@ std::string Model::compile_multiphase(std::vector<std::vector<int>>& f_slots) {
         for (int q = P.pm_ptr[pm]; q < P.pm_ptr[pm + 1]; ++q) {
           if (!P.pm_counted[q]) continue;
           if (k < v.njac(i)) {
-            if (v.phase_jac(i, 0, k) > 0) addj(v.phase_jac(i, 0, k), kJsSimpolGP, inst, q, 0, 0.0);
-            if (v.phase_jac(i, 1, k) > 0) addj(v.phase_jac(i, 1, k), kJsSimpolAP, inst, q, 0, 0.0);
+            if (v.phase_jac(i, 0, k) > 0) addj(v.phase_jac(i, 0, k), kJsSimpolGP, inst, q, P.pit_ptr[pi] + k, 0.0);
+            if (v.phase_jac(i, 1, k) > 0) addj(v.phase_jac(i, 1, k), kJsSimpolAP, inst, q, P.pit_ptr[pi] + k, 0.0);
           }
           ++k;
         }

@@ -189,8 +189,12 @@ struct Program {
   std::vector<double> pi_dp;
   std::vector<int> pm_ptr, pm_counted;
   std::vector<double> pm_mw, pm_dens;
+  // the counted species of every phase instance ("items", instance i's at
+  // [pit_ptr[i], pit_ptr[i + 1])): state id, instance, MW, density
+  std::vector<int> pit_ptr, pit_state, pit_pi;
+  std::vector<double> pit_mw, pit_dens;
   // ZSR items (one per sub model and phase) and their JACOBSON ion pairs
-  std::vector<int> zi_water, zi_gw, zi_sub, zi_pair_ptr;
+  std::vector<int> zi_water, zi_gw, zi_sub, zi_pair_ptr, zp_zi;
   std::vector<int> zp_cat, zp_an, zp_ncat, zp_nan, zp_ny, zp_jgw, zp_jcat, zp_jan;
   std::vector<double> zp_catmw, zp_anmw, zp_lowrh, zp_y;   // zp_y: 8 per pair
   int n_sub_env = 0;
@@ -202,6 +206,7 @@ struct Program {
   std::vector<double> aq_small_water;
   int n_slots = 0;
   // special Jacobian records per reaction element: {kind, instance, p1, p2}, c
+  // (p2 of a phase element: its item)
   std::vector<int> js_ptr, js_a;
   std::vector<double> js_c;
   // solver element e = sum over [jm_ptr[e], jm_ptr[e+1]) of J_rxn[jm_rxn] * J_params[jm_param]

@@ -21,7 +21,7 @@
 namespace camp {
 
 constexpr int kAeroSlots = 8;           // per phase instance in LDS
-constexpr int kSpScalars = 13;          // per SIMPOL instance in LDS
+constexpr int kSpScalars = 17;          // per SIMPOL instance
 constexpr int kAqScalars = 6;           // per aqueous-equilibrium instance
 
 // --- transition-regime condensation (util.h:19-68), all double -------------
@@ -42,79 +42,109 @@ __host__ __device__ __forceinline__ double mp_dcond_rate_dr(double D, double mfp
 // --- aerosol state of one cell (aero_rep_update_state) ---------------------
 // s_aero[i*8]: mass, average MW, number concentration (cached, as the
 // representation caches them), then the mass and mole sums (dd) of the
-// current state, which the MW partial derivatives use
-__host__ __device__ __forceinline__ void mp_phase_sums(const DevProgram& P, int i, const double* s_state,
-                                              dd* mass_out, dd* moles_out, double* vol_out) {
-  int st0 = P.pi_start[i], pm = P.pi_model[i];
-  dd mass = {P.min_mass_hi, P.min_mass_lo};
-  dd moles = {P.min_moles_hi, P.min_moles_lo};
-  double vol = P.min_volume;
-  for (int q = P.pm_ptr[pm], k = 0; q < P.pm_ptr[pm + 1]; ++q, ++k) {
-    if (!P.pm_counted[q]) continue;
-    double x = s_state[st0 + k];
-    mass = dd_add(mass, dd_from(x));
-    moles = dd_add(moles, dd_div_d(dd_from(x), P.pm_mw[q]));
-    vol += x / P.pm_dens[q];
+// current state, which the MW partial derivatives use, and its volume
+// The sums run over the counted species of each phase instance ("items",
+// Program::pit_ptr).  A lane per phase, as the sums' order suggests, leaves 8
+// of 64 lanes with 29 double-double divisions one after another; the quotients
+// x / MW and x / density are formed by a lane per item into scratch and only
+// the additions stay in order, the three sums of a phase on three lanes.
+
+// mass, moles (dd) and volume of every phase into s_aero[3..7]
+__device__ __forceinline__ void mp_phase_sums(const DevProgram& P, int lane, const double* s_state,
+                                              double* s_aero, double* scratch) {
+  for (int it = lane; it < P.n_it; it += kWave) {
+    double x = s_state[P.pit_state[it]];
+    dd m = dd_div_d(dd_from(x), P.pit_mw[it]);
+    double* q = scratch + 4 * it;
+    q[0] = x;
+    q[1] = m.hi;
+    q[2] = m.lo;
+    q[3] = x / P.pit_dens[it];
   }
-  *mass_out = mass;
-  *moles_out = moles;
-  *vol_out = vol;
+  wsync();
+  for (int t = lane; t < 3 * P.n_pi; t += kWave) {
+    const int i = t / 3, w = t - 3 * i;
+    const int k0 = P.pit_ptr[i], k1 = P.pit_ptr[i + 1];
+    const double* q = scratch + (w == 0 ? 0 : w == 1 ? 1 : 3);
+    dd s = w == 0 ? dd{P.min_mass_hi, P.min_mass_lo}
+                  : w == 1 ? dd{P.min_moles_hi, P.min_moles_lo} : dd{P.min_volume, 0.0};
+    for (int k = k0; k < k1; ++k) {
+      dd v = {q[4 * k], w == 1 ? q[4 * k + 1] : 0.0};
+      const double plain = s.hi + v.hi;
+      s = dd_add(s, v);
+      if (w == 2) s = dd{plain, 0.0};
+    }
+    double* a = s_aero + kAeroSlots * i + 3 + 2 * w;
+    a[0] = s.hi;
+    if (w < 2) a[1] = s.lo;
+  }
+  wsync();
 }
 
-__host__ __device__ __forceinline__ void mp_phase_update(const DevProgram& P, int i, const double* s_state,
-                                                double* a) {
-  dd mass, moles;
-  double vol;
-  mp_phase_sums(P, i, s_state, &mass, &moles, &vol);
-  double mass_d = dd_round(mass);
-  a[0] = mass_d;
-  a[1] = dd_round(dd_div(dd_from(mass_d), moles));
-  double r = P.pi_dp[i] / 2.0;
-  a[2] = vol * 3.0 / (4.0 * kPi) / cr_powi(r, 3);
+// --- ZSR water of every (sub model, phase) item (:216-301) -----------------
+// A lane per ion for the exponentials, a lane per ion pair for its molality and
+// contribution, a lane per item to add the pairs in order; scratch holds 6
+// doubles per pair (cation, anion, their exponentials, the contribution).
+__device__ __forceinline__ void mp_zsr_ions(const DevProgram& P, int lane, const double* s_state,
+                                            double* scratch) {
+  for (int t = lane; t < 2 * P.n_zp; t += kWave) {
+    const bool an = t >= P.n_zp;
+    const int x = an ? t - P.n_zp : t;
+    // ion concentrations are double expressions (state / int / MW / 1000)
+    double c = s_state[an ? P.zp_an[x] : P.zp_cat[x]] / (double)(an ? P.zp_nan[x] : P.zp_ncat[x]) /
+               (an ? P.zp_anmw[x] : P.zp_catmw[x]) / 1000.0;
+    scratch[6 * x + (an ? 1 : 0)] = c;
+    scratch[6 * x + (an ? 3 : 2)] = cr_exp(-100.0 * c);
+  }
+  wsync();
 }
 
-// sums of the state after the sub models ran (the getters' partials see it)
-__host__ __device__ __forceinline__ void mp_phase_partial_sums(const DevProgram& P, int i,
-                                                      const double* s_state, double* a) {
-  dd mass, moles;
-  double vol;
-  mp_phase_sums(P, i, s_state, &mass, &moles, &vol);
-  a[3] = mass.hi;
-  a[4] = mass.lo;
-  a[5] = moles.hi;
-  a[6] = moles.lo;
-}
-
-// --- ZSR water of one (sub model, phase) item (:216-301) -------------------
-__host__ __device__ __forceinline__ void mp_zsr_water(const DevProgram& P, int z, const double* s_sub_env,
-                                             double* s_state) {
-  // a_w = PPM_TO_RH * state: a double product (both operands double)
-  dd aw = dd_from(s_sub_env[P.zi_sub[z]] * s_state[P.zi_gw[z]]);
-  double water = 1.0e-30;
-  for (int x = P.zi_pair_ptr[z]; x < P.zi_pair_ptr[z + 1]; ++x) {
+__device__ __forceinline__ void mp_zsr(const DevProgram& P, int lane, const double* s_sub_env,
+                                       double* s_state, double* scratch) {
+  mp_zsr_ions(P, lane, s_state, scratch);
+  for (int x = lane; x < P.n_zp; x += kWave) {
+    const int z = P.zp_zi[x];
+    // a_w = PPM_TO_RH * state: a double product (both operands double)
+    dd aw = dd_from(s_sub_env[P.zi_sub[z]] * s_state[P.zi_gw[z]]);
     double low = P.zp_lowrh[x];
     dd jaw = dd_gt(aw, low) ? aw : dd_from(low);
     double jaw_d = dd_round(jaw);
+    // the powers of jaw (cr_powi) as one chain: each continues the last
     dd mol = dd_from(0.0);
-    for (int k = 0; k < P.zp_ny[x]; ++k) mol = dd_add(mol, dd_from(P.zp_y[8 * x + k] * cr_powi(jaw_d, k)));
+    dd pw = dd_from(fabs(jaw_d));
+    for (int k = 0; k < P.zp_ny[x]; ++k) {
+      double pk = k == 0 ? 1.0 : dd_round(pw);
+      if (jaw_d < 0.0 && (k & 1)) pk = -pk;
+      if (k > 0) pw = dd_mul_d(pw, fabs(jaw_d));
+      mol = dd_add(mol, dd_from(P.zp_y[8 * x + k] * pk));
+    }
     mol = dd_mul(mol, mol);
-    // ion concentrations are double expressions (state / int / MW / 1000)
-    dd cat = dd_from(s_state[P.zp_cat[x]] / (double)P.zp_ncat[x] / P.zp_catmw[x] / 1000.0);
-    dd an = dd_from(s_state[P.zp_an[x]] / (double)P.zp_nan[x] / P.zp_anmw[x] / 1000.0);
-    dd e_ac = dd_from(cr_exp(-100.0 * cat.hi));
-    dd e_aa = dd_from(cr_exp(-100.0 * an.hi));
+    double* q = scratch + 6 * x;
+    dd cat = dd_from(q[0]), an = dd_from(q[1]), e_ac = dd_from(q[2]), e_aa = dd_from(q[3]);
     dd conc = dd_div(dd_add(dd_mul(cat, e_ac), dd_mul(an, e_aa)), dd_add(e_ac, e_aa));
-    water = dd_round(dd_add(dd_from(water), dd_mul(dd_div(conc, mol), dd_from(1000.0))));
+    dd v = dd_mul(dd_div(conc, mol), dd_from(1000.0));
+    q[4] = v.hi;
+    q[5] = v.lo;
   }
-  s_state[P.zi_water[z]] = water;
+  wsync();
+  for (int z = lane; z < P.n_zi; z += kWave) {
+    double water = 1.0e-30;
+    for (int x = P.zi_pair_ptr[z]; x < P.zi_pair_ptr[z + 1]; ++x)
+      water = dd_round(dd_add(dd_from(water), dd{scratch[6 * x + 4], scratch[6 * x + 5]}));
+    s_state[P.zi_water[z]] = water;
+  }
+  wsync();
 }
 
-// --- ZSR parameter Jacobian of one item (:314-~440), added into s_jp -------
-__host__ __device__ __forceinline__ void mp_zsr_jac(const DevProgram& P, int z, const double* s_sub_env,
-                                           const double* s_state, double* s_jp) {
-  double ppm = s_sub_env[P.zi_sub[z]];
-  dd aw = dd_from(ppm * s_state[P.zi_gw[z]]);
-  for (int x = P.zi_pair_ptr[z]; x < P.zi_pair_ptr[z + 1]; ++x) {
+// --- ZSR parameter Jacobian (:314-~440), added into s_jp: a lane per pair,
+// then a lane per item adds its pairs in order ------------------------------
+__device__ __forceinline__ void mp_zsr_jac(const DevProgram& P, int lane, const double* s_sub_env,
+                                           const double* s_state, double* s_jp, double* scratch) {
+  mp_zsr_ions(P, lane, s_state, scratch);
+  for (int x = lane; x < P.n_zp; x += kWave) {
+    const int z = P.zp_zi[x];
+    double ppm = s_sub_env[P.zi_sub[z]];
+    dd aw = dd_from(ppm * s_state[P.zi_gw[z]]);
     double low = P.zp_lowrh[x];
     bool above = dd_gt(aw, low);
     dd jaw = above ? aw : dd_from(low);
@@ -127,12 +157,10 @@ __host__ __device__ __forceinline__ void mp_zsr_jac(const DevProgram& P, int z, 
       dmol = dd_add(dmol, dd_from(Y[k] * k * cr_powi(jaw_d, k - 1)));
     }
     dmol = dd_mul(dmol, djaw);
-    dd cat = dd_from(s_state[P.zp_cat[x]] / (double)P.zp_ncat[x] / P.zp_catmw[x] / 1000.0);
+    double* q = scratch + 6 * x;
+    dd cat = dd_from(q[0]), an = dd_from(q[1]), e_ac = dd_from(q[2]), e_aa = dd_from(q[3]);
     double dcat = 1.0 / (double)P.zp_ncat[x] / P.zp_catmw[x] / 1000.0;
-    dd an = dd_from(s_state[P.zp_an[x]] / (double)P.zp_nan[x] / P.zp_anmw[x] / 1000.0);
     double dan = 1.0 / (double)P.zp_nan[x] / P.zp_anmw[x] / 1000.0;
-    dd e_ac = dd_from(cr_exp(-100.0 * cat.hi));
-    dd e_aa = dd_from(cr_exp(-100.0 * an.hi));
     dd conc = dd_div(dd_add(dd_mul(cat, e_ac), dd_mul(an, e_aa)), dd_add(e_ac, e_aa));
     dd den = dd_mul(dd_add(e_ac, e_aa), dd_add(e_ac, e_aa));
     // (1 - ALPHA*anion + ALPHA*cation), ALPHA = -100
@@ -149,10 +177,25 @@ __host__ __device__ __forceinline__ void mp_zsr_jac(const DevProgram& P, int z, 
     double t2 = 1.0 / p2 * 1000.0;
     dd v_an = dd_mul(dd_mul(dd_from(t2), dcda), dd_from(dan));
     dd v_cat = dd_mul(dd_mul(dd_from(t2), dcdc), dd_from(dcat));
-    s_jp[P.zp_jgw[x]] = dd_round(dd_add(dd_from(s_jp[P.zp_jgw[x]]), v_gw));
-    s_jp[P.zp_jan[x]] = dd_round(dd_add(dd_from(s_jp[P.zp_jan[x]]), v_an));
-    s_jp[P.zp_jcat[x]] = dd_round(dd_add(dd_from(s_jp[P.zp_jcat[x]]), v_cat));
+    q[0] = v_gw.hi;
+    q[1] = v_gw.lo;
+    q[2] = v_an.hi;
+    q[3] = v_an.lo;
+    q[4] = v_cat.hi;
+    q[5] = v_cat.lo;
   }
+  wsync();
+  for (int z = lane; z < P.n_zi; z += kWave)
+    for (int x = P.zi_pair_ptr[z]; x < P.zi_pair_ptr[z + 1]; ++x) {
+      const double* q = scratch + 6 * x;
+      double* j = s_jp + P.zp_jgw[x];
+      *j = dd_round(dd_add(dd_from(*j), dd{q[0], q[1]}));
+      j = s_jp + P.zp_jan[x];
+      *j = dd_round(dd_add(dd_from(*j), dd{q[2], q[3]}));
+      j = s_jp + P.zp_jcat[x];
+      *j = dd_round(dd_add(dd_from(*j), dd{q[4], q[5]}));
+    }
+  wsync();
 }
 
 // --- per-instance quantities shared by f and J ------------------------------
@@ -240,7 +283,8 @@ __host__ __device__ __forceinline__ void mp_aqeq_f(const DevProgram& P, int i, c
 
 // --- Jacobian scalars of one SIMPOL instance (rxn_SIMPOL_phase_transfer.c:
 // 415-~590), kSpScalars doubles: N, kp, kc, evap0 (dd), cond (dd), evap
-// (dd), d_cond_d_radius, d_evap_d_radius, d_evap_d_mass, d_evap_d_MW.  evap0
+// (dd), d_cond_d_radius, d_evap_d_radius, d_evap_d_mass, d_evap_d_MW, evap /
+// kp (dd), cond / kp (dd).  evap0
 // is k_c*Keq*MW/mass before the activity coefficient and the aerosol factor.
 __host__ __device__ __forceinline__ void mp_simpol_jscalars(const DevProgram& P, int i,
                                                    const double* s_state, const double* s_k,
@@ -270,6 +314,11 @@ __host__ __device__ __forceinline__ void mp_simpol_jscalars(const DevProgram& P,
   o[10] = dedr;
   o[11] = dedm;
   o[12] = dedw;
+  dd ek = dd_div_d(evap, e[3]), ck = dd_div_d(cond, e[3]);
+  o[13] = ek.hi;
+  o[14] = ek.lo;
+  o[15] = ck.hi;
+  o[16] = ck.lo;
 }
 
 // --- Jacobian scalars of one aqueous-equilibrium instance (:403-~430):
@@ -299,7 +348,7 @@ __host__ __device__ __forceinline__ void mp_aqeq_jscalars(const DevProgram& P, i
 // PRODUCTION contributions add, LOSS contributions subtract (Jacobian.c:
 // 223-241 keeps them in separate long double sums and outputs prod - loss).
 __host__ __device__ __forceinline__ dd mp_jac_record(const DevProgram& P, int4 a, double c,
-                                            const double* s_state, const double* s_aero,
+                                            const double* s_state, const double* s_part,
                                             const double* s_jsc, dd D) {
   const double* aq0 = s_jsc + kSpScalars * P.n_sp;
   if (a.x <= kJsSimpolAP) {
@@ -320,28 +369,24 @@ __host__ __device__ __forceinline__ dd mp_jac_record(const DevProgram& P, int4 a
       case kJsSimpolAA:  // LOSS N * evap_rate * act / kp
         D = dd_sub(D, dd_div_d(dd_mul(dd_from(N), evap0), kp));
         break;
-      default: {  // phase element: species a.z of the instance's phase
-        int pi = P.sp_pi[a.y];
-        const double* ag = s_aero + kAeroSlots * pi;
-        double dens = P.pm_dens[a.z], mw = P.pm_mw[a.z];
-        double factor = 3.0 / (4.0 * kPi) / cr_powi(P.pi_dp[pi] / 2.0, 3);
-        double numj = 1.0 / dens * factor;
+      default: {  // phase element: item a.w, whose partials s_part holds
+        double numj = s_part[2 * a.w], mwj = s_part[2 * a.w + 1];
         double massj = 1.0;
-        dd lm = {ag[3], ag[4]}, mo = {ag[5], ag[6]};
-        double mwj = dd_round(dd_div(dd_sub(mo, dd_mul(dd_from(1.0 / mw), lm)), dd_mul(mo, mo)));
         double radj = 0.0;
+        // (a radius term is an exact zero unless its factor overflowed)
+        auto term = [](dd d, double v) { return v == 0.0 ? d : dd_add(d, dd_from(v)); };
         if (a.x == kJsSimpolGP) {
-          D = dd_add(D, dd_from(N * dedr * radj));
-          D = dd_sub(D, dd_from(N * dcdr * radj));
+          D = term(D, N * dedr * radj);
+          D = term(D, -(N * dcdr * radj));
           D = dd_add(D, dd_mul(evap, dd_from(numj)));
           D = dd_sub(D, dd_mul(cond, dd_from(numj)));
           D = dd_add(D, dd_from(N * dedm * massj));
           D = dd_add(D, dd_from(N * dedw * mwj));
         } else {
-          D = dd_sub(D, dd_from(N * dedr / kp * radj));
-          D = dd_add(D, dd_from(N * dcdr / kp * radj));
-          D = dd_sub(D, dd_mul(dd_div_d(evap, kp), dd_from(numj)));
-          D = dd_add(D, dd_mul(dd_div_d(cond, kp), dd_from(numj)));
+          D = term(D, -(N * dedr / kp * radj));
+          D = term(D, N * dcdr / kp * radj);
+          D = dd_sub(D, dd_mul(dd{s[13], s[14]}, dd_from(numj)));
+          D = dd_add(D, dd_mul(dd{s[15], s[16]}, dd_from(numj)));
           D = dd_sub(D, dd_from(N * dedm / kp * massj));
           D = dd_sub(D, dd_from(N * dedw / kp * mwj));
         }
@@ -380,14 +425,6 @@ __host__ __device__ __forceinline__ dd mp_jac_record(const DevProgram& P, int4 a
   return D;
 }
 
-// All special Jacobian records of one reaction element, added to D.
-__host__ __device__ __forceinline__ dd mp_jac_records(const DevProgram& P, int e, const double* s_state,
-                                             const double* s_aero, const double* s_jsc, dd D) {
-  for (int q = P.js_ptr[e]; q < P.js_ptr[e + 1]; ++q)
-    D = mp_jac_record(P, P.js_a[q], P.js_c[q], s_state, s_aero, s_jsc, D);
-  return D;
-}
-
 // --- per-cell LDS of the multi-phase extras ----------------------------------
 struct MpLds {
   double *sub_env, *aero, *slot, *jsc, *jp;
@@ -397,9 +434,17 @@ struct MpLds {
 // parameter Jacobian); the per-instance Jacobian scalars (used only while J
 // is assembled) get their own mp_jsc_doubles(P) region, in LDS or in
 // per-wavefront global scratch as the caller places it.
+// The slots also serve as scratch while none holds a contribution: 4 doubles
+// per phase item (mp_phase_sums) or 6 per ion pair (mp_zsr) ahead of f's
+// contributions, 2 per phase item (s_part) while J is assembled.
+__host__ __device__ inline size_t mp_slot_doubles(const DevProgram& P) {
+  size_t n = 2 * (size_t)P.n_slots;
+  n = n > 4 * (size_t)P.n_it ? n : 4 * (size_t)P.n_it;
+  return n > 6 * (size_t)P.n_zp ? n : 6 * (size_t)P.n_zp;
+}
 __host__ __device__ inline size_t mp_lds_doubles(const DevProgram& P) {
   if (!P.mp) return 0;
-  return (size_t)P.n_sub_env + kAeroSlots * (size_t)P.n_pi + 2 * (size_t)P.n_slots + P.pnnz;
+  return (size_t)P.n_sub_env + kAeroSlots * (size_t)P.n_pi + mp_slot_doubles(P) + P.pnnz;
 }
 __host__ __device__ inline size_t mp_jsc_doubles(const DevProgram& P) {
   if (!P.mp) return 0;
@@ -411,7 +456,7 @@ __device__ __forceinline__ MpLds mp_lds(const DevProgram& P, double* base, doubl
   L.sub_env = base;
   L.aero = L.sub_env + P.n_sub_env;
   L.slot = L.aero + kAeroSlots * P.n_pi;
-  L.jp = L.slot + 2 * P.n_slots;
+  L.jp = L.slot + mp_slot_doubles(P);
   L.jsc = jsc;
   return L;
 }
@@ -430,10 +475,17 @@ __device__ __forceinline__ void mp_cell_env(const DevProgram& P, int lane, doubl
 // update sees the water that f() left.
 __device__ __forceinline__ void mp_refresh(const DevProgram& P, int lane, double* s_state, MpLds L) {
   lane = phase_lane(lane);
-  for (int i = lane; i < P.n_pi; i += kWave) mp_phase_update(P, i, s_state, L.aero + kAeroSlots * i);
+  mp_phase_sums(P, lane, s_state, L.aero, L.slot);
+  for (int i = lane; i < P.n_pi; i += kWave) {
+    double* a = L.aero + kAeroSlots * i;
+    double mass_d = dd_round(dd{a[3], a[4]});
+    a[0] = mass_d;
+    a[1] = dd_round(dd_div(dd_from(mass_d), dd{a[5], a[6]}));
+    double r = P.pi_dp[i] / 2.0;
+    a[2] = a[7] * 3.0 / (4.0 * kPi) / cr_powi(r, 3);
+  }
   wsync();
-  for (int z = lane; z < P.n_zi; z += kWave) mp_zsr_water(P, z, L.sub_env, s_state);
-  wsync();
+  mp_zsr(P, lane, L.sub_env, s_state, L.slot);
 }
 
 // The per-cell start of f(): refresh, then the contributions of the
@@ -453,11 +505,22 @@ __device__ __forceinline__ void mp_f_prologue(const DevProgram& P, int lane, dou
 __device__ __forceinline__ void mp_j_prologue(const DevProgram& P, int lane, const double* s_state,
                                               const double* s_k, MpLds L) {
   lane = phase_lane(lane);
-  for (int i = lane; i < P.n_pi; i += kWave)
-    mp_phase_partial_sums(P, i, s_state, L.aero + kAeroSlots * i);
+  mp_phase_sums(P, lane, s_state, L.aero, L.slot);
   for (int q = lane; q < P.pnnz; q += kWave) L.jp[q] = 0.0;
   wsync();
-  for (int z = lane; z < P.n_zi; z += kWave) mp_zsr_jac(P, z, L.sub_env, s_state, L.jp);
+  mp_zsr_jac(P, lane, L.sub_env, s_state, L.jp, L.slot);
+  // the partial derivatives of each phase's number concentration and average
+  // MW by its species (aero_phase_solver.c:78-150 and the representation's
+  // getters): one division per item instead of one per record that uses it
+  for (int it = lane; it < P.n_it; it += kWave) {
+    const int pi = P.pit_pi[it];
+    const double* ag = L.aero + kAeroSlots * pi;
+    double factor = 3.0 / (4.0 * kPi) / cr_powi(P.pi_dp[pi] / 2.0, 3);
+    L.slot[2 * it] = 1.0 / P.pit_dens[it] * factor;
+    dd lm = {ag[3], ag[4]}, mo = {ag[5], ag[6]};
+    L.slot[2 * it + 1] = dd_round(
+        dd_div(dd_sub(mo, dd_mul(dd_from(1.0 / P.pit_mw[it]), lm)), dd_mul(mo, mo)));
+  }
   for (int i = lane; i < P.n_sp; i += kWave)
     mp_simpol_jscalars(P, i, s_state, s_k, L.aero, L.jsc + kSpScalars * i);
   for (int i = lane; i < P.n_aq; i += kWave)
@@ -472,7 +535,7 @@ __device__ __forceinline__ void mp_j_prologue(const DevProgram& P, int lane, con
 // mp_jac_record does, padding not at all.
 __device__ __forceinline__ dd mp_jac_stream_record(const DevProgram& P, int4 a, int4 b,
                                                    const double* s_state, const double* s_k,
-                                                   double h, const double* s_aero,
+                                                   double h, const double* s_part,
                                                    const double* s_jsc, dd D) {
   const double c = hilo_to_double(b.w, b.z);
   if (a.x == -1) {
@@ -485,7 +548,7 @@ __device__ __forceinline__ dd mp_jac_stream_record(const DevProgram& P, int4 a, 
     return dd_add(D, dd{c * v, 0.0});
   }
   if (a.x == 0) return D;
-  return mp_jac_record(P, a, c, s_state, s_aero, s_jsc, D);
+  return mp_jac_record(P, a, c, s_state, s_part, s_jsc, D);
 }
 
 // J of a multi-phase cell: the reaction Jacobian into Jr (global scratch,
@@ -510,7 +573,7 @@ __device__ __forceinline__ void cell_jac_mp(const DevProgram& P, int lane, const
       const int4* nx = rec + 2 * (size_t)(k + 1) * kWave;
       a = nx[0];
       b = nx[1];
-      D = mp_jac_stream_record(P, ca, cb, s_state, s_k, h, L.aero, L.jsc, D);
+      D = mp_jac_stream_record(P, ca, cb, s_state, s_k, h, L.slot, L.jsc, D);
     }
     if (e >= 0) Jr[e] = D.hi;
   }

@@ -140,13 +140,15 @@ void Solver::setup_device() {
     P.min_moles_hi = (double)mo;
     P.min_moles_lo = (double)(mo - (long double)P.min_moles_hi);
     P.min_volume = (double)mv;
-    P.pi_start = dev_upload(G.pi_start, owned);
-    P.pi_model = dev_upload(G.pi_model, owned);
     P.pi_dp = dev_upload(G.pi_dp, owned);
-    P.pm_ptr = dev_upload(G.pm_ptr, owned);
-    P.pm_counted = dev_upload(G.pm_counted, owned);
-    P.pm_mw = dev_upload(G.pm_mw, owned);
-    P.pm_dens = dev_upload(G.pm_dens, owned);
+    P.n_it = (int)G.pit_state.size();
+    P.n_zp = (int)G.zp_cat.size();
+    P.pit_ptr = dev_upload(G.pit_ptr, owned);
+    P.pit_state = dev_upload(G.pit_state, owned);
+    P.pit_pi = dev_upload(G.pit_pi, owned);
+    P.pit_mw = dev_upload(G.pit_mw, owned);
+    P.pit_dens = dev_upload(G.pit_dens, owned);
+    P.zp_zi = dev_upload(G.zp_zi, owned);
     P.zi_water = dev_upload(G.zi_water, owned);
     P.zi_gw = dev_upload(G.zi_gw, owned);
     P.zi_sub = dev_upload(G.zi_sub, owned);
@@ -192,6 +194,14 @@ void Solver::setup_device() {
     P.jm_param = dev_upload(G.jm_param, owned);
   }
 
+  // beyond 64 KiB of LDS per block is opted into per kernel
+  const size_t fj_lds = fj_waves_per_block(P) * fj_lds_doubles(P) * sizeof(double);
+  if (fj_lds > 65536) {
+    (void)hipFuncSetAttribute((const void*)k_deriv, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)fj_lds);
+    (void)hipFuncSetAttribute((const void*)k_jac, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)fj_lds);
+  }
   size_t nc = m.nc;
   d_state = dev_alloc<double>(nc * G.ns, owned);
   d_env = dev_alloc<double>(nc * 2, owned);
