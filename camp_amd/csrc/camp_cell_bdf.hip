@@ -78,11 +78,14 @@ struct UDouble {
 };
 
 // MP selects the multi-phase instantiation: gas-phase programs run a kernel
-// without the aerosol code (smaller code and register footprint).  KG: the
-// rate constants are read in place in global memory (s_k) and, for the f
-// terms, held by the lanes (kt).
-template <bool MP, bool KG>
+// without the aerosol code (smaller code and register footprint).  PL: the
+// placement.  KG: the rate constants are read in place in global memory (s_k)
+// and, for the f terms, held by the lanes (kt).  GH: the J history lives in
+// global memory, with a copy in f's order in the wavefront's scratch (E).
+template <bool MP, int PL>
 struct CellCv {
+  static constexpr bool KG = !MP && PL == kPlaceGlobal, GH = MP || PL != kPlaceLds;
+
   // The kernel argument's program, read from kernarg memory anew where a phase
   // begins: the pointer is opaque to the compiler there, so the phase's fields
   // come with a few scalar loads.  Loaded once at the kernel's start, as the
@@ -96,7 +99,7 @@ struct CellCv {
   }
   int lane, nv;
   double *s_state, *s_k, *s_rate, *z01, *z2, *ewt, *acor, *y, *tempv, *ftemp, *last, *acinit,
-      *w, *lu, *slu, *s_fb;
+      *w, *lu, *slu, *s_fb, *E;
   double *Js, *Jy, *Jf;
   MpLds mpl;   // multi-phase extras (LDS); unused for gas-phase programs
   double* Jr;  // reaction Jacobian scratch (global) of multi-phase programs
@@ -165,14 +168,24 @@ struct CellCv {
     const DevProgram& P = program();
     long long t0 = tick();
     double ts = next_h > 0.0 ? next_h : init_h;
+    FLoad F;
+    if (!MP) {
+      f_load_terms(P, lane, F);
+      f_load_gather(P, lane, F);
+    }
     int bad = cell_set_state(P, lane, y, s_state);
     if (!bad) {
-      if (MP) mp_f_prologue(P, lane, s_state, s_k, mpl);
-      cell_rates<KG>(P, lane, s_state, s_k, s_rate, kt);
+      if (MP) {
+        mp_f_prologue(P, lane, s_state, s_k, mpl);
+        f_load_terms(P, lane, F);
+      }
+      cell_rates<KG>(P, lane, s_state, s_k, s_rate, F, kt);
+      if (MP) f_load_gather(P, lane, F);
       wsync();
       long long t1 = tick();
       if (prof && est) c_fr += t1 - t0;
-      cell_deriv(P, lane, s_state, s_rate, y, Js, Jy, Jf, est, ts, ftemp, s_fb, mpl.slot);
+      cell_deriv<GH>(P, lane, s_state, s_rate, y, GH ? E : Js, Jy, Jf, est, ts, ftemp, s_fb,
+                     KG ? tempv : w, F, MP ? mpl.slot : nullptr);
       wsync();
       if (prof && est) c_fg += clock64() - t1;
     }
@@ -206,7 +219,11 @@ struct CellCv {
     }
     __threadfence_block();
     wsync();
+    stage_history(P);
     if (prof) c_j += clock64() - t0;
+  }
+  __device__ __forceinline__ void stage_history(const DevProgram& P) {
+    if (GH) est_stage(P, lane, Js, Jf, E);
   }
 
   // The history updates below work on one row of the Nordsieck array at a
@@ -1021,7 +1038,7 @@ __global__ void __launch_bounds__(256)
   double* scratch = GH ? a.wave_scratch + ((size_t)blockIdx.x * (blockDim.x / kWave) + wv) *
                                               cell_bdf_wave_scratch(P, kPlace)
                        : nullptr;
-  CellCv<MP, !MP && PL == kPlaceGlobal> cv;
+  CellCv<MP, PL> cv;
   cv.lane = lane;
   cv.nv = nv;
   cv.s_state = base;
@@ -1032,6 +1049,7 @@ __global__ void __launch_bounds__(256)
     cv.s_k = sk_end;
     sk_end += P.n_env;
   }
+  sk_end = cv.s_state + even_up(sk_end - cv.s_state);
   cv.mpl = mp_lds(P, sk_end,
                   MP ? scratch + 2 * (P.lu_nnz + kWave + 1) + P.rnnz : nullptr);
   cv.s_rate = sk_end + mp_lds_doubles(P);
@@ -1062,6 +1080,10 @@ __global__ void __launch_bounds__(256)
   cv.z2 = vh; vh += 4 * (size_t)nv;
   cv.last = vh; vh += nv;
   cv.acinit = vh; vh += nv;
+  cv.E = nullptr;
+  if (GH) {
+    cv.E = vh; vh += est_doubles(P);
+  }
   cv.acor = v; v += nv;
   cv.y = v; v += nv;
   // the column solve's scratch w (nv > 128 only: smaller programs solve in
@@ -1173,6 +1195,7 @@ __global__ void __launch_bounds__(256)
         cv.zn0()[i] = s > 1.0e-60 ? s : 1.0e-60;
       }
       wsync();
+      cv.stage_history(P);
       cv.c_f = cv.c_j = cv.c_lu = cv.c_sol = cv.c_fr = cv.c_fg = 0;
       long long c_start = cv.tick();
       int flag;

@@ -20,6 +20,8 @@
 namespace camp {
 
 constexpr int kWave = 64;
+// doubles rounded up to whole 16-byte pairs
+__host__ __device__ constexpr size_t even_up(size_t n) { return n + (n & 1); }
 
 struct DevProgram {
   int ns, nv, nnz, n_env, n_terms, lu_nnz, n_rxn;
@@ -51,11 +53,12 @@ struct DevProgram {
   const double* je_c;
   const int* fs_species;             // lane slot -> species of the f gather
   const int4* t_rec;                 // per term: {k index | flags << 28, reactants x3}
-  const int4* fl_hdr;                // per pass: -, -, re_ell offset, width
-  const int2* re_ell;                // row-view entries in slot-major order
+  int es_n;                          // f estimate (Program::es_hdr and following)
+  const int4 *es_col, *es_fin;
+  const int2* es_hdr;
+  const int* es_src;
   int fb_rows, fb_nparts;            // balanced f gather: rows per lane, partials
   const int4* fb_rec;                // {index | target << 16, guard | flags << 24, coef}
-  const int2* fb_fin;                // per species: {first partial, count}
   // rate-constant program (rxn_update_env_state)
   const int *rx_type, *rx_fidx, *rx_eidx, *rx_nreact;
   const double* rx_float;
@@ -288,12 +291,52 @@ __device__ __forceinline__ void cell_rate_constants(const DevProgram& P, int lan
 // (n_terms double-doubles): k * prod(reactants) as the per-type
 // calc_deriv_contrib computes it (rxn_arrhenius.c:143-147 and alike);
 // first-order loss rounds k * y to double (rxn_first_order_loss.c:150).
+// What f(y) reads of the program before any of it depends on y: the lane's
+// first terms, the first records of its gather bin and the first batches of
+// the estimate.  Loaded ahead of f's start, so that one trip to the caches
+// covers what were five, one after another (each 300 to 600 cycles of the
+// 13000 of a gas-phase f).
+constexpr int kTermRegs = 4;
+constexpr int kEstSets = 4, kEstAhead = 2;  // register sets; batches whose values are ahead
+// One batch of the estimate's stream: the lane's columns, {position of its
+// first value, stride between entries | (pass the batch ends + 1) << 16} and
+// the values.  (The header comes by lane: a scalar load would be waited on at
+// once.)
+struct EstBatch {
+  int4 c;
+  int2 h;
+  double v[kEstBatch];
+};
+struct FLoad {
+  int4 tr[kTermRegs], a[4], fin;
+  EstBatch B[kEstSets];
+};
+__device__ __forceinline__ void est_prog(const DevProgram& P, int lane, int n, EstBatch& S) {
+  S.c = P.es_col[(size_t)n * kWave + lane];
+  S.h = P.es_hdr[(size_t)n * kWave + lane];
+}
+__device__ __forceinline__ void f_load_terms(const DevProgram& P, int lane, FLoad& F) {
+  lane = phase_lane(lane);
+#pragma unroll
+  for (int g = 0; g < kTermRegs; ++g) {
+    int t = lane + g * kWave;
+    F.tr[g] = t < P.n_terms ? P.t_rec[t] : make_int4(0, -1, -1, -1);
+  }
+}
+__device__ __forceinline__ void f_load_gather(const DevProgram& P, int lane, FLoad& F) {
+  lane = phase_lane(lane);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) F.a[g] = P.fb_rec[g * kWave + lane];
+#pragma unroll
+  for (int u = 0; u < kEstSets; ++u) est_prog(P, lane, u, F.B[u]);
+  F.fin = P.es_fin[lane];
+}
+
 // KT: the constants of a lane's first kTermRegs terms are in its registers
 // (kt), the others' in global memory.
-constexpr int kTermRegs = 4;
 template <bool KT = false>
-__host__ __device__ __forceinline__ void cell_rates(const DevProgram& P, int lane, const double* s_state,
-                                           const double* s_k, double* s_rate,
+__device__ __forceinline__ void cell_rates(const DevProgram& P, int lane, const double* s_state,
+                                           const double* s_k, double* s_rate, const FLoad& F,
                                            const double* kt = nullptr) {
   lane = phase_lane(lane);
   // a lane's terms in groups of four whose program loads are issued together
@@ -303,7 +346,8 @@ __host__ __device__ __forceinline__ void cell_rates(const DevProgram& P, int lan
 #pragma unroll
     for (int g = 0; g < TG; ++g) {
       int t = t0 + g * kWave;
-      tr[g] = t < P.n_terms ? P.t_rec[t] : make_int4(0, -1, -1, -1);
+      tr[g] = F.tr[g];
+      if (t0 != lane) tr[g] = t < P.n_terms ? P.t_rec[t] : make_int4(0, -1, -1, -1);
     }
 #pragma unroll
     for (int g = 0; g < TG; ++g) {
@@ -321,8 +365,7 @@ __host__ __device__ __forceinline__ void cell_rates(const DevProgram& P, int lan
         rate = tr[g].z >= 0 ? dd_mul_d(rate, y1) : rate;
         rate = tr[g].w >= 0 ? dd_mul_d(rate, y2) : rate;
       }
-      s_rate[2 * t] = rate.hi;
-      s_rate[2 * t + 1] = rate.lo;
+      reinterpret_cast<double2*>(s_rate)[t] = make_double2(rate.hi, rate.lo);
     }
   }
 }
@@ -356,21 +399,21 @@ __host__ __device__ inline size_t fb_sink_doubles(const DevProgram& P) {
 // (exact up to the rounding of lo * c); p joins the running sum Dh with an
 // error-free TwoSum whose error, with e, goes to Dl, so Dh + Dl is the
 // record sum to about 2^-100 of the magnitudes S (the reference's long
-// double production/loss sums keep 2^-64).  The running sums are stored at
-// the piece's target after every record -- the last store of a piece is its
-// value -- and a piece's last record (flag 16) restarts them from zero.
+// double production/loss sums keep 2^-64).  A piece's last record (flag 16)
+// stores the sums at the piece's target and restarts them from zero.
 struct FOps {
   double hi, lo, sg;
 };
-__host__ __device__ __forceinline__ FOps f_operands(int4 rec, const double* s_state,
+__device__ __forceinline__ FOps f_operands(int4 rec, const double* s_state,
                                            const double* s_rate, const double* s_slot) {
   int flags = (int)((unsigned)rec.y >> 24);
   int g = (rec.y << 8) >> 8;  // sign-extended 24-bit guard (-1 = none)
   const double* src = (flags & 4) ? s_slot : s_rate;
   int idx = rec.x & 0xFFFF;
   FOps o;
-  o.hi = src[2 * idx];
-  o.lo = src[2 * idx + 1];
+  const double2 v = reinterpret_cast<const double2*>(src)[idx];  // (16-byte aligned)
+  o.hi = v.x;
+  o.lo = v.y;
   o.sg = s_state[g >= 0 ? g : 0];
   return o;
 }
@@ -395,15 +438,51 @@ __host__ __device__ __forceinline__ void f_record(int4 rec, FOps o, double h, in
   // whole species: value Dh + Dl at [t], S at [nv + t]; partial: (Dh, Dl,
   // S) at [t], [t + 1], [t + 2] (the lo store first, so that for a whole
   // species the value overwrites it)
-  int t = (int)((unsigned)rec.x >> 16);
-  bool part = flags & 32;
-  s_fb[part ? t + 1 : t] = Dl;
-  s_fb[t] = part ? Dh : Dh + Dl;
-  s_fb[part ? t + 2 : nv + t] = S;
   if (flags & 16) {
+    int t = (int)((unsigned)rec.x >> 16);
+    bool part = flags & 32;
+    s_fb[part ? t + 1 : t] = Dl;
+    s_fb[t] = part ? Dh : Dh + Dl;
+    s_fb[part ? t + 2 : nv + t] = S;
     Dh = 0.0;
     Dl = 0.0;
     S = 0.0;
+  }
+}
+
+// The f estimate's J history in the order its stream reads it (Program::es_hdr),
+// then J_deriv by lane slot: est_doubles(P) doubles of the wavefront's scratch,
+// refreshed with the history.  An entry per lane is then one run of
+// consecutive doubles; read in place the elements were a cache line each (8
+// lines an instruction against 64).
+__host__ __device__ inline size_t est_doubles(const DevProgram& P) {
+  return (size_t)P.es_n + (size_t)(P.nv + kWave - 1) / kWave * kWave;
+}
+__device__ __forceinline__ void est_stage(const DevProgram& P, int lane, const double* Js,
+                                          const double* Jf, double* E) {
+  lane = phase_lane(lane);
+  for (int p = lane; p < P.es_n; p += kWave) {
+    const int e = P.es_src[p];
+    E[p] = e >= 0 ? Js[e] : 0.0;
+  }
+  for (int s = lane; s < P.nv; s += kWave) E[P.es_n + s] = Jf[P.fs_species[s]];
+  __threadfence_block();
+  wsync();
+}
+
+// (STAGED: values in the stream's order, else the Jacobian's elements)
+template <bool STAGED>
+__device__ __forceinline__ void est_vals(const DevProgram& P, const double* Js, EstBatch& S) {
+  int p = S.h.x;
+  const int stride = S.h.y & 0xFFFF;
+#pragma unroll
+  for (int u = 0; u < kEstBatch; ++u, p += stride) {
+    if (STAGED) {
+      S.v[u] = Js[p];
+    } else {
+      const int e = P.es_src[p];
+      S.v[u] = Js[e >= 0 ? e : 0];
+    }
   }
 }
 
@@ -415,21 +494,31 @@ __host__ __device__ __forceinline__ void f_record(int4 rec, FOps o, double h, in
 // are processed and each batch's LDS operands read before the batch is
 // accumulated.  Phase 3: lane per species, the pieces of a split species
 // are added in order, the Jacobian-based estimate J_hist (y - y_hist) +
-// f_hist is formed (ELL over the row view), and the precision-loss blend of
-// time_derivative.c:58-64 gives f.  s_fb is LDS scratch of fb_lds_doubles.
-__host__ __device__ __forceinline__ void cell_deriv(const DevProgram& P, int lane, const double* s_state,
+// f_hist is formed (a stream of batches over the rows, y - y_hist once per
+// species in dy), and the precision-loss blend of time_derivative.c:58-64
+// gives f.  s_fb is LDS scratch of fb_lds_doubles, dy (use_est) of nv.
+// STAGED: Js is est_stage's copy of the history (Jf unused).
+template <bool STAGED>
+__device__ __forceinline__ void cell_deriv(const DevProgram& P, int lane, const double* s_state,
                                            const double* s_rate, const double* y,
                                            const double* Js, const double* Jy,
                                            const double* Jf, bool use_est, double h,
-                                           double* out, double* s_fb,
+                                           double* out, double* s_fb, double* dy, FLoad& F,
                                            const double* s_slot = nullptr) {
   lane = phase_lane(lane);
   const int nv = P.nv, L = P.fb_rows;
   const double* slot_or_rate = s_slot ? s_slot : s_rate;
+  double jf = 0.0;
+  if (use_est) {
+#pragma unroll
+    for (int u = 0; u < kEstAhead; ++u) est_vals<STAGED>(P, Js, F.B[u]);
+    jf = STAGED ? Js[P.es_n + lane] : F.fin.x >= 0 ? Jf[F.fin.x] : 0.0;
+    for (int i = lane; i < nv; i += kWave) dy[i] = y[i] - Jy[i];
+  }
   {
     const int4* fr = P.fb_rec + lane;
     // fb_rec has padding rows up to a multiple of 4 plus 4 beyond fb_rows
-    int4 a0 = fr[0], a1 = fr[kWave], a2 = fr[2 * kWave], a3 = fr[3 * kWave];
+    int4 a0 = F.a[0], a1 = F.a[1], a2 = F.a[2], a3 = F.a[3];
     double Dh = 0.0, Dl = 0.0, S = 0.0;
     for (int j = 0; j < L; j += 4) {
       int4 c0 = a0, c1 = a1, c2 = a2, c3 = a3;
@@ -449,52 +538,20 @@ __host__ __device__ __forceinline__ void cell_deriv(const DevProgram& P, int lan
   }
   wsync();
   const double* part = s_fb + 2 * nv;
-  for (int pass = 0; pass * kWave < nv; ++pass) {
-    int slot = pass * kWave + lane;
-    int i = slot < nv ? P.fs_species[slot] : -1;
-    int4 hd = ld_uniform(P.fl_hdr, pass);
-    const int2* er = P.re_ell + hd.z + lane;
-    double acc = 0.0;
-    if (use_est) {
-      // re_ell has padding rows up to a multiple of kEstBatch plus kEstBatch
-      // beyond hd.w; a batch's J-history loads are all issued before the
-      // first is used
-      constexpr int EB = kEstBatch;
-      int2 b[EB];
-#pragma unroll
-      for (int u = 0; u < EB; ++u) b[u] = er[u * kWave];
-      for (int j = 0; j < hd.w; j += EB) {
-        int2 c[EB];
-#pragma unroll
-        for (int u = 0; u < EB; ++u) {
-          c[u] = b[u];
-          b[u] = er[(j + EB + u) * kWave];
-        }
-        double jv[EB], yv[EB], jyv[EB];
-#pragma unroll
-        for (int u = 0; u < EB; ++u) {
-          int e = c[u].x >= 0 ? c[u].x : 0, col = c[u].x >= 0 ? c[u].y : 0;
-          jv[u] = Js[e];
-          yv[u] = y[col];
-          jyv[u] = Jy[col];
-        }
-#pragma unroll
-        for (int u = 0; u < EB; ++u)
-          if (c[u].x >= 0) acc += jv[u] * (yv[u] - jyv[u]);
-      }
-    }
-    if (i < 0) continue;
-    int2 fin = P.fb_fin[i];
+  // a species' value from its pieces, blended with its estimate
+  auto finish = [&](int4 fin, double jf, double acc) {
+    const int i = fin.x;
+    if (i < 0) return;
     double Dhi = 0.0, S = 0.0;
-    if (fin.y == 0) {
+    if (fin.z == 0) {
       Dhi = s_fb[i];
       S = s_fb[nv + i];
-    } else if (fin.y > 0) {
+    } else if (fin.z > 0) {
       // the partials' (hi, lo) pairs are not normalised: TwoSum each first
-      dd D = two_sum(part[3 * fin.x], part[3 * fin.x + 1]);
-      S = part[3 * fin.x + 2];
-      for (int k = 1; k < fin.y; ++k) {
-        const double* q = part + 3 * (fin.x + k);
+      dd D = two_sum(part[3 * fin.y], part[3 * fin.y + 1]);
+      S = part[3 * fin.y + 2];
+      for (int k = 1; k < fin.z; ++k) {
+        const double* q = part + 3 * (fin.y + k);
         D = dd_add(D, two_sum(q[0], q[1]));
         S += q[2];
       }
@@ -503,7 +560,7 @@ __host__ __device__ __forceinline__ void cell_deriv(const DevProgram& P, int lan
     double v = 0.0;
     if (S != 0.0) {
       if (use_est) {
-        double est = Jf[i] + acc;
+        double est = jf + acc;
         double inv = 1.0 / S;
         double sf = inv / (inv + 1.0e-14 / fabs(Dhi));
         v = sf * Dhi + (1.0 - sf) * est;
@@ -512,6 +569,46 @@ __host__ __device__ __forceinline__ void cell_deriv(const DevProgram& P, int lan
       }
     }
     out[i] = v;
+  };
+  if (!use_est) {
+    for (int slot = lane; slot < (nv + kWave - 1) / kWave * kWave; slot += kWave)
+      finish(P.es_fin[slot], 0.0, 0.0);
+    return;
+  }
+  constexpr int NS = kEstSets, AH = kEstAhead;
+  EstBatch(&B)[NS] = F.B;
+  int4 fin = F.fin;
+  double acc = 0.0;
+  for (int n = 0;; n += NS) {
+#pragma unroll
+    for (int u = 0; u < NS; ++u) {
+      EstBatch& S = B[u];
+      est_vals<STAGED>(P, Js, B[(u + AH) % NS]);
+      const int cw[4] = {S.c.x, S.c.y, S.c.z, S.c.w};
+      double d[kEstBatch];
+#pragma unroll
+      for (int q = 0; q < kEstBatch; ++q) {
+        const int col = q % 2 ? (unsigned)cw[q / 2] >> 16 : cw[q / 2] & 0xFFFF;
+        d[q] = dy[col == 0xFFFF ? 0 : col];
+      }
+      __builtin_amdgcn_sched_barrier(0);  // (the loads ahead of their uses)
+#pragma unroll
+      for (int q = 0; q < kEstBatch; ++q) {
+        const int col = q % 2 ? (unsigned)cw[q / 2] >> 16 : cw[q / 2] & 0xFFFF;
+        const double t = acc + S.v[q] * d[q];
+        acc = col == 0xFFFF ? acc : t;
+      }
+      const int pass = (__builtin_amdgcn_readfirstlane(S.h.y) >> 16) - 1;
+      if (pass >= 0) {
+        finish(fin, jf, acc);
+        acc = 0.0;
+        const int next = (pass + 1) * kWave;
+        if (next >= nv) return;
+        fin = P.es_fin[next + lane];
+        jf = STAGED ? Js[P.es_n + next + lane] : fin.x >= 0 ? Jf[fin.x] : 0.0;
+      }
+      est_prog(P, lane, n + u + NS, S);
+    }
   }
 }
 
@@ -520,13 +617,25 @@ __host__ __device__ __forceinline__ void cell_deriv(const DevProgram& P, int lan
 __device__ __forceinline__ int cell_set_state(const DevProgram& P, int lane, const double* y,
                                               double* s_state) {
   lane = phase_lane(lane);
-  int bad = 0;
-  for (int i = lane; i < P.nv; i += kWave) bad |= (y[i] < -1.0e-30);
+  constexpr int R = 2;  // rows a lane keeps between the check and the copy
+  double v[R];
+  int to[R], bad = 0;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = lane + r * kWave;
+    v[r] = i < P.nv ? y[i] : 0.0;
+    to[r] = i < P.nv ? P.dep_state[i] : -1;
+    bad |= v[r] < -1.0e-30;
+  }
+  for (int i = lane + R * kWave; i < P.nv; i += kWave) bad |= (y[i] < -1.0e-30);
   bad = wave_or(bad);
   if (bad) return 1;
-  for (int i = lane; i < P.nv; i += kWave) {
-    double v = y[i];
-    s_state[P.dep_state[i]] = v > -1.0e-30 ? v : 1.0e-60;
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (to[r] >= 0) s_state[to[r]] = v[r] > -1.0e-30 ? v[r] : 1.0e-60;
+  for (int i = lane + R * kWave; i < P.nv; i += kWave) {
+    double w = y[i];
+    s_state[P.dep_state[i]] = w > -1.0e-30 ? w : 1.0e-60;
   }
   wsync();
   return 0;

@@ -52,8 +52,9 @@ __global__ void __launch_bounds__(256) k_deriv(DevProgram P, int nc, const doubl
   int wpb = blockDim.x / kWave;
   double* s_state = smem + (size_t)wv * fj_lds_doubles(P);
   double* s_k = s_state + P.ns;
-  double* s_rate = s_k + P.n_env + mp_lds_doubles(P);
-  MpLds L = mp_lds(P, s_k + P.n_env, s_rate + 2 * (size_t)P.n_terms);
+  double* s_mp = s_state + even_up((size_t)P.ns + P.n_env);
+  double* s_rate = s_mp + mp_lds_doubles(P);
+  MpLds L = mp_lds(P, s_mp, s_rate + 2 * (size_t)P.n_terms);
   double* s_fb = s_rate + 2 * (size_t)P.n_terms + mp_jsc_doubles(P);
   for (int c = blockIdx.x * wpb + wv; c < nc; c += gridDim.x * wpb) {
     stage_cell(P, lane, state + (size_t)c * P.ns, rxn_env + (size_t)c * P.n_env, s_state, s_k);
@@ -66,10 +67,14 @@ __global__ void __launch_bounds__(256) k_deriv(DevProgram P, int nc, const doubl
       mp_cell_env(P, lane, env[2 * c], env[2 * c + 1], L);
       mp_f_prologue(P, lane, s_state, s_k, L);
     }
-    cell_rates(P, lane, s_state, s_k, s_rate);
+    FLoad F;
+    f_load_terms(P, lane, F);
+    f_load_gather(P, lane, F);
+    cell_rates(P, lane, s_state, s_k, s_rate, F);
     wsync();
-    cell_deriv(P, lane, s_state, s_rate, yc, Js + (size_t)c * P.nnz, Jy + (size_t)c * P.nv,
-               Jf + (size_t)c * P.nv, use_est != 0, h, fout + (size_t)c * P.nv, s_fb, L.slot);
+    cell_deriv<false>(P, lane, s_state, s_rate, yc, Js + (size_t)c * P.nnz, Jy + (size_t)c * P.nv,
+                      Jf + (size_t)c * P.nv, use_est != 0, h, fout + (size_t)c * P.nv, s_fb,
+                      s_fb + fb_lds_doubles(P), F, P.mp ? L.slot : nullptr);
     wsync();
   }
 }
@@ -86,8 +91,9 @@ __global__ void __launch_bounds__(256) k_jac(DevProgram P, int nc, const double*
   int wpb = blockDim.x / kWave;
   double* s_state = smem + (size_t)wv * fj_lds_doubles(P);
   double* s_k = s_state + P.ns;
-  double* s_rate = s_k + P.n_env + mp_lds_doubles(P);
-  MpLds L = mp_lds(P, s_k + P.n_env, s_rate + 2 * (size_t)P.n_terms);
+  double* s_mp = s_state + even_up((size_t)P.ns + P.n_env);
+  double* s_rate = s_mp + mp_lds_doubles(P);
+  MpLds L = mp_lds(P, s_mp, s_rate + 2 * (size_t)P.n_terms);
   for (int c = blockIdx.x * wpb + wv; c < nc; c += gridDim.x * wpb) {
     stage_cell(P, lane, state + (size_t)c * P.ns, rxn_env + (size_t)c * P.n_env, s_state, s_k);
     if (cell_set_state(P, lane, y + (size_t)c * P.nv, s_state)) continue;
@@ -711,10 +717,13 @@ __device__ __forceinline__ int fd_f(const DevProgram& P, int lane, const double*
                                    double h_ts, double* out) {
   if (cell_set_state(P, lane, yp, s_state)) return 1;
   if (P.mp) mp_f_prologue(P, lane, s_state, s_k, L);
-  cell_rates(P, lane, s_state, s_k, s_rate);
+  FLoad F;
+  f_load_terms(P, lane, F);
+  f_load_gather(P, lane, F);
+  cell_rates(P, lane, s_state, s_k, s_rate, F);
   wsync();
-  cell_deriv(P, lane, s_state, s_rate, yp, nullptr, nullptr, nullptr, false, h_ts, out, s_fb,
-             L.slot);
+  cell_deriv<false>(P, lane, s_state, s_rate, yp, nullptr, nullptr, nullptr, false, h_ts, out,
+                    s_fb, nullptr, F, P.mp ? L.slot : nullptr);
   wsync();
   return 0;
 }
@@ -729,8 +738,9 @@ __global__ void __launch_bounds__(64) k_check_jac(DevProgram P, int nc, const do
   const int lane = threadIdx.x;
   double* s_state = smem;
   double* s_k = s_state + P.ns;
-  double* s_rate = s_k + P.n_env + mp_lds_doubles(P);
-  MpLds L = mp_lds(P, s_k + P.n_env, s_rate + 2 * (size_t)P.n_terms);
+  double* s_mp = s_state + even_up((size_t)P.ns + P.n_env);
+  double* s_rate = s_mp + mp_lds_doubles(P);
+  MpLds L = mp_lds(P, s_mp, s_rate + 2 * (size_t)P.n_terms);
   double* s_fb = s_rate + 2 * (size_t)P.n_terms + mp_jsc_doubles(P);
   double* f0 = smem + fj_lds_doubles(P);
   double* f1 = f0 + P.nv;

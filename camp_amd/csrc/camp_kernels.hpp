@@ -59,11 +59,11 @@ __host__ __device__ inline size_t cell_lu_lds(const DevProgram& P) {
 }
 __host__ __device__ inline size_t cell_bdf_lds_doubles(const DevProgram& P, int place) {
   const bool g = cell_placement(P, place) != kPlaceLds;
-  return (size_t)P.ns + cell_lds_env(P, place) + mp_lds_doubles(P) + 2 * (size_t)P.n_terms +
-         (size_t)cell_lds_vectors(P, place) * P.nv + fb_sink_doubles(P) +
+  return even_up(P.ns + cell_lds_env(P, place)) + mp_lds_doubles(P) +
+         even_up(2 * (size_t)P.n_terms + (size_t)cell_lds_vectors(P, place) * P.nv + fb_sink_doubles(P) +
          (cell_lu_global(P, place) ? 0 : cell_placement(P, place) == kPlaceGlobal ? cell_lu_lds(P)
                                                                        : (size_t)P.lu_nnz) +
-         (g ? 0 : (size_t)P.nnz + 2 * (size_t)P.nv) + 24;
+         (g ? 0 : (size_t)P.nnz + 2 * (size_t)P.nv) + 24);
 }
 // Global scratch doubles per wavefront: the LU factors where they are global
 // (with the factorisation's 64 sink slots and the solve's zero slot; for
@@ -71,12 +71,13 @@ __host__ __device__ inline size_t cell_bdf_lds_doubles(const DevProgram& P, int 
 // multi-phase programs then the reaction Jacobian and the per-instance
 // Jacobian scalars, then (kPlaceGlobal, kPlaceGlobalLu) the Nordsieck
 // history and the work vectors not in LDS (11 vectors; 7 for gas-phase
-// kPlaceGlobal).
+// kPlaceGlobal) and the J history in f's order.
 __host__ __device__ inline size_t cell_bdf_wave_scratch(const DevProgram& P, int place) {
   if (P.mp)
-    return 2 * ((size_t)P.lu_nnz + kWave + 1) + P.rnnz + mp_jsc_doubles(P) + 11 * (size_t)P.nv;
-  if (place == kPlaceGlobalLu) return (size_t)P.lu_nnz + kWave + 1 + 11 * (size_t)P.nv;
-  return place == kPlaceGlobal ? 7 * (size_t)P.nv : 0;
+    return 2 * ((size_t)P.lu_nnz + kWave + 1) + P.rnnz + mp_jsc_doubles(P) + 11 * (size_t)P.nv +
+           est_doubles(P);
+  if (place == kPlaceGlobalLu) return (size_t)P.lu_nnz + kWave + 1 + 11 * (size_t)P.nv + est_doubles(P);
+  return place == kPlaceGlobal ? 7 * (size_t)P.nv + est_doubles(P) : 0;
 }
 
 // The no-allocation entry point's scratch (a file-scope device array of
@@ -137,8 +138,8 @@ __global__ void k_jac(DevProgram P, int nc, const double* y, const double* state
 // LDS doubles per wavefront of k_deriv and k_jac, and wavefronts per block
 // (one for multi-phase programs, whose per-cell extras are large)
 __host__ __device__ inline size_t fj_lds_doubles(const DevProgram& P) {
-  return (size_t)P.ns + P.n_env + mp_lds_doubles(P) + 2 * (size_t)P.n_terms + mp_jsc_doubles(P) +
-         fb_lds_doubles(P);
+  return even_up((size_t)P.ns + P.n_env) + mp_lds_doubles(P) +
+         even_up(2 * (size_t)P.n_terms + mp_jsc_doubles(P) + fb_lds_doubles(P) + P.nv);
 }
 inline int fj_waves_per_block(const DevProgram& P) { return P.mp ? 1 : 4; }
 

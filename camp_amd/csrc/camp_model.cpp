@@ -1059,35 +1059,44 @@ std::string Model::initialize() {
       return P.r_ptr[a + 1] - P.r_ptr[a] > P.r_ptr[b + 1] - P.r_ptr[b];
     });
     P.fs_species = order;
-    P.fl_hdr.clear();
-    P.re_ell.clear();
-    int npass = (nv + W - 1) / W;
+    P.es_hdr.clear();
+    P.es_col.clear();
+    P.es_src.clear();
+    const int npass = (nv + W - 1) / W;
     for (int pass = 0; pass < npass; ++pass) {
-      int cr = 0;
-      for (int l = 0; l < W && pass * W + l < nv; ++l) {
-        int i = order[pass * W + l];
-        cr = std::max(cr, P.r_ptr[i + 1] - P.r_ptr[i]);
-      }
-      P.fl_hdr.push_back(0);
-      P.fl_hdr.push_back(0);
-      P.fl_hdr.push_back((int)(P.re_ell.size() / 2));
-      P.fl_hdr.push_back(cr);
-      // rows padded (with -1 entries) to a multiple of kEstBatch plus
-      // kEstBatch, so that the estimate's batches and its loads a batch ahead
-      // need no checks
-      int cr_alloc = (cr + kEstBatch - 1) / kEstBatch * kEstBatch + kEstBatch;
-      for (int j = 0; j < cr_alloc; ++j)
+      auto len = [&](int l) {
+        int slot = pass * W + l;
+        return slot < nv ? P.r_ptr[order[slot] + 1] - P.r_ptr[order[slot]] : 0;
+      };
+      for (int j = 0; j == 0 || j < len(0); j += kEstBatch) {
+        int cnt = 0;
+        while (cnt < W && len(cnt) > j) ++cnt;
+        const bool last = j + kEstBatch >= len(0);
         for (int l = 0; l < W; ++l) {
-          int slot = pass * W + l, q = -1;
-          if (slot < nv) {
-            int i = order[slot];
-            if (j < P.r_ptr[i + 1] - P.r_ptr[i]) q = P.r_ptr[i] + j;
-          }
-          P.re_ell.push_back(q >= 0 ? P.r_elem[q] : -1);
-          P.re_ell.push_back(q >= 0 ? P.r_col[q] : -1);
+          P.es_hdr.push_back((int)P.es_src.size() + std::max(0, std::min(l, cnt - 1)));
+          P.es_hdr.push_back(cnt | (last ? (pass + 1) << 16 : 0));
         }
+        for (int l = 0; l < W; ++l)
+          for (int u = 0; u < kEstBatch; u += 2) {
+            int w = 0;
+            for (int h = 0; h < 2; ++h) {
+              int c = j + u + h < len(l) ? P.r_col[P.r_ptr[order[pass * W + l]] + j + u + h]
+                                         : 0xFFFF;
+              w |= c << (16 * h);
+            }
+            P.es_col.push_back(w);
+          }
+        for (int u = 0; u < kEstBatch; ++u)
+          for (int l = 0; l < cnt; ++l)
+            P.es_src.push_back(j + u < len(l) ? P.r_elem[P.r_ptr[order[pass * W + l]] + j + u]
+                                              : -1);
+      }
     }
-    if (P.re_ell.empty()) P.re_ell.assign(2, -1);
+    P.es_n = (int)P.es_src.size();
+    for (int q = 0; q < kEstPad; ++q) {
+      P.es_hdr.insert(P.es_hdr.end(), (size_t)2 * W, 0);
+      P.es_col.insert(P.es_col.end(), (size_t)W * kEstBatch / 2, -1);
+    }
   }
   {
     // balanced bins of the f gather
@@ -1323,6 +1332,12 @@ std::string Model::initialize() {
     h[3] = P.diag_pos[k];
   }
   initialized = true;
+  // the f gather's final pass in slot order: {species, first partial, count}
+  P.es_fin.clear();
+  for (int slot = 0; slot < (nv + 63) / 64 * 64; ++slot) {
+    const int i = slot < nv ? P.fs_species[slot] : -1;
+    P.es_fin.insert(P.es_fin.end(), {i, i < 0 ? 0 : P.fb_fin[2 * i], i < 0 ? -1 : P.fb_fin[2 * i + 1], 0});
+  }
   return std::string();
 }
 

@@ -28,8 +28,10 @@ constexpr int kLuRowBatch = 5;
 // programs' empty batches past the end, which the look-ahead loads.
 constexpr int kTriInPlace = 128;
 constexpr int kTriPad = 4;
-// Row-view entries of the f estimate's ELL a lane reads per batch.
+// Entries of the f estimate a lane reads per batch, and its empty batches past
+// the end, which the look-ahead loads.
 constexpr int kEstBatch = 8;
+constexpr int kEstPad = 4;
 
 // src/camp_common.h:34-45, src/time_derivative.h:18
 constexpr int kVariable = 1;
@@ -89,11 +91,16 @@ struct Program {
   std::vector<int> fe_rec;
   // The per-species pass of f(y) (estimate and blend) in lane-slot order:
   // species are assigned to slots by row length, longest first (slot s =
-  // pass * 64 + lane), fs_species[slot] is the species, and per pass fl_hdr
-  // = {0, 0, offset and width of re_ell ({element, column}, padding -1,
-  // rows padded to a multiple of 4 plus 4)}; entry j of lane l is at
-  // offset + j * 64 + l, so a wavefront's loads are contiguous.
-  std::vector<int> fs_species, fl_hdr, re_ell;
+  // pass * 64 + lane), fs_species[slot] is the species.  The estimate's
+  // entries are a stream of batches of kEstBatch entries per lane: es_hdr =
+  // per batch and lane {position of the lane's first value, lanes with
+  // entries (the first cnt) | (pass the batch ends + 1) << 16}, es_col = the
+  // columns as 16-bit words (0xFFFF past the row); entry u's value is u * cnt
+  // further on in the values' order, es_src[position] = its Jacobian element
+  // (-1 padding); then kEstPad empty batches.  es_fin = {species or -1, first
+  // partial, count, 0} per slot (fb_fin).
+  std::vector<int> fs_species, es_hdr, es_col, es_src, es_fin;
+  int es_n = 0;
   // The f gather in balanced bins: the species' record lists are cut into
   // pieces of at most fb_rows records (a species longer than that is split
   // into near-equal pieces) and the pieces packed longest first into 64

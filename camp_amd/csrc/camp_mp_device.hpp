@@ -440,11 +440,11 @@ struct MpLds {
 __host__ __device__ inline size_t mp_slot_doubles(const DevProgram& P) {
   size_t n = 2 * (size_t)P.n_slots;
   n = n > 4 * (size_t)P.n_it ? n : 4 * (size_t)P.n_it;
-  return n > 6 * (size_t)P.n_zp ? n : 6 * (size_t)P.n_zp;
+  return n > 6 * (size_t)P.n_zp ? n : 6 * (size_t)P.n_zp;  // (even)
 }
 __host__ __device__ inline size_t mp_lds_doubles(const DevProgram& P) {
   if (!P.mp) return 0;
-  return (size_t)P.n_sub_env + kAeroSlots * (size_t)P.n_pi + mp_slot_doubles(P) + P.pnnz;
+  return even_up((size_t)P.n_sub_env + kAeroSlots * (size_t)P.n_pi + mp_slot_doubles(P) + P.pnnz);
 }
 __host__ __device__ inline size_t mp_jsc_doubles(const DevProgram& P) {
   if (!P.mp) return 0;
@@ -453,10 +453,10 @@ __host__ __device__ inline size_t mp_jsc_doubles(const DevProgram& P) {
 
 __device__ __forceinline__ MpLds mp_lds(const DevProgram& P, double* base, double* jsc) {
   MpLds L;
-  L.sub_env = base;
+  L.slot = base;  // (16-byte aligned: the f gather reads (hi, lo) pairs)
+  L.sub_env = L.slot + mp_slot_doubles(P);
   L.aero = L.sub_env + P.n_sub_env;
-  L.slot = L.aero + kAeroSlots * P.n_pi;
-  L.jp = L.slot + mp_slot_doubles(P);
+  L.jp = L.aero + kAeroSlots * P.n_pi;
   L.jsc = jsc;
   return L;
 }

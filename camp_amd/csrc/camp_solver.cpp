@@ -96,12 +96,14 @@ void Solver::setup_device() {
   P.lf_hdr = reinterpret_cast<const int4*>(dev_upload(G.lf_hdr, owned));
   P.fs_species = dev_upload(G.fs_species, owned);
   P.t_rec = reinterpret_cast<const int4*>(dev_upload(G.t_rec, owned));
-  P.fl_hdr = reinterpret_cast<const int4*>(dev_upload(G.fl_hdr, owned));
-  P.re_ell = reinterpret_cast<const int2*>(dev_upload(G.re_ell, owned));
+  P.es_n = G.es_n;
+  P.es_hdr = reinterpret_cast<const int2*>(dev_upload(G.es_hdr, owned));
+  P.es_col = reinterpret_cast<const int4*>(dev_upload(G.es_col, owned));
+  P.es_src = dev_upload(G.es_src, owned);
+  P.es_fin = reinterpret_cast<const int4*>(dev_upload(G.es_fin, owned));
   P.fb_rows = G.fb_rows;
   P.fb_nparts = G.fb_nparts;
   P.fb_rec = reinterpret_cast<const int4*>(dev_upload(G.fb_rec, owned));
-  P.fb_fin = reinterpret_cast<const int2*>(dev_upload(G.fb_fin, owned));
   P.je_a = reinterpret_cast<const int4*>(dev_upload(G.je_a, owned));
   P.je_b = dev_upload(G.je_b, owned);
   P.je_c = dev_upload(G.je_c, owned);
