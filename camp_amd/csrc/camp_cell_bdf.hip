@@ -99,7 +99,7 @@ struct CellCv {
   }
   int lane, nv;
   double *s_state, *s_k, *s_rate, *z01, *z2, *ewt, *acor, *y, *tempv, *ftemp, *last, *acinit,
-      *w, *lu, *slu, *s_fb, *E;
+      *w, *lu, *s_fb, *E;
   double *Js, *Jy, *Jf;
   MpLds mpl;   // multi-phase extras (LDS); unused for gas-phase programs
   double* Jr;  // reaction Jacobian scratch (global) of multi-phase programs
@@ -456,8 +456,7 @@ struct CellCv {
   __device__ __forceinline__ int factor() {
     const DevProgram& P = program();
     long long t0 = tick();
-    int rc = cell_lu_factor(P, lane, Js, gamma, lu);
-    if (MP) cell_lu_order(P, lane, lu, slu);
+    int rc = cell_lu_factor(P, lane, Js, gamma, lu, s_fb);
     if (prof) c_lu += clock64() - t0;
     return rc;
   }
@@ -465,7 +464,7 @@ struct CellCv {
   __device__ __forceinline__ void lsolve(double* b) {
     const DevProgram& P = program();
     long long t0 = tick();
-    cell_lu_solve<MP>(P, lane, MP ? slu : lu, b, w);
+    cell_lu_solve<MP>(P, lane, lu, b, w);
     if (prof) c_sol += clock64() - t0;
     if (uc(gamrat != 1.0)) {
       double s = 2.0 / (1.0 + gamrat);
@@ -1051,14 +1050,14 @@ __global__ void __launch_bounds__(256)
   }
   sk_end = cv.s_state + even_up(sk_end - cv.s_state);
   cv.mpl = mp_lds(P, sk_end,
-                  MP ? scratch + 2 * (P.lu_nnz + kWave + 1) + P.rnnz : nullptr);
+                  MP ? scratch + (P.lu_nnz + kWave + 1) + P.rnnz : nullptr);
   cv.s_rate = sk_end + mp_lds_doubles(P);
   double* v = cv.s_rate + 2 * (size_t)P.n_terms;
   // With GH the Nordsieck history and the work vectors other than y, acor
   // and w live in the wavefront's global scratch (after the LU where it is
   // global, and for multi-phase programs the J_rxn and Jacobian scalars);
   // else all in LDS.
-  double* g = MP   ? scratch + 2 * (P.lu_nnz + kWave + 1) + P.rnnz + mp_jsc_doubles(P)
+  double* g = MP   ? scratch + (P.lu_nnz + kWave + 1) + P.rnnz + mp_jsc_doubles(P)
               : GL ? scratch + P.lu_nnz + kWave + 1
                    : scratch;
   double*& vh = GH ? g : v;
@@ -1100,8 +1099,7 @@ __global__ void __launch_bounds__(256)
   // the f gather's scratch follows the LU values (gas: also the LU's sinks)
   if (MP) {
     cv.lu = scratch;
-    cv.slu = scratch + P.lu_nnz + kWave + 1;
-    cv.Jr = cv.slu + P.lu_nnz + kWave + 1;
+    cv.Jr = scratch + P.lu_nnz + kWave + 1;
     cv.s_fb = v; v += fb_sink_doubles(P);
   } else {
     cv.Jr = nullptr;

@@ -38,16 +38,15 @@ struct DevProgram {
   const int *r_ptr, *r_elem, *r_col;  // row view of the solver pattern
   int n_cs;                            // state variables that are not solver variables
   const int* cs_ids;
-  const int *perm, *m_to_lu, *diag_pos, *e_diag;
-  const uint64_t* up_rec;  // LU update records: dst | l << 16 | u << 32, rows of 64
-  const int* lf_pos;        // L positions the factorisation scales, rows of 64
-  const int4* lf_hdr;       // per pivot: {lf_pos row start, up_rec row start,
-                            //  L rows | update rows << 16, diag position}
+  const int *perm, *diag_pos;
+  // LU factorisation (Program::lg_rec and following)
+  int lu_d, lg_n;
+  const int4* lg_rec;
+  const int* lt_pos;
   // triangular solves (Program::tri_e and following)
   int tri_s, tri_d, tri_nf, tri_nb, tt_nf, tt_nb;
   const int4 *tri_e, *tt;
   const int2* tri_r;
-  const int *tri_diag, *tri_src;
   const int4* je_a;  // packed J records (see Program in camp_model.hpp)
   const int* je_b;
   const double* je_c;
@@ -383,11 +382,14 @@ __host__ __device__ inline size_t fb_lds_doubles(const DevProgram& P) {
   return 2 * (size_t)P.nv + 3 * ((size_t)P.fb_nparts + 1);
 }
 // The per-cell kernel places the f gather's scratch right after the LU
-// values, where it also serves as the factorisation's 64 sink slots and
-// the triangular solve's zero slot (the 65th).
+// values, where it also serves as the zero slot of the factorisation and the
+// triangular solve (the 65th) and as the factorisation's tail buffers.
+// the LU tail's buffers: a pivot's row and column, 8 groups of up to 5 doubles
+constexpr int kLuTailStride = kLuTail / 8 + 1, kLuTailBuf = 2 * 8 * kLuTailStride;
 __host__ __device__ inline size_t fb_sink_doubles(const DevProgram& P) {
   size_t n = fb_lds_doubles(P);
-  return n > (size_t)kWave + 1 ? n : (size_t)kWave + 1;
+  const size_t m = kLuTailBuf > kWave + 1 ? kLuTailBuf : kWave + 1;
+  return n > m ? n : m;
 }
 
 // One record of the f gather, without branches: the term's rate (or a
@@ -742,115 +744,170 @@ __device__ __forceinline__ void cell_jac(const DevProgram& P, int lane, const do
 
 // ---------------------------------------------------------------------
 // Sparse LU of M = I - gamma*J (SUNMatScaleAddI) with the static pivot
-// order of the program; right-looking, one pivot at a time.  Returns 1 on
-// a zero or non-finite pivot (a recoverable linear-setup failure).  lu
-// holds lu_nnz values and 64 sink slots after them (scratch).
+// order of the program.  Returns 1 on a zero or non-finite pivot (a
+// recoverable linear-setup failure).  lu holds lu_nnz values and, at lu_nnz +
+// 64, the zero slot; buf is LDS scratch of kLuTailBuf doubles.
+//
+// One pivot after another, the factorisation is nv dependent steps whose lists
+// of updates are read from L2 as they come up (1300 cycles a pivot for the
+// CB05-scale mechanism, 2300 to 5000 for multi-phase cells, whose LU lives in
+// global memory).  The elimination order has far fewer levels (46 of 72, 65 of
+// 304 pivots), and most of them are the dense last pivots.  So every LU value is
+// a task -- its products in pivot order, the same operations the pivot-wise
+// elimination does on it, so the values are the same bit for bit -- and the
+// host packs the tasks into groups of 64 lanes, longest chain first, each at
+// least kLuDist groups after the values it reads are stored: a group's
+// operands are loaded while the one before it runs.  The last kLuTail pivots
+// are a dense block in registers (lane l holds rows 8 a + l / 8 and columns
+// 8 b + l % 8), a pivot's row and column going through LDS.
+// Cycles per factorisation: one CB05-scale cell 84k -> 55k (2000 cells 95k ->
+// 63k), one multi-phase cell 743k -> 339k (1024 cells 1.60M -> 0.57M); a third of
+// the gas one is tasks, the rest the register block (850 a pivot: an LDS round
+// trip, a division and 25 products).
 // ---------------------------------------------------------------------
-// One pivot of the factorisation's program: its header {lf_pos row start,
-// up_rec row start, L rows | update rows << 16, diagonal position}, the
-// lane's first L position and its first kLuRowBatch update records.
-struct LuPivot {
-  int4 h;
-  int l_p;
-  uint64_t rec[kLuRowBatch];
+struct LuGroup {
+  int4 r, h;
+  double src, a[4], b[4], dg;
 };
-__device__ __forceinline__ void lu_fetch_pivot(const DevProgram& P, int lane, int k, LuPivot& S) {
-  // lf_hdr has two empty pivots past the end; later ones are never used
-  S.h = ld_uniform(P.lf_hdr, k < P.nv + 2 ? k : P.nv + 1);
-  S.l_p = P.lf_pos[S.h.x + lane];
-#pragma unroll
-  for (int r = 0; r < kLuRowBatch; ++r) S.rec[r] = P.up_rec[S.h.y + r * kWave + lane];
+__device__ __forceinline__ void lu_prog(const DevProgram& P, int lane, int n, LuGroup& S) {
+  S.r = P.lg_rec[(size_t)(2 * n) * kWave + lane];
+  S.h = P.lg_rec[(size_t)(2 * n + 1) * kWave + lane];
 }
-// Eliminate one pivot; returns true on a zero or non-finite pivot.
-template <int R>
-__device__ __forceinline__ bool lu_pivot(const DevProgram& P, int lane, const LuPivot& S,
-                                         double* lu) {
-  const int nb = S.h.z >> 16;
-  double piv = lu[S.h.w];
-  double lval = lu[S.l_p];
-  double od[R], oa[R], ob[R];
+__device__ __forceinline__ void lu_src(const double* J, LuGroup& S) {
+  S.src = J[S.h.x >= 0 ? S.h.x : 0];
+}
+__device__ __forceinline__ void lu_vals(const double* lu, LuGroup& S) {
+  const int e[4] = {S.r.x, S.r.y, S.r.z, S.r.w};
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    od[r] = lu[(int)(S.rec[r] & 0xFFFF)];
-    oa[r] = lu[(int)((S.rec[r] >> 16) & 0xFFFF)];
-    ob[r] = lu[(int)((S.rec[r] >> 32) & 0xFFFF)];
+  for (int u = 0; u < 4; ++u) {
+    S.a[u] = lu[e[u] & 0xFFFF];
+    S.b[u] = lu[(unsigned)e[u] >> 16];
   }
-  // a zero or non-finite pivot fails the factorisation; the check is
-  // folded into a flag tested after the loop, so it does not make the
-  // pivot's load a wait ahead of the others (the values computed after a
-  // bad pivot are discarded with the failure)
-  bool bad = !(piv != 0.0 && isfinite(piv));
-  double rinv = 1.0 / piv;
-  lu[S.l_p] = lval * rinv;
-  for (int r = 1; r < (S.h.z & 0xFFFF); ++r) {
-    int p = P.lf_pos[S.h.x + r * kWave + lane];
-    lu[p] = lu[p] * rinv;
+  S.dg = lu[(unsigned)S.h.y >> 16];
+}
+// One group: the tasks' next four products; acc carries a task that goes on.
+__device__ __forceinline__ void lu_run(const LuGroup& S, double gamma, double* lu, double& acc,
+                                       bool& bad) {
+  const int fl = S.h.z;
+  double v = S.h.x >= 0 ? -gamma * S.src : 0.0;
+  v = (fl & 8) ? v + 1.0 : v;
+  acc = (fl & 1) ? v : acc;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) acc = acc - S.a[u] * S.b[u];
+  const double scaled = acc * (1.0 / S.dg);
+  acc = (fl & 4) ? scaled : acc;
+  if (fl & 2) {
+    // (a pivot of the register block is checked there)
+    bad |= (fl & 16) && !(acc != 0.0 && isfinite(acc));
+    lu[S.h.y & 0xFFFF] = acc;
   }
+  wsync();
+}
+
+// The dense block of the last lu_d pivots, NB blocks of 8.  A pivot's row and
+// column go through LDS (buf) by lane: the NB values a lane needs of either are
+// consecutive.
+template <int NB>
+__device__ __forceinline__ bool lu_tail(const DevProgram& P, int lane, double* lu, double* buf) {
+  constexpr int W = kLuTailStride;  // doubles per lane group of 8
+  const int d = P.lu_d, r = lane >> 3, c = lane & 7;
+  double a[NB][NB];
 #pragma unroll
-  for (int r = 0; r < R; ++r) lu[(int)(S.rec[r] & 0xFFFF)] = od[r] - (oa[r] * rinv) * ob[r];
-  if (nb > R) {
-    // the remaining rows (pivots of the dense trailing block) read the
-    // scaled L values; they go in batches of R rows whose loads are all
-    // issued before the first is used (the program pads them to whole
-    // batches: a per-row selection on a loaded record made the compiler
-    // wait for each load before issuing the next)
-    wsync();
-    for (int b = R; b < nb; b += R) {
-      uint64_t x[R];
+  for (int p = 0; p < NB; ++p)
 #pragma unroll
-      for (int r = 0; r < R; ++r) x[r] = P.up_rec[S.h.y + (b + r) * kWave + lane];
+    for (int q = 0; q < NB; ++q) {
+      const int at = P.lt_pos[(NB * p + q) * kWave + lane];
+      a[p][q] = lu[at >= 0 ? at : P.lu_nnz + kWave];
+    }
+  double *ub = buf, *lb = buf + 8 * W;
+  wsync();
+  bool bad = false;
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        od[r] = lu[(int)(x[r] & 0xFFFF)];
-        oa[r] = lu[(int)((x[r] >> 16) & 0xFFFF)];
-        ob[r] = lu[(int)((x[r] >> 32) & 0xFFFF)];
+  for (int kp = 0; kp < NB; ++kp) {
+    for (int kr = 0; kr < 8; ++kr) {
+      if (8 * kp + kr >= d) break;
+      if (r == kr) {
+#pragma unroll
+        for (int q = kp; q < NB; ++q) ub[W * c + q] = a[kp][q];
       }
+      if (c == kr) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) lu[(int)(x[r] & 0xFFFF)] = od[r] - oa[r] * ob[r];
+        for (int p = kp; p < NB; ++p) lb[W * r + p] = a[p][kp];
+      }
+      wsync();
+      const double piv = ub[W * kr + kp];
+      double l[NB], u[NB];
+#pragma unroll
+      for (int p = kp; p < NB; ++p) {
+        l[p] = lb[W * r + p];
+        u[p] = ub[W * c + p];
+      }
+      bad |= !(piv != 0.0 && isfinite(piv));
+      const double rinv = 1.0 / piv;
+#pragma unroll
+      for (int p = kp; p < NB; ++p) l[p] = l[p] * rinv;
+#pragma unroll
+      for (int p = kp; p < NB; ++p)
+#pragma unroll
+        for (int q = kp; q < NB; ++q) {
+          const double v = a[p][q] - l[p] * u[q];
+          a[p][q] = (p > kp || r > kr) && (q > kp || c > kr) ? v : a[p][q];
+        }
+      // the pivot's column keeps the scaled values
+#pragma unroll
+      for (int p = kp; p < NB; ++p) a[p][kp] = c == kr && (p > kp || r > kr) ? l[p] : a[p][kp];
+      wsync();
     }
   }
+#pragma unroll
+  for (int p = 0; p < NB; ++p)
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+      const int at = P.lt_pos[(NB * p + q) * kWave + lane];
+      if (at >= 0) lu[at] = a[p][q];
+    }
   wsync();
   return bad;
 }
 
 __device__ __forceinline__ int cell_lu_factor(const DevProgram& P, int lane, const double* J,
-                                              double gamma, double* lu) {
+                                              double gamma, double* lu, double* buf) {
   lane = phase_lane(lane);
+  if (lane == 0) lu[P.lu_nnz + kWave] = 0.0;
+  wsync();
   vm_drain();
-  for (int p = lane; p < P.lu_nnz; p += kWave) lu[p] = 0.0;
-  wsync();
-  for (int e = lane; e < P.nnz; e += kWave) {
-    double v = -gamma * J[e];
-    if (P.e_diag[e]) v = v + 1.0;
-    lu[P.m_to_lu[e]] = v;
-  }
-  wsync();
-  // Software pipeline over pivots, unrolled by two over two register sets:
-  // a pivot's header (scalar), first row of L positions and first R rows of
-  // update records are fetched two pivots before it is eliminated, so their
-  // latency hides behind the pivot in between (a rotation through copies
-  // would make every pivot wait for the newest loads).  The program pads
-  // every pivot to at least R rows of update records and its L positions to
-  // whole rows of 64, with entries that write the lane's own sink slot
-  // lu[lu_nnz + lane], so every load and store is unconditional.  Within one
-  // pivot every update has a distinct destination (neither the pivot's L
-  // column nor its U row).  A wavefront's LDS accesses execute in program
-  // order, so the pivot, the L values and every update operand are read
-  // before any of them is written: the updates use the unscaled L value
-  // times the pivot's reciprocal -- the same product that is stored as the
-  // scaled L value -- and the pivot needs a single wavefront sync.
-  constexpr int R = kLuRowBatch;
+  constexpr int NS = 4;  // register sets (NS <= kLuPad)
+  LuGroup S[NS];
+  double acc = 0.0;
   bool bad = false;
-  LuPivot A, B;
-  lu_fetch_pivot(P, lane, 0, A);
-  lu_fetch_pivot(P, lane, 1, B);
-  for (int k = 0; k < P.nv; k += 2) {
-    bad |= lu_pivot<R>(P, lane, A, lu);
-    lu_fetch_pivot(P, lane, k + 2, A);
-    if (k + 1 < P.nv) bad |= lu_pivot<R>(P, lane, B, lu);
-    lu_fetch_pivot(P, lane, k + 3, B);
+#pragma unroll
+  for (int u = 0; u < NS; ++u) lu_prog(P, lane, u, S[u]);
+  lu_src(J, S[0]);
+  lu_src(J, S[1]);
+  lu_vals(lu, S[0]);
+  bool done = P.lg_n == 0;
+  for (int n = 0; !done; n += NS) {
+#pragma unroll
+    for (int u = 0; u < NS; ++u) {
+      if (n + u >= P.lg_n) {
+        done = true;
+        break;
+      }
+      lu_vals(lu, S[(u + 1) % NS]);
+      lu_src(J, S[(u + 2) % NS]);
+      __builtin_amdgcn_sched_barrier(0);  // (the loads ahead of the chain)
+      lu_run(S[u], gamma, lu, acc, bad);
+      lu_prog(P, lane, n + u + NS, S[u]);
+    }
   }
-  return bad ? 1 : 0;
+  switch ((P.lu_d + 7) / 8) {
+    case 1: bad |= lu_tail<1>(P, lane, lu, buf); break;
+    case 2: bad |= lu_tail<2>(P, lane, lu, buf); break;
+    case 3: bad |= lu_tail<3>(P, lane, lu, buf); break;
+    case 4: bad |= lu_tail<4>(P, lane, lu, buf); break;
+    default: bad |= lu_tail<5>(P, lane, lu, buf); break;
+  }
+  return wave_or(bad ? 1 : 0);
 }
 
 __device__ __forceinline__ double readlane_d(double v, int l) {
@@ -1025,7 +1082,7 @@ __device__ __forceinline__ void tri_solve(const DevProgram& P, int lane, const d
   const bool on = lane < P.tri_d;
   const int r = on ? P.tri_s + lane : 0;
   const int ix = FMA ? P.perm[r] : r;
-  const double dg = on ? lu[P.tri_diag[r]] : 1.0;
+  const double dg = on ? lu[P.diag_pos[r]] : 1.0;
   tri_head<true, FMA, AH, NS>(P, lane, lu, X);
   double x = on ? X[ix] : 0.0;
   tri_tail<true, FMA, AH>(P, lane, lu, 1.0, 1.0, x);
@@ -1038,23 +1095,9 @@ __device__ __forceinline__ void tri_solve(const DevProgram& P, int lane, const d
   tri_head<false, FMA, AH, NS>(P, lane, lu, X);
 }
 
-// The factors of multi-phase programs (in global memory) in the order the
-// solve reads them (Program::tri_src), the zero slot after them: a batch's
-// loads of one entry per lane are then consecutive addresses (a row-major
-// gather touches a cache line per lane, and the solves outnumber the
-// factorisations eight to one).
-__device__ __forceinline__ void cell_lu_order(const DevProgram& P, int lane, const double* lu,
-                                              double* out) {
-  lane = phase_lane(lane);
-  for (int p = lane; p < P.lu_nnz; p += kWave) out[p] = lu[P.tri_src[p]];
-  if (lane == 0) out[P.lu_nnz + kWave] = 0.0;
-  __threadfence_block();
-  wsync();
-}
-
 // Solve (LU) x = b in place; b in dep order, w a scratch vector (nv) in LDS,
-// used past kTriInPlace.  FAR: the factors are those of cell_lu_order, in
-// global memory, and are fetched two batches ahead instead of one.
+// used past kTriInPlace.  FAR: the factors live in global memory (multi-phase
+// programs) and are fetched two batches ahead instead of one.
 template <bool FAR>
 __device__ __forceinline__ void cell_lu_solve(const DevProgram& P, int lane, double* lu, double* b,
                                               double* w) {

@@ -424,14 +424,14 @@ __global__ void __launch_bounds__(64) k_lu_factor(DevProgram P, int nc, const do
   int lane = threadIdx.x;
   double* s_lu = smem;
   for (int c = blockIdx.x; c < nc; c += gridDim.x) {
-    int bad = cell_lu_factor(P, lane, J + (size_t)c * P.nnz, gamma, s_lu);
+    int bad = cell_lu_factor(P, lane, J + (size_t)c * P.nnz, gamma, s_lu,
+                             s_lu + P.lu_nnz + kWave + 1);
     if (bad) {
       if (lane == 0) atomicOr(fail, 1);
       continue;
     }
     double* out = LU + (size_t)c * P.lu_nnz;
-    // (multi-phase programs: in the order the solve reads them)
-    for (int p = lane; p < P.lu_nnz; p += kWave) out[p] = s_lu[P.mp ? P.tri_src[p] : p];
+    for (int p = lane; p < P.lu_nnz; p += kWave) out[p] = s_lu[p];
     wsync();
   }
 }

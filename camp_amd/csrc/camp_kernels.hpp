@@ -66,15 +66,13 @@ __host__ __device__ inline size_t cell_bdf_lds_doubles(const DevProgram& P, int 
          (g ? 0 : (size_t)P.nnz + 2 * (size_t)P.nv) + 24);
 }
 // Global scratch doubles per wavefront: the LU factors where they are global
-// (with the factorisation's 64 sink slots and the solve's zero slot; for
-// multi-phase programs a second copy in the solve's order), for
-// multi-phase programs then the reaction Jacobian and the per-instance
+// (with the zero slot), for multi-phase programs then the reaction Jacobian and the per-instance
 // Jacobian scalars, then (kPlaceGlobal, kPlaceGlobalLu) the Nordsieck
 // history and the work vectors not in LDS (11 vectors; 7 for gas-phase
 // kPlaceGlobal) and the J history in f's order.
 __host__ __device__ inline size_t cell_bdf_wave_scratch(const DevProgram& P, int place) {
   if (P.mp)
-    return 2 * ((size_t)P.lu_nnz + kWave + 1) + P.rnnz + mp_jsc_doubles(P) + 11 * (size_t)P.nv +
+    return (size_t)P.lu_nnz + kWave + 1 + P.rnnz + mp_jsc_doubles(P) + 11 * (size_t)P.nv +
            est_doubles(P);
   if (place == kPlaceGlobalLu) return (size_t)P.lu_nnz + kWave + 1 + 11 * (size_t)P.nv + est_doubles(P);
   return place == kPlaceGlobal ? 7 * (size_t)P.nv + est_doubles(P) : 0;
@@ -167,6 +165,10 @@ inline size_t group_lds_bytes(const DevProgram& P, int lanes, bool fsum) {
 // out contiguously.
 inline size_t group_jac_lds_bytes(const DevProgram& P, int lanes) {
   return group_lds_bytes(P, lanes, false) + (size_t)(kWave / lanes) * P.nnz * sizeof(double);
+}
+// LDS of k_lu_factor: the LU values, the zero slot and the tail's buffers
+inline size_t lu_factor_lds_bytes(const DevProgram& P) {
+  return ((size_t)P.lu_nnz + kWave + 1 + kLuTailBuf) * sizeof(double);
 }
 __global__ void k_lu_factor(DevProgram P, int nc, const double* J, double gamma, double* LU,
                             int* fail);

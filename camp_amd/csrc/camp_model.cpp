@@ -571,8 +571,8 @@ static void build_tri_program(Program& P, const std::vector<char>& F,
         P.tt.push_back(w);
       }
   };
-  P.tri_diag = P.diag_pos;
-  P.tri_src.clear();
+  P.lu_at.resize(P.lu_nnz);
+  for (int p = 0; p < P.lu_nnz; ++p) P.lu_at[p] = p;
   P.tt_nf = P.tt_nb = 0;
   for (int kb = 0; kb < d - 1; kb += 8, ++P.tt_nf) block(kb, 1);
   for (int q = 0; q < kTriPad; ++q) block(d, 1);
@@ -580,17 +580,13 @@ static void build_tri_program(Program& P, const std::vector<char>& F,
   for (int q = 0; q < kTriPad; ++q) block(-1, -1);
   if (!P.mp) return;
   // renumber the LU values in the order the batches and blocks read them,
-  // lane after lane for each entry, the diagonals first
+  // lane after lane for each entry, the diagonals first: in global memory a
+  // load of one entry per lane is then a run of addresses
   std::vector<int> to(zero + 1, -1);
+  int n_to = 0;
   to[zero] = zero;
-  auto take = [&](int p) {
-    if (to[p] < 0) {
-      to[p] = (int)P.tri_src.size();
-      P.tri_src.push_back(p);
-    }
-    return to[p];
-  };
-  for (int k = 0; k < nv; ++k) P.tri_diag[k] = take(P.diag_pos[k]);
+  auto take = [&](int p) { return to[p] >= 0 ? to[p] : to[p] = n_to++; };
+  for (int k = 0; k < nv; ++k) take(P.diag_pos[k]);
   auto head = [&](int b0, int nb) {
     for (int b = b0; b < b0 + nb; ++b)
       for (int u = 0; u < 8; ++u)
@@ -615,6 +611,135 @@ static void build_tri_program(Program& P, const std::vector<char>& F,
   head(P.tri_nf + kTriPad, P.tri_nb);
   for (size_t q = 0; q < P.tri_r.size(); q += 2)
     if ((P.tri_r[q] & 0xFFFF) != 0xFFFF) P.tri_r[q + 1] = to[P.tri_r[q + 1]];
+  for (int p = 0; p < P.lu_nnz; ++p) P.lu_at[p] = take(p);
+  for (int k = 0; k < nv; ++k) P.diag_pos[k] = to[P.diag_pos[k]];
+}
+
+// The factorisation's program (Program::lg_rec) of the filled pattern F with
+// value positions pos.
+static void build_lu_program(Program& P, const std::vector<char>& F,
+                             const std::vector<int>& row_major) {
+  const int nv = P.nv, zero = P.lu_nnz + 64;
+  // (the positions are those the solve reads: Program::lu_at)
+  std::vector<int> pos = row_major;
+  for (int& p : pos)
+    if (p >= 0) p = P.lu_at[p];
+  const int d = P.lu_d = std::min(kLuTail, nv), s = nv - d;
+  struct Task {
+    int i, j, waits = 0;
+    std::vector<int> k;   // the pivots whose products it takes
+    std::vector<int> out; // tasks that wait on it
+    long path = 0;        // groups from its start to the end of the longest chain
+  };
+  std::vector<Task> t(P.lu_nnz);
+  for (int i = 0; i < nv; ++i)
+    for (int j = 0; j < nv; ++j) {
+      const int p = pos[(size_t)i * nv + j];
+      if (p < 0) continue;
+      Task& a = t[p];
+      a.i = i;
+      a.j = j;
+      const int top = std::min(std::min(i, j), s);
+      for (int k = 0; k < top; ++k)
+        if (F[(size_t)i * nv + k] && F[(size_t)k * nv + j]) a.k.push_back(k);
+      auto wait = [&](int q) {
+        t[q].out.push_back(p);
+        ++a.waits;
+      };
+      for (int k : a.k) {
+        wait(pos[(size_t)i * nv + k]);
+        wait(pos[(size_t)k * nv + j]);
+      }
+      if (i > j && j < s) wait(pos[(size_t)j * nv + j]);
+    }
+  auto groups = [&](const Task& a) { return std::max<long>(1, ((long)a.k.size() + 3) / 4); };
+  // longest chains, from the last tasks back (min(i, j) orders them; within
+  // one pivot the diagonal and its row precede the column)
+  std::vector<int> order(P.lu_nnz);
+  for (int p = 0; p < P.lu_nnz; ++p) order[p] = p;
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+    const int mx = std::min(t[x].i, t[x].j), my = std::min(t[y].i, t[y].j);
+    return mx != my ? mx > my : (t[x].i > t[x].j) > (t[y].i > t[y].j);
+  });
+  for (int p : order) {
+    for (int q : t[p].out) t[p].path = std::max(t[p].path, t[q].path + kLuDist - 1);
+    t[p].path += groups(t[p]);
+  }
+  std::vector<int> j_of(P.lu_nnz, -1);
+  for (int e = 0; e < P.nnz; ++e) j_of[P.lu_at[P.m_to_lu[e]]] = e;
+  // list scheduling: the ready task with the longest chain to a free lane
+  typedef std::pair<long, int> Ready;  // {path, -task}
+  std::vector<Ready> heap;
+  std::vector<std::vector<int>> due;   // tasks that become ready at a group
+  auto at = [&](size_t g) -> std::vector<int>& {
+    if (due.size() <= g) due.resize(g + 1);
+    return due[g];
+  };
+  for (int p = 0; p < P.lu_nnz; ++p)
+    if (t[p].waits == 0) at(0).push_back(p);
+  std::vector<int> lane_task(64, -1), lane_step(64, 0);
+  std::vector<size_t> ready_at(P.lu_nnz, 0);
+  long left = P.lu_nnz;
+  P.lg_rec.clear();
+  P.lg_n = 0;
+  while (left > 0) {
+    const size_t g = (size_t)P.lg_n++;
+    if (g < due.size())
+      for (int p : due[g]) {
+        heap.push_back({t[p].path, -p});
+        std::push_heap(heap.begin(), heap.end());
+      }
+    const size_t r0 = P.lg_rec.size();
+    P.lg_rec.resize(r0 + 64 * 8, 0);
+    for (int l = 0; l < 64; ++l) {
+      if (lane_task[l] < 0 && !heap.empty()) {
+        std::pop_heap(heap.begin(), heap.end());
+        lane_task[l] = -heap.back().second;
+        lane_step[l] = 0;
+        heap.pop_back();
+      }
+      int* rec = &P.lg_rec[r0 + (size_t)l * 4];
+      int* hdr = &P.lg_rec[r0 + 64 * 4 + (size_t)l * 4];
+      for (int u = 0; u < 4; ++u) rec[u] = zero | (zero << 16);
+      hdr[0] = -1;
+      hdr[1] = zero | (zero << 16);
+      const int p = lane_task[l];
+      if (p < 0) continue;
+      Task& a = t[p];
+      for (int u = 0; u < 4; ++u) {
+        const size_t q = (size_t)lane_step[l] * 4 + u;
+        if (q < a.k.size())
+          rec[u] = pos[(size_t)a.i * nv + a.k[q]] | (pos[(size_t)a.k[q] * nv + a.j] << 16);
+      }
+      const bool scaled = a.i > a.j && a.j < s;
+      const bool first = lane_step[l] == 0, last = lane_step[l] + 1 == groups(a);
+      if (first) hdr[0] = j_of[p];
+      hdr[1] = p | ((scaled ? pos[(size_t)a.j * nv + a.j] : zero) << 16);
+      hdr[2] = (first ? 1 : 0) | (last ? 2 : 0) | (scaled && last ? 4 : 0) | (a.i == a.j ? 8 : 0) |
+               (a.i == a.j && a.j < s ? 16 : 0);
+      ++lane_step[l];
+      if (last) {
+        lane_task[l] = -1;
+        --left;
+        for (int q : a.out) {
+          ready_at[q] = std::max(ready_at[q], g + kLuDist);
+          if (--t[q].waits == 0) at(ready_at[q]).push_back(q);
+        }
+      }
+    }
+  }
+  for (int q = 0; q < kLuPad; ++q)
+    for (int l = 0; l < 64 * 8; ++l)
+      P.lg_rec.push_back(l < 64 * 4 ? zero | (zero << 16)
+                                    : l % 4 == 0 ? -1 : l % 4 == 1 ? zero | (zero << 16) : 0);
+  P.lt_pos.clear();
+  const int nb = (d + 7) / 8;
+  for (int a = 0; a < nb; ++a)
+    for (int b = 0; b < nb; ++b)
+      for (int l = 0; l < 64; ++l) {
+        const int i = 8 * a + l / 8, j = 8 * b + l % 8;
+        P.lt_pos.push_back(i < d && j < d ? pos[(size_t)(s + i) * nv + s + j] : -1);
+      }
 }
 
 std::string Model::initialize() {
@@ -1260,11 +1385,9 @@ std::string Model::initialize() {
   P.lu_nnz = p;
   if (P.lu_nnz > 65535) return "LU fill exceeds 65535 entries per cell";
   P.m_to_lu.resize(P.nnz);
-  P.e_diag.assign(P.nnz, 0);
   for (int j = 0; j < nv; ++j)
     for (int e = P.colptr[j]; e < P.colptr[j + 1]; ++e) {
       P.m_to_lu[e] = pos[(size_t)P.iperm[P.rowval[e]] * nv + P.iperm[j]];
-      P.e_diag[e] = P.rowval[e] == j;
     }
   P.diag_pos.resize(nv);
   for (int k = 0; k < nv; ++k) P.diag_pos[k] = pos[(size_t)k * nv + k];
@@ -1297,40 +1420,7 @@ std::string Model::initialize() {
   }
   if (P.lu_nnz + 64 > 65535) return "LU fill exceeds 65471 entries per cell";
   build_tri_program(P, F, pos);
-  // The factorisation's program: per pivot, the L positions to scale and the
-  // update records {dst, l, u}, each padded to whole rows of 64 (at least
-  // one row of L positions) with entries that write lane l's sink slot
-  // lu_nnz + l, so the device loops need no per-lane bounds checks; every
-  // pivot's updates are padded with rows of sinks to a whole number (at
-  // least one) of batches of kLuRowBatch rows, so that the device loads a
-  // batch with no per-row selection; lf_hdr[k] = {first L position, first
-  // update record, L rows | update rows << 16, diagonal position} (two empty
-  // pivots past the end).
-  P.lf_pos.clear();
-  P.up_rec.clear();
-  P.lf_hdr.assign((size_t)4 * (nv + 2), 0);
-  for (int k = 0; k < nv; ++k) {
-    int* h = &P.lf_hdr[(size_t)4 * k];
-    h[0] = (int)P.lf_pos.size();
-    h[1] = (int)P.up_rec.size();
-    int nl = P.l_ptr[k + 1] - P.l_ptr[k], nu = P.up_ptr[k + 1] - P.up_ptr[k];
-    int rl = std::max(1, (nl + 63) / 64);
-    int ru = std::max(kLuRowBatch, (nu + 63) / 64);
-    ru = (ru + kLuRowBatch - 1) / kLuRowBatch * kLuRowBatch;
-    for (int q = 0; q < 64 * rl; ++q)
-      P.lf_pos.push_back(q < nl ? P.l_pos[P.l_ptr[k] + q] : P.lu_nnz + q % 64);
-    for (int q = 0; q < 64 * ru; ++q) {
-      if (q < nu) {
-        size_t e = (size_t)P.up_ptr[k] + q;
-        P.up_rec.push_back((uint64_t)P.up_dst[e] | ((uint64_t)P.up_l[e] << 16) |
-                           ((uint64_t)P.up_u[e] << 32));
-      } else {
-        P.up_rec.push_back((uint64_t)(P.lu_nnz + q % 64));
-      }
-    }
-    h[2] = rl | (ru << 16);
-    h[3] = P.diag_pos[k];
-  }
+  build_lu_program(P, F, pos);
   initialized = true;
   // the f gather's final pass in slot order: {species, first partial, count}
   P.es_fin.clear();

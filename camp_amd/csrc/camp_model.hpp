@@ -18,10 +18,12 @@
 
 namespace camp {
 
-// Rows of 64 LU update records the per-cell factorisation processes
-// together: a pivot's first kLuRowBatch rows, then its further rows in
-// batches of kLuRowBatch (the program pads those to whole batches).
-constexpr int kLuRowBatch = 5;
+// The LU factorisation: the last pivots (up to kLuTail) are factorised as a
+// dense block in registers; the program's empty groups past the end, which the
+// look-ahead loads, and the groups between a value's store and its first use.
+constexpr int kLuTail = 40;
+constexpr int kLuPad = 4;
+constexpr int kLuDist = 2;
 // The triangular solves: programs of up to kTriInPlace solver variables solve
 // in the right-hand side with fused multiply-adds and reciprocal diagonals,
 // larger ones in a scratch vector with separate products and divisions; the
@@ -124,16 +126,25 @@ struct Program {
   std::vector<int> r_ptr, r_elem, r_col;            // row view of the pattern
   // LU (positions in the permuted LU value array)
   std::vector<int> perm, iperm;                     // perm[k] = dep index of pivot k
-  std::vector<int> m_to_lu, diag_pos, e_diag;       // [nnz], [nv], [nnz]
+  std::vector<int> m_to_lu, diag_pos;               // [nnz], [nv]
   std::vector<int> l_ptr, l_pos, l_row;             // per pivot k: L(:,k) below k
   std::vector<int> u_ptr, u_pos, u_row;             // per pivot k: U(:,k) above k
   std::vector<int> up_ptr;                          // per pivot k: update range
   std::vector<uint16_t> up_dst, up_l, up_u;         // LU[dst] -= LU[l] * LU[u]
-  // the factorisation's program (built in Model::initialize): per pivot L
-  // positions (lf_pos) and update records dst | l << 16 | u << 32 (up_rec),
-  // each padded to rows of 64 with writes to the lanes' sink slots past the
-  // LU values, and lf_hdr = 4 ints per pivot
-  std::vector<int> lf_pos, lf_hdr;
+  // The factorisation's program (built by build_lu_program).  Every LU value is
+  // one task: its matrix entry, then the products l * u it receives, in pivot
+  // order, then (below the diagonal) the pivot's reciprocal.  Values of the
+  // last lu_d pivots' block take the products of earlier pivots only; the
+  // block itself is factorised in registers.  Tasks run in groups of 64 lanes;
+  // a lane works on one task for as many groups of 4 products as it has.
+  // lg_rec: per group and lane two int4 -- 4 products {position of l |
+  // position of u << 16}, and {Jacobian element or -1, position | position of
+  // the pivot << 16, flags: 1 first group, 2 last, 4 times the pivot's
+  // reciprocal, 8 diagonal, 16 a pivot before the block, 0}; lg_n groups, then kLuPad empty ones.  lt_pos:
+  // the block's positions (-1 none), entry (8 a + l / 8, 8 b + l % 8) of lane l
+  // at (nb a + b) * 64 + l, nb = (lu_d + 7) / 8.
+  int lu_d = 0, lg_n = 0;
+  std::vector<int> lg_rec, lt_pos;
   // The triangular solves' program (built by build_tri_program).  The last
   // tri_d = min(64, nv) pivots are the tail, whose unknowns sit one per lane;
   // the tri_s = nv - tri_d pivots before it are the head.
@@ -150,14 +161,12 @@ struct Program {
   //    no entry), tt_nf forward blocks, kTriPad empty ones, tt_nb backward
   //    blocks, kTriPad empty ones.
   // Unknowns are indexed by solver variable where the solve works in the
-  // right-hand side itself (nv <= kTriInPlace), else by pivot.  The LU
-  // values are read at the factorisation's positions; by multi-phase programs
-  // from a copy in the solve's own order, position p of it being tri_src[p] of
-  // the factorisation (tri_diag: the diagonals' positions as the solve reads
-  // them).
+  // right-hand side itself (nv <= kTriInPlace), else by pivot.  LU
+  // values are numbered by rows; those of multi-phase programs, whose factors
+  // live in global memory, in the order the solve reads them (lu_at: position
+  // by rows -> position).
   int tri_s = 0, tri_d = 0, tri_nf = 0, tri_nb = 0, tt_nf = 0, tt_nb = 0;
-  std::vector<int> tri_e, tri_r, tt, tri_diag, tri_src;
-  std::vector<uint64_t> up_rec;
+  std::vector<int> tri_e, tri_r, tt, lu_at;
   long n_updates() const { return (long)up_dst.size(); }
 
   // ---- lane-group f and J (gas-phase programs) ------------------------------

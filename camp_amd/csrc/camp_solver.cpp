@@ -77,9 +77,11 @@ void Solver::setup_device() {
     P.cs_ids = dev_upload(cs, owned);
   }
   P.perm = dev_upload(G.perm, owned);
-  P.m_to_lu = dev_upload(G.m_to_lu, owned);
   P.diag_pos = dev_upload(G.diag_pos, owned);
-  P.e_diag = dev_upload(G.e_diag, owned);
+  P.lu_d = G.lu_d;
+  P.lg_n = G.lg_n;
+  P.lg_rec = reinterpret_cast<const int4*>(dev_upload(G.lg_rec, owned));
+  P.lt_pos = dev_upload(G.lt_pos, owned);
   P.tri_s = G.tri_s;
   P.tri_d = G.tri_d;
   P.tri_nf = G.tri_nf;
@@ -89,11 +91,6 @@ void Solver::setup_device() {
   P.tri_e = reinterpret_cast<const int4*>(dev_upload(G.tri_e, owned));
   P.tri_r = reinterpret_cast<const int2*>(dev_upload(G.tri_r, owned));
   P.tt = reinterpret_cast<const int4*>(dev_upload(G.tt, owned));
-  P.tri_diag = dev_upload(G.tri_diag, owned);
-  P.tri_src = dev_upload(G.tri_src, owned);
-  P.up_rec = dev_upload(G.up_rec, owned);
-  P.lf_pos = dev_upload(G.lf_pos, owned);
-  P.lf_hdr = reinterpret_cast<const int4*>(dev_upload(G.lf_hdr, owned));
   P.fs_species = dev_upload(G.fs_species, owned);
   P.t_rec = reinterpret_cast<const int4*>(dev_upload(G.t_rec, owned));
   P.es_n = G.es_n;
@@ -687,7 +684,7 @@ struct BlockCv {
     }
     HIP_OK(hipMemsetAsync(S.d_fail, 0, sizeof(int), s));
     hipLaunchKernelGGL(k_lu_factor, dim3(std::min(nc, 16384)), dim3(64),
-                       ((size_t)S.P.lu_nnz + kWave) * sizeof(double), s, S.P, nc, S.d_Js, gamma, S.d_LU,
+                       lu_factor_lds_bytes(S.P), s, S.P, nc, S.d_Js, gamma, S.d_LU,
                        S.d_fail);
     return check_fail();
   }
@@ -1886,7 +1883,7 @@ extern "C" int camp_eval_lu_solve(void* solver_data, const double* jac, double g
   HIP_OK(hipMemcpyAsync(d_b, b, (size_t)nc * P.nv * sizeof(double), hipMemcpyHostToDevice, s->stream));
   HIP_OK(hipMemsetAsync(s->d_fail, 0, sizeof(int), s->stream));
   hipLaunchKernelGGL(camp::k_lu_factor, dim3(std::min(nc, 16384)), dim3(64),
-                     ((size_t)P.lu_nnz + camp::kWave) * sizeof(double), s->stream, P, nc, d_J,
+                     camp::lu_factor_lds_bytes(P), s->stream, P, nc, d_J,
                      gamma, d_LU, s->d_fail);
   hipLaunchKernelGGL(camp::k_lu_solve, dim3(std::min(nc, 16384)), dim3(64),
                      ((size_t)P.lu_nnz + camp::kWave + 1 + 2 * (size_t)P.nv) * sizeof(double),
