@@ -84,7 +84,7 @@ struct UDouble {
 // global memory, with a copy in f's order in the wavefront's scratch (E).
 template <bool MP, int PL>
 struct CellCv {
-  static constexpr bool KG = !MP && PL == kPlaceGlobal, GH = MP || PL != kPlaceLds;
+  static constexpr bool GH = MP || PL != kPlaceLds, KG = GH && !MP;
 
   // The kernel argument's program, read from kernarg memory anew where a phase
   // begins: the pointer is opaque to the compiler there, so the phase's fields
@@ -205,7 +205,7 @@ struct CellCv {
       cell_jac_mp(P, lane, s_state, s_k, ts, mpl, Jr, Js);
     } else {
       const double* k = s_k;
-      if (KG) {
+      if (KG && PL != kPlaceGlobalLu) {
         // J reads its constants at random: staged where the LU goes next
         for (int i = lane; i < P.n_env; i += kWave) lu[i] = s_k[i];
         wsync();
@@ -464,7 +464,7 @@ struct CellCv {
   __device__ __forceinline__ void lsolve(double* b) {
     const DevProgram& P = program();
     long long t0 = tick();
-    cell_lu_solve<MP>(P, lane, lu, b, w);
+    cell_lu_solve<MP || PL == kPlaceGlobalLu>(P, lane, lu, b, w);
     if (prof) c_sol += clock64() - t0;
     if (uc(gamrat != 1.0)) {
       double s = 2.0 / (1.0 + gamrat);
@@ -1041,7 +1041,7 @@ __global__ void __launch_bounds__(256)
   cv.lane = lane;
   cv.nv = nv;
   cv.s_state = base;
-  constexpr bool kNewtonLds = !MP && PL == kPlaceGlobal;
+  constexpr bool kNewtonLds = GH && !MP;
   // (kNewtonLds: no rate constants in LDS, see CellCv::kt)
   double* sk_end = cv.s_state + P.ns;
   if (!kNewtonLds) {
@@ -1076,9 +1076,11 @@ __global__ void __launch_bounds__(256)
     cv.tempv = vh; vh += nv;
     cv.ftemp = vh; vh += nv;
   }
-  cv.z2 = vh; vh += 4 * (size_t)nv;
-  cv.last = vh; vh += nv;
-  cv.acinit = vh; vh += nv;
+  // (where the LU is global there is room in LDS for all of the history)
+  double*& v2 = !MP && GL ? v : vh;
+  cv.z2 = v2; v2 += 4 * (size_t)nv;
+  cv.last = v2; v2 += nv;
+  cv.acinit = v2; v2 += nv;
   cv.E = nullptr;
   if (GH) {
     cv.E = vh; vh += est_doubles(P);

@@ -676,6 +676,14 @@ __global__ void k_state_gather(DevProgram P, int nc, const double* __restrict__ 
   double v = state[(size_t)c * P.ns + P.dep_state[d]];
   y[g] = v > 1.0e-60 ? v : 1.0e-60;
 }
+// (as given: the layer entry points evaluate the caller's state)
+__global__ void k_state_take(DevProgram P, int nc, const double* __restrict__ state,
+                             double* __restrict__ y) {
+  long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= (long)nc * P.nv) return;
+  int c = (int)(g / P.nv), d = (int)(g % P.nv);
+  y[g] = state[(size_t)c * P.ns + P.dep_state[d]];
+}
 __global__ void k_state_scatter(DevProgram P, int nc, const double* __restrict__ y,
                                 double* __restrict__ state) {
   long g = (long)blockIdx.x * blockDim.x + threadIdx.x;

@@ -47,11 +47,12 @@ __host__ __device__ inline bool cell_lu_global(const DevProgram& P, int place) {
 // weights, y, acor, tempv and ftemp; otherwise y, acor and the solve's w
 __host__ __device__ inline int cell_lds_vectors(const DevProgram& P, int place) {
   const int pl = cell_placement(P, place);
-  return pl == kPlaceLds ? 14 : (!P.mp && pl == kPlaceGlobal) ? 7 : 3;
+  return pl == kPlaceLds ? 14 : P.mp ? 3 : pl == kPlaceGlobal ? 7 : 13;
 }
-// rate constants in LDS (gas-phase kPlaceGlobal reads them in global memory)
+// rate constants in LDS (gas-phase cells with the J history in global memory
+// read them there too)
 __host__ __device__ inline size_t cell_lds_env(const DevProgram& P, int place) {
-  return !P.mp && cell_placement(P, place) == kPlaceGlobal ? 0 : (size_t)P.n_env;
+  return !P.mp && cell_placement(P, place) != kPlaceLds ? 0 : (size_t)P.n_env;
 }
 // gas-phase kPlaceGlobal: the LU's LDS, where J(y) also stages the rate constants
 __host__ __device__ inline size_t cell_lu_lds(const DevProgram& P) {
@@ -74,7 +75,7 @@ __host__ __device__ inline size_t cell_bdf_wave_scratch(const DevProgram& P, int
   if (P.mp)
     return (size_t)P.lu_nnz + kWave + 1 + P.rnnz + mp_jsc_doubles(P) + 11 * (size_t)P.nv +
            est_doubles(P);
-  if (place == kPlaceGlobalLu) return (size_t)P.lu_nnz + kWave + 1 + 11 * (size_t)P.nv + est_doubles(P);
+  if (place == kPlaceGlobalLu) return (size_t)P.lu_nnz + kWave + 1 + (size_t)P.nv + est_doubles(P);
   return place == kPlaceGlobal ? 7 * (size_t)P.nv + est_doubles(P) : 0;
 }
 
@@ -213,6 +214,7 @@ __global__ void k_scatter_rates(int n_cells, int n_upd, const int* upd_off, cons
                                 int n_env, double* renv);
 __global__ void k_clamp_constants(DevProgram P, int nc, const int* var_type, double* state);
 __global__ void k_state_gather(DevProgram P, int nc, const double* state, double* y);
+__global__ void k_state_take(DevProgram P, int nc, const double* state, double* y);
 __global__ void k_state_scatter(DevProgram P, int nc, const double* y, double* state);
 
 }  // namespace camp

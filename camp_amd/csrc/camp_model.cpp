@@ -578,10 +578,9 @@ static void build_tri_program(Program& P, const std::vector<char>& F,
   for (int q = 0; q < kTriPad; ++q) block(d, 1);
   for (int kb = d - 1; kb >= 0; kb -= 8, ++P.tt_nb) block(kb, -1);
   for (int q = 0; q < kTriPad; ++q) block(-1, -1);
-  if (!P.mp) return;
   // renumber the LU values in the order the batches and blocks read them,
-  // lane after lane for each entry, the diagonals first: in global memory a
-  // load of one entry per lane is then a run of addresses
+  // lane after lane for each entry, the diagonals first: a load of one entry
+  // per lane is then a run of addresses (whole cache lines, no bank conflicts)
   std::vector<int> to(zero + 1, -1);
   int n_to = 0;
   to[zero] = zero;

@@ -162,9 +162,8 @@ struct Program {
   //    blocks, kTriPad empty ones.
   // Unknowns are indexed by solver variable where the solve works in the
   // right-hand side itself (nv <= kTriInPlace), else by pivot.  LU
-  // values are numbered by rows; those of multi-phase programs, whose factors
-  // live in global memory, in the order the solve reads them (lu_at: position
-  // by rows -> position).
+  // values are numbered in the order the solves read them (lu_at: number by
+  // rows -> position).
   int tri_s = 0, tri_d = 0, tri_nf = 0, tri_nb = 0, tt_nf = 0, tt_nb = 0;
   std::vector<int> tri_e, tri_r, tt, lu_at;
   long n_updates() const { return (long)up_dst.size(); }

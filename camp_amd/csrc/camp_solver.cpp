@@ -305,9 +305,26 @@ void Solver::cell_launch_shape(long nq, int* grid, int* block, size_t* lds, int 
   *grid = (int)std::max<long>(1, std::min<long>((long)per_cu * ncu, (nq + cpb - 1) / cpb));
 }
 
+// The placement of a launch of n cells.  With the LU in global memory a
+// CB05-scale cell needs 13 KB of LDS instead of 26 and eight cells share a CU
+// instead of six, but a cell alone is slower: a step of 777 cells takes 16.9
+// instead of 16.0 ms, of 3000 19.3 instead of 17.4, of 10000 36.4 instead of
+// 38.0, of 100000 337 instead of 357.  So it is taken where it holds more cells
+// and the launch is at least four times what it holds.
+int Solver::run_place(long n) const {
+  if (!place_auto || P.mp || n < 4096) return place;
+  int g1 = 0, g2 = 0, block = 0;
+  size_t lds = 0;
+  cell_launch_shape(1L << 30, &g1, &block, &lds, place);
+  cell_launch_shape(1L << 30, &g2, &block, &lds, kPlaceGlobalLu);
+  return g2 > g1 && n >= 4L * g2 * (block / kWave) ? kPlaceGlobalLu : place;
+}
+
 int Solver::run_cells(double* st, double* env, double t0, double t1, double* noalloc,
                       size_t noalloc_doubles) {
   CellBdfArgs a = cell_args();
+  const int place = noalloc ? this->place : run_place(m.nc);
+  a.place = cell_placement(P, place);
   a.nc = m.nc;
   a.state = st;
   a.env = env;
@@ -327,7 +344,7 @@ int Solver::run_cells(double* st, double* env, double t0, double t1, double* noa
   }
   int grid = 0, block = 0;
   size_t lds = 0;
-  cell_launch_shape(m.nc, &grid, &block, &lds);
+  cell_launch_shape(m.nc, &grid, &block, &lds, place);
   int dev = 0;
   HIP_OK(hipGetDevice(&dev));
   if (noalloc) {
@@ -375,7 +392,8 @@ int Solver::run_cells(double* st, double* env, double t0, double t1, double* noa
   }
   bstats = s;
   stats_from_cells = true;
-  if (!explicit_order && (d_order || !noalloc)) {
+  // (cells that all start at once need no order, nor the copy of one)
+  if (!explicit_order && (d_order || !noalloc) && m.nc > (long)grid * (block / kWave)) {
     // Next call's queue order: the cells by this call's BDF step count,
     // most first (a counting sort on quarter octaves), so that a launch's
     // tail holds the cheap cells.  A cell's result does not depend on the
@@ -1465,7 +1483,10 @@ extern "C" long camp_solver_cell_lds_bytes(void* solver_data, int place) {
 extern "C" int camp_solver_set_placement(void* solver_data, int place) {
   using namespace camp;
   Solver* s = SD(solver_data);
-  if (place >= 0 && place < kNumPlacements) s->place = place;
+  if (place >= 0 && place < kNumPlacements) {
+    s->place = place;
+    s->place_auto = false;
+  }
   return cell_placement(s->P, s->place);
 }
 
@@ -1581,6 +1602,7 @@ extern "C" int camp_solver_autotune(void* solver_data, const double* d_state,
   for (void* p : tmp) HIP_OK(hipFree(p));
   s->cells_per_block = best;
   s->place = best_place;
+  s->place_auto = false;
   return best + 100 * best_place;
 }
 
@@ -1739,12 +1761,8 @@ static void eval_prepare(Solver* s, const double* state, const double* env, doub
   hipLaunchKernelGGL(camp::k_rates, dim3(camp::nblk((long)nc * s->m.n_rxn)), dim3(256), 0,
                      s->stream, P, nc, s->d_env, s->d_renv);
   // the solver variables, taken from the state as given (no clamping)
-  std::vector<double> y((size_t)nc * P.nv);
-  for (int c = 0; c < nc; ++c)
-    for (int d = 0; d < P.nv; ++d)
-      y[(size_t)c * P.nv + d] = state[(size_t)c * P.ns + s->m.prog.dep_state[d]];
-  HIP_OK(hipMemcpyAsync(d_y, y.data(), y.size() * sizeof(double), hipMemcpyHostToDevice, s->stream));
-  HIP_OK(hipStreamSynchronize(s->stream));
+  hipLaunchKernelGGL(camp::k_state_take, dim3(camp::nblk((long)nc * P.nv)), dim3(256), 0,
+                     s->stream, P, nc, s->d_state, d_y);
 }
 
 extern "C" int camp_eval_deriv(void* solver_data, const double* state, const double* env,
@@ -1753,10 +1771,11 @@ extern "C" int camp_eval_deriv(void* solver_data, const double* state, const dou
   s->ensure_device();
   int nc = s->m.nc;
   const camp::DevProgram& P = s->P;
-  std::vector<void*> tmp;
-  double* d_y = camp::dev_alloc<double>((size_t)nc * P.nv, tmp);
-  double* d_f = camp::dev_alloc<double>((size_t)nc * P.nv, tmp);
+  double* d_y = s->kept(s->d_eval_y, (size_t)nc * P.nv);
+  double* d_f = s->kept(s->d_eval_f, (size_t)nc * P.nv);
   eval_prepare(s, state, env, d_y);
+  // (a cell whose f fails keeps zeros)
+  HIP_OK(hipMemsetAsync(d_f, 0, (size_t)nc * P.nv * sizeof(double), s->stream));
   HIP_OK(hipMemsetAsync(s->d_fail, 0, sizeof(int), s->stream));
   if (s->eval_group && !P.mp) {
     s->refresh_kval();
@@ -1773,7 +1792,6 @@ extern "C" int camp_eval_deriv(void* solver_data, const double* state, const dou
   HIP_OK(hipMemcpyAsync(deriv, d_f, (size_t)nc * P.nv * sizeof(double), hipMemcpyDeviceToHost,
                         s->stream));
   HIP_OK(hipStreamSynchronize(s->stream));
-  for (void* p : tmp) (void)hipFree(p);
   return fail;
 }
 
@@ -1784,7 +1802,7 @@ extern "C" int camp_eval_jac(void* solver_data, const double* state, const doubl
   int nc = s->m.nc;
   const camp::DevProgram& P = s->P;
   std::vector<void*> tmp;
-  double* d_y = camp::dev_alloc<double>((size_t)nc * P.nv, tmp);
+  double* d_y = s->kept(s->d_eval_y, (size_t)nc * P.nv);
   eval_prepare(s, state, env, d_y);
   HIP_OK(hipMemsetAsync(s->d_fail, 0, sizeof(int), s->stream));
   int wpb = camp::fj_waves_per_block(P);
@@ -1875,10 +1893,11 @@ extern "C" int camp_eval_lu_solve(void* solver_data, const double* jac, double g
   s->ensure_device();
   int nc = s->m.nc;
   const camp::DevProgram& P = s->P;
-  std::vector<void*> tmp;
-  double* d_J = camp::dev_alloc<double>((size_t)nc * P.nnz, tmp);
-  double* d_LU = camp::dev_alloc<double>((size_t)nc * P.lu_nnz, tmp);
-  double* d_b = camp::dev_alloc<double>((size_t)nc * P.nv, tmp);
+  double* d_J = s->kept(s->d_eval_J, (size_t)nc * P.nnz);
+  double* d_LU = s->kept(s->d_eval_LU, (size_t)nc * P.lu_nnz);
+  double* d_b = s->kept(s->d_eval_f, (size_t)nc * P.nv);
+  // (a cell whose factorisation fails is solved with zeros)
+  HIP_OK(hipMemsetAsync(d_LU, 0, (size_t)nc * P.lu_nnz * sizeof(double), s->stream));
   HIP_OK(hipMemcpyAsync(d_J, jac, (size_t)nc * P.nnz * sizeof(double), hipMemcpyHostToDevice, s->stream));
   HIP_OK(hipMemcpyAsync(d_b, b, (size_t)nc * P.nv * sizeof(double), hipMemcpyHostToDevice, s->stream));
   HIP_OK(hipMemsetAsync(s->d_fail, 0, sizeof(int), s->stream));
@@ -1892,7 +1911,6 @@ extern "C" int camp_eval_lu_solve(void* solver_data, const double* jac, double g
   HIP_OK(hipMemcpyAsync(&fail, s->d_fail, sizeof(int), hipMemcpyDeviceToHost, s->stream));
   HIP_OK(hipMemcpyAsync(b, d_b, (size_t)nc * P.nv * sizeof(double), hipMemcpyDeviceToHost, s->stream));
   HIP_OK(hipStreamSynchronize(s->stream));
-  for (void* p : tmp) (void)hipFree(p);
   return fail;
 }
 

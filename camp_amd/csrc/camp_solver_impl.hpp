@@ -63,6 +63,10 @@ struct Solver {
   // per-cell kernel variant (cell_placement): history in global memory, the
   // fastest for the CB05-scale mechanism (six cells per CU instead of four)
   int place = kPlaceGlobal;
+  // until the caller or the autotuner chooses: run_place picks by the number
+  // of cells of a launch
+  bool place_auto = true;
+  int run_place(long n) const;
   int guess_on = 1;
   bool renv_dirty = true;
   hipStream_t stream = nullptr;
@@ -164,6 +168,11 @@ struct Solver {
     if (!stream) setup_device();
   }
   void upload_renv();
+  // The layer entry points' (camp_eval_deriv, camp_eval_jac) solver variables
+  // and f(y) of all cells, made by the first such call
+  double *d_eval_y = nullptr, *d_eval_f = nullptr;
+  double *d_eval_J = nullptr, *d_eval_LU = nullptr;  // camp_eval_lu_solve
+  double* kept(double*& p, size_t n) { return p ? p : p = dev_alloc<double>(n, owned); }
   // Per-cell kernel arguments with the solver's program and controls filled
   // in (buffers left to the caller), and the launch shape for nq queued cells.
   CellBdfArgs cell_args() const;

@@ -202,11 +202,14 @@ int camp_solver_set_graphs(void *solver_data, int on);
 int camp_solver_set_cells_per_block(void *solver_data, int cells_per_block);
 
 /* Cell placement of the per-cell kernel (gas-phase programs; multi-phase
- * programs always use 1): 0 = each cell's Nordsieck history, work vectors
- * and J history in LDS (fewer cells per compute unit), 1 = those in global
- * memory (more cells per compute unit, two wavefronts per SIMD; the
- * default), 2 = those and the LU factors in global memory.  Returns the
- * placement in effect.  Results do not depend on it. */
+ * programs always use 1): 0 = everything in LDS (fewest cells per compute
+ * unit), 1 = the higher Nordsieck vectors, the rate constants and the J
+ * history in global memory (two wavefronts per SIMD), 2 = the LU factors, the
+ * rate constants and the J history in global memory (most cells per compute
+ * unit).  Until it is set (or autotuned) each launch takes 1, or 2 where 2
+ * holds more cells at once and the launch has at least four times as many.
+ * Returns the placement set (1 by default; a negative place only asks).
+ * Results do not depend on it. */
 int camp_solver_set_placement(void *solver_data, int place);
 
 /* LDS bytes one cell of the per-cell kernel uses with the given placement
