@@ -12,6 +12,7 @@
 // camp_solver.c:1111-1114) is in HBM, because CAMP keeps it across calls.
 #include <cstdio>
 #include <mutex>
+#include <type_traits>
 
 #include "camp_device.hpp"
 #include "camp_kernels.hpp"
@@ -137,6 +138,38 @@ struct CellCv {
     else znh(j)[i] = v;
   }
 
+  // body(i, on) over the lane's rows, two at a time where there are more than
+  // 64: the second row's loads then overlap the first's (a second trip of the
+  // loop costs its full latency, for 8 rows of a CB05-scale cell).  A lane
+  // without a second row repeats its first one (on[1] false): same loads,
+  // same stores.
+  template <class B>
+  __device__ __forceinline__ void rows(B body) const {
+    for (int i0 = 0; i0 < nv; i0 += 2 * kWave) {
+      const int i = i0 + lane;
+      if (i0 + kWave < nv) {
+        const bool two = i + kWave < nv;
+        const int id[2] = {i, two ? i + kWave : i};
+        body(id, two, std::integral_constant<int, 2>());
+      } else if (i < nv) {
+        const int id[2] = {i, i};
+        body(id, false, std::integral_constant<int, 1>());
+      }
+    }
+  }
+  // f(order) with the method's order as a constant: the history loops then
+  // have fixed bounds
+  template <class F>
+  __device__ __forceinline__ void by_order(F f) const {
+    switch (q) {
+      case 1: f(std::integral_constant<int, 1>()); break;
+      case 2: f(std::integral_constant<int, 2>()); break;
+      case 3: f(std::integral_constant<int, 3>()); break;
+      case 4: f(std::integral_constant<int, 4>()); break;
+      default: f(std::integral_constant<int, 5>()); break;
+    }
+  }
+
   __device__ __forceinline__ double wrms(const double* x) {
     double s = 0.0;
     for (int i = lane; i < nv; i += kWave) {
@@ -151,12 +184,22 @@ struct CellCv {
   __device__ __forceinline__ double ewt_set() {
     const DevProgram& P = program();
     double s = 0.0;
-    for (int i = lane; i < nv; i += kWave) {
-      double z = zn0()[i], wt = 1.0 / (rtol * fabs(z) + P.abs_tol_dep[i]);
-      ewt[i] = wt;
-      double p = z * wt;
-      s += p * p;
-    }
+    rows([&](const int* id, bool two, auto R) {
+      double wt[R], z[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        z[r] = zn0()[id[r]];
+        wt[r] = P.abs_tol_dep[id[r]];
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) wt[r] = 1.0 / (rtol * fabs(z[r]) + wt[r]);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        ewt[id[r]] = wt[r];
+        double p = z[r] * wt[r];
+        s += r == 0 || two ? p * p : 0.0;
+      }
+    });
     wsync();
     return sqrt(wave_sum(s) / nv);
   }
@@ -246,13 +289,19 @@ struct CellCv {
       fac[j] = factor;
       factor *= eta;
     }
-    for (int i = lane; i < nv; i += kWave) {
-      double z[QMAX + 1];
-      hist_load(i, z);
+    by_order([&](auto Q) {
+      rows([&](const int* id, bool, auto R) {
+        double z[R][QMAX + 1];
 #pragma unroll
-      for (int j = 1; j <= QMAX; ++j)
-        if (j <= q) zset(j, i, z[j] * fac[j]);
-    }
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int j = 1; j <= Q; ++j) z[r][j] = zget(j, id[r]);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int j = 1; j <= Q; ++j) zset(j, id[r], z[r][j] * fac[j]);
+      });
+    });
     h = hscale * eta;
     next_h = h;
     hscale = h;
@@ -264,22 +313,29 @@ struct CellCv {
   template <int SIGN>
   __device__ __forceinline__ double pascal() {
     double mn = 1.0e308;
-    for (int i = lane; i < nv; i += kWave) {
-      double z[QMAX + 1];
-      hist_load(i, z);
+    by_order([&](auto Q) {
+      rows([&](const int* id, bool, auto R) {
+        double z[R][QMAX + 1];
 #pragma unroll
-      for (int k = 1; k <= QMAX; ++k)
+        for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int j = QMAX; j >= k; --j)
-          if (j <= q) z[j - 1] = SIGN > 0 ? z[j - 1] + z[j] : z[j - 1] - z[j];
+          for (int j = 0; j <= Q; ++j) z[r][j] = zget(j, id[r]);
 #pragma unroll
-      for (int j = 0; j < QMAX; ++j)
-        if (j < q) zset(j, i, z[j]);
-      if (SIGN > 0) {
-        y[i] = z[0];
-        mn = fmin(mn, z[0]);
-      }
-    }
+        for (int r = 0; r < R; ++r) {
+#pragma unroll
+          for (int k = 1; k <= Q; ++k)
+#pragma unroll
+            for (int j = Q; j >= k; --j)
+              z[r][j - 1] = SIGN > 0 ? z[r][j - 1] + z[r][j] : z[r][j - 1] - z[r][j];
+#pragma unroll
+          for (int j = 0; j < Q; ++j) zset(j, id[r], z[r][j]);
+          if (SIGN > 0) {
+            y[id[r]] = z[r][0];
+            mn = fmin(mn, z[r][0]);
+          }
+        }
+      });
+    });
     wsync();
     return mn;
   }
@@ -501,10 +557,16 @@ struct CellCv {
   // (y holds the iterate), else the nonlinear solve's outcome.  m, del and
   // delp carry the iteration count and the last two correction norms.
   __device__ __forceinline__ int newton_pass(int& m, UDouble& delp) {
-    for (int i = lane; i < nv; i += kWave) {
-      double t = rl1 * zn1()[i] + acor[i];
-      tempv[i] = gamma * ftemp[i] - t;
-    }
+    rows([&](const int* id, bool, auto R) {
+      double t[R], fv[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        t[r] = rl1 * zn1()[id[r]] + acor[id[r]];
+        fv[r] = ftemp[id[r]];
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) tempv[id[r]] = gamma * fv[r] - t[r];
+    });
     wsync();
     lsolve(tempv);
     nni++;
@@ -512,16 +574,28 @@ struct CellCv {
     // of the new correction's norm in one pass over the rows (one round
     // trip for the error weights and zn[0] instead of two)
     double s_del = 0.0, s_acor = 0.0;
-    for (int i = lane; i < nv; i += kWave) {
-      double t = tempv[i], wt = ewt[i];
-      double p = t * wt;
-      s_del += p * p;
-      double a = acor[i] + t;
-      acor[i] = a;
-      y[i] = zn0()[i] + a;
-      double pa = a * wt;
-      s_acor += pa * pa;
-    }
+    rows([&](const int* id, bool two, auto R) {
+      double t[R], wt[R], a[R], z[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        t[r] = tempv[id[r]];
+        wt[r] = ewt[id[r]];
+        a[r] = acor[id[r]];
+        z[r] = zn0()[id[r]];
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        double p = t[r] * wt[r];
+        a[r] += t[r];
+        double pa = a[r] * wt[r];
+        if (r == 0 || two) {
+          s_del += p * p;
+          s_acor += pa * pa;
+        }
+        acor[id[r]] = a[r];
+        y[id[r]] = z[r] + a[r];
+      }
+    });
     double del = sqrt(wave_sum(s_del) / nv);
     wsync();
     if (m > 0) crate = fmax(CRDOWN * crate, del / delp);
@@ -608,28 +682,36 @@ struct CellCv {
     tau[1] = h;
     qwait--;
     bool save = (qwait == 1) && (q != QMAX);
-    double lj[QMAX + 1];
+    by_order([&](auto Q) {
+      double lj[Q + 1];
 #pragma unroll
-    for (int j = 0; j <= QMAX; ++j) lj[j] = j <= q ? l[j] : 0.0;
-    for (int i = lane; i < nv; i += kWave) {
-      double a = acor[i];
-      double z[QMAX + 1];
-      hist_load(i, z);
+      for (int j = 0; j <= Q; ++j) lj[j] = l[j];
+      rows([&](const int* id, bool, auto R) {
+        double z[R][QMAX + 1], a[R];
 #pragma unroll
-      for (int j = 0; j <= QMAX; ++j)
-        if (j <= q) z[j] += lj[j] * a;
-      // after a projection, components at TINY restart flat
-      if (projected && y[i] == 1.0e-60) {
-        z[0] = 1.0e-60;
+        for (int r = 0; r < R; ++r) {
+          a[r] = acor[id[r]];
 #pragma unroll
-        for (int j = 1; j <= QMAX; ++j) z[j] = 0.0;
-      }
+          for (int j = 0; j <= Q; ++j) z[r][j] = zget(j, id[r]);
+        }
 #pragma unroll
-      for (int j = 0; j <= QMAX; ++j)
-        if (j <= q) zset(j, i, z[j]);
-      if (save) znh(QMAX)[i] = a;
-      last[i] = z[0];
-    }
+        for (int r = 0; r < R; ++r) {
+          const int i = id[r];
+#pragma unroll
+          for (int j = 0; j <= Q; ++j) z[r][j] += lj[j] * a[r];
+          // after a projection, components at TINY restart flat
+          if (projected && y[i] == 1.0e-60) {
+            z[r][0] = 1.0e-60;
+#pragma unroll
+            for (int j = 1; j <= Q; ++j) z[r][j] = 0.0;
+          }
+#pragma unroll
+          for (int j = 0; j <= Q; ++j) zset(j, i, z[r][j]);
+          if (save) znh(QMAX)[i] = a[r];
+          last[i] = z[r][0];
+        }
+      });
+    });
     if (save) saved_tq5 = tq[5];
     wsync();
   }
