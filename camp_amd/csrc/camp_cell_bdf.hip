@@ -556,12 +556,16 @@ struct CellCv {
   // One Newton iteration up to the next f(y): NEWTON_F where it needs one
   // (y holds the iterate), else the nonlinear solve's outcome.  m, del and
   // delp carry the iteration count and the last two correction norms.
+  // (the first iteration starts from the guess, or zero)
+  __device__ __forceinline__ double correction(int m, int i) const {
+    return m > 0 ? acor[i] : use_acinit ? acinit[i] : 0.0;
+  }
   __device__ __forceinline__ int newton_pass(int& m, UDouble& delp) {
     rows([&](const int* id, bool, auto R) {
       double t[R], fv[R];
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        t[r] = rl1 * zn1()[id[r]] + acor[id[r]];
+        t[r] = rl1 * zn1()[id[r]] + correction(m, id[r]);
         fv[r] = ftemp[id[r]];
       }
 #pragma unroll
@@ -580,7 +584,7 @@ struct CellCv {
       for (int r = 0; r < R; ++r) {
         t[r] = tempv[id[r]];
         wt[r] = ewt[id[r]];
-        a[r] = acor[id[r]];
+        a[r] = correction(m, id[r]);
         z[r] = zn0()[id[r]];
       }
 #pragma unroll
@@ -1016,8 +1020,6 @@ struct CellCv {
           break;
         case ACT_NEWTON:
           if (m < 0) {
-            for (int i = lane; i < nv; i += kWave) acor[i] = use_acinit ? acinit[i] : 0.0;
-            wsync();
             m = 0;
             delp = 0.0;
           }
@@ -1061,8 +1063,6 @@ struct CellCv {
           complete_step();
           prepare_next_step(dsm);
           etamax = (nst <= SMALL_NST) ? ETAMX2 : ETAMX3;
-          for (int i = lane; i < nv; i += kWave) acor[i] *= tq[2];
-          wsync();
           nstloc++;
           act = ACT_MAIN;
           if (uc((tn - tout) * h >= 0.0)) {

@@ -757,13 +757,13 @@ __device__ __forceinline__ void cell_jac(const DevProgram& P, int lane, const do
 // elimination does on it, so the values are the same bit for bit -- and the
 // host packs the tasks into groups of 64 lanes, longest chain first, each at
 // least kLuDist groups after the values it reads are stored: a group's
-// operands are loaded while the one before it runs.  The last kLuTail pivots
-// are a dense block in registers (lane l holds rows 8 a + l / 8 and columns
+// operands are loaded while the one before it runs.  The last lu_d pivots
+// (up to kLuTail) are a dense block in registers (lane l holds rows 8 a + l / 8 and columns
 // 8 b + l % 8), a pivot's row and column going through LDS.
-// Cycles per factorisation: one CB05-scale cell 84k -> 55k (2000 cells 95k ->
-// 63k), one multi-phase cell 743k -> 339k (1024 cells 1.60M -> 0.57M); a third of
-// the gas one is tasks, the rest the register block (850 a pivot: an LDS round
-// trip, a division and 25 products).
+// Cycles per factorisation: one CB05-scale cell 84k -> 49k (2000 cells 95k ->
+// 55k), CB05cl_ae5 66k -> 21k, one multi-phase cell 743k -> 339k (1024 cells
+// 1.60M -> 0.57M); half of the gas one is tasks, the rest the register block (a
+// pivot: an LDS round trip, a division and up to 25 products, 350 to 850).
 // ---------------------------------------------------------------------
 struct LuGroup {
   int4 r, h;

@@ -615,15 +615,16 @@ static void build_tri_program(Program& P, const std::vector<char>& F,
 }
 
 // The factorisation's program (Program::lg_rec) of the filled pattern F with
-// value positions pos.
+// value positions row_major,
+// for a register block of the last `tail` pivots.
 static void build_lu_program(Program& P, const std::vector<char>& F,
-                             const std::vector<int>& row_major) {
+                             const std::vector<int>& row_major, int tail) {
   const int nv = P.nv, zero = P.lu_nnz + 64;
   // (the positions are those the solve reads: Program::lu_at)
   std::vector<int> pos = row_major;
   for (int& p : pos)
     if (p >= 0) p = P.lu_at[p];
-  const int d = P.lu_d = std::min(kLuTail, nv), s = nv - d;
+  const int d = P.lu_d = std::min(tail, nv), s = nv - d;
   struct Task {
     int i, j, waits = 0;
     std::vector<int> k;   // the pivots whose products it takes
@@ -1419,7 +1420,23 @@ std::string Model::initialize() {
   }
   if (P.lu_nnz + 64 > 65535) return "LU fill exceeds 65471 entries per cell";
   build_tri_program(P, F, pos);
-  build_lu_program(P, F, pos);
+  // The block's size by what a factorisation then costs: the tasks' groups
+  // (about 600 cycles each) against the block's pivots, whose cost grows with
+  // its size (350 to 850 cycles, measured).  CB05cl_ae5, two thirds of whose
+  // last 40 x 40 are zeros, takes 16 (42k -> 21k cycles), the CB05-scale
+  // mechanism 32 (55k -> 49k).  Large factors end in a dense block: all 40.
+  int best = kLuTail;
+  double best_cost = 0.0;
+  for (int d = 8; P.lu_nnz <= 4096 && d <= kLuTail; d += 8) {
+    build_lu_program(P, F, pos, d);
+    const double cost = 600.0 * P.lg_n + P.lu_d * (230.0 + 125.0 * (d / 8));
+    if (d == 8 || cost < best_cost) {
+      best = d;
+      best_cost = cost;
+    }
+    if (d >= nv) break;
+  }
+  build_lu_program(P, F, pos, best);
   initialized = true;
   // the f gather's final pass in slot order: {species, first partial, count}
   P.es_fin.clear();
