@@ -509,6 +509,8 @@ __device__ __forceinline__ void cell_deriv(const DevProgram& P, int lane, const 
                                            const double* s_slot = nullptr) {
   lane = phase_lane(lane);
   const int nv = P.nv, L = P.fb_rows;
+  // (no solver variables: the estimate's stream is empty, and ends nowhere)
+  use_est = use_est && nv > 0;
   const double* slot_or_rate = s_slot ? s_slot : s_rate;
   double jf = 0.0;
   if (use_est) {
@@ -901,6 +903,7 @@ __device__ __forceinline__ int cell_lu_factor(const DevProgram& P, int lane, con
     }
   }
   switch ((P.lu_d + 7) / 8) {
+    case 0: break;  // no solver variables
     case 1: bad |= lu_tail<1>(P, lane, lu, buf); break;
     case 2: bad |= lu_tail<2>(P, lane, lu, buf); break;
     case 3: bad |= lu_tail<3>(P, lane, lu, buf); break;

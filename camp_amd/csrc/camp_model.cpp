@@ -1439,8 +1439,9 @@ std::string Model::initialize() {
   build_lu_program(P, F, pos, best);
   initialized = true;
   // the f gather's final pass in slot order: {species, first partial, count}
+  // (at least one pass: f loads the first one ahead)
   P.es_fin.clear();
-  for (int slot = 0; slot < (nv + 63) / 64 * 64; ++slot) {
+  for (int slot = 0; slot < std::max((nv + 63) / 64, 1) * 64; ++slot) {
     const int i = slot < nv ? P.fs_species[slot] : -1;
     P.es_fin.insert(P.es_fin.end(), {i, i < 0 ? 0 : P.fb_fin[2 * i], i < 0 ? -1 : P.fb_fin[2 * i + 1], 0});
   }

@@ -1761,8 +1761,9 @@ static void eval_prepare(Solver* s, const double* state, const double* env, doub
   hipLaunchKernelGGL(camp::k_rates, dim3(camp::nblk((long)nc * s->m.n_rxn)), dim3(256), 0,
                      s->stream, P, nc, s->d_env, s->d_renv);
   // the solver variables, taken from the state as given (no clamping)
-  hipLaunchKernelGGL(camp::k_state_take, dim3(camp::nblk((long)nc * P.nv)), dim3(256), 0,
-                     s->stream, P, nc, s->d_state, d_y);
+  if (P.nv > 0)
+    hipLaunchKernelGGL(camp::k_state_take, dim3(camp::nblk((long)nc * P.nv)), dim3(256), 0,
+                       s->stream, P, nc, s->d_state, d_y);
 }
 
 extern "C" int camp_eval_deriv(void* solver_data, const double* state, const double* env,
