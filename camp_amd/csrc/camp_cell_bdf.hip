@@ -1336,10 +1336,6 @@ static const void* cell_bdf_fn(const DevProgram& P, int place) {
     default: return (const void*)k_cell_bdf<false, kPlaceLds>;
   }
 }
-static void allow_lds(const void* fn, size_t lds) {
-  if (lds > 65536)
-    (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-}
 
 void launch_cell_bdf(const CellBdfArgs& a, int grid, int block, size_t lds, hipStream_t s) {
   allow_lds(cell_bdf_fn(a.P, a.place), lds);
@@ -1373,7 +1369,7 @@ void launch_cell_bdf_bench(const CellBdfArgs& a, int grid, int block, size_t lds
 }
 
 int cell_bdf_blocks_per_cu(const DevProgram& P, int place, int block, size_t lds) {
-  if (block > 256 || lds > 160 * 1024) return 0;
+  if (block > 256 || lds > kMaxLds) return 0;
   const void* fn = cell_bdf_fn(P, place);
   allow_lds(fn, lds);
   int n = 0;

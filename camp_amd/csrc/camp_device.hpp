@@ -499,8 +499,9 @@ __device__ __forceinline__ void est_vals(const DevProgram& P, const double* Js, 
 // f_hist is formed (a stream of batches over the rows, y - y_hist once per
 // species in dy), and the precision-loss blend of time_derivative.c:58-64
 // gives f.  s_fb is LDS scratch of fb_lds_doubles, dy (use_est) of nv.
-// STAGED: Js is est_stage's copy of the history (Jf unused).
-template <bool STAGED>
+// STAGED: Js is est_stage's copy of the history (Jf unused).  DY: with dy; a
+// program whose dy does not fit LDS forms y - y_hist for every entry.
+template <bool STAGED, bool DY = true>
 __device__ __forceinline__ void cell_deriv(const DevProgram& P, int lane, const double* s_state,
                                            const double* s_rate, const double* y,
                                            const double* Js, const double* Jy,
@@ -517,7 +518,8 @@ __device__ __forceinline__ void cell_deriv(const DevProgram& P, int lane, const 
 #pragma unroll
     for (int u = 0; u < kEstAhead; ++u) est_vals<STAGED>(P, Js, F.B[u]);
     jf = STAGED ? Js[P.es_n + lane] : F.fin.x >= 0 ? Jf[F.fin.x] : 0.0;
-    for (int i = lane; i < nv; i += kWave) dy[i] = y[i] - Jy[i];
+    if (DY)
+      for (int i = lane; i < nv; i += kWave) dy[i] = y[i] - Jy[i];
   }
   {
     const int4* fr = P.fb_rec + lane;
@@ -593,7 +595,8 @@ __device__ __forceinline__ void cell_deriv(const DevProgram& P, int lane, const 
 #pragma unroll
       for (int q = 0; q < kEstBatch; ++q) {
         const int col = q % 2 ? (unsigned)cw[q / 2] >> 16 : cw[q / 2] & 0xFFFF;
-        d[q] = dy[col == 0xFFFF ? 0 : col];
+        const int at = col == 0xFFFF ? 0 : col;
+        d[q] = DY ? dy[at] : y[at] - Jy[at];
       }
       __builtin_amdgcn_sched_barrier(0);  // (the loads ahead of their uses)
 #pragma unroll

@@ -56,6 +56,7 @@ __global__ void __launch_bounds__(256) k_deriv(DevProgram P, int nc, const doubl
   double* s_rate = s_mp + mp_lds_doubles(P);
   MpLds L = mp_lds(P, s_mp, s_rate + 2 * (size_t)P.n_terms);
   double* s_fb = s_rate + 2 * (size_t)P.n_terms + mp_jsc_doubles(P);
+  double* s_dy = fj_dy(P) ? smem + (size_t)wv * fj_lds_doubles(P) + fj_lds_doubles_no_dy(P) : nullptr;
   for (int c = blockIdx.x * wpb + wv; c < nc; c += gridDim.x * wpb) {
     stage_cell(P, lane, state + (size_t)c * P.ns, rxn_env + (size_t)c * P.n_env, s_state, s_k);
     const double* yc = y + (size_t)c * P.nv;
@@ -72,9 +73,16 @@ __global__ void __launch_bounds__(256) k_deriv(DevProgram P, int nc, const doubl
     f_load_gather(P, lane, F);
     cell_rates(P, lane, s_state, s_k, s_rate, F);
     wsync();
-    cell_deriv<false>(P, lane, s_state, s_rate, yc, Js + (size_t)c * P.nnz, Jy + (size_t)c * P.nv,
-                      Jf + (size_t)c * P.nv, use_est != 0, h, fout + (size_t)c * P.nv, s_fb,
-                      s_fb + fb_lds_doubles(P), F, P.mp ? L.slot : nullptr);
+    const double *Jsc = Js + (size_t)c * P.nnz, *Jyc = Jy + (size_t)c * P.nv,
+                 *Jfc = Jf + (size_t)c * P.nv;
+    double* fc = fout + (size_t)c * P.nv;
+    const double* slot = P.mp ? L.slot : nullptr;
+    if (s_dy)
+      cell_deriv<false>(P, lane, s_state, s_rate, yc, Jsc, Jyc, Jfc, use_est != 0, h, fc, s_fb,
+                        s_dy, F, slot);
+    else
+      cell_deriv<false, false>(P, lane, s_state, s_rate, yc, Jsc, Jyc, Jfc, use_est != 0, h, fc,
+                               s_fb, nullptr, F, slot);
     wsync();
   }
 }
@@ -374,9 +382,7 @@ static void launch_group_fj(bool jac, const DevProgram& P, int nc, const double*
   blocks = blocks < 1 ? 1 : blocks > (1 << 22) ? (1 << 22) : blocks;
   if (jac) {
     const size_t lds = group_jac_lds_bytes(P, G);
-    if (lds > 65536)
-      (void)hipFuncSetAttribute((const void*)k_jac_g<G>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    allow_lds((const void*)k_jac_g<G>, lds);
     hipLaunchKernelGGL((k_jac_g<G>), dim3(blocks), dim3(kWave), lds, st, P, nc, y, state, kval,
                        out, h);
   } else if (use_est) {
@@ -718,7 +724,7 @@ __global__ void k_scatter_rates(int n_cells, int n_upd, const int* upd_off, cons
 // at the smallest steps the rounding error admits almost any value, so the
 // best quotient is used instead.)  One wavefront per cell; cell_fails[c] =
 // failing elements (-1: f() failed at y).  LDS per wavefront:
-// fj_lds_doubles(P) + 4 nv + 2 nnz.
+// fj_lds_doubles_no_dy(P) + 4 nv + 2 nnz.
 // ---------------------------------------------------------------------
 __device__ __forceinline__ int fd_f(const DevProgram& P, int lane, const double* yp, double* s_state,
                                    double* s_k, MpLds& L, double* s_rate, double* s_fb,
@@ -750,7 +756,7 @@ __global__ void __launch_bounds__(64) k_check_jac(DevProgram P, int nc, const do
   double* s_rate = s_mp + mp_lds_doubles(P);
   MpLds L = mp_lds(P, s_mp, s_rate + 2 * (size_t)P.n_terms);
   double* s_fb = s_rate + 2 * (size_t)P.n_terms + mp_jsc_doubles(P);
-  double* f0 = smem + fj_lds_doubles(P);
+  double* f0 = smem + fj_lds_doubles_no_dy(P);
   double* f1 = f0 + P.nv;
   double* f2 = f1 + P.nv;
   double* yp = f2 + P.nv;

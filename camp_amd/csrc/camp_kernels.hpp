@@ -11,6 +11,16 @@
 namespace camp {
 
 constexpr int kCellStats = 10;  // nst nfe nsetups netf nni ncfn nje flag hu next_h
+
+// LDS of a CU.  A kernel opts into more than 64 KiB a block once and for all
+// (the limit belongs to the function, which solvers and threads share: set to
+// each launch's own size it would lower another's).
+constexpr size_t kMaxLds = 160 * 1024;
+inline void allow_lds(const void* fn, size_t lds) {
+  if (lds > 65536 && lds <= kMaxLds)
+    (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds);
+}
+
 // shader cycles per cell: f, Jac, LU factor, LU solve, whole solve, and the
 // two parts of f (state update + rates, species gather + estimate blend)
 constexpr int kCellProf = 7;
@@ -134,13 +144,25 @@ __global__ void k_deriv(DevProgram P, int nc, const double* y, const double* sta
 // Jr: reaction-Jacobian scratch [nc][rnnz] of multi-phase programs (else unused)
 __global__ void k_jac(DevProgram P, int nc, const double* y, const double* state,
                       const double* env, const double* rxn_env, double* J, double h, double* Jr);
-// LDS doubles per wavefront of k_deriv and k_jac, and wavefronts per block
-// (one for multi-phase programs, whose per-cell extras are large)
-__host__ __device__ inline size_t fj_lds_doubles(const DevProgram& P) {
+// LDS doubles per wavefront of k_deriv and k_jac (the estimate's dy last, where
+// it fits; without: k_check_jac, whose f takes no estimate), and wavefronts per
+// block: one for multi-phase programs, whose per-cell extras are large, else up
+// to four, as many as fit.
+__host__ __device__ inline size_t fj_lds_doubles_no_dy(const DevProgram& P) {
   return even_up((size_t)P.ns + P.n_env) + mp_lds_doubles(P) +
-         even_up(2 * (size_t)P.n_terms + mp_jsc_doubles(P) + fb_lds_doubles(P) + P.nv);
+         even_up(2 * (size_t)P.n_terms + mp_jsc_doubles(P) + fb_lds_doubles(P));
 }
-inline int fj_waves_per_block(const DevProgram& P) { return P.mp ? 1 : 4; }
+__host__ __device__ inline bool fj_dy(const DevProgram& P) {
+  return (fj_lds_doubles_no_dy(P) + even_up(P.nv)) * sizeof(double) <= kMaxLds;
+}
+__host__ __device__ inline size_t fj_lds_doubles(const DevProgram& P) {
+  return fj_lds_doubles_no_dy(P) + (fj_dy(P) ? even_up(P.nv) : 0);
+}
+inline int fj_waves_per_block(const DevProgram& P) {
+  int w = P.mp ? 1 : 4;
+  while (w > 1 && w * fj_lds_doubles(P) * sizeof(double) > kMaxLds) w /= 2;
+  return w;
+}
 
 // Lane-group f(y) and J(y) of gas-phase programs (lanes per cell = 8, 16
 // or 32; camp_kernels.hip) and the compact rate-constant array they read.
@@ -207,7 +229,7 @@ __global__ void k_check_jac(DevProgram P, int nc, const double* y, const double*
                             const double* env, const double* rxn_env, const double* J, double h_ts,
                             int* cell_fails);
 inline size_t check_jac_lds_doubles(const DevProgram& P) {
-  return fj_lds_doubles(P) + 4 * (size_t)P.nv + 2 * (size_t)P.nnz;
+  return fj_lds_doubles_no_dy(P) + 4 * (size_t)P.nv + 2 * (size_t)P.nnz;
 }
 // renv[c][upd_off[u]] = rates[c][u] for c < n_cells, u < n_upd
 __global__ void k_scatter_rates(int n_cells, int n_upd, const int* upd_off, const double* rates,

@@ -193,14 +193,6 @@ void Solver::setup_device() {
     P.jm_param = dev_upload(G.jm_param, owned);
   }
 
-  // beyond 64 KiB of LDS per block is opted into per kernel
-  const size_t fj_lds = fj_waves_per_block(P) * fj_lds_doubles(P) * sizeof(double);
-  if (fj_lds > 65536) {
-    (void)hipFuncSetAttribute((const void*)k_deriv, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)fj_lds);
-    (void)hipFuncSetAttribute((const void*)k_jac, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)fj_lds);
-  }
   size_t nc = m.nc;
   d_state = dev_alloc<double>(nc * G.ns, owned);
   d_env = dev_alloc<double>(nc * 2, owned);
@@ -234,29 +226,41 @@ void Solver::refresh_kval() {
 
 void Solver::launch_deriv(const double* y, const double* st, const double* env, double* out,
                           double h, int use_est, int* fail) {
-  int nc = m.nc;
   if (!P.mp) {
-    launch_group_deriv(f_lanes, P, nc, y, st, kval(), d_Js, d_Jy, d_Jf, out, h, nullptr, use_est,
+    launch_group_deriv(f_lanes, P, m.nc, y, st, kval(), d_Js, d_Jy, d_Jf, out, h, nullptr, use_est,
                        fail, stream);
     return;
   }
-  int wpb = fj_waves_per_block(P);
+  launch_wave_deriv(y, st, env, out, h, use_est, fail);
+}
+
+void Solver::launch_wave_deriv(const double* y, const double* st, const double* env, double* out,
+                               double h, int use_est, int* fail) {
+  int nc = m.nc, wpb = fj_waves_per_block(P);
   size_t lds = wpb * fj_lds_doubles(P) * sizeof(double);
+  allow_lds((const void*)k_deriv, lds);
   hipLaunchKernelGGL(k_deriv, dim3(std::min(nblk(nc, wpb), 4096)), dim3(64 * wpb), lds, stream, P,
                      nc, y, st, env, d_renv, d_Js, d_Jy, d_Jf, out, h, use_est, fail);
+  HIP_OK(hipGetLastError());
 }
 
 void Solver::launch_jac(const double* y, const double* st, const double* env, double* J, double h,
                         double* jr) {
-  int nc = m.nc;
   if (!P.mp) {
-    launch_group_jac(j_lanes, P, nc, y, st, kval(), J, h, stream);
+    launch_group_jac(j_lanes, P, m.nc, y, st, kval(), J, h, stream);
     return;
   }
-  int wpb = fj_waves_per_block(P);
+  launch_wave_jac(y, st, env, J, h, jr);
+}
+
+void Solver::launch_wave_jac(const double* y, const double* st, const double* env, double* J,
+                             double h, double* jr) {
+  int nc = m.nc, wpb = fj_waves_per_block(P);
   size_t lds = wpb * fj_lds_doubles(P) * sizeof(double);
+  allow_lds((const void*)k_jac, lds);
   hipLaunchKernelGGL(k_jac, dim3(std::min(nblk(nc, wpb), 4096)), dim3(64 * wpb), lds, stream, P,
                      nc, y, st, env, d_renv, J, h, jr);
+  HIP_OK(hipGetLastError());
 }
 
 int Solver::run(double* st, double* env, double t0, double t1) {
@@ -1782,11 +1786,7 @@ extern "C" int camp_eval_deriv(void* solver_data, const double* state, const dou
     s->refresh_kval();
     s->launch_deriv(d_y, s->d_state, s->d_env, d_f, time_step, use_deriv_est, s->d_fail);
   } else {
-    int wpb = camp::fj_waves_per_block(P);
-    size_t lds = wpb * camp::fj_lds_doubles(P) * sizeof(double);
-    hipLaunchKernelGGL(camp::k_deriv, dim3(std::min(camp::nblk(nc, wpb), 4096)), dim3(64 * wpb),
-                       lds, s->stream, P, nc, d_y, s->d_state, s->d_env, s->d_renv, s->d_Js,
-                       s->d_Jy, s->d_Jf, d_f, time_step, use_deriv_est, s->d_fail);
+    s->launch_wave_deriv(d_y, s->d_state, s->d_env, d_f, time_step, use_deriv_est, s->d_fail);
   }
   int fail = 0;
   HIP_OK(hipMemcpyAsync(&fail, s->d_fail, sizeof(int), hipMemcpyDeviceToHost, s->stream));
@@ -1806,19 +1806,13 @@ extern "C" int camp_eval_jac(void* solver_data, const double* state, const doubl
   double* d_y = s->kept(s->d_eval_y, (size_t)nc * P.nv);
   eval_prepare(s, state, env, d_y);
   HIP_OK(hipMemsetAsync(s->d_fail, 0, sizeof(int), s->stream));
-  int wpb = camp::fj_waves_per_block(P);
-  size_t lds = wpb * camp::fj_lds_doubles(P) * sizeof(double);
   double* d_jr = P.mp ? camp::dev_alloc<double>((size_t)nc * P.rnnz, tmp) : nullptr;
-  hipLaunchKernelGGL(camp::k_deriv, dim3(std::min(camp::nblk(nc, wpb), 4096)), dim3(64 * wpb), lds,
-                     s->stream, P, nc, d_y, s->d_state, s->d_env, s->d_renv, s->d_Js, s->d_Jy,
-                     s->d_Jf, s->d_Jf, time_step, 0, s->d_fail);
+  s->launch_wave_deriv(d_y, s->d_state, s->d_env, s->d_Jf, time_step, 0, s->d_fail);
   if (s->eval_group && !P.mp) {
     s->refresh_kval();
     s->launch_jac(d_y, s->d_state, s->d_env, s->d_Js, time_step, nullptr);
   } else {
-    hipLaunchKernelGGL(camp::k_jac, dim3(std::min(camp::nblk(nc, wpb), 4096)), dim3(64 * wpb),
-                       lds, s->stream, P, nc, d_y, s->d_state, s->d_env, s->d_renv, s->d_Js,
-                       time_step, d_jr);
+    s->launch_wave_jac(d_y, s->d_state, s->d_env, s->d_Js, time_step, d_jr);
   }
   HIP_OK(hipMemcpyAsync(s->d_Jy, d_y, (size_t)nc * P.nv * sizeof(double), hipMemcpyDeviceToDevice,
                         s->stream));
@@ -1838,9 +1832,7 @@ void check_jac_device(Solver* s, const double* d_y, const double* d_state, const
                       const double* d_J, double time_step, int* d_fails) {
   const DevProgram& P = s->P;
   size_t lds = check_jac_lds_doubles(P) * sizeof(double);
-  if (lds > 65536)
-    (void)hipFuncSetAttribute((const void*)k_check_jac,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  allow_lds((const void*)k_check_jac, lds);
   hipLaunchKernelGGL(k_check_jac, dim3(std::min(s->m.nc, 16384)), dim3(64), lds, s->stream, P,
                      s->m.nc, d_y, d_state, d_env, s->d_renv, d_J, time_step, d_fails);
   HIP_OK(hipGetLastError());

@@ -126,6 +126,11 @@ struct Solver {
                     int use_est, int* fail);
   void launch_jac(const double* y, const double* st, const double* env, double* J, double h,
                   double* jr);
+  // the same with one wavefront per cell (the per-cell kernel's code)
+  void launch_wave_deriv(const double* y, const double* st, const double* env, double* out,
+                         double h, int use_est, int* fail);
+  void launch_wave_jac(const double* y, const double* st, const double* env, double* J, double h,
+                       double* jr);
   std::vector<double> h_red;
   BlockStats bstats;
   bool stats_from_cells = false;

@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from camp_amd.core import CampSolver
-from camp_amd.mechanisms import box_mechanism, synthetic_cells
+from camp_amd.mechanisms import Mechanism, Reaction, box_mechanism, synthetic_cells
 
 pytestmark = pytest.mark.gpu
 
@@ -28,3 +28,62 @@ def test_no_solver_variables(oracle_lib):
     a, b = cells.state.copy(), cells.state.copy()
     assert gpu.solve(a, cells.env, 0.0, 60.0) == ref.run(b, cells.env, 0.0, 60.0, mode=1)
     assert np.array_equal(a, b)
+
+
+def ring_mechanism(n):
+    """n species, each turning into the next at 1e-3 / s: a sparse Jacobian
+    whose factors fill little, so that vectors, not factors, take the LDS."""
+    rx = [Reaction("ARRHENIUS", [i], [((i + 1) % n, 1.0)], {"A": 1.0e-3}) for i in range(n)]
+    return Mechanism(["S%d" % i for i in range(n)], [1] * n, [1.0e-10] * n, rx, rel_tol=1.0e-6)
+
+
+def ring_solution(y0, t):
+    """The ring's exact solution: its modes are Fourier modes."""
+    n = y0.shape[1]
+    w = np.exp(-2j * np.pi * np.arange(n) / n) - 1.0
+    return np.fft.ifft(np.fft.fft(y0, axis=1) * np.exp(1.0e-3 * t * w), axis=1).real
+
+
+ENV = np.array([298.0, 101325.0])
+
+
+@pytest.mark.parametrize("n", [720, 1300])
+def test_layers_of_a_wide_mechanism(n):
+    """Four cells of 720 species, or two of 1300, are more than a CU's LDS: f
+    and J run with fewer wavefronts a block (the rates are 1e-3 y to rounding),
+    also after a small solver has launched the same kernels, and the step does
+    not see an error that the layers' set-up left behind.  The step is not
+    stiff: an error per step of 1e-6 of the solution over at most some hundred
+    steps stays under 1e-3."""
+    n_cells = 3
+    gpu = CampSolver(ring_mechanism(n), n_cells)
+    env = np.tile(ENV, (n_cells, 1))
+    y0 = np.random.default_rng(3).uniform(1.0, 2.0, (n_cells, n))
+    small = CampSolver(ring_mechanism(100), n_cells)
+    assert small.eval_deriv(y0[:, :100], env)[0] == 0
+    want = 1.0e-3 * (np.roll(y0, 1, axis=1) - y0)
+    for est in (False, True):
+        rc, f = gpu.eval_deriv(y0, env, 1.0, est)
+        assert rc == 0 and np.allclose(f, want, rtol=1e-12, atol=1e-15)
+        rc, jac = gpu.eval_jac(y0, env, 1.0)
+        assert rc == 0 and np.allclose(np.abs(jac), 1.0e-3, rtol=1e-12, atol=0.0)
+    y = y0.copy()
+    assert gpu.solve(y, env, 0.0, 60.0) == 0
+    assert np.allclose(y, ring_solution(y0, 60.0), rtol=1e-3, atol=0.0)
+
+
+def test_layers_where_the_estimate_has_no_scratch():
+    """400 species in a ring of 6300 reactions: f's own LDS fits a CU, its
+    vector y - y_hist does not and is formed entry by entry."""
+    n, n_rxn, n_cells = 400, 6300, 2
+    rx = [Reaction("ARRHENIUS", [r % n], [((r + 1) % n, 1.0)], {"A": 2.0 ** -14})
+          for r in range(n_rxn)]
+    mech = Mechanism(["S%d" % i for i in range(n)], [1] * n, [1.0e-10] * n, rx, rel_tol=1.0e-6)
+    gpu = CampSolver(mech, n_cells)
+    env = np.tile(ENV, (n_cells, 1))
+    y0 = np.random.default_rng(4).uniform(1.0, 2.0, (n_cells, n))
+    rate = y0 * np.bincount(np.arange(n_rxn) % n) * 2.0 ** -14
+    want = np.roll(rate, 1, axis=1) - rate
+    assert gpu.eval_jac(y0, env, 1.0)[0] == 0
+    rc, f = gpu.eval_deriv(y0, env, 1.0, True)
+    assert rc == 0 and np.allclose(f, want, rtol=1e-12, atol=1e-15)
