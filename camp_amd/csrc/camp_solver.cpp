@@ -309,26 +309,9 @@ void Solver::cell_launch_shape(long nq, int* grid, int* block, size_t* lds, int 
   *grid = (int)std::max<long>(1, std::min<long>((long)per_cu * ncu, (nq + cpb - 1) / cpb));
 }
 
-// The placement of a launch of n cells.  With the LU in global memory a
-// CB05-scale cell needs 13 KB of LDS instead of 26 and eight cells share a CU
-// instead of six, but a cell alone is slower: a step of 777 cells takes 16.9
-// instead of 16.0 ms, of 3000 19.3 instead of 17.4, of 10000 36.4 instead of
-// 38.0, of 100000 337 instead of 357.  So it is taken where it holds more cells
-// and the launch is at least four times what it holds.
-int Solver::run_place(long n) const {
-  if (!place_auto || P.mp || n < 4096) return place;
-  int g1 = 0, g2 = 0, block = 0;
-  size_t lds = 0;
-  cell_launch_shape(1L << 30, &g1, &block, &lds, place);
-  cell_launch_shape(1L << 30, &g2, &block, &lds, kPlaceGlobalLu);
-  return g2 > g1 && n >= 4L * g2 * (block / kWave) ? kPlaceGlobalLu : place;
-}
-
 int Solver::run_cells(double* st, double* env, double t0, double t1, double* noalloc,
                       size_t noalloc_doubles) {
   CellBdfArgs a = cell_args();
-  const int place = noalloc ? this->place : run_place(m.nc);
-  a.place = cell_placement(P, place);
   a.nc = m.nc;
   a.state = st;
   a.env = env;
@@ -348,7 +331,7 @@ int Solver::run_cells(double* st, double* env, double t0, double t1, double* noa
   }
   int grid = 0, block = 0;
   size_t lds = 0;
-  cell_launch_shape(m.nc, &grid, &block, &lds, place);
+  cell_launch_shape(m.nc, &grid, &block, &lds);
   int dev = 0;
   HIP_OK(hipGetDevice(&dev));
   if (noalloc) {
@@ -1487,10 +1470,7 @@ extern "C" long camp_solver_cell_lds_bytes(void* solver_data, int place) {
 extern "C" int camp_solver_set_placement(void* solver_data, int place) {
   using namespace camp;
   Solver* s = SD(solver_data);
-  if (place >= 0 && place < kNumPlacements) {
-    s->place = place;
-    s->place_auto = false;
-  }
+  if (place >= 0 && place < kNumPlacements) s->place = place;
   return cell_placement(s->P, s->place);
 }
 
@@ -1606,7 +1586,6 @@ extern "C" int camp_solver_autotune(void* solver_data, const double* d_state,
   for (void* p : tmp) HIP_OK(hipFree(p));
   s->cells_per_block = best;
   s->place = best_place;
-  s->place_auto = false;
   return best + 100 * best_place;
 }
 

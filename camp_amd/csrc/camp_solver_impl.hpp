@@ -60,13 +60,14 @@ struct Solver {
   Model m;
   int mode = CAMP_MODE_PER_CELL;
   int cells_per_block = 1;
-  // per-cell kernel variant (cell_placement): history in global memory, the
-  // fastest for the CB05-scale mechanism (six cells per CU instead of four)
+  // per-cell kernel variant (cell_placement) until the caller or the autotuner
+  // chooses.  A CB05-scale CU holds six cells with kPlaceGlobal and eight with
+  // kPlaceGlobalLu, whose factorisation and solves are slower; one 180 s step
+  // in ms, kPlaceGlobal / kPlaceGlobalLu: 16384 cells spun up for five steps
+  // 17.3 / 19.1, as they start 313 / 312, relaxed and disturbed by 3 % 57.3 /
+  // 57.0; 60000 cells 48.1 / 48.5, 1115 / 1118, 205 / 202; 60000 CB05cl_ae5
+  // cells (6 s) 11.6 / 12.1.  No size or state tried gains more than 2 %.
   int place = kPlaceGlobal;
-  // until the caller or the autotuner chooses: run_place picks by the number
-  // of cells of a launch
-  bool place_auto = true;
-  int run_place(long n) const;
   int guess_on = 1;
   bool renv_dirty = true;
   hipStream_t stream = nullptr;

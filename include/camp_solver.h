@@ -206,10 +206,8 @@ int camp_solver_set_cells_per_block(void *solver_data, int cells_per_block);
  * unit), 1 = the higher Nordsieck vectors, the rate constants and the J
  * history in global memory (two wavefronts per SIMD), 2 = the LU factors, the
  * rate constants and the J history in global memory (most cells per compute
- * unit).  Until it is set (or autotuned) each launch takes 1, or 2 where 2
- * holds more cells at once and the launch has at least four times as many.
- * Returns the placement set (1 by default; a negative place only asks).
- * Results do not depend on it. */
+ * unit).  Returns the placement in effect (1 by default; a negative place
+ * only asks).  Results do not depend on it. */
 int camp_solver_set_placement(void *solver_data, int place);
 
 /* LDS bytes one cell of the per-cell kernel uses with the given placement

@@ -87,3 +87,15 @@ def test_layers_where_the_estimate_has_no_scratch():
     assert gpu.eval_jac(y0, env, 1.0)[0] == 0
     rc, f = gpu.eval_deriv(y0, env, 1.0, True)
     assert rc == 0 and np.allclose(f, want, rtol=1e-12, atol=1e-15)
+
+
+def test_large_launch_of_a_wide_mechanism():
+    """1300 species: the default placement fits a CU's LDS, the placement with
+    the factors in global memory (and all vectors in LDS) does not.  A launch
+    of many cells runs all the same (tolerance as above)."""
+    n, n_cells = 1300, 4100
+    gpu = CampSolver(ring_mechanism(n), n_cells)
+    y0 = np.tile(np.random.default_rng(3).uniform(1.0, 2.0, (4, n)), (n_cells // 4, 1))
+    y = y0.copy()
+    assert gpu.solve(y, np.tile(ENV, (n_cells, 1)), 0.0, 60.0) == 0
+    assert np.allclose(y, ring_solution(y0, 60.0), rtol=1e-3, atol=0.0)
