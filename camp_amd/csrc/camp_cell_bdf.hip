@@ -80,7 +80,7 @@ struct UDouble {
 
 // MP selects the multi-phase instantiation: gas-phase programs run a kernel
 // without the aerosol code (smaller code and register footprint).  PL: the
-// placement.  KG: the rate constants are read in place in global memory (s_k)
+// variant.  KG: the rate constants are read in place in global memory (s_k)
 // and, for the f terms, held by the lanes (kt).  GH: the J history lives in
 // global memory, with a copy in f's order in the wavefront's scratch (E).
 template <bool MP, int PL>
@@ -228,7 +228,7 @@ struct CellCv {
       long long t1 = tick();
       if (prof && est) c_fr += t1 - t0;
       cell_deriv<GH>(P, lane, s_state, s_rate, y, GH ? E : Js, Jy, Jf, est, ts, ftemp, s_fb,
-                     KG ? tempv : w, F, MP ? mpl.slot : nullptr);
+                     KG && PL != kPlaceWide ? tempv : w, F, MP ? mpl.slot : nullptr);
       wsync();
       if (prof && est) c_fg += clock64() - t1;
     }
@@ -248,7 +248,7 @@ struct CellCv {
       cell_jac_mp(P, lane, s_state, s_k, ts, mpl, Jr, Js);
     } else {
       const double* k = s_k;
-      if (KG && PL != kPlaceGlobalLu) {
+      if (!MP && PL == kPlaceGlobal) {
         // J reads its constants at random: staged where the LU goes next
         for (int i = lane; i < P.n_env; i += kWave) lu[i] = s_k[i];
         wsync();
@@ -520,7 +520,7 @@ struct CellCv {
   __device__ __forceinline__ void lsolve(double* b) {
     const DevProgram& P = program();
     long long t0 = tick();
-    cell_lu_solve<MP || PL == kPlaceGlobalLu>(P, lane, lu, b, w);
+    cell_lu_solve<MP || PL == kPlaceGlobalLu || PL == kPlaceWide>(P, lane, lu, b, w);
     if (prof) c_sol += clock64() - t0;
     if (uc(gamrat != 1.0)) {
       double s = 2.0 / (1.0 + gamrat);
@@ -1094,21 +1094,18 @@ struct CellCv {
 
 }  // namespace
 
-// MP: multi-phase program; PL: the placement (kPlaceLds, kPlaceGlobal:
-// the Nordsieck history, 5 of the 8 work vectors and the J history in
-// global memory, kPlaceGlobalLu: the LU factors as well; multi-phase
-// programs run kPlaceGlobal with global LU factors).  Each variant is
-// compiled for the wavefronts per SIMD its LDS footprint lets onto a CU
-// (1, 2 and 3 for the CB05-scale mechanism), which bounds its registers.
+// MP: multi-phase program (PL then kPlaceGlobal); PL: the variant (see
+// kPlaceLds and following).  Each is compiled for the wavefronts per SIMD its
+// LDS footprint lets onto a CU (one or two), which bounds its registers.
 // BENCH: the measurement variant (bench_phases instead of the solve).
 template <bool MP, int PL, bool BENCH = false>
 __global__ void __launch_bounds__(256)
-    __attribute__((amdgpu_waves_per_eu(MP || PL == kPlaceLds ? 1 : 2)))
+    __attribute__((amdgpu_waves_per_eu(MP || PL == kPlaceLds || PL == kPlaceWide ? 1 : 2)))
     k_cell_bdf(CellBdfArgs a) {
   extern __shared__ double smem[];
   const DevProgram& P = a.P;
   constexpr bool GH = MP || PL != kPlaceLds;
-  constexpr bool GL = MP || PL == kPlaceGlobalLu;
+  constexpr bool GL = MP || PL == kPlaceGlobalLu || PL == kPlaceWide;
   constexpr int kPlace = MP ? kPlaceGlobal : PL;
   // the wavefront index is uniform: a scalar, so the cell's LDS and scratch
   // pointers derived from it live in scalar registers
@@ -1123,10 +1120,10 @@ __global__ void __launch_bounds__(256)
   cv.lane = lane;
   cv.nv = nv;
   cv.s_state = base;
-  constexpr bool kNewtonLds = GH && !MP;
-  // (kNewtonLds: no rate constants in LDS, see CellCv::kt)
+  constexpr bool kConstLds = MP || !GH;  // (else see CellCv::kt)
+  constexpr bool kNewtonLds = GH && !MP && PL != kPlaceWide;
   double* sk_end = cv.s_state + P.ns;
-  if (!kNewtonLds) {
+  if (kConstLds) {
     cv.s_k = sk_end;
     sk_end += P.n_env;
   }
@@ -1158,8 +1155,8 @@ __global__ void __launch_bounds__(256)
     cv.tempv = vh; vh += nv;
     cv.ftemp = vh; vh += nv;
   }
-  // (where the LU is global there is room in LDS for all of the history)
-  double*& v2 = !MP && GL ? v : vh;
+  // (kPlaceGlobalLu has room in LDS for all of the history)
+  double*& v2 = !MP && PL == kPlaceGlobalLu ? v : vh;
   cv.z2 = v2; v2 += 4 * (size_t)nv;
   cv.last = v2; v2 += nv;
   cv.acinit = v2; v2 += nv;
@@ -1256,7 +1253,7 @@ __global__ void __launch_bounds__(256)
           state_c[i] = s;
         }
       }
-      if (kNewtonLds)
+      if (!kConstLds)
         cv.s_k = renv_c;
       else
         for (int i = lane; i < P.n_env; i += kWave) cv.s_k[i] = renv_c[i];
@@ -1266,7 +1263,7 @@ __global__ void __launch_bounds__(256)
       cell_rate_constants(P, lane, T, Pa, cv.s_k);
       wsync();
       if (MP) mp_cell_env(P, lane, T, Pa, cv.mpl);
-      if (kNewtonLds) {
+      if (!kConstLds) {
         __threadfence_block();
         cv.load_term_constants();
       } else {
@@ -1330,9 +1327,10 @@ __global__ void __launch_bounds__(256)
 // cells per workgroup) is opted into per kernel; gfx950 has 160 KiB per CU.
 static const void* cell_bdf_fn(const DevProgram& P, int place) {
   if (P.mp) return (const void*)k_cell_bdf<true, kPlaceGlobal>;
-  switch (cell_placement(P, place)) {
+  switch (place) {
     case kPlaceGlobal: return (const void*)k_cell_bdf<false, kPlaceGlobal>;
     case kPlaceGlobalLu: return (const void*)k_cell_bdf<false, kPlaceGlobalLu>;
+    case kPlaceWide: return (const void*)k_cell_bdf<false, kPlaceWide>;
     default: return (const void*)k_cell_bdf<false, kPlaceLds>;
   }
 }
@@ -1341,10 +1339,12 @@ void launch_cell_bdf(const CellBdfArgs& a, int grid, int block, size_t lds, hipS
   allow_lds(cell_bdf_fn(a.P, a.place), lds);
   if (a.P.mp)
     hipLaunchKernelGGL((k_cell_bdf<true, kPlaceGlobal>), dim3(grid), dim3(block), lds, s, a);
-  else if (cell_placement(a.P, a.place) == kPlaceGlobal)
+  else if (a.place == kPlaceGlobal)
     hipLaunchKernelGGL((k_cell_bdf<false, kPlaceGlobal>), dim3(grid), dim3(block), lds, s, a);
-  else if (cell_placement(a.P, a.place) == kPlaceGlobalLu)
+  else if (a.place == kPlaceGlobalLu)
     hipLaunchKernelGGL((k_cell_bdf<false, kPlaceGlobalLu>), dim3(grid), dim3(block), lds, s, a);
+  else if (a.place == kPlaceWide)
+    hipLaunchKernelGGL((k_cell_bdf<false, kPlaceWide>), dim3(grid), dim3(block), lds, s, a);
   else
     hipLaunchKernelGGL((k_cell_bdf<false, kPlaceLds>), dim3(grid), dim3(block), lds, s, a);
 }
@@ -1356,11 +1356,11 @@ void launch_cell_bdf_bench(const CellBdfArgs& a, int grid, int block, size_t lds
     allow_lds((const void*)k_cell_bdf<true, kPlaceGlobal, true>, lds);
     hipLaunchKernelGGL((k_cell_bdf<true, kPlaceGlobal, true>), dim3(grid), dim3(block), lds, s,
                        a);
-  } else if (cell_placement(a.P, a.place) == kPlaceGlobal) {
+  } else if (a.place == kPlaceGlobal) {
     allow_lds((const void*)k_cell_bdf<false, kPlaceGlobal, true>, lds);
     hipLaunchKernelGGL((k_cell_bdf<false, kPlaceGlobal, true>), dim3(grid), dim3(block), lds, s,
                        a);
-  } else if (cell_placement(a.P, a.place) == kPlaceLds) {
+  } else if (a.place == kPlaceLds) {
     allow_lds((const void*)k_cell_bdf<false, kPlaceLds, true>, lds);
     hipLaunchKernelGGL((k_cell_bdf<false, kPlaceLds, true>), dim3(grid), dim3(block), lds, s, a);
   } else {
@@ -1431,7 +1431,7 @@ extern "C" int camp_solver_run_device_noalloc(void* solver_data, double* d_state
                          "timing or the Jacobian check\n");
     return CAMP_NOALLOC_UNSUPPORTED;
   }
-  const size_t per_wave = cell_bdf_wave_scratch(s->P, s->place);
+  const size_t per_wave = cell_bdf_wave_scratch(s->P, s->variant());
   if (per_wave > kNoAllocScratchDoubles - kNoAllocHeaderDoubles) {
     std::fprintf(stderr, "camp_solver_run_device_noalloc: one wavefront needs %zu doubles of "
                          "scratch, more than the %zu available\n",

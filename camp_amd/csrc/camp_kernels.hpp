@@ -25,68 +25,71 @@ inline void allow_lds(const void* fn, size_t lds) {
 // two parts of f (state update + rates, species gather + estimate blend)
 constexpr int kCellProf = 7;
 
-// Where a cell's working set lives in the persistent kernel.
-//  kPlaceLds     everything in LDS: state, rate data, per-term rates,
-//                Nordsieck history (6 vectors), 8 work vectors, the f
-//                gather's scratch, the LU factors, the J history and 24
-//                slots for the BDF coefficient arrays l, tq and tau (gas
-//                phase only: 4 cells per CU for the CB05-scale mechanism);
-//  kPlaceGlobal  the Nordsieck history and most work vectors in
-//                per-wavefront global scratch (gas phase: all but zn[0], zn[1],
-//                the error weights, y, acor, tempv and ftemp; multi-phase: all but y, acor and w) and
-//                the J history used in place in HBM, so that more cells fit
-//                a CU's LDS (6 for the CB05-scale mechanism; compiled for
-//                two wavefronts per SIMD).  Multi-phase programs always run
-//                so, with their LU factors, reaction Jacobian and
-//                per-instance Jacobian scalars in the scratch as well.
-//  kPlaceGlobalLu  the Nordsieck history, 5 of the 8 work vectors and the
-//                LU factors (with the factorisation's sink slots and the
-//                solve's zero slot) in the scratch (gas phase: 12 cells per
-//                CU for the CB05-scale mechanism, compiled for two
-//                wavefronts per SIMD).
-constexpr int kPlaceLds = 0, kPlaceGlobal = 1, kPlaceGlobalLu = 2, kNumPlacements = 3;
-__host__ __device__ inline int cell_placement(const DevProgram& P, int place) {
-  return P.mp ? kPlaceGlobal : place;
-}
+// Where a cell's working set lives in the persistent kernel.  Every variant
+// keeps the state, the per-term rates, y, acor, the f gather's scratch and the
+// BDF coefficient arrays l, tq and tau (24 slots) in LDS.
+//  kPlaceLds     everything else too: rate constants, Nordsieck history (6
+//                vectors), 8 work vectors, LU factors, J history (gas phase
+//                only: 4 cells per CU for the CB05-scale mechanism);
+//  kPlaceGlobal  gas phase: zn[0], zn[1], the error weights, tempv, ftemp and
+//                the LU factors in LDS; Nordsieck vectors 2 to 5, last,
+//                acinit, w and the J history in f's order in the wavefront's
+//                global scratch; rate constants and J history in place in HBM
+//                (6 cells per CU).  Multi-phase programs always run this
+//                variant, with y, acor, w and the rate constants in LDS and
+//                their other vectors, LU factors, reaction Jacobian and
+//                per-instance Jacobian scalars in the scratch.
+//  kPlaceGlobalLu  gas phase: the LU factors, w and the J history in f's order
+//                in the scratch, all other vectors in LDS, rate constants and
+//                J history in HBM (8 cells per CU).
+//  kPlaceWide    gas phase: all vectors but y, acor and w, and the LU factors,
+//                in the scratch.  Needs the least LDS; for programs of which no
+//                cell fits with the placement asked for (the vectors in LDS
+//                outgrow it with the number of solver variables).
+// All but kPlaceLds and the multi-phase kernel are compiled for two wavefronts
+// per SIMD, kPlaceWide for one.
+constexpr int kPlaceLds = 0, kPlaceGlobal = 1, kPlaceGlobalLu = 2, kNumPlacements = 3,
+              kPlaceWide = 3;
 // LU factors in the wavefront's global scratch
 __host__ __device__ inline bool cell_lu_global(const DevProgram& P, int place) {
-  return P.mp || place == kPlaceGlobalLu;
+  return P.mp || place == kPlaceGlobalLu || place == kPlaceWide;
 }
-// vectors of a cell in LDS: all 14 with the history in LDS; for
-// gas-phase cells with the history in global memory zn[0], zn[1], the error
-// weights, y, acor, tempv and ftemp; otherwise y, acor and the solve's w
+// vectors of a cell in LDS
 __host__ __device__ inline int cell_lds_vectors(const DevProgram& P, int place) {
-  const int pl = cell_placement(P, place);
-  return pl == kPlaceLds ? 14 : P.mp ? 3 : pl == kPlaceGlobal ? 7 : 13;
+  return P.mp || place == kPlaceWide ? 3 : place == kPlaceLds ? 14 : place == kPlaceGlobal ? 7 : 13;
 }
 // rate constants in LDS (gas-phase cells with the J history in global memory
 // read them there too)
 __host__ __device__ inline size_t cell_lds_env(const DevProgram& P, int place) {
-  return !P.mp && cell_placement(P, place) != kPlaceLds ? 0 : (size_t)P.n_env;
+  return P.mp || place == kPlaceLds ? (size_t)P.n_env : 0;
 }
 // gas-phase kPlaceGlobal: the LU's LDS, where J(y) also stages the rate constants
 __host__ __device__ inline size_t cell_lu_lds(const DevProgram& P) {
   return P.lu_nnz > P.n_env ? P.lu_nnz : P.n_env;
 }
+// LDS doubles of a cell; place: the variant launched (any for multi-phase)
 __host__ __device__ inline size_t cell_bdf_lds_doubles(const DevProgram& P, int place) {
-  const bool g = cell_placement(P, place) != kPlaceLds;
+  const bool lds = !P.mp && place == kPlaceLds;
   return even_up(P.ns + cell_lds_env(P, place)) + mp_lds_doubles(P) +
          even_up(2 * (size_t)P.n_terms + (size_t)cell_lds_vectors(P, place) * P.nv + fb_sink_doubles(P) +
-         (cell_lu_global(P, place) ? 0 : cell_placement(P, place) == kPlaceGlobal ? cell_lu_lds(P)
-                                                                       : (size_t)P.lu_nnz) +
-         (g ? 0 : (size_t)P.nnz + 2 * (size_t)P.nv) + 24);
+         (cell_lu_global(P, place) ? 0 : place == kPlaceGlobal ? cell_lu_lds(P) : (size_t)P.lu_nnz) +
+         (lds ? (size_t)P.nnz + 2 * (size_t)P.nv : 0) + 24);
+}
+// The variant that runs placement `place`, cpb cells a workgroup: itself where
+// it fits a CU, else kPlaceWide.
+inline int cell_placement(const DevProgram& P, int place, int cpb = 1) {
+  if (P.mp) return kPlaceGlobal;
+  return cpb * cell_bdf_lds_doubles(P, place) * sizeof(double) <= kMaxLds ? place : kPlaceWide;
 }
 // Global scratch doubles per wavefront: the LU factors where they are global
-// (with the zero slot), for multi-phase programs then the reaction Jacobian and the per-instance
-// Jacobian scalars, then (kPlaceGlobal, kPlaceGlobalLu) the Nordsieck
-// history and the work vectors not in LDS (11 vectors; 7 for gas-phase
-// kPlaceGlobal) and the J history in f's order.
+// (with the zero slot), for multi-phase programs then the reaction Jacobian and
+// the per-instance Jacobian scalars, then the vectors not in LDS (of 14) and
+// the J history in f's order.
 __host__ __device__ inline size_t cell_bdf_wave_scratch(const DevProgram& P, int place) {
-  if (P.mp)
-    return (size_t)P.lu_nnz + kWave + 1 + P.rnnz + mp_jsc_doubles(P) + 11 * (size_t)P.nv +
-           est_doubles(P);
-  if (place == kPlaceGlobalLu) return (size_t)P.lu_nnz + kWave + 1 + (size_t)P.nv + est_doubles(P);
-  return place == kPlaceGlobal ? 7 * (size_t)P.nv + est_doubles(P) : 0;
+  if (!P.mp && place == kPlaceLds) return 0;
+  return (cell_lu_global(P, place) ? (size_t)P.lu_nnz + kWave + 1 : 0) +
+         (P.mp ? P.rnnz + mp_jsc_doubles(P) : 0) +
+         (size_t)(14 - cell_lds_vectors(P, place)) * P.nv + est_doubles(P);
 }
 
 // The no-allocation entry point's scratch (a file-scope device array of
@@ -114,12 +117,12 @@ struct CellBdfArgs {
   const double* cell_t1 = nullptr;
   double* prof = nullptr;  // [cells][kCellProf] when phase timing is on
   int* fail_count = nullptr;  // per cell: incremented on each failed solve
-  double* wave_scratch = nullptr;  // [grid waves][cell_bdf_wave_scratch] (kPlaceGlobal)
+  double* wave_scratch = nullptr;  // [grid waves][cell_bdf_wave_scratch]
   // Optional: cell solves cell_nsteps[cell] consecutive timesteps over
   // [t0, t1] in this launch, each exactly as a separate launch would
   // (state written back and restaged between them); nullptr: one.
   const int* cell_nsteps = nullptr;
-  int place = kPlaceLds;  // cell_placement(P, place) selects the kernel variant
+  int place = kPlaceLds;  // the kernel variant (cell_placement)
   // Check of per-cell independence: when non-zero, every wavefront fills its
   // whole working memory (the cell's LDS region and, for multi-phase
   // programs, its global scratch) with quiet NaNs before it stages each

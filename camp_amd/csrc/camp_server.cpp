@@ -487,7 +487,7 @@ extern "C" int camp_server_add_mechanism(void* server, void* solver_data, long m
   // list and wavefront scratch are allocated here, per stream, at that size
   int grid = 0, block = 0;
   size_t lds = 0;
-  A->place = cell_placement(S->P, S->place);
+  A->place = S->variant();
   S->cell_launch_shape(1L << 30, &grid, &block, &lds, A->place);
   A->chunk = 2L * grid * (block / kWave);
   size_t waves = (size_t)grid * (block / kWave);

@@ -292,13 +292,13 @@ CellBdfArgs Solver::cell_args() const {
   a.max_steps = m.max_steps;
   a.max_conv_fails = m.max_conv_fails;
   a.guess_on = guess_on;
-  a.place = cell_placement(P, place);
+  a.place = variant();
   return a;
 }
 
 void Solver::cell_launch_shape(long nq, int* grid, int* block, size_t* lds, int at_place) const {
   int cpb = cells_per_block;
-  const int place = at_place < 0 ? this->place : at_place;
+  const int place = at_place < 0 ? variant() : at_place;
   *block = kWave * cpb;
   *lds = (size_t)cpb * cell_bdf_lds_doubles(P, place) * sizeof(double);
   int dev = 0, ncu = 0;
@@ -337,7 +337,7 @@ int Solver::run_cells(double* st, double* env, double t0, double t1, double* noa
   if (noalloc) {
     // the queue counter in the scratch's first 256 bytes, the wavefronts'
     // scratch after it; as many workgroups as the scratch holds
-    const size_t per_wave = cell_bdf_wave_scratch(P, place);
+    const size_t per_wave = cell_bdf_wave_scratch(P, a.place);
     if (per_wave > 0) {
       long waves_fit = (long)((noalloc_doubles - kNoAllocHeaderDoubles) / per_wave);
       grid = (int)std::max<long>(1, std::min<long>(grid, waves_fit / (block / kWave)));
@@ -346,7 +346,7 @@ int Solver::run_cells(double* st, double* env, double t0, double t1, double* noa
     a.wave_scratch = per_wave > 0 ? noalloc + kNoAllocHeaderDoubles : nullptr;
     hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, stream, 1L, 0.0, noalloc);
   } else {
-    a.wave_scratch = wave_scratch((size_t)grid * (block / kWave), place);
+    a.wave_scratch = wave_scratch((size_t)grid * (block / kWave), a.place);
     HIP_OK(hipMemsetAsync(d_counter, 0, sizeof(int), stream));
   }
   HIP_OK(hipEventRecord(ev0, stream));
@@ -1444,9 +1444,10 @@ extern "C" int camp_solver_set_cells_per_block(void* solver_data, int cpb) {
   Solver* s = SD(solver_data);
   if (cpb == 0) cpb = 1;
   if (cpb == 1 || cpb == 2 || cpb == 4 || cpb == 8 || cpb == 16 || cpb == 32) {
-    size_t lds = (size_t)cpb * cell_bdf_lds_doubles(s->P, s->place) * sizeof(double);
+    const int pl = cell_placement(s->P, s->place, cpb);
+    size_t lds = (size_t)cpb * cell_bdf_lds_doubles(s->P, pl) * sizeof(double);
     if (!s->m.initialized || !s->stream ||
-        cell_bdf_blocks_per_cu(s->P, s->place, kWave * cpb, lds) > 0)
+        cell_bdf_blocks_per_cu(s->P, pl, kWave * cpb, lds) > 0)
       s->cells_per_block = cpb;
   }
   return s->cells_per_block;
@@ -1471,7 +1472,7 @@ extern "C" int camp_solver_set_placement(void* solver_data, int place) {
   using namespace camp;
   Solver* s = SD(solver_data);
   if (place >= 0 && place < kNumPlacements) s->place = place;
-  return cell_placement(s->P, s->place);
+  return s->P.mp ? kPlaceGlobal : s->place;
 }
 
 // Autotuner for the persistent per-cell kernel.  Candidates: the cell
@@ -1529,7 +1530,7 @@ extern "C" int camp_solver_autotune(void* solver_data, const double* d_state,
   }
   const int cand[6] = {1, 2, 4, 8, 16, 32};
   const int keep_cpb = s->cells_per_block, keep_place = s->place;
-  int best = keep_cpb, best_place = cell_placement(P, keep_place);
+  int best = keep_cpb, best_place = P.mp ? kPlaceGlobal : keep_place;
   double best_ms = -1.0;
   for (int pl = 0; pl < kNumPlacements; ++pl) {
     const int place = pl;
@@ -1537,8 +1538,8 @@ extern "C" int camp_solver_autotune(void* solver_data, const double* d_state,
       double* slot = ms_out ? &ms_out[pl * 6 + k] : nullptr;
       if (slot) *slot = -1.0;
       // multi-phase programs have one placement
-      if (cell_placement(P, place) != place) continue;
       int cpb = cand[k];
+      if (cell_placement(P, place, cpb) != place) continue;
       size_t lds = (size_t)cpb * cell_bdf_lds_doubles(P, place) * sizeof(double);
       if (cell_bdf_blocks_per_cu(P, place, kWave * cpb, lds) <= 0) continue;
       gather(d_state, P.ns, st);
@@ -1602,7 +1603,7 @@ extern "C" int camp_solver_phase_cycles(void* solver_data, const double* d_state
   Solver* s = SD(solver_data);
   if (!s->m.initialized || reps < 1) return 1;
   s->ensure_device();
-  if (cell_placement(s->P, s->place) == kPlaceGlobalLu) return 1;
+  if (s->variant() != kPlaceLds && s->variant() != kPlaceGlobal) return 1;
   s->upload_renv();
   const DevProgram& P = s->P;
   long nc = s->m.nc;

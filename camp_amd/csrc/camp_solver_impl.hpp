@@ -68,6 +68,8 @@ struct Solver {
   // 57.0; 60000 cells 48.1 / 48.5, 1115 / 1118, 205 / 202; 60000 CB05cl_ae5
   // cells (6 s) 11.6 / 12.1.  No size or state tried gains more than 2 %.
   int place = kPlaceGlobal;
+  // the variant of this solver's launches
+  int variant() const { return cell_placement(P, place, cells_per_block); }
   int guess_on = 1;
   bool renv_dirty = true;
   hipStream_t stream = nullptr;
@@ -182,7 +184,7 @@ struct Solver {
   // Per-cell kernel arguments with the solver's program and controls filled
   // in (buffers left to the caller), and the launch shape for nq queued cells.
   CellBdfArgs cell_args() const;
-  // (at_place < 0: the solver's own placement)
+  // (at_place < 0: the solver's own variant)
   void cell_launch_shape(long nq, int* grid, int* block, size_t* lds, int at_place = -1) const;
   int run(double* d_state_in, double* d_env_in, double t0, double t1);
   // noalloc: the no-allocation entry point's scratch (device pointer and

@@ -206,7 +206,8 @@ int camp_solver_set_cells_per_block(void *solver_data, int cells_per_block);
  * unit), 1 = the higher Nordsieck vectors, the rate constants and the J
  * history in global memory (two wavefronts per SIMD), 2 = the LU factors, the
  * rate constants and the J history in global memory (most cells per compute
- * unit).  Returns the placement in effect (1 by default; a negative place
+ * unit).  Cells that do not fit a compute unit's LDS with the placement set
+ * run with most of their vectors in global memory.  Returns the placement set (1 by default; a negative place
  * only asks).  Results do not depend on it. */
 int camp_solver_set_placement(void *solver_data, int place);
 

@@ -99,3 +99,22 @@ def test_large_launch_of_a_wide_mechanism():
     y = y0.copy()
     assert gpu.solve(y, np.tile(ENV, (n_cells, 1)), 0.0, 60.0) == 0
     assert np.allclose(y, ring_solution(y0, 60.0), rtol=1e-3, atol=0.0)
+
+
+@pytest.mark.parametrize("n, cells_per_block", [(300, 4), (1300, 1), (1500, 1)])
+def test_placements_that_do_not_fit(n, cells_per_block):
+    """Four cells of 300 species a workgroup fit with placement 1 only, one of
+    1300 with placement 1 only, one of 1500 with none: the others run with
+    their vectors in global memory, and the result is the same bit for bit."""
+    n_cells = 5
+    y0 = np.random.default_rng(5).uniform(1.0, 2.0, (n_cells, n))
+    got = []
+    for place in (1, 0, 2):
+        gpu = CampSolver(ring_mechanism(n), n_cells)
+        assert gpu.set_placement(place) == place
+        assert gpu.set_cells_per_block(cells_per_block) == cells_per_block
+        y = y0.copy()
+        assert gpu.solve(y, np.tile(ENV, (n_cells, 1)), 0.0, 60.0) == 0
+        got.append(y)
+    assert np.allclose(got[0], ring_solution(y0, 60.0), rtol=1e-3, atol=0.0)
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
