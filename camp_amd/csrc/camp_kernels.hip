@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(256) k_deriv(DevProgram P, int nc, const doubl
   double* s_mp = s_state + even_up((size_t)P.ns + P.n_env);
   double* s_rate = s_mp + mp_lds_doubles(P);
   MpLds L = mp_lds(P, s_mp, s_rate + 2 * (size_t)P.n_terms);
-  double* s_fb = s_rate + 2 * (size_t)P.n_terms + mp_jsc_doubles(P);
+  double* s_fb = s_rate + 2 * (size_t)P.n_terms;
   double* s_dy = fj_dy(P) ? smem + (size_t)wv * fj_lds_doubles(P) + fj_lds_doubles_no_dy(P) : nullptr;
   for (int c = blockIdx.x * wpb + wv; c < nc; c += gridDim.x * wpb) {
     stage_cell(P, lane, state + (size_t)c * P.ns, rxn_env + (size_t)c * P.n_env, s_state, s_k);
@@ -755,7 +755,7 @@ __global__ void __launch_bounds__(64) k_check_jac(DevProgram P, int nc, const do
   double* s_mp = s_state + even_up((size_t)P.ns + P.n_env);
   double* s_rate = s_mp + mp_lds_doubles(P);
   MpLds L = mp_lds(P, s_mp, s_rate + 2 * (size_t)P.n_terms);
-  double* s_fb = s_rate + 2 * (size_t)P.n_terms + mp_jsc_doubles(P);
+  double* s_fb = s_rate + 2 * (size_t)P.n_terms;
   double* f0 = smem + fj_lds_doubles_no_dy(P);
   double* f1 = f0 + P.nv;
   double* f2 = f1 + P.nv;

@@ -147,13 +147,14 @@ __global__ void k_deriv(DevProgram P, int nc, const double* y, const double* sta
 // Jr: reaction-Jacobian scratch [nc][rnnz] of multi-phase programs (else unused)
 __global__ void k_jac(DevProgram P, int nc, const double* y, const double* state,
                       const double* env, const double* rxn_env, double* J, double h, double* Jr);
-// LDS doubles per wavefront of k_deriv and k_jac (the estimate's dy last, where
-// it fits; without: k_check_jac, whose f takes no estimate), and wavefronts per
+// LDS doubles per wavefront of k_deriv and k_jac (f's gather scratch and J's
+// per-instance scalars share a place; the estimate's dy last, where it fits; without: k_check_jac, whose f takes no estimate), and wavefronts per
 // block: one for multi-phase programs, whose per-cell extras are large, else up
 // to four, as many as fit.
 __host__ __device__ inline size_t fj_lds_doubles_no_dy(const DevProgram& P) {
   return even_up((size_t)P.ns + P.n_env) + mp_lds_doubles(P) +
-         even_up(2 * (size_t)P.n_terms + mp_jsc_doubles(P) + fb_lds_doubles(P));
+         even_up(2 * (size_t)P.n_terms +
+                 (mp_jsc_doubles(P) > fb_lds_doubles(P) ? mp_jsc_doubles(P) : fb_lds_doubles(P)));
 }
 __host__ __device__ inline bool fj_dy(const DevProgram& P) {
   return (fj_lds_doubles_no_dy(P) + even_up(P.nv)) * sizeof(double) <= kMaxLds;

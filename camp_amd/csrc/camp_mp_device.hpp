@@ -48,154 +48,191 @@ __host__ __device__ __forceinline__ double mp_dcond_rate_dr(double D, double mfp
 // of 64 lanes with 29 double-double divisions one after another; the quotients
 // x / MW and x / density are formed by a lane per item into scratch and only
 // the additions stay in order, the three sums of a phase on three lanes.
+//
+// The scratch (here, in the ZSR passes and for J's partial derivatives) is the
+// LDS of f's contribution slots and of the per-term rates after them, which
+// hold nothing yet: mp_scratch_doubles(P) of it.  What does not fit at once
+// goes in chunks, each continuing the sums of the last.
+__host__ __device__ inline size_t mp_slot_doubles(const DevProgram& P) {
+  const size_t n = 2 * (size_t)P.n_slots;
+  return n > 6 ? n : 6;  // (one item or ion pair at least)
+}
+__host__ __device__ inline int mp_scratch_doubles(const DevProgram& P) {
+  return (int)(mp_slot_doubles(P) + 2 * (size_t)P.n_terms);
+}
 
 // mass, moles (dd) and volume of every phase into s_aero[3..7]
 __device__ __forceinline__ void mp_phase_sums(const DevProgram& P, int lane, const double* s_state,
                                               double* s_aero, double* scratch) {
-  for (int it = lane; it < P.n_it; it += kWave) {
-    double x = s_state[P.pit_state[it]];
-    dd m = dd_div_d(dd_from(x), P.pit_mw[it]);
-    double* q = scratch + 4 * it;
-    q[0] = x;
-    q[1] = m.hi;
-    q[2] = m.lo;
-    q[3] = x / P.pit_dens[it];
-  }
-  wsync();
-  for (int t = lane; t < 3 * P.n_pi; t += kWave) {
-    const int i = t / 3, w = t - 3 * i;
-    const int k0 = P.pit_ptr[i], k1 = P.pit_ptr[i + 1];
-    const double* q = scratch + (w == 0 ? 0 : w == 1 ? 1 : 3);
-    dd s = w == 0 ? dd{P.min_mass_hi, P.min_mass_lo}
-                  : w == 1 ? dd{P.min_moles_hi, P.min_moles_lo} : dd{P.min_volume, 0.0};
-    for (int k = k0; k < k1; ++k) {
-      dd v = {q[4 * k], w == 1 ? q[4 * k + 1] : 0.0};
-      const double plain = s.hi + v.hi;
-      s = dd_add(s, v);
-      if (w == 2) s = dd{plain, 0.0};
+  const int cap = mp_scratch_doubles(P) / 4;
+  int b = 0;
+  do {
+    const int end = min(b + cap, P.n_it);
+    for (int it = b + lane; it < end; it += kWave) {
+      double x = s_state[P.pit_state[it]];
+      dd m = dd_div_d(dd_from(x), P.pit_mw[it]);
+      double* q = scratch + 4 * (it - b);
+      q[0] = x;
+      q[1] = m.hi;
+      q[2] = m.lo;
+      q[3] = x / P.pit_dens[it];
     }
-    double* a = s_aero + kAeroSlots * i + 3 + 2 * w;
-    a[0] = s.hi;
-    if (w < 2) a[1] = s.lo;
-  }
-  wsync();
+    wsync();
+    for (int t = lane; t < 3 * P.n_pi; t += kWave) {
+      const int i = t / 3, w = t - 3 * i;
+      const int k0 = max(P.pit_ptr[i], b), k1 = min(P.pit_ptr[i + 1], end);
+      double* a = s_aero + kAeroSlots * i + 3 + 2 * w;
+      const double* q = scratch + 4 * (k0 - b) + (w == 0 ? 0 : w == 1 ? 1 : 3);
+      dd s = w == 0 ? dd{P.min_mass_hi, P.min_mass_lo}
+                    : w == 1 ? dd{P.min_moles_hi, P.min_moles_lo} : dd{P.min_volume, 0.0};
+      if (b > 0) s = dd{a[0], w < 2 ? a[1] : 0.0};
+      for (int k = k0; k < k1; ++k, q += 4) {
+        dd v = {q[0], w == 1 ? q[1] : 0.0};
+        const double plain = s.hi + v.hi;
+        s = dd_add(s, v);
+        if (w == 2) s = dd{plain, 0.0};
+      }
+      a[0] = s.hi;
+      if (w < 2) a[1] = s.lo;
+    }
+    wsync();
+    b += cap;
+  } while (b < P.n_it);
 }
 
 // --- ZSR water of every (sub model, phase) item (:216-301) -----------------
 // A lane per ion for the exponentials, a lane per ion pair for its molality and
 // contribution, a lane per item to add the pairs in order; scratch holds 6
 // doubles per pair (cation, anion, their exponentials, the contribution).
-__device__ __forceinline__ void mp_zsr_ions(const DevProgram& P, int lane, const double* s_state,
-                                            double* scratch) {
-  for (int t = lane; t < 2 * P.n_zp; t += kWave) {
-    const bool an = t >= P.n_zp;
-    const int x = an ? t - P.n_zp : t;
+// (pairs x0 to x1, pair x's scratch at 6 (x - x0))
+__device__ __forceinline__ void mp_zsr_ions(const DevProgram& P, int lane, int x0, int x1,
+                                            const double* s_state, double* scratch) {
+  for (int t = lane; t < 2 * (x1 - x0); t += kWave) {
+    const bool an = t >= x1 - x0;
+    const int x = x0 + (an ? t - (x1 - x0) : t);
     // ion concentrations are double expressions (state / int / MW / 1000)
     double c = s_state[an ? P.zp_an[x] : P.zp_cat[x]] / (double)(an ? P.zp_nan[x] : P.zp_ncat[x]) /
                (an ? P.zp_anmw[x] : P.zp_catmw[x]) / 1000.0;
-    scratch[6 * x + (an ? 1 : 0)] = c;
-    scratch[6 * x + (an ? 3 : 2)] = cr_exp(-100.0 * c);
+    scratch[6 * (x - x0) + (an ? 1 : 0)] = c;
+    scratch[6 * (x - x0) + (an ? 3 : 2)] = cr_exp(-100.0 * c);
   }
   wsync();
 }
 
 __device__ __forceinline__ void mp_zsr(const DevProgram& P, int lane, const double* s_sub_env,
                                        double* s_state, double* scratch) {
-  mp_zsr_ions(P, lane, s_state, scratch);
-  for (int x = lane; x < P.n_zp; x += kWave) {
-    const int z = P.zp_zi[x];
-    // a_w = PPM_TO_RH * state: a double product (both operands double)
-    dd aw = dd_from(s_sub_env[P.zi_sub[z]] * s_state[P.zi_gw[z]]);
-    double low = P.zp_lowrh[x];
-    dd jaw = dd_gt(aw, low) ? aw : dd_from(low);
-    double jaw_d = dd_round(jaw);
-    // the powers of jaw (cr_powi) as one chain: each continues the last
-    dd mol = dd_from(0.0);
-    dd pw = dd_from(fabs(jaw_d));
-    for (int k = 0; k < P.zp_ny[x]; ++k) {
-      double pk = k == 0 ? 1.0 : dd_round(pw);
-      if (jaw_d < 0.0 && (k & 1)) pk = -pk;
-      if (k > 0) pw = dd_mul_d(pw, fabs(jaw_d));
-      mol = dd_add(mol, dd_from(P.zp_y[8 * x + k] * pk));
+  const int cap = mp_scratch_doubles(P) / 6;
+  int x0 = 0;
+  do {
+    const int x1 = min(x0 + cap, P.n_zp);
+    mp_zsr_ions(P, lane, x0, x1, s_state, scratch);
+    for (int x = x0 + lane; x < x1; x += kWave) {
+      const int z = P.zp_zi[x];
+      // a_w = PPM_TO_RH * state: a double product (both operands double)
+      dd aw = dd_from(s_sub_env[P.zi_sub[z]] * s_state[P.zi_gw[z]]);
+      double low = P.zp_lowrh[x];
+      dd jaw = dd_gt(aw, low) ? aw : dd_from(low);
+      double jaw_d = dd_round(jaw);
+      // the powers of jaw (cr_powi) as one chain: each continues the last
+      dd mol = dd_from(0.0);
+      dd pw = dd_from(fabs(jaw_d));
+      for (int k = 0; k < P.zp_ny[x]; ++k) {
+        double pk = k == 0 ? 1.0 : dd_round(pw);
+        if (jaw_d < 0.0 && (k & 1)) pk = -pk;
+        if (k > 0) pw = dd_mul_d(pw, fabs(jaw_d));
+        mol = dd_add(mol, dd_from(P.zp_y[8 * x + k] * pk));
+      }
+      mol = dd_mul(mol, mol);
+      double* q = scratch + 6 * (x - x0);
+      dd cat = dd_from(q[0]), an = dd_from(q[1]), e_ac = dd_from(q[2]), e_aa = dd_from(q[3]);
+      dd conc = dd_div(dd_add(dd_mul(cat, e_ac), dd_mul(an, e_aa)), dd_add(e_ac, e_aa));
+      dd v = dd_mul(dd_div(conc, mol), dd_from(1000.0));
+      q[4] = v.hi;
+      q[5] = v.lo;
     }
-    mol = dd_mul(mol, mol);
-    double* q = scratch + 6 * x;
-    dd cat = dd_from(q[0]), an = dd_from(q[1]), e_ac = dd_from(q[2]), e_aa = dd_from(q[3]);
-    dd conc = dd_div(dd_add(dd_mul(cat, e_ac), dd_mul(an, e_aa)), dd_add(e_ac, e_aa));
-    dd v = dd_mul(dd_div(conc, mol), dd_from(1000.0));
-    q[4] = v.hi;
-    q[5] = v.lo;
-  }
-  wsync();
-  for (int z = lane; z < P.n_zi; z += kWave) {
-    double water = 1.0e-30;
-    for (int x = P.zi_pair_ptr[z]; x < P.zi_pair_ptr[z + 1]; ++x)
-      water = dd_round(dd_add(dd_from(water), dd{scratch[6 * x + 4], scratch[6 * x + 5]}));
-    s_state[P.zi_water[z]] = water;
-  }
-  wsync();
+    wsync();
+    for (int z = lane; z < P.n_zi; z += kWave) {
+      double water = x0 > 0 ? s_state[P.zi_water[z]] : 1.0e-30;
+      const int e = min(P.zi_pair_ptr[z + 1], x1);
+      for (int x = max(P.zi_pair_ptr[z], x0); x < e; ++x) {
+        const double* q = scratch + 6 * (x - x0);
+        water = dd_round(dd_add(dd_from(water), dd{q[4], q[5]}));
+      }
+      s_state[P.zi_water[z]] = water;
+    }
+    wsync();
+    x0 += cap;
+  } while (x0 < P.n_zp);
 }
 
 // --- ZSR parameter Jacobian (:314-~440), added into s_jp: a lane per pair,
 // then a lane per item adds its pairs in order ------------------------------
 __device__ __forceinline__ void mp_zsr_jac(const DevProgram& P, int lane, const double* s_sub_env,
                                            const double* s_state, double* s_jp, double* scratch) {
-  mp_zsr_ions(P, lane, s_state, scratch);
-  for (int x = lane; x < P.n_zp; x += kWave) {
-    const int z = P.zp_zi[x];
-    double ppm = s_sub_env[P.zi_sub[z]];
-    dd aw = dd_from(ppm * s_state[P.zi_gw[z]]);
-    double low = P.zp_lowrh[x];
-    bool above = dd_gt(aw, low);
-    dd jaw = above ? aw : dd_from(low);
-    double jaw_d = dd_round(jaw);
-    dd djaw = above ? dd_from(ppm) : dd_from(0.0);
-    const double* Y = P.zp_y + 8 * x;
-    dd mol = dd_from(Y[0]), dmol = dd_from(0.0);
-    for (int k = 1; k < P.zp_ny[x]; ++k) {
-      mol = dd_add(mol, dd_from(Y[k] * cr_powi(jaw_d, k)));
-      dmol = dd_add(dmol, dd_from(Y[k] * k * cr_powi(jaw_d, k - 1)));
+  const int cap = mp_scratch_doubles(P) / 6;
+  int x0 = 0;
+  do {
+    const int x1 = min(x0 + cap, P.n_zp);
+    mp_zsr_ions(P, lane, x0, x1, s_state, scratch);
+    for (int x = x0 + lane; x < x1; x += kWave) {
+      const int z = P.zp_zi[x];
+      double ppm = s_sub_env[P.zi_sub[z]];
+      dd aw = dd_from(ppm * s_state[P.zi_gw[z]]);
+      double low = P.zp_lowrh[x];
+      bool above = dd_gt(aw, low);
+      dd jaw = above ? aw : dd_from(low);
+      double jaw_d = dd_round(jaw);
+      dd djaw = above ? dd_from(ppm) : dd_from(0.0);
+      const double* Y = P.zp_y + 8 * x;
+      dd mol = dd_from(Y[0]), dmol = dd_from(0.0);
+      for (int k = 1; k < P.zp_ny[x]; ++k) {
+        mol = dd_add(mol, dd_from(Y[k] * cr_powi(jaw_d, k)));
+        dmol = dd_add(dmol, dd_from(Y[k] * k * cr_powi(jaw_d, k - 1)));
+      }
+      dmol = dd_mul(dmol, djaw);
+      double* q = scratch + 6 * (x - x0);
+      dd cat = dd_from(q[0]), an = dd_from(q[1]), e_ac = dd_from(q[2]), e_aa = dd_from(q[3]);
+      double dcat = 1.0 / (double)P.zp_ncat[x] / P.zp_catmw[x] / 1000.0;
+      double dan = 1.0 / (double)P.zp_nan[x] / P.zp_anmw[x] / 1000.0;
+      dd conc = dd_div(dd_add(dd_mul(cat, e_ac), dd_mul(an, e_aa)), dd_add(e_ac, e_aa));
+      dd den = dd_mul(dd_add(e_ac, e_aa), dd_add(e_ac, e_aa));
+      // (1 - ALPHA*anion + ALPHA*cation), ALPHA = -100
+      dd kc = dd_add(dd_add(dd_from(1.0), dd_mul(dd_from(100.0), an)), dd_mul(dd_from(-100.0), cat));
+      dd ka = dd_add(dd_add(dd_from(1.0), dd_mul(dd_from(100.0), cat)), dd_mul(dd_from(-100.0), an));
+      dd dcdc = dd_div(dd_add(dd_mul(e_ac, e_ac), dd_mul(dd_mul(e_ac, e_aa), kc)), den);
+      dd dcda = dd_div(dd_add(dd_mul(e_aa, e_aa), dd_mul(dd_mul(e_ac, e_aa), ka)), den);
+      double mol_d = dd_round(mol);
+      double p3 = cr_powi(mol_d, 3), p2 = cr_powi(mol_d, 2);
+      // J[...] += value: each a double += (long double) rounded to double
+      // -2.0 * conc / pow(m, 3) * 1000.0 * dm and 1.0 / pow(m, 2) * 1000.0 * dc * dion,
+      // evaluated left to right as the reference does
+      dd v_gw = dd_mul(dd_mul(dd_div_d(dd_mul(dd_from(-2.0), conc), p3), dd_from(1000.0)), dmol);
+      double t2 = 1.0 / p2 * 1000.0;
+      dd v_an = dd_mul(dd_mul(dd_from(t2), dcda), dd_from(dan));
+      dd v_cat = dd_mul(dd_mul(dd_from(t2), dcdc), dd_from(dcat));
+      q[0] = v_gw.hi;
+      q[1] = v_gw.lo;
+      q[2] = v_an.hi;
+      q[3] = v_an.lo;
+      q[4] = v_cat.hi;
+      q[5] = v_cat.lo;
     }
-    dmol = dd_mul(dmol, djaw);
-    double* q = scratch + 6 * x;
-    dd cat = dd_from(q[0]), an = dd_from(q[1]), e_ac = dd_from(q[2]), e_aa = dd_from(q[3]);
-    double dcat = 1.0 / (double)P.zp_ncat[x] / P.zp_catmw[x] / 1000.0;
-    double dan = 1.0 / (double)P.zp_nan[x] / P.zp_anmw[x] / 1000.0;
-    dd conc = dd_div(dd_add(dd_mul(cat, e_ac), dd_mul(an, e_aa)), dd_add(e_ac, e_aa));
-    dd den = dd_mul(dd_add(e_ac, e_aa), dd_add(e_ac, e_aa));
-    // (1 - ALPHA*anion + ALPHA*cation), ALPHA = -100
-    dd kc = dd_add(dd_add(dd_from(1.0), dd_mul(dd_from(100.0), an)), dd_mul(dd_from(-100.0), cat));
-    dd ka = dd_add(dd_add(dd_from(1.0), dd_mul(dd_from(100.0), cat)), dd_mul(dd_from(-100.0), an));
-    dd dcdc = dd_div(dd_add(dd_mul(e_ac, e_ac), dd_mul(dd_mul(e_ac, e_aa), kc)), den);
-    dd dcda = dd_div(dd_add(dd_mul(e_aa, e_aa), dd_mul(dd_mul(e_ac, e_aa), ka)), den);
-    double mol_d = dd_round(mol);
-    double p3 = cr_powi(mol_d, 3), p2 = cr_powi(mol_d, 2);
-    // J[...] += value: each a double += (long double) rounded to double
-    // -2.0 * conc / pow(m, 3) * 1000.0 * dm and 1.0 / pow(m, 2) * 1000.0 * dc * dion,
-    // evaluated left to right as the reference does
-    dd v_gw = dd_mul(dd_mul(dd_div_d(dd_mul(dd_from(-2.0), conc), p3), dd_from(1000.0)), dmol);
-    double t2 = 1.0 / p2 * 1000.0;
-    dd v_an = dd_mul(dd_mul(dd_from(t2), dcda), dd_from(dan));
-    dd v_cat = dd_mul(dd_mul(dd_from(t2), dcdc), dd_from(dcat));
-    q[0] = v_gw.hi;
-    q[1] = v_gw.lo;
-    q[2] = v_an.hi;
-    q[3] = v_an.lo;
-    q[4] = v_cat.hi;
-    q[5] = v_cat.lo;
-  }
-  wsync();
-  for (int z = lane; z < P.n_zi; z += kWave)
-    for (int x = P.zi_pair_ptr[z]; x < P.zi_pair_ptr[z + 1]; ++x) {
-      const double* q = scratch + 6 * x;
-      double* j = s_jp + P.zp_jgw[x];
-      *j = dd_round(dd_add(dd_from(*j), dd{q[0], q[1]}));
-      j = s_jp + P.zp_jan[x];
-      *j = dd_round(dd_add(dd_from(*j), dd{q[2], q[3]}));
-      j = s_jp + P.zp_jcat[x];
-      *j = dd_round(dd_add(dd_from(*j), dd{q[4], q[5]}));
+    wsync();
+    for (int z = lane; z < P.n_zi; z += kWave) {
+      const int e = min(P.zi_pair_ptr[z + 1], x1);
+      for (int x = max(P.zi_pair_ptr[z], x0); x < e; ++x) {
+        const double* q = scratch + 6 * (x - x0);
+        double* j = s_jp + P.zp_jgw[x];
+        *j = dd_round(dd_add(dd_from(*j), dd{q[0], q[1]}));
+        j = s_jp + P.zp_jan[x];
+        *j = dd_round(dd_add(dd_from(*j), dd{q[2], q[3]}));
+        j = s_jp + P.zp_jcat[x];
+        *j = dd_round(dd_add(dd_from(*j), dd{q[4], q[5]}));
+      }
     }
-  wsync();
+    wsync();
+    x0 += cap;
+  } while (x0 < P.n_zp);
 }
 
 // --- per-instance quantities shared by f and J ------------------------------
@@ -344,12 +381,28 @@ __host__ __device__ __forceinline__ void mp_aqeq_jscalars(const DevProgram& P, i
   o[5] = w < 1.0e-4 * P.aq_small_water[i] ? 1.0 : 0.0;
 }
 
+// The partial derivatives of an item's phase's number concentration and average
+// MW by the item's species (aero_phase_solver.c:78-150 and the representation's
+// getters).
+__host__ __device__ __forceinline__ void mp_item_partials(const DevProgram& P, int it,
+                                                          const double* s_aero, double& numj,
+                                                          double& mwj) {
+  const int pi = P.pit_pi[it];
+  const double* ag = s_aero + kAeroSlots * pi;
+  double factor = 3.0 / (4.0 * kPi) / cr_powi(P.pi_dp[pi] / 2.0, 3);
+  numj = 1.0 / P.pit_dens[it] * factor;
+  dd lm = {ag[3], ag[4]}, mo = {ag[5], ag[6]};
+  mwj = dd_round(dd_div(dd_sub(mo, dd_mul(dd_from(1.0 / P.pit_mw[it]), lm)), dd_mul(mo, mo)));
+}
+
 // --- one special Jacobian record {kind, instance, p1, p2}, c, added to D ----
 // PRODUCTION contributions add, LOSS contributions subtract (Jacobian.c:
 // 223-241 keeps them in separate long double sums and outputs prod - loss).
+// s_part: the items' partials (mp_item_partials), or nullptr where they do not
+// fit the scratch and are formed here.
 __host__ __device__ __forceinline__ dd mp_jac_record(const DevProgram& P, int4 a, double c,
                                             const double* s_state, const double* s_part,
-                                            const double* s_jsc, dd D) {
+                                            const double* s_aero, const double* s_jsc, dd D) {
   const double* aq0 = s_jsc + kSpScalars * P.n_sp;
   if (a.x <= kJsSimpolAP) {
     const double* s = s_jsc + kSpScalars * a.y;
@@ -369,8 +422,14 @@ __host__ __device__ __forceinline__ dd mp_jac_record(const DevProgram& P, int4 a
       case kJsSimpolAA:  // LOSS N * evap_rate * act / kp
         D = dd_sub(D, dd_div_d(dd_mul(dd_from(N), evap0), kp));
         break;
-      default: {  // phase element: item a.w, whose partials s_part holds
-        double numj = s_part[2 * a.w], mwj = s_part[2 * a.w + 1];
+      default: {  // phase element: item a.w
+        double numj, mwj;
+        if (s_part) {
+          numj = s_part[2 * a.w];
+          mwj = s_part[2 * a.w + 1];
+        } else {
+          mp_item_partials(P, a.w, s_aero, numj, mwj);
+        }
         double massj = 1.0;
         double radj = 0.0;
         // (a radius term is an exact zero unless its factor overflowed)
@@ -434,17 +493,15 @@ struct MpLds {
 // parameter Jacobian); the per-instance Jacobian scalars (used only while J
 // is assembled) get their own mp_jsc_doubles(P) region, in LDS or in
 // per-wavefront global scratch as the caller places it.
-// The slots also serve as scratch while none holds a contribution: 4 doubles
-// per phase item (mp_phase_sums) or 6 per ion pair (mp_zsr) ahead of f's
-// contributions, 2 per phase item (s_part) while J is assembled.
-__host__ __device__ inline size_t mp_slot_doubles(const DevProgram& P) {
-  size_t n = 2 * (size_t)P.n_slots;
-  n = n > 4 * (size_t)P.n_it ? n : 4 * (size_t)P.n_it;
-  return n > 6 * (size_t)P.n_zp ? n : 6 * (size_t)P.n_zp;  // (even)
+// The slots come last, before the per-term rates, so that both together serve
+// as scratch (mp_scratch_doubles).  While J is assembled it holds the items'
+// partials, where they fit.
+__host__ __device__ inline bool mp_part(const DevProgram& P) {
+  return 2 * (long)P.n_it <= (long)mp_scratch_doubles(P);
 }
 __host__ __device__ inline size_t mp_lds_doubles(const DevProgram& P) {
   if (!P.mp) return 0;
-  return even_up((size_t)P.n_sub_env + kAeroSlots * (size_t)P.n_pi + mp_slot_doubles(P) + P.pnnz);
+  return even_up((size_t)P.n_sub_env + kAeroSlots * (size_t)P.n_pi + P.pnnz) + mp_slot_doubles(P);
 }
 __host__ __device__ inline size_t mp_jsc_doubles(const DevProgram& P) {
   if (!P.mp) return 0;
@@ -453,10 +510,11 @@ __host__ __device__ inline size_t mp_jsc_doubles(const DevProgram& P) {
 
 __device__ __forceinline__ MpLds mp_lds(const DevProgram& P, double* base, double* jsc) {
   MpLds L;
-  L.slot = base;  // (16-byte aligned: the f gather reads (hi, lo) pairs)
-  L.sub_env = L.slot + mp_slot_doubles(P);
+  L.sub_env = base;
   L.aero = L.sub_env + P.n_sub_env;
   L.jp = L.aero + kAeroSlots * P.n_pi;
+  // (16-byte aligned: the f gather reads (hi, lo) pairs)
+  L.slot = base + even_up((size_t)P.n_sub_env + kAeroSlots * (size_t)P.n_pi + P.pnnz);
   L.jsc = jsc;
   return L;
 }
@@ -509,18 +567,10 @@ __device__ __forceinline__ void mp_j_prologue(const DevProgram& P, int lane, con
   for (int q = lane; q < P.pnnz; q += kWave) L.jp[q] = 0.0;
   wsync();
   mp_zsr_jac(P, lane, L.sub_env, s_state, L.jp, L.slot);
-  // the partial derivatives of each phase's number concentration and average
-  // MW by its species (aero_phase_solver.c:78-150 and the representation's
-  // getters): one division per item instead of one per record that uses it
-  for (int it = lane; it < P.n_it; it += kWave) {
-    const int pi = P.pit_pi[it];
-    const double* ag = L.aero + kAeroSlots * pi;
-    double factor = 3.0 / (4.0 * kPi) / cr_powi(P.pi_dp[pi] / 2.0, 3);
-    L.slot[2 * it] = 1.0 / P.pit_dens[it] * factor;
-    dd lm = {ag[3], ag[4]}, mo = {ag[5], ag[6]};
-    L.slot[2 * it + 1] = dd_round(
-        dd_div(dd_sub(mo, dd_mul(dd_from(1.0 / P.pit_mw[it]), lm)), dd_mul(mo, mo)));
-  }
+  // one division per item instead of one per record that uses it
+  if (mp_part(P))
+    for (int it = lane; it < P.n_it; it += kWave)
+      mp_item_partials(P, it, L.aero, L.slot[2 * it], L.slot[2 * it + 1]);
   for (int i = lane; i < P.n_sp; i += kWave)
     mp_simpol_jscalars(P, i, s_state, s_k, L.aero, L.jsc + kSpScalars * i);
   for (int i = lane; i < P.n_aq; i += kWave)
@@ -536,7 +586,8 @@ __device__ __forceinline__ void mp_j_prologue(const DevProgram& P, int lane, con
 __device__ __forceinline__ dd mp_jac_stream_record(const DevProgram& P, int4 a, int4 b,
                                                    const double* s_state, const double* s_k,
                                                    double h, const double* s_part,
-                                                   const double* s_jsc, dd D) {
+                                                   const double* s_aero, const double* s_jsc,
+                                                   dd D) {
   const double c = hilo_to_double(b.w, b.z);
   if (a.x == -1) {
     double v = s_k[a.y];
@@ -548,7 +599,7 @@ __device__ __forceinline__ dd mp_jac_stream_record(const DevProgram& P, int4 a, 
     return dd_add(D, dd{c * v, 0.0});
   }
   if (a.x == 0) return D;
-  return mp_jac_record(P, a, c, s_state, s_part, s_jsc, D);
+  return mp_jac_record(P, a, c, s_state, s_part, s_aero, s_jsc, D);
 }
 
 // J of a multi-phase cell: the reaction Jacobian into Jr (global scratch,
@@ -559,6 +610,7 @@ __device__ __forceinline__ void cell_jac_mp(const DevProgram& P, int lane, const
                                             double* J) {
   lane = phase_lane(lane);
   vm_drain();
+  const double* part = mp_part(P) ? L.slot : nullptr;
   // elements in the program's order, whose rows share their record kinds;
   // each lane reads its element's records as a stream, the next record in
   // flight while the current one is added
@@ -573,7 +625,7 @@ __device__ __forceinline__ void cell_jac_mp(const DevProgram& P, int lane, const
       const int4* nx = rec + 2 * (size_t)(k + 1) * kWave;
       a = nx[0];
       b = nx[1];
-      D = mp_jac_stream_record(P, ca, cb, s_state, s_k, h, L.slot, L.jsc, D);
+      D = mp_jac_stream_record(P, ca, cb, s_state, s_k, h, part, L.aero, L.jsc, D);
     }
     if (e >= 0) Jr[e] = D.hi;
   }

@@ -6,6 +6,7 @@ import pytest
 
 from camp_amd.core import CampSolver
 from camp_amd.mechanisms import Mechanism, Reaction, box_mechanism, synthetic_cells
+from camp_amd.multiphase import multiphase_cells, multiphase_mechanism
 
 pytestmark = pytest.mark.gpu
 
@@ -118,3 +119,32 @@ def test_placements_that_do_not_fit(n, cells_per_block):
         got.append(y)
     assert np.allclose(got[0], ring_solution(y0, 60.0), rtol=1e-3, atol=0.0)
     assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
+def test_many_aerosol_species_and_few_reactions(oracle_lib):
+    """80 bins of 11 solutes, two of them partitioning: the phases' and ion
+    pairs' quotients do not fit the scratch at once and go in chunks, and the
+    species' partial derivatives not at all.  No more LDS is taken for them:
+    two cells a workgroup fit.  f and J as in the oracle (1e-12 relative: both
+    accumulate in extended precision, and the chunks keep the order), the step
+    as the oracle's at the 1e-4 / 1e-8 bar of the other multi-phase tests."""
+    mp = multiphase_mechanism(1, n_bins=80, n_simpol=2, n_aqeq=1)
+    n = 2
+    cells = multiphase_cells(mp, n, seed=2)
+    kw = dict(rel_tol=1e-8, abs_tol=np.full(mp.n_state, 1e-12), max_steps=100000)
+    gpu, ref = CampSolver(mp, n, **kw), oracle_lib.Oracle(mp, n, **kw)
+    for s in (gpu, ref):
+        s.set_rates(cells.rates)
+    st, env = cells.state, cells.env
+    ref.update_env(env)
+    rc, jac = gpu.eval_jac(st, env, 10.0)
+    want = np.stack([ref.eval_jac(c, st[c], 10.0)[1] for c in range(n)])
+    assert rc == 0 and (np.abs(jac - want) <= 1e-12 * np.abs(want) + 1e-280).all()
+    rc, f = gpu.eval_deriv(st, env, 10.0, False)
+    want = np.stack([ref.eval_f(c, st[c], 10.0, False)[1] for c in range(n)])
+    assert rc == 0 and (np.abs(f - want) <= 1e-12 * np.abs(want) + 1e-280).all()
+    assert gpu.set_cells_per_block(2) == 2
+    a, b = st.copy(), st.copy()
+    assert gpu.solve(a, env, 0.0, 1.0) == 0
+    assert ref.run(b, env, 0.0, 1.0, mode=1) == 0
+    assert (np.abs(a - b) <= 1e-4 * np.abs(b) + 1e-8).all()
