@@ -93,9 +93,10 @@ __host__ __device__ inline size_t cell_bdf_wave_scratch(const DevProgram& P, int
 }
 
 // The no-allocation entry point's scratch (a file-scope device array of
-// kNoAllocScratchDoubles doubles, 64 MiB): the first kNoAllocHeaderDoubles
+// kNoAllocScratchDoubles doubles, 96 MiB, 316 wavefronts of the CB05-scale
+// mechanism with eight aerosol bins): the first kNoAllocHeaderDoubles
 // (256 bytes) hold the queue counter, the rest the wavefronts' scratch.
-constexpr size_t kNoAllocScratchDoubles = (size_t)8 << 20;
+constexpr size_t kNoAllocScratchDoubles = (size_t)12 << 20;
 constexpr size_t kNoAllocHeaderDoubles = 32;
 
 struct CellBdfArgs {

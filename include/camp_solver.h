@@ -268,7 +268,7 @@ int camp_solver_run_device(void *solver_data, double *d_state, double *d_env,
 /* No counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid it).  Same as camp_solver_run_device, but the per-cell kernel's
- * queue counter and wavefront scratch come from a fixed 64 MiB device array
+ * queue counter and wavefront scratch come from a fixed 96 MiB device array
  * in the library (one per GPU, kept until the process ends) and nothing is
  * allocated, on the device or on the host.  Per-cell mode only, without
  * phase timing or the Jacobian check; the solver's own buffers must exist
