@@ -7,6 +7,8 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
+#include <functional>
+#include <limits>
 
 namespace camp {
 
@@ -207,29 +209,39 @@ std::vector<int> markowitz_order(int n, const std::vector<int>& colptr,
   std::vector<char> A((size_t)n * n, 0);
   for (int j = 0; j < n; ++j)
     for (int k = colptr[j]; k < colptr[j + 1]; ++k) A[(size_t)rowval[k] * n + j] = 1;
-  std::vector<char> alive(n, 1);
-  std::vector<int> order;
-  for (int s = 0; s < n; ++s) {
-    long best = -1;
-    int bj = -1;
-    for (int j = 0; j < n; ++j) {
-      if (!alive[j]) continue;
-      long r = -1, c = -1;
-      for (int u = 0; u < n; ++u)
-        if (alive[u]) {
-          r += A[(size_t)j * n + u];
-          c += A[(size_t)u * n + j];
+  // entries of each row and column among the pivots left, the diagonal aside
+  std::vector<long> row(n, -1), col(n, -1);
+  for (int i = 0; i < n; ++i)
+    for (int j = 0; j < n; ++j)
+      if (A[(size_t)i * n + j]) {
+        ++row[i];
+        ++col[j];
+      }
+  std::vector<int> order, left(n), across;
+  for (int j = 0; j < n; ++j) left[j] = j;
+  while (!left.empty()) {
+    int b = left[0];
+    for (int j : left)
+      if (row[j] * col[j] < row[b] * col[b]) b = j;
+    left.erase(std::find(left.begin(), left.end(), b));
+    across.clear();
+    for (int c : left)
+      if (A[(size_t)b * n + c]) {
+        across.push_back(c);
+        --col[c];
+      }
+    for (int i : left) {
+      char* r = &A[(size_t)i * n];
+      if (!r[b]) continue;
+      --row[i];
+      for (int c : across)
+        if (!r[c]) {
+          r[c] = 1;
+          ++row[i];
+          ++col[c];
         }
-      long m = r * c;
-      if (best < 0 || m < best) best = m, bj = j;
     }
-    for (int i = 0; i < n; ++i) {
-      if (!alive[i] || i == bj || !A[(size_t)i * n + bj]) continue;
-      for (int c = 0; c < n; ++c)
-        if (alive[c] && c != bj && A[(size_t)bj * n + c]) A[(size_t)i * n + c] = 1;
-    }
-    order.push_back(bj);
-    alive[bj] = 0;
+    order.push_back(b);
   }
   return order;
 }
@@ -614,131 +626,189 @@ static void build_tri_program(Program& P, const std::vector<char>& F,
   for (int k = 0; k < nv; ++k) P.diag_pos[k] = to[P.diag_pos[k]];
 }
 
-// The factorisation's program (Program::lg_rec) of the filled pattern F with
-// value positions row_major,
-// for a register block of the last `tail` pivots.
-static void build_lu_program(Program& P, const std::vector<char>& F,
-                             const std::vector<int>& row_major, int tail) {
-  const int nv = P.nv, zero = P.lu_nnz + 64;
-  // (the positions are those the solve reads: Program::lu_at)
-  std::vector<int> pos = row_major;
-  for (int& p : pos)
-    if (p >= 0) p = P.lu_at[p];
-  const int d = P.lu_d = std::min(tail, nv), s = nv - d;
-  struct Task {
-    int i, j, waits = 0;
-    std::vector<int> k;   // the pivots whose products it takes
-    std::vector<int> out; // tasks that wait on it
-    long path = 0;        // groups from its start to the end of the longest chain
-  };
-  std::vector<Task> t(P.lu_nnz);
-  for (int i = 0; i < nv; ++i)
-    for (int j = 0; j < nv; ++j) {
-      const int p = pos[(size_t)i * nv + j];
-      if (p < 0) continue;
-      Task& a = t[p];
-      a.i = i;
-      a.j = j;
-      const int top = std::min(std::min(i, j), s);
-      for (int k = 0; k < top; ++k)
-        if (F[(size_t)i * nv + k] && F[(size_t)k * nv + j]) a.k.push_back(k);
-      auto wait = [&](int q) {
-        t[q].out.push_back(p);
-        ++a.waits;
-      };
-      for (int k : a.k) {
-        wait(pos[(size_t)i * nv + k]);
-        wait(pos[(size_t)k * nv + j]);
+// The factorisation's tasks (Program::lg_rec) for a filled pattern: what does not
+// depend on the register block's size, so that sizes can be compared.
+struct LuProduct {
+  uint16_t dst, l, u;
+};
+struct LuTasks {
+  int nv = 0;
+  std::vector<int> pos;               // (row, column) -> task (LU position) or -1
+  std::vector<int> row, col;          // of each task
+  std::vector<int> k_ptr, k;          // per task: the pivots whose products it takes, in order
+  std::vector<int> out_ptr, out;      // per task: the tasks that read it
+  std::vector<int> order;             // the tasks from the last pivot back
+  std::vector<int> j_of;              // Jacobian element or -1
+
+  LuTasks(const Program& P, const std::vector<LuProduct>& products,
+          const std::vector<int>& positions)
+      : nv(P.nv), pos(positions) {
+    const int n = P.lu_nnz;
+    row.resize(n);
+    col.resize(n);
+    for (int i = 0; i < nv; ++i)
+      for (int j = 0; j < nv; ++j) {
+        const int p = pos[(size_t)i * nv + j];
+        if (p < 0) continue;
+        row[p] = i;
+        col[p] = j;
       }
-      if (i > j && j < s) wait(pos[(size_t)j * nv + j]);
+    k_ptr.assign(n + 1, 0);
+    out_ptr.assign(n + 1, 0);
+    for (const LuProduct& x : products) {
+      ++k_ptr[x.dst + 1];
+      ++out_ptr[x.l + 1];
+      ++out_ptr[x.u + 1];
     }
-  auto groups = [&](const Task& a) { return std::max<long>(1, ((long)a.k.size() + 3) / 4); };
-  // longest chains, from the last tasks back (min(i, j) orders them; within
-  // one pivot the diagonal and its row precede the column)
-  std::vector<int> order(P.lu_nnz);
-  for (int p = 0; p < P.lu_nnz; ++p) order[p] = p;
-  std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-    const int mx = std::min(t[x].i, t[x].j), my = std::min(t[y].i, t[y].j);
-    return mx != my ? mx > my : (t[x].i > t[x].j) > (t[y].i > t[y].j);
-  });
-  for (int p : order) {
-    for (int q : t[p].out) t[p].path = std::max(t[p].path, t[q].path + kLuDist - 1);
-    t[p].path += groups(t[p]);
+    for (int p = 0; p < n; ++p)
+      if (row[p] > col[p]) ++out_ptr[diag(col[p]) + 1];
+    for (int p = 0; p < n; ++p) {
+      k_ptr[p + 1] += k_ptr[p];
+      out_ptr[p + 1] += out_ptr[p];
+    }
+    k.resize(k_ptr[n]);
+    out.resize(out_ptr[n]);
+    std::vector<int> k_at(k_ptr.begin(), k_ptr.end() - 1), at(out_ptr.begin(), out_ptr.end() - 1);
+    for (const LuProduct& x : products) {
+      k[k_at[x.dst]++] = col[x.l];
+      out[at[x.l]++] = x.dst;
+      out[at[x.u]++] = x.dst;
+    }
+    for (int p = 0; p < n; ++p)
+      if (row[p] > col[p]) out[at[diag(col[p])]++] = p;
+    // min(row, column) orders the tasks; within one pivot the diagonal and its
+    // row precede the column
+    order.resize(n);
+    for (int p = 0; p < n; ++p) order[p] = p;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+      const int mx = pivot(x), my = pivot(y);
+      return mx != my ? mx > my : (row[x] > col[x]) > (row[y] > col[y]);
+    });
+    j_of.assign(n, -1);
+    for (int e = 0; e < P.nnz; ++e) j_of[P.lu_at[P.m_to_lu[e]]] = e;
   }
-  std::vector<int> j_of(P.lu_nnz, -1);
-  for (int e = 0; e < P.nnz; ++e) j_of[P.lu_at[P.m_to_lu[e]]] = e;
-  // list scheduling: the ready task with the longest chain to a free lane
-  typedef std::pair<long, int> Ready;  // {path, -task}
-  std::vector<Ready> heap;
-  std::vector<std::vector<int>> due;   // tasks that become ready at a group
-  auto at = [&](size_t g) -> std::vector<int>& {
-    if (due.size() <= g) due.resize(g + 1);
-    return due[g];
+  int diag(int k) const { return pos[(size_t)k * nv + k]; }
+  // the pivot at which a task's value is final (and read by others)
+  int pivot(int p) const { return std::min(row[p], col[p]); }
+};
+
+// What a lane does in a group: step `step` of a task, 4 products.
+struct LuSlot {
+  int group, lane, task, step;
+};
+// Schedules the tasks for a register block of the last `tail` pivots into slots
+// and returns the number of groups, or `most` where it takes as many or more.
+static int schedule_lu(const LuTasks& T, int tail, int most, std::vector<LuSlot>& slots) {
+  slots.clear();
+  const int n = (int)T.row.size();
+  if (n == 0) return 0;
+  const int s = T.nv - std::min(tail, T.nv);
+  std::vector<int> groups(n), waits(n);
+  for (int p = 0; p < n; ++p) {
+    const int* k0 = T.k.data() + T.k_ptr[p];
+    const int c = (int)(std::lower_bound(k0, T.k.data() + T.k_ptr[p + 1], s) - k0);
+    groups[p] = std::max(1, (c + 3) / 4);
+    waits[p] = 2 * c + (T.row[p] > T.col[p] && T.col[p] < s ? 1 : 0);
+  }
+  // longest chains (groups from a task's start), from the last tasks back
+  std::vector<int> path(n, 0);
+  for (int p : T.order) {
+    if (T.pivot(p) < s)
+      for (int q = T.out_ptr[p]; q < T.out_ptr[p + 1]; ++q)
+        path[p] = std::max(path[p], path[T.out[q]] + kLuDist - 1);
+    path[p] += groups[p];
+  }
+  // list scheduling: the ready task with the longest chain (of equals the first)
+  // to a free lane; ready[c]: the ready tasks with a chain of c, a heap of their
+  // numbers, top: the longest
+  std::vector<std::vector<int>> ready(1 + *std::max_element(path.begin(), path.end()));
+  int top = 0;
+  // tasks that become ready at a group: linked lists (a group's tasks enter the
+  // heap together, so their order does not matter)
+  std::vector<int> due, next(n, -1), ready_at(n, 0);
+  auto put = [&](int g, int p) {
+    if ((int)due.size() <= g) due.resize(g + 1, -1);
+    next[p] = due[g];
+    due[g] = p;
   };
-  for (int p = 0; p < P.lu_nnz; ++p)
-    if (t[p].waits == 0) at(0).push_back(p);
-  std::vector<int> lane_task(64, -1), lane_step(64, 0);
-  std::vector<size_t> ready_at(P.lu_nnz, 0);
-  long left = P.lu_nnz;
-  P.lg_rec.clear();
-  P.lg_n = 0;
-  while (left > 0) {
-    const size_t g = (size_t)P.lg_n++;
-    if (g < due.size())
-      for (int p : due[g]) {
-        heap.push_back({t[p].path, -p});
-        std::push_heap(heap.begin(), heap.end());
+  for (int p = 0; p < n; ++p)
+    if (waits[p] == 0) put(0, p);
+  int lane_task[64], lane_step[64], left = n, g = 0;
+  std::fill(lane_task, lane_task + 64, -1);
+  for (; left > 0; ++g) {
+    if (g == most) return most;
+    if (g < (int)due.size())
+      for (int p = due[g]; p >= 0; p = next[p]) {
+        auto& h = ready[path[p]];
+        h.push_back(p);
+        std::push_heap(h.begin(), h.end(), std::greater<int>());
+        top = std::max(top, path[p]);
       }
-    const size_t r0 = P.lg_rec.size();
-    P.lg_rec.resize(r0 + 64 * 8, 0);
     for (int l = 0; l < 64; ++l) {
-      if (lane_task[l] < 0 && !heap.empty()) {
-        std::pop_heap(heap.begin(), heap.end());
-        lane_task[l] = -heap.back().second;
+      if (lane_task[l] < 0) {
+        while (top > 0 && ready[top].empty()) --top;
+        if (top == 0) continue;
+        auto& h = ready[top];
+        std::pop_heap(h.begin(), h.end(), std::greater<int>());
+        lane_task[l] = h.back();
         lane_step[l] = 0;
-        heap.pop_back();
+        h.pop_back();
       }
-      int* rec = &P.lg_rec[r0 + (size_t)l * 4];
-      int* hdr = &P.lg_rec[r0 + 64 * 4 + (size_t)l * 4];
-      for (int u = 0; u < 4; ++u) rec[u] = zero | (zero << 16);
-      hdr[0] = -1;
-      hdr[1] = zero | (zero << 16);
       const int p = lane_task[l];
-      if (p < 0) continue;
-      Task& a = t[p];
-      for (int u = 0; u < 4; ++u) {
-        const size_t q = (size_t)lane_step[l] * 4 + u;
-        if (q < a.k.size())
-          rec[u] = pos[(size_t)a.i * nv + a.k[q]] | (pos[(size_t)a.k[q] * nv + a.j] << 16);
-      }
-      const bool scaled = a.i > a.j && a.j < s;
-      const bool first = lane_step[l] == 0, last = lane_step[l] + 1 == groups(a);
-      if (first) hdr[0] = j_of[p];
-      hdr[1] = p | ((scaled ? pos[(size_t)a.j * nv + a.j] : zero) << 16);
-      hdr[2] = (first ? 1 : 0) | (last ? 2 : 0) | (scaled && last ? 4 : 0) | (a.i == a.j ? 8 : 0) |
-               (a.i == a.j && a.j < s ? 16 : 0);
-      ++lane_step[l];
-      if (last) {
-        lane_task[l] = -1;
-        --left;
-        for (int q : a.out) {
-          ready_at[q] = std::max(ready_at[q], g + kLuDist);
-          if (--t[q].waits == 0) at(ready_at[q]).push_back(q);
-        }
+      slots.push_back({g, l, p, lane_step[l]});
+      if (++lane_step[l] < groups[p]) continue;
+      lane_task[l] = -1;
+      --left;
+      if (T.pivot(p) >= s) continue;
+      for (int q = T.out_ptr[p]; q < T.out_ptr[p + 1]; ++q) {
+        const int t = T.out[q];
+        ready_at[t] = std::max(ready_at[t], g + kLuDist);
+        if (--waits[t] == 0) put(ready_at[t], t);
       }
     }
   }
-  for (int q = 0; q < kLuPad; ++q)
-    for (int l = 0; l < 64 * 8; ++l)
-      P.lg_rec.push_back(l < 64 * 4 ? zero | (zero << 16)
-                                    : l % 4 == 0 ? -1 : l % 4 == 1 ? zero | (zero << 16) : 0);
+  return g;
+}
+
+// The factorisation's program (Program::lg_rec) of a schedule for a register
+// block of the last `tail` pivots.
+static void build_lu_program(Program& P, const LuTasks& T, int tail, int n_groups,
+                             const std::vector<LuSlot>& slots) {
+  const int nv = P.nv, zero = P.lu_nnz + 64;
+  const int d = P.lu_d = std::min(tail, nv), s = nv - d;
+  P.lg_n = n_groups;
+  P.lg_rec.resize((size_t)(n_groups + kLuPad) * 64 * 8);
+  for (size_t q = 0; q < P.lg_rec.size(); q += 4) {
+    const bool rec = q / 256 % 2 == 0;
+    int* w = &P.lg_rec[q];
+    w[0] = rec ? zero | (zero << 16) : -1;
+    w[1] = zero | (zero << 16);
+    w[2] = w[3] = rec ? zero | (zero << 16) : 0;
+  }
+  for (const LuSlot& x : slots) {
+    int* rec = &P.lg_rec[(size_t)x.group * 64 * 8 + (size_t)x.lane * 4];
+    int* hdr = rec + 64 * 4;
+    const int p = x.task, i = T.row[p], j = T.col[p];
+    const int* k0 = T.k.data() + T.k_ptr[p];
+    const int c = (int)(std::lower_bound(k0, T.k.data() + T.k_ptr[p + 1], s) - k0);
+    for (int u = 0; u < 4 && x.step * 4 + u < c; ++u) {
+      const int k = k0[x.step * 4 + u];
+      rec[u] = T.pos[(size_t)i * nv + k] | (T.pos[(size_t)k * nv + j] << 16);
+    }
+    const bool scaled = i > j && j < s, first = x.step == 0,
+               last = x.step + 1 == std::max(1, (c + 3) / 4);
+    if (first) hdr[0] = T.j_of[p];
+    hdr[1] = p | ((scaled ? T.diag(j) : zero) << 16);
+    hdr[2] = (first ? 1 : 0) | (last ? 2 : 0) | (scaled && last ? 4 : 0) | (i == j ? 8 : 0) |
+             (i == j && j < s ? 16 : 0);
+  }
   P.lt_pos.clear();
   const int nb = (d + 7) / 8;
   for (int a = 0; a < nb; ++a)
     for (int b = 0; b < nb; ++b)
       for (int l = 0; l < 64; ++l) {
         const int i = 8 * a + l / 8, j = 8 * b + l % 8;
-        P.lt_pos.push_back(i < d && j < d ? pos[(size_t)(s + i) * nv + s + j] : -1);
+        P.lt_pos.push_back(i < d && j < d ? T.pos[(size_t)(s + i) * nv + s + j] : -1);
       }
 }
 
@@ -1391,52 +1461,53 @@ std::string Model::initialize() {
     }
   P.diag_pos.resize(nv);
   for (int k = 0; k < nv; ++k) P.diag_pos[k] = pos[(size_t)k * nv + k];
-  P.l_ptr.assign(1, 0);
-  P.u_ptr.assign(1, 0);
-  P.up_ptr.assign(1, 0);
-  for (int k = 0; k < nv; ++k) {
-    for (int i = k + 1; i < nv; ++i)
-      if (F[(size_t)i * nv + k]) {
-        P.l_pos.push_back(pos[(size_t)i * nv + k]);
-        P.l_row.push_back(i);
-      }
-    for (int i = 0; i < k; ++i)
-      if (F[(size_t)i * nv + k]) {
-        P.u_pos.push_back(pos[(size_t)i * nv + k]);
-        P.u_row.push_back(i);
-      }
-    for (int i = k + 1; i < nv; ++i) {
-      if (!F[(size_t)i * nv + k]) continue;
-      for (int j = k + 1; j < nv; ++j) {
-        if (!F[(size_t)k * nv + j]) continue;
-        P.up_dst.push_back((uint16_t)pos[(size_t)i * nv + j]);
-        P.up_l.push_back((uint16_t)pos[(size_t)i * nv + k]);
-        P.up_u.push_back((uint16_t)pos[(size_t)k * nv + j]);
-      }
-    }
-    P.l_ptr.push_back((int)P.l_pos.size());
-    P.u_ptr.push_back((int)P.u_pos.size());
-    P.up_ptr.push_back((int)P.up_dst.size());
-  }
   if (P.lu_nnz + 64 > 65535) return "LU fill exceeds 65471 entries per cell";
   build_tri_program(P, F, pos);
+  // (from here on the positions are those the solve reads: Program::lu_at)
+  for (int& q : pos)
+    if (q >= 0) q = P.lu_at[q];
+  // the elimination's products LU[dst] -= LU[l] * LU[u], in pivot order
+  std::vector<LuProduct> products;
+  products.reserve((size_t)4 * P.lu_nnz);
+  std::vector<int> u;
+  for (int k = 0; k < nv; ++k) {
+    u.clear();
+    for (int j = k + 1; j < nv; ++j)
+      if (pos[(size_t)k * nv + j] >= 0) u.push_back(j);
+    for (int i = k + 1; i < nv; ++i) {
+      const int* pi = &pos[(size_t)i * nv];
+      if (pi[k] < 0) continue;
+      ++P.n_lower;
+      for (int j : u)
+        products.push_back({(uint16_t)pi[j], (uint16_t)pi[k], (uint16_t)pos[(size_t)k * nv + j]});
+    }
+  }
+  P.n_updates = (long)products.size();
   // The block's size by what a factorisation then costs: the tasks' groups
   // (about 600 cycles each) against the block's pivots, whose cost grows with
   // its size (350 to 850 cycles, measured).  CB05cl_ae5, two thirds of whose
   // last 40 x 40 are zeros, takes 16 (42k -> 21k cycles), the CB05-scale
   // mechanism 32 (55k -> 49k).  Large factors end in a dense block: all 40.
-  int best = kLuTail;
+  const LuTasks tasks(P, products, pos);
+  std::vector<LuSlot> slots, trial;
+  int best = kLuTail, n_groups = 0;
   double best_cost = 0.0;
-  for (int d = 8; P.lu_nnz <= 4096 && d <= kLuTail; d += 8) {
-    build_lu_program(P, F, pos, d);
-    const double cost = 600.0 * P.lg_n + P.lu_d * (230.0 + 125.0 * (d / 8));
-    if (d == 8 || cost < best_cost) {
-      best = d;
-      best_cost = cost;
-    }
-    if (d >= nv) break;
+  // (from the largest down, as long as the cost falls: the schedule's chain grows
+  // with every pivot outside the block)
+  for (int d = std::max(8, std::min(kLuTail, (nv + 7) / 8 * 8)); d >= 8; d -= 8) {
+    const double block = std::min(d, nv) * (230.0 + 125.0 * (d / 8));
+    const int most = best_cost > 0.0 ? (int)std::max(0.0, (best_cost - block) / 600.0) + 1
+                                     : std::numeric_limits<int>::max();
+    const int n = schedule_lu(tasks, d, most, trial);
+    const double cost = 600.0 * n + block;
+    if (best_cost > 0.0 && cost >= best_cost) break;
+    best = d;
+    best_cost = cost;
+    n_groups = n;
+    std::swap(slots, trial);
+    if (P.lu_nnz > 4096) break;
   }
-  build_lu_program(P, F, pos, best);
+  build_lu_program(P, tasks, best, n_groups, slots);
   initialized = true;
   // the f gather's final pass in slot order: {species, first partial, count}
   // (at least one pass: f loads the first one ahead)

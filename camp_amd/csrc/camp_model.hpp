@@ -127,10 +127,7 @@ struct Program {
   // LU (positions in the permuted LU value array)
   std::vector<int> perm, iperm;                     // perm[k] = dep index of pivot k
   std::vector<int> m_to_lu, diag_pos;               // [nnz], [nv]
-  std::vector<int> l_ptr, l_pos, l_row;             // per pivot k: L(:,k) below k
-  std::vector<int> u_ptr, u_pos, u_row;             // per pivot k: U(:,k) above k
-  std::vector<int> up_ptr;                          // per pivot k: update range
-  std::vector<uint16_t> up_dst, up_l, up_u;         // LU[dst] -= LU[l] * LU[u]
+  long n_lower = 0, n_updates = 0;                  // entries of L, products l * u
   // The factorisation's program (built by build_lu_program).  Every LU value is
   // one task: its matrix entry, then the products l * u it receives, in pivot
   // order, then (below the diagonal) the pivot's reciprocal.  Values of the
@@ -166,7 +163,6 @@ struct Program {
   // rows -> position).
   int tri_s = 0, tri_d = 0, tri_nf = 0, tri_nb = 0, tt_nf = 0, tt_nb = 0;
   std::vector<int> tri_e, tri_r, tt, lu_at;
-  long n_updates() const { return (long)up_dst.size(); }
 
   // ---- lane-group f and J (gas-phase programs) ------------------------------
   // G lanes integrate one cell's f(y) or J(y), 64 / G cells per wavefront,

@@ -1926,7 +1926,7 @@ extern "C" void camp_solver_work_model(void* solver_data, double* out8) {
     f += 40.0 * G.n_pi + 60.0 * G.n_zi + 80.0 * G.n_sp + 60.0 * G.n_aq;
     j += 12.0 * (G.js_ptr.back()) + 2.0 * G.jm_rxn.size() + 120.0 * G.n_sp + 40.0 * G.n_aq;
   }
-  double lu = 2.0 * G.nnz + (double)G.l_pos.size() + 2.0 * G.up_dst.size();
+  double lu = 2.0 * G.nnz + (double)G.n_lower + 2.0 * G.n_updates;
   double sv = 2.0 * (G.lu_nnz - G.nv) + G.nv;
   double nr = G.n_terms;
   out8[0] = f;
