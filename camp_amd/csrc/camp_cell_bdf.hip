@@ -10,6 +10,7 @@
 // in LDS (Nordsieck history, work vectors, rate constants, LU factors);
 // only the cell's saved Jacobian history (J_solver, J_state, J_deriv,
 // camp_solver.c:1111-1114) is in HBM, because CAMP keeps it across calls.
+#include <cstddef>
 #include <cstdio>
 #include <mutex>
 #include <type_traits>
@@ -93,6 +94,7 @@ struct CellCv {
   // compiler would otherwise, the ~90 pointers overflow the scalar registers
   // into lanes of vector registers, and each use costs a v_readlane pair (24
   // cycles each).
+  static_assert(offsetof(CellBdfArgs, P) == 0, "the program is read at the kernel arguments' start");
   __device__ __forceinline__ static const DevProgram& program() {
     auto k = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(k));
