@@ -463,9 +463,19 @@ __host__ __device__ inline size_t est_doubles(const DevProgram& P) {
 __device__ __forceinline__ void est_stage(const DevProgram& P, int lane, const double* Js,
                                           const double* Jf, double* E) {
   lane = phase_lane(lane);
-  for (int p = lane; p < P.es_n; p += kWave) {
-    const int e = P.es_src[p];
-    E[p] = e >= 0 ? Js[e] : 0.0;
+  // eight elements a lane at a time, the loads of each kind together (one after
+  // another they are two trips to the caches per row of 64)
+  constexpr int B = 8;
+  for (int p0 = lane; p0 < P.es_n; p0 += B * kWave) {
+    int e[B];
+    double v[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) e[u] = P.es_src[min(p0 + u * kWave, P.es_n - 1)];
+#pragma unroll
+    for (int u = 0; u < B; ++u) v[u] = Js[e[u] >= 0 ? e[u] : 0];
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      if (p0 + u * kWave < P.es_n) E[p0 + u * kWave] = e[u] >= 0 ? v[u] : 0.0;
   }
   for (int s = lane; s < P.nv; s += kWave) E[P.es_n + s] = Jf[P.fs_species[s]];
   __threadfence_block();
