@@ -514,7 +514,7 @@ struct CellCv {
   __device__ __forceinline__ int factor() {
     const DevProgram& P = program();
     long long t0 = tick();
-    int rc = cell_lu_factor(P, lane, Js, gamma, lu, s_fb);
+    int rc = cell_lu_factor<false>(P, lane, Js, gamma, lu, s_fb);
     if (prof) c_lu += clock64() - t0;
     return rc;
   }
@@ -522,7 +522,7 @@ struct CellCv {
   __device__ __forceinline__ void lsolve(double* b) {
     const DevProgram& P = program();
     long long t0 = tick();
-    cell_lu_solve<MP || PL == kPlaceGlobalLu || PL == kPlaceWide>(P, lane, lu, b, w);
+    cell_lu_solve<MP || PL == kPlaceGlobalLu || PL == kPlaceWide, false>(P, lane, lu, b, w);
     if (prof) c_sol += clock64() - t0;
     if (uc(gamrat != 1.0)) {
       double s = 2.0 / (1.0 + gamrat);

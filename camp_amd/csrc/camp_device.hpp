@@ -819,10 +819,45 @@ __device__ __forceinline__ void lu_run(const LuGroup& S, double gamma, double* l
   wsync();
 }
 
-// The dense block of the last lu_d pivots, NB blocks of 8.  A pivot's row and
+// The block of the last lu_d pivots in memory, pivot by pivot, products of its
+// entries only.  The dense elimination below also multiplies entries the pattern
+// does not have; as zeros they change nothing unless a value is not finite.
+__device__ __forceinline__ bool lu_tail_sparse(const DevProgram& P, int lane, double* lu) {
+  const int d = P.lu_d, nb = (d + 7) / 8, r = lane >> 3, c = lane & 7;
+  auto at = [&](int i, int j) {
+    return i < d && j < d ? P.lt_pos[((i >> 3) * nb + (j >> 3)) * kWave + (i & 7) * 8 + (j & 7)]
+                          : -1;
+  };
+  bool bad = false;
+#pragma nounroll
+  for (int k = 0; k < d; ++k) {
+    const double piv = lu[at(k, k)];
+    bad |= !(piv != 0.0 && isfinite(piv));
+    const double rinv = 1.0 / piv;
+    wsync();
+#pragma nounroll
+    for (int i = k + 1 + lane; i < d; i += kWave) {
+      const int p = at(i, k);
+      if (p >= 0) lu[p] = lu[p] * rinv;
+    }
+    wsync();
+#pragma nounroll
+    for (int b = (k >> 3) * (nb + 1); b < nb * nb; ++b) {
+      const int i = 8 * (b / nb) + r, j = 8 * (b % nb) + c;
+      if (i <= k || j <= k) continue;
+      const int p = at(i, j), l = at(i, k), u = at(k, j);
+      if (p >= 0 && l >= 0 && u >= 0) lu[p] = lu[p] - lu[l] * lu[u];
+    }
+    wsync();
+  }
+  return bad;
+}
+
+// The dense block of the last lu_d pivots, NB blocks of 8.  Returns whether a
+// pivot is zero or not finite; EXACT: or any value, and then stores nothing.  A pivot's row and
 // column go through LDS (buf) by lane: the NB values a lane needs of either are
 // consecutive.
-template <int NB>
+template <int NB, bool EXACT>
 __device__ __forceinline__ bool lu_tail(const DevProgram& P, int lane, double* lu, double* buf) {
   constexpr int W = kLuTailStride;  // doubles per lane group of 8
   const int d = P.lu_d, r = lane >> 3, c = lane & 7;
@@ -874,6 +909,13 @@ __device__ __forceinline__ bool lu_tail(const DevProgram& P, int lane, double* l
       wsync();
     }
   }
+  if (EXACT) {
+#pragma unroll
+    for (int p = 0; p < NB; ++p)
+#pragma unroll
+      for (int q = 0; q < NB; ++q) bad |= !isfinite(a[p][q]);
+    if (__builtin_amdgcn_ballot_w64(bad) != 0) return true;
+  }
 #pragma unroll
   for (int p = 0; p < NB; ++p)
 #pragma unroll
@@ -885,6 +927,10 @@ __device__ __forceinline__ bool lu_tail(const DevProgram& P, int lane, double* l
   return bad;
 }
 
+// EXACT: the block entry by entry where a value is not finite (lu_tail_sparse).
+// The integrator does without: to it such factors are a failed set-up as a bad
+// pivot is, and the code costs it registers (1 to 2 % of a step).
+template <bool EXACT>
 __device__ __forceinline__ int cell_lu_factor(const DevProgram& P, int lane, const double* J,
                                               double gamma, double* lu, double* buf) {
   lane = phase_lane(lane);
@@ -915,14 +961,17 @@ __device__ __forceinline__ int cell_lu_factor(const DevProgram& P, int lane, con
       lu_prog(P, lane, n + u + NS, S[u]);
     }
   }
+  bool odd = false;
   switch ((P.lu_d + 7) / 8) {
     case 0: break;  // no solver variables
-    case 1: bad |= lu_tail<1>(P, lane, lu, buf); break;
-    case 2: bad |= lu_tail<2>(P, lane, lu, buf); break;
-    case 3: bad |= lu_tail<3>(P, lane, lu, buf); break;
-    case 4: bad |= lu_tail<4>(P, lane, lu, buf); break;
-    default: bad |= lu_tail<5>(P, lane, lu, buf); break;
+    case 1: odd = lu_tail<1, EXACT>(P, lane, lu, buf); break;
+    case 2: odd = lu_tail<2, EXACT>(P, lane, lu, buf); break;
+    case 3: odd = lu_tail<3, EXACT>(P, lane, lu, buf); break;
+    case 4: odd = lu_tail<4, EXACT>(P, lane, lu, buf); break;
+    default: odd = lu_tail<5, EXACT>(P, lane, lu, buf); break;
   }
+  if (EXACT && odd) odd = lu_tail_sparse(P, lane, lu);
+  bad |= odd;
   return wave_or(bad ? 1 : 0);
 }
 
@@ -948,7 +997,8 @@ __device__ __forceinline__ double readlane_d(double v, int l) {
 //    in LDS, so that a batch costs one LDS round trip and independent rows
 //    (the aerosol's size bins) run side by side.
 // Every row adds its entries in elimination order, one product at a time, so
-// the results are those of the pivot-by-pivot sweeps bit for bit.  All LU
+// the results are those of the pivot-by-pivot sweeps bit for bit, as long as they
+// are finite and quot's operands in range (see cell_lu_solve).  All LU
 // values and positions are known before the sweep and are loaded ahead of it
 // (AH batches; the program NS ahead), so a batch waits on the unknowns only.
 // Cycles per solve: 1024 multi-phase cells 557k -> 84k, one cell 381k -> 54k;
@@ -1042,11 +1092,18 @@ __device__ __forceinline__ void tail_vals(const double* lu, TailBlock& S) {
 // x / dg for every lane: the quotient from the correctly rounded reciprocal y
 // with two residual corrections, which is the correctly rounded quotient (P.
 // Markstein, IBM J. Res. Dev. 34(1), 1990) in a third of the latency of the
-// division, which sits on the chain of every pivot.
+// division, which sits on the chain of every pivot -- as long as nothing on the
+// way over- or underflows.  quot_ok: the reciprocal and the first quotient are
+// normal and the residual x - dg q, a multiple of 2^-104 of x, is exact.
 __device__ __forceinline__ double quot(double x, double dg, double y) {
   double q = x * y;
   q = fma(fma(-dg, q, x), y, q);
   return fma(fma(-dg, q, x), y, q);
+}
+__device__ __forceinline__ bool quot_ok(double x, double dg, double q) {
+  const double ax = fabs(x), ad = fabs(dg), aq = fabs(q);
+  return ad >= 0x1p-1000 && ad <= 0x1p1000 &&
+         (x == 0.0 || (ax >= 0x1p-900 && ax <= 0x1p1000 && aq >= 0x1p-900 && aq <= 0x1p1000));
 }
 // Eight pivots of the tail, k0 onwards (or downwards).
 template <bool FWD, bool FMA>
@@ -1091,8 +1148,10 @@ __device__ __forceinline__ void tri_tail(const DevProgram& P, int lane, const do
 }
 
 // x in X (LDS): indexed by solver variable for FMA programs, else by pivot.
+// Returns false where a quotient of the tail may not be the correctly rounded
+// one (non-FMA programs).
 template <bool FMA, int AH, int NS>
-__device__ __forceinline__ void tri_solve(const DevProgram& P, int lane, const double* lu,
+__device__ __forceinline__ bool tri_solve(const DevProgram& P, int lane, const double* lu,
                                           double* X) {
   vm_drain();
   const bool on = lane < P.tri_d;
@@ -1105,16 +1164,73 @@ __device__ __forceinline__ void tri_solve(const DevProgram& P, int lane, const d
   const double y = 1.0 / dg;
   if (FMA) x *= y;
   tri_tail<false, FMA, AH>(P, lane, lu, dg, y, x);
-  if (!FMA) x = quot(x, dg, y);
+  bool ok = true;
+  if (!FMA) {
+    const double q = quot(x, dg, y);
+    ok = !on || quot_ok(x, dg, q);
+    x = q;
+  }
   if (on) X[ix] = x;
   wsync();
   tri_head<false, FMA, AH, NS>(P, lane, lu, X);
+  return ok;
+}
+
+// The same solve of a program with separate products, entry by entry: no
+// product with the padding's zeros, divisions by the diagonal.  With values
+// that are not finite, or too small for quot, these are not the same.
+__device__ __forceinline__ void tri_solve_sparse(const DevProgram& P, int lane, const double* lu,
+                                                 double* X) {
+  const int zero = P.lu_nnz + kWave;
+  auto head = [&](bool fwd) {
+    const int n0 = fwd ? 0 : P.tri_nf + kTriPad, nb = fwd ? P.tri_nf : P.tri_nb;
+#pragma nounroll
+    for (int n = 0; n < nb; ++n) {
+      const int* e = (const int*)P.tri_e + (size_t)(n0 + n) * 2 * kWave * 4 + 4 * lane;
+      const int2 r = P.tri_r[(size_t)(n0 + n) * kWave + lane];
+      const int row = r.x & 0xFFFF;
+      double acc = X[row == 0xFFFF ? 0 : row];
+#pragma nounroll
+      for (int u = 0; u < 8; ++u) {
+        const int w = e[(u >> 2) * kWave * 4 + (u & 3)];
+        if ((w & 0xFFFF) != zero) acc = acc - lu[w & 0xFFFF] * X[(unsigned)w >> 16];
+      }
+      if (!fwd && (r.x & (1 << 17))) acc = acc / lu[r.y];
+      if (row != 0xFFFF) X[row] = acc;
+      wsync();
+    }
+  };
+  const int d = P.tri_d;
+  auto tail = [&](bool fwd, double dg, double& x) {
+    const int4* tb = P.tt + (size_t)(fwd ? 0 : P.tt_nf + kTriPad) * kWave + lane;
+#pragma nounroll
+    for (int k = 0; k < d; ++k) {
+      const int* t = (const int*)(tb + (size_t)(k >> 3) * kWave);
+      const int p = (int)(((unsigned)t[(k & 7) >> 1] >> (16 * (k & 1))) & 0xFFFF);
+      const double xk = readlane_d(fwd ? x : x / dg, fwd ? k : d - 1 - k);
+      if (p != zero && !(fwd && k == d - 1)) x = x - lu[p] * xk;
+    }
+  };
+  const bool on = lane < d;
+  const int r = on ? P.tri_s + lane : 0;
+  const double dg = on ? lu[P.diag_pos[r]] : 1.0;
+  head(true);
+  double x = on ? X[r] : 0.0;
+  tail(true, 1.0, x);
+  tail(false, dg, x);
+  if (on) X[r] = x / dg;
+  wsync();
+  head(false);
 }
 
 // Solve (LU) x = b in place; b in dep order, w a scratch vector (nv) in LDS,
 // used past kTriInPlace.  FAR: the factors live in global memory (multi-phase
-// programs) and are fetched two batches ahead instead of one.
-template <bool FAR>
+// programs) and are fetched two batches ahead instead of one.  EXACT: a solution
+// with values that are not finite, or quotients outside quot's range, is that of
+// the pivot-by-pivot sweeps too: entry by entry past kTriInPlace, NaN as a whole
+// up to it.  The integrator does without: it rejects a correction that is not
+// finite whatever values it has, and an ulp of one under 2^-900 decides nothing.
+template <bool FAR, bool EXACT>
 __device__ __forceinline__ void cell_lu_solve(const DevProgram& P, int lane, double* lu, double* b,
                                               double* w) {
   lane = phase_lane(lane);
@@ -1125,12 +1241,26 @@ __device__ __forceinline__ void cell_lu_solve(const DevProgram& P, int lane, dou
     wsync();
   }
   if (P.nv <= kTriInPlace) {
-    tri_solve<true, FAR ? 2 : 1, 4>(P, lane, lu, b);
+    (void)tri_solve<true, FAR ? 2 : 1, 4>(P, lane, lu, b);
+    if (!EXACT) return;
+    bool odd = false;
+    for (int i = lane; i < P.nv; i += kWave) odd |= !isfinite(b[i]);
+    if (__builtin_amdgcn_ballot_w64(odd) != 0)
+      for (int i = lane; i < P.nv; i += kWave) b[i] = __builtin_nan("");
+    wsync();
     return;
   }
   for (int k = lane; k < P.nv; k += kWave) w[k] = b[P.perm[k]];
   wsync();
-  tri_solve<false, FAR ? 2 : 1, 4>(P, lane, lu, w);
+  bool ok = tri_solve<false, FAR ? 2 : 1, 4>(P, lane, lu, w);
+  if (EXACT) {
+    for (int k = lane; k < P.nv; k += kWave) ok = ok && isfinite(w[k]);
+    if (__builtin_amdgcn_ballot_w64(!ok) != 0) {
+      for (int k = lane; k < P.nv; k += kWave) w[k] = b[P.perm[k]];
+      wsync();
+      tri_solve_sparse(P, lane, lu, w);
+    }
+  }
   for (int k = lane; k < P.nv; k += kWave) b[P.perm[k]] = w[k];
   wsync();
 }

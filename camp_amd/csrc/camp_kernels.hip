@@ -430,7 +430,7 @@ __global__ void __launch_bounds__(64) k_lu_factor(DevProgram P, int nc, const do
   int lane = threadIdx.x;
   double* s_lu = smem;
   for (int c = blockIdx.x; c < nc; c += gridDim.x) {
-    int bad = cell_lu_factor(P, lane, J + (size_t)c * P.nnz, gamma, s_lu,
+    int bad = cell_lu_factor<true>(P, lane, J + (size_t)c * P.nnz, gamma, s_lu,
                              s_lu + P.lu_nnz + kWave + 1);
     if (bad) {
       if (lane == 0) atomicOr(fail, 1);
@@ -458,7 +458,7 @@ __global__ void __launch_bounds__(64) k_lu_solve(DevProgram P, int nc, const dou
     double* bc = b + (size_t)c * P.nv;
     for (int i = lane; i < P.nv; i += kWave) s_b[i] = bc[i];
     wsync();
-    cell_lu_solve<false>(P, lane, s_lu, s_b, s_w);
+    cell_lu_solve<false, true>(P, lane, s_lu, s_b, s_w);
     for (int i = lane; i < P.nv; i += kWave) bc[i] = s != 1.0 ? s_b[i] * s : s_b[i];
     wsync();
   }
