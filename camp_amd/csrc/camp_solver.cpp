@@ -1756,8 +1756,9 @@ extern "C" int camp_eval_deriv(void* solver_data, const double* state, const dou
   s->ensure_device();
   int nc = s->m.nc;
   const camp::DevProgram& P = s->P;
-  double* d_y = s->kept(s->d_eval_y, (size_t)nc * P.nv);
-  double* d_f = s->kept(s->d_eval_f, (size_t)nc * P.nv);
+  Solver::EvalArrays mem(*s, 2 * (size_t)nc * P.nv);
+  double* d_y = mem.take((size_t)nc * P.nv);
+  double* d_f = mem.take((size_t)nc * P.nv);
   eval_prepare(s, state, env, d_y);
   // (a cell whose f fails keeps zeros)
   HIP_OK(hipMemsetAsync(d_f, 0, (size_t)nc * P.nv * sizeof(double), s->stream));
@@ -1783,7 +1784,8 @@ extern "C" int camp_eval_jac(void* solver_data, const double* state, const doubl
   int nc = s->m.nc;
   const camp::DevProgram& P = s->P;
   std::vector<void*> tmp;
-  double* d_y = s->kept(s->d_eval_y, (size_t)nc * P.nv);
+  Solver::EvalArrays mem(*s, (size_t)nc * P.nv);
+  double* d_y = mem.take((size_t)nc * P.nv);
   eval_prepare(s, state, env, d_y);
   HIP_OK(hipMemsetAsync(s->d_fail, 0, sizeof(int), s->stream));
   double* d_jr = P.mp ? camp::dev_alloc<double>((size_t)nc * P.rnnz, tmp) : nullptr;
@@ -1866,9 +1868,10 @@ extern "C" int camp_eval_lu_solve(void* solver_data, const double* jac, double g
   s->ensure_device();
   int nc = s->m.nc;
   const camp::DevProgram& P = s->P;
-  double* d_J = s->kept(s->d_eval_J, (size_t)nc * P.nnz);
-  double* d_LU = s->kept(s->d_eval_LU, (size_t)nc * P.lu_nnz);
-  double* d_b = s->kept(s->d_eval_f, (size_t)nc * P.nv);
+  Solver::EvalArrays mem(*s, (size_t)nc * (P.nnz + P.lu_nnz + P.nv));
+  double* d_J = mem.take((size_t)nc * P.nnz);
+  double* d_LU = mem.take((size_t)nc * P.lu_nnz);
+  double* d_b = mem.take((size_t)nc * P.nv);
   // (a cell whose factorisation fails is solved with zeros)
   HIP_OK(hipMemsetAsync(d_LU, 0, (size_t)nc * P.lu_nnz * sizeof(double), s->stream));
   HIP_OK(hipMemcpyAsync(d_J, jac, (size_t)nc * P.nnz * sizeof(double), hipMemcpyHostToDevice, s->stream));

@@ -164,6 +164,7 @@ struct Solver {
     if (h_fail_pin) (void)hipHostFree(h_fail_pin);
     for (void* p : owned) (void)hipFree(p);
     if (d_wave_scratch) (void)hipFree(d_wave_scratch);
+    drop_eval();
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (stream) (void)hipStreamDestroy(stream);
@@ -176,11 +177,43 @@ struct Solver {
     if (!stream) setup_device();
   }
   void upload_renv();
-  // The layer entry points' (camp_eval_deriv, camp_eval_jac) solver variables
-  // and f(y) of all cells, made by the first such call
-  double *d_eval_y = nullptr, *d_eval_f = nullptr;
-  double *d_eval_J = nullptr, *d_eval_LU = nullptr;  // camp_eval_lu_solve
-  double* kept(double*& p, size_t n) { return p ? p : p = dev_alloc<double>(n, owned); }
+  // The layer entry points' (camp_eval_*) device arrays: one block that the next
+  // such call uses again.  A call that needs more than kEvalKept returns it at
+  // its end: allocating it (and clearing what needs it) is 0.1 ms, little against
+  // the copies of so many cells, and a solver that is called once for a large
+  // grid does not hold on to gigabytes.
+  static constexpr size_t kEvalKept = (size_t)512 << 20;
+  double* d_eval = nullptr;
+  size_t eval_bytes = 0;
+  struct EvalArrays {
+    Solver& S;
+    double* at;
+    // doubles: of all arrays that take() will hand out
+    EvalArrays(Solver& s, size_t doubles) : S(s) {
+      const size_t bytes = std::max<size_t>(doubles, 1) * sizeof(double);
+      if (bytes > S.eval_bytes) {
+        S.drop_eval();
+        HIP_OK(hipMalloc(&S.d_eval, bytes));
+        S.eval_bytes = bytes;
+      }
+      at = S.d_eval;
+    }
+    ~EvalArrays() {
+      if (S.eval_bytes > kEvalKept) S.drop_eval();
+    }
+    EvalArrays(const EvalArrays&) = delete;
+    EvalArrays& operator=(const EvalArrays&) = delete;
+    double* take(size_t n) {
+      double* p = at;
+      at += n;
+      return p;
+    }
+  };
+  void drop_eval() {
+    if (d_eval) (void)hipFree(d_eval);
+    d_eval = nullptr;
+    eval_bytes = 0;
+  }
   // Per-cell kernel arguments with the solver's program and controls filled
   // in (buffers left to the caller), and the launch shape for nq queued cells.
   CellBdfArgs cell_args() const;

@@ -3,9 +3,11 @@ import dataclasses
 
 import numpy as np
 import pytest
+import torch
 
 from camp_amd.core import CampSolver
-from camp_amd.mechanisms import Mechanism, Reaction, box_mechanism, synthetic_cells
+from camp_amd.mechanisms import (Mechanism, Reaction, box_mechanism, cb05_scale_mechanism,
+                                 synthetic_cells)
 from camp_amd.multiphase import multiphase_cells, multiphase_mechanism
 
 pytestmark = pytest.mark.gpu
@@ -148,3 +150,25 @@ def test_many_aerosol_species_and_few_reactions(oracle_lib):
     assert gpu.solve(a, env, 0.0, 1.0) == 0
     assert ref.run(b, env, 0.0, 1.0, mode=1) == 0
     assert (np.abs(a - b) <= 1e-4 * np.abs(b) + 1e-8).all()
+
+
+def test_layer_calls_of_a_large_grid_return_their_memory():
+    """f, then one factorisation and solve of 30000 cells (680 MB of device
+    arrays): what the second call took is free again, and the calls give the
+    same results as before, whichever came before them."""
+    n = 30000
+    mech = cb05_scale_mechanism(1)
+    gpu = CampSolver(mech, n)
+    cells = synthetic_cells(mech, 1, seed=2)
+    state, env = np.tile(cells.state, (n, 1)), np.tile(cells.env, (n, 1))
+    gpu.set_rates({k: np.repeat(v, n) for k, v in cells.rates.items()})
+    f0 = gpu.eval_deriv(state, env)[1]
+    free = torch.cuda.mem_get_info()[0]
+    rows = gpu.pattern()["rowval"]
+    cols = np.repeat(np.arange(gpu.nv), np.diff(gpu.pattern()["colptr"]))
+    jac = np.tile(np.where(rows == cols, -1.0, 1e-3), (n, 1))
+    b = np.ones((n, gpu.nv))
+    x0 = gpu.eval_lu_solve(jac, 0.5, b)[1]
+    assert torch.cuda.mem_get_info()[0] > free - (64 << 20)
+    assert np.array_equal(gpu.eval_deriv(state, env)[1], f0)
+    assert np.array_equal(gpu.eval_lu_solve(jac, 0.5, b)[1], x0)
