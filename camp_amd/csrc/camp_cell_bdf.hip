@@ -1168,9 +1168,8 @@ __global__ void __launch_bounds__(256)
   }
   cv.acor = v; v += nv;
   cv.y = v; v += nv;
-  // the column solve's scratch w (nv > 128 only: smaller programs solve in
-  // registers) stays in LDS except for gas-phase cells with the history in
-  // global memory, whose LDS it would push past six cells per CU
+  // the solve's scratch w (used past kTriInPlace only) stays in LDS except where
+  // it would take a place from another cell of a small program
   if (kNewtonLds) {
     cv.w = vh; vh += nv;
   } else {
@@ -1179,11 +1178,11 @@ __global__ void __launch_bounds__(256)
   // Without GH the J history (J_solver, J_state, J_deriv) is staged in LDS
   // for the whole solve; with GH it is used in place in HBM.
   double *h_js = nullptr, *h_jy = nullptr, *h_jf = nullptr;
-  // the f gather's scratch follows the LU values (gas: also the LU's sinks)
+  // the f gather's scratch follows the LU values (their zero slot lies in it)
   if (MP) {
     cv.lu = scratch;
     cv.Jr = scratch + P.lu_nnz + kWave + 1;
-    cv.s_fb = v; v += fb_sink_doubles(P);
+    cv.s_fb = v; v += fb_scratch_doubles(P);
   } else {
     cv.Jr = nullptr;
     if (GL) {
@@ -1192,7 +1191,7 @@ __global__ void __launch_bounds__(256)
       cv.lu = v;
       v += kNewtonLds ? cell_lu_lds(P) : P.lu_nnz;
     }
-    cv.s_fb = v; v += fb_sink_doubles(P);
+    cv.s_fb = v; v += fb_scratch_doubles(P);
     if (!GH) {
       h_js = v; v += P.nnz;
       h_jy = v; v += nv;

@@ -4,8 +4,8 @@
 // Execution model: one wavefront (64 lanes) owns one grid cell at a time.
 // The cell's state, rate constants, BDF vectors and LU factors live in LDS;
 // lanes split the work of each sparse phase (rate terms and species in
-// f(y), Jacobian elements in J(y), updates of one pivot in the LU, the
-// column of one pivot in the triangular solves).  Every decision that
+// f(y), Jacobian elements in J(y), entries of the LU factors in the
+// factorisation, ready rows in the triangular solves).  Every decision that
 // controls the cell's integration is made on wave-uniform values (lane 0's
 // reduction result is broadcast), so a wavefront never diverges between
 // cells and never needs a workgroup barrier.
@@ -26,7 +26,6 @@ __host__ __device__ constexpr size_t even_up(size_t n) { return n + (n & 1); }
 struct DevProgram {
   int ns, nv, nnz, n_env, n_terms, lu_nnz, n_rxn;
   const int* dep_state;
-  const int* j_ptr;
   const int *colptr, *rowval;  // solver pattern (dep ids, CSC)
   // lane-group f/J programs (gas-phase programs; Program::gf_rec), one per
   // group width (8, 16, 32 lanes per cell)
@@ -47,9 +46,6 @@ struct DevProgram {
   int tri_s, tri_d, tri_nf, tri_nb, tt_nf, tt_nb;
   const int4 *tri_e, *tt;
   const int2* tri_r;
-  const int4* je_a;  // packed J records (see Program in camp_model.hpp)
-  const int* je_b;
-  const double* je_c;
   const int* fs_species;             // lane slot -> species of the f gather
   const int4* t_rec;                 // per term: {k index | flags << 28, reactants x3}
   int es_n;                          // f estimate (Program::es_hdr and following)
@@ -76,9 +72,6 @@ struct DevProgram {
   const double* sp_radius;
   const int *aq_nr, *aq_np, *aq_sp, *aq_water, *aq_env, *aq_flt, *aq_slot;
   const double* aq_small_water;
-  const int* js_ptr;
-  const int4* js_a;
-  const double* js_c;
   const int *jm_ptr, *jm_rxn, *jm_param;
   const int* mj_elist;  // J_rxn assembly order (Program::mj_elist)
   int mj_rows;
@@ -386,7 +379,7 @@ __host__ __device__ inline size_t fb_lds_doubles(const DevProgram& P) {
 // triangular solve (the 65th) and as the factorisation's tail buffers.
 // the LU tail's buffers: a pivot's row and column, 8 groups of up to 5 doubles
 constexpr int kLuTailStride = kLuTail / 8 + 1, kLuTailBuf = 2 * 8 * kLuTailStride;
-__host__ __device__ inline size_t fb_sink_doubles(const DevProgram& P) {
+__host__ __device__ inline size_t fb_scratch_doubles(const DevProgram& P) {
   size_t n = fb_lds_doubles(P);
   const size_t m = kLuTailBuf > kWave + 1 ? kLuTailBuf : kWave + 1;
   return n > m ? n : m;
@@ -663,28 +656,6 @@ __device__ __forceinline__ int cell_set_state(const DevProgram& P, int lane, con
 // calc_jac_contrib + jacobian_output + jac_map (camp_solver.c:1052-1106,
 // Jacobian.c:223-241).
 // ---------------------------------------------------------------------
-// Mass-action contributions to Jacobian element e of the gather space
-// (solver elements, or reaction-pattern elements for multi-phase programs).
-__host__ __device__ __forceinline__ dd jac_elem_mass_action(const DevProgram& P, int e, const double* s_state,
-                                                   const double* s_k, double h) {
-  dd D = {0.0, 0.0};
-  for (int q = P.j_ptr[e]; q < P.j_ptr[e + 1]; ++q) {
-    int4 a = P.je_a[q];
-    double c = P.je_c[q];
-    double v = s_k[a.x];
-    if (a.y >= 0) v *= s_state[a.y];
-    if (a.z >= 0) v *= s_state[a.z];
-    if (c == -1.0) {
-      D = dd_add(D, dd{-v, 0.0});
-    } else {
-      int g = P.je_b[q];
-      if (g >= 0 && !(-v * s_state[a.w] * c * h <= s_state[g])) continue;
-      D = dd_add(D, dd{c * v, 0.0});
-    }
-  }
-  return D;
-}
-
 // Operands of one J record.
 struct GjOps {
   int e, last, g, h1, h2;
@@ -1235,8 +1206,8 @@ __device__ __forceinline__ void cell_lu_solve(const DevProgram& P, int lane, dou
                                               double* w) {
   lane = phase_lane(lane);
   if (!FAR) {
-    // the zero slot, after the LU values and the factorisation's sinks (the
-    // f gather's scratch shares it)
+    // the zero slot, 64 places after the LU values (the f gather's scratch
+    // shares it)
     if (lane == 0) lu[P.lu_nnz + kWave] = 0.0;
     wsync();
   }

@@ -449,7 +449,7 @@ __global__ void __launch_bounds__(64) k_lu_solve(DevProgram P, int nc, const dou
   extern __shared__ double smem[];
   int lane = threadIdx.x;
   if (sp) s = *sp;  // scale from device memory (graph replays)
-  double* s_lu = smem;  // LU values, then the factorisation's sinks and the solve's zero slot
+  double* s_lu = smem;  // LU values and the zero slot
   double* s_b = s_lu + P.lu_nnz + kWave + 1;
   double* s_w = s_b + P.nv;
   for (int c = blockIdx.x; c < nc; c += gridDim.x) {

@@ -71,7 +71,7 @@ __host__ __device__ inline size_t cell_lu_lds(const DevProgram& P) {
 __host__ __device__ inline size_t cell_bdf_lds_doubles(const DevProgram& P, int place) {
   const bool lds = !P.mp && place == kPlaceLds;
   return even_up(P.ns + cell_lds_env(P, place)) + mp_lds_doubles(P) +
-         even_up(2 * (size_t)P.n_terms + (size_t)cell_lds_vectors(P, place) * P.nv + fb_sink_doubles(P) +
+         even_up(2 * (size_t)P.n_terms + (size_t)cell_lds_vectors(P, place) * P.nv + fb_scratch_doubles(P) +
          (cell_lu_global(P, place) ? 0 : place == kPlaceGlobal ? cell_lu_lds(P) : (size_t)P.lu_nnz) +
          (lds ? (size_t)P.nnz + 2 * (size_t)P.nv : 0) + 24);
 }

@@ -581,8 +581,8 @@ __device__ __forceinline__ void mp_j_prologue(const DevProgram& P, int lane, con
 }
 
 // One record of a J_rxn row stream (Program::mj_rec) added to D: a
-// mass-action record as jac_elem_mass_action adds it, a special record as
-// mp_jac_record does, padding not at all.
+// mass-action record as gj_acc adds it, a special record as mp_jac_record does,
+// padding not at all.
 __device__ __forceinline__ dd mp_jac_stream_record(const DevProgram& P, int4 a, int4 b,
                                                    const double* s_state, const double* s_k,
                                                    double h, const double* s_part,

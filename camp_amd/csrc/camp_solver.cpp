@@ -43,7 +43,6 @@ void Solver::setup_device() {
   P.lu_nnz = G.lu_nnz;
   P.n_rxn = m.n_rxn;
   P.dep_state = dev_upload(G.dep_state, owned);
-  P.j_ptr = dev_upload(G.j_ptr, owned);
   P.colptr = dev_upload(G.colptr, owned);
   P.rowval = dev_upload(G.rowval, owned);
   P.n_k = G.n_k;
@@ -101,9 +100,6 @@ void Solver::setup_device() {
   P.fb_rows = G.fb_rows;
   P.fb_nparts = G.fb_nparts;
   P.fb_rec = reinterpret_cast<const int4*>(dev_upload(G.fb_rec, owned));
-  P.je_a = reinterpret_cast<const int4*>(dev_upload(G.je_a, owned));
-  P.je_b = dev_upload(G.je_b, owned);
-  P.je_c = dev_upload(G.je_c, owned);
   std::vector<int> rx_type(m.n_rxn), rx_fidx(m.n_rxn), rx_eidx(m.n_rxn), rx_nreact(m.n_rxn);
   for (int r = 0; r < m.n_rxn; ++r) {
     int* id = m.rint(r);
@@ -181,9 +177,6 @@ void Solver::setup_device() {
     P.aq_flt = dev_upload(G.aq_flt, owned);
     P.aq_slot = dev_upload(G.aq_slot, owned);
     P.aq_small_water = dev_upload(G.aq_small_water, owned);
-    P.js_ptr = dev_upload(G.js_ptr, owned);
-    P.js_a = reinterpret_cast<const int4*>(dev_upload(G.js_a, owned));
-    P.js_c = dev_upload(G.js_c, owned);
     P.mj_rows = G.mj_rows;
     P.mj_elist = dev_upload(G.mj_elist, owned);
     P.mj_rec = reinterpret_cast<const int4*>(dev_upload(G.mj_rec, owned));
@@ -1478,7 +1471,7 @@ extern "C" int camp_solver_set_placement(void* solver_data, int place) {
 // Autotuner for the persistent per-cell kernel.  Candidates: the cell
 // placement (history in LDS: fewer cells per CU; history in global memory:
 // more cells per CU, two wavefronts per SIMD; history and LU factors in
-// global memory: three wavefronts per SIMD) times cells per workgroup
+// global memory: more still) times cells per workgroup
 // {1, 2, 4, 8, 16, 32}; every candidate that fits a compute unit solves the
 // same sample of cells (every (nc / n_sample)-th cell, copied with its rate
 // data and J history, so the solver's own cells are untouched) over

@@ -108,7 +108,8 @@ def test_large_launch_of_a_wide_mechanism():
 def test_placements_that_do_not_fit(n, cells_per_block):
     """Four cells of 300 species a workgroup fit with placement 1 only, one of
     1300 with placement 1 only, one of 1500 with none: the others run with
-    their vectors in global memory, and the result is the same bit for bit."""
+    their vectors in global memory, and the result is the same bit for bit, also
+    with every wavefront's memory filled with NaNs before each cell."""
     n_cells = 5
     y0 = np.random.default_rng(5).uniform(1.0, 2.0, (n_cells, n))
     got = []
@@ -116,6 +117,7 @@ def test_placements_that_do_not_fit(n, cells_per_block):
         gpu = CampSolver(ring_mechanism(n), n_cells)
         assert gpu.set_placement(place) == place
         assert gpu.set_cells_per_block(cells_per_block) == cells_per_block
+        gpu.set_poison(place == 2)
         y = y0.copy()
         assert gpu.solve(y, np.tile(ENV, (n_cells, 1)), 0.0, 60.0) == 0
         got.append(y)
@@ -172,3 +174,25 @@ def test_layer_calls_of_a_large_grid_return_their_memory():
     assert torch.cuda.mem_get_info()[0] > free - (64 << 20)
     assert np.array_equal(gpu.eval_deriv(state, env)[1], f0)
     assert np.array_equal(gpu.eval_lu_solve(jac, 0.5, b)[1], x0)
+
+
+@pytest.mark.parametrize("n, per_species", [(50, 18), (100, 3), (200, 2)])
+@pytest.mark.parametrize("place", [0, 1, 2])
+def test_more_reactions_than_a_lane_holds_and_than_factors(n, per_species, place):
+    """Rings with several reactions a species: more than 256 terms, whose rate
+    constants the lanes no longer hold all of, more rate constants than LU
+    factors (J stages them in the factors' place), and more than 128 solver
+    variables (solved in a scratch vector), one step with every placement and
+    every wavefront's memory filled with NaNs (tolerance as above)."""
+    n_cells = 5
+    rx = [Reaction("ARRHENIUS", [i], [((i + 1) % n, 1.0)], {"A": 1.0e-3 / per_species})
+          for _ in range(per_species) for i in range(n)]
+    mech = Mechanism(["S%d" % i for i in range(n)], [1] * n, [1.0e-10] * n, rx, rel_tol=1.0e-6)
+    gpu = CampSolver(mech, n_cells)
+    assert len(rx) > 256 and (n > 128 or len(rx) > gpu.lu_nnz)
+    gpu.set_placement(place)
+    gpu.set_poison(True)
+    y0 = np.random.default_rng(6).uniform(1.0, 2.0, (n_cells, n))
+    y = y0.copy()
+    assert gpu.solve(y, np.tile(ENV, (n_cells, 1)), 0.0, 60.0) == 0
+    assert np.allclose(y, ring_solution(y0, 60.0), rtol=1e-3, atol=0.0)
