@@ -55,16 +55,19 @@ __device__ __forceinline__ double rpoweri(double b, int e) {
 // execution masks, with its control state copied between vector registers).
 __device__ __forceinline__ bool uc(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
 
-// A wave-uniform double kept in scalar registers: every assignment reads the
-// first active lane's value (all lanes hold the same one), so the value
-// lives in an SGPR pair between uses instead of occupying two VGPRs for the
-// whole solve (the integrator's step-control scalars).
+// A step-control value, the same in every lane, held in vector registers: in
+// scalar ones each assignment was a v_readfirstlane pair and each use a copy
+// back, 1k to 3k cycles of a step (10 species 46.7k -> 45.8k, with everything in
+// LDS 56.1k -> 52.0k; CB05-scale, everything in LDS, 75.4k -> 72.5k).  A class of
+// its own: as plain doubles the compiler, at the two-wavefront register bound,
+// spills f's rate constants instead of the history passes' values (2000
+// CB05-scale cells: f 13.8k instead of 13.3k cycles).
 struct UDouble {
   double v;
   UDouble() = default;
-  __device__ UDouble(double x) : v(uni(x)) {}
+  __device__ UDouble(double x) : v(x) {}
   __device__ UDouble& operator=(double x) {
-    v = uni(x);
+    v = x;
     return *this;
   }
   __device__ UDouble& operator+=(double x) { return *this = v + x; }
@@ -72,11 +75,6 @@ struct UDouble {
   __device__ UDouble& operator*=(double x) { return *this = v * x; }
   __device__ UDouble& operator/=(double x) { return *this = v / x; }
   __device__ operator double() const { return v; }
-  __device__ static double uni(double x) {
-    int lo = __builtin_amdgcn_readfirstlane(__double2loint(x));
-    int hi = __builtin_amdgcn_readfirstlane(__double2hiint(x));
-    return __hiloint2double(hi, lo);
-  }
 };
 
 // MP selects the multi-phase instantiation: gas-phase programs run a kernel
