@@ -188,9 +188,10 @@ struct Solver {
   struct EvalArrays {
     Solver& S;
     double* at;
-    // doubles: of all arrays that take() will hand out
+    // doubles: of all (up to four) arrays that take() will hand out, each on a
+    // 256-byte line as an allocation of its own would be
     EvalArrays(Solver& s, size_t doubles) : S(s) {
-      const size_t bytes = std::max<size_t>(doubles, 1) * sizeof(double);
+      const size_t bytes = (doubles + 4 * 32) * sizeof(double);
       if (bytes > S.eval_bytes) {
         S.drop_eval();
         HIP_OK(hipMalloc(&S.d_eval, bytes));
@@ -205,7 +206,7 @@ struct Solver {
     EvalArrays& operator=(const EvalArrays&) = delete;
     double* take(size_t n) {
       double* p = at;
-      at += n;
+      at += (n + 31) / 32 * 32;
       return p;
     }
   };
