@@ -718,10 +718,15 @@ static int schedule_lu(const LuTasks& T, int tail, int most, std::vector<LuSlot>
         path[p] = std::max(path[p], path[T.out[q]] + kLuDist - 1);
     path[p] += groups[p];
   }
+  // (no schedule is shorter than the longest chain, or than the lanes allow)
+  const int longest = *std::max_element(path.begin(), path.end());
+  long total = 0;
+  for (int c : groups) total += c;
+  if (std::max<long>(longest, (total + 63) / 64) >= most) return most;
   // list scheduling: the ready task with the longest chain (of equals the first)
   // to a free lane; ready[c]: the ready tasks with a chain of c, a heap of their
   // numbers, top: the longest
-  std::vector<std::vector<int>> ready(1 + *std::max_element(path.begin(), path.end()));
+  std::vector<std::vector<int>> ready(1 + longest);
   int top = 0;
   // tasks that become ready at a group: linked lists (a group's tasks enter the
   // heap together, so their order does not matter)
