@@ -6,10 +6,11 @@
 // algorithm that CAMP's solver_run drives (camp_solver.c:544-693; CVODE:
 // Hindmarsh et al., ACM TOMS 31(3), 2005) -- but with order, step size,
 // Newton iteration, Jacobian reuse and error test decided per cell instead
-// of once for the whole block of cells.  Everything a step touches lives
-// in LDS (Nordsieck history, work vectors, rate constants, LU factors);
-// only the cell's saved Jacobian history (J_solver, J_state, J_deriv,
-// camp_solver.c:1111-1114) is in HBM, because CAMP keeps it across calls.
+// of once for the whole block of cells.  What a step touches lives in LDS
+// as far as it fits (Nordsieck history, work vectors, rates, LU factors; kPlaceLds
+// and following say what lies where); the cell's saved Jacobian history (J_solver,
+// J_state, J_deriv, camp_solver.c:1111-1114) has its place in HBM, because CAMP
+// keeps it across calls.
 #include <cstddef>
 #include <cstdio>
 #include <mutex>

@@ -46,8 +46,8 @@ constexpr int kCellProf = 7;
 //                in the scratch.  Needs the least LDS; for programs of which no
 //                cell fits with the placement asked for (the vectors in LDS
 //                outgrow it with the number of solver variables).
-// All but kPlaceLds and the multi-phase kernel are compiled for two wavefronts
-// per SIMD, kPlaceWide for one.
+// The gas-phase kernels of kPlaceGlobal and kPlaceGlobalLu are compiled for two
+// wavefronts per SIMD, the others for one.
 constexpr int kPlaceLds = 0, kPlaceGlobal = 1, kPlaceGlobalLu = 2, kNumPlacements = 3,
               kPlaceWide = 3;
 // LU factors in the wavefront's global scratch

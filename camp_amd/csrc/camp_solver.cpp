@@ -232,6 +232,7 @@ void Solver::launch_wave_deriv(const double* y, const double* st, const double* 
   int nc = m.nc, wpb = fj_waves_per_block(P);
   size_t lds = wpb * fj_lds_doubles(P) * sizeof(double);
   allow_lds((const void*)k_deriv, lds);
+  (void)hipGetLastError();  // (an error that the caller's own calls left is not ours)
   hipLaunchKernelGGL(k_deriv, dim3(std::min(nblk(nc, wpb), 4096)), dim3(64 * wpb), lds, stream, P,
                      nc, y, st, env, d_renv, d_Js, d_Jy, d_Jf, out, h, use_est, fail);
   HIP_OK(hipGetLastError());
@@ -251,6 +252,7 @@ void Solver::launch_wave_jac(const double* y, const double* st, const double* en
   int nc = m.nc, wpb = fj_waves_per_block(P);
   size_t lds = wpb * fj_lds_doubles(P) * sizeof(double);
   allow_lds((const void*)k_jac, lds);
+  (void)hipGetLastError();  // (an error that the caller's own calls left is not ours)
   hipLaunchKernelGGL(k_jac, dim3(std::min(nblk(nc, wpb), 4096)), dim3(64 * wpb), lds, stream, P,
                      nc, y, st, env, d_renv, J, h, jr);
   HIP_OK(hipGetLastError());

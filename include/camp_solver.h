@@ -207,13 +207,13 @@ int camp_solver_set_cells_per_block(void *solver_data, int cells_per_block);
  * history in global memory (two wavefronts per SIMD), 2 = the LU factors, the
  * rate constants and the J history in global memory (most cells per compute
  * unit).  Cells that do not fit a compute unit's LDS with the placement set
- * run with most of their vectors in global memory.  Returns the placement set (1 by default; a negative place
- * only asks).  Results do not depend on it. */
+ * run with most of their vectors in global memory.  Returns the placement set
+ * (1 by default; a negative place only asks).  Results do not depend on it. */
 int camp_solver_set_placement(void *solver_data, int place);
 
 /* LDS bytes one cell of the per-cell kernel uses with the given placement
- * (-1 for an unknown placement or an uninitialised solver; makes the
- * solver's device buffers). */
+ * (where it does not fit, of what runs in its place; -1 for an unknown
+ * placement or an uninitialised solver; makes the solver's device buffers). */
 long camp_solver_cell_lds_bytes(void *solver_data, int place);
 
 /* Autotuner for the per-cell kernel: solves a sample of n_sample cells

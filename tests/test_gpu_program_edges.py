@@ -1,4 +1,5 @@
 """Programs at the edges of what the kernels' tables can describe."""
+import ctypes
 import dataclasses
 
 import numpy as np
@@ -196,3 +197,20 @@ def test_more_reactions_than_a_lane_holds_and_than_factors(n, per_species, place
     y = y0.copy()
     assert gpu.solve(y, np.tile(ENV, (n_cells, 1)), 0.0, 60.0) == 0
     assert np.allclose(y, ring_solution(y0, 60.0), rtol=1e-3, atol=0.0)
+
+
+def test_layers_ignore_an_error_left_by_the_caller():
+    """A HIP call of the caller's that failed (a device that is not there) leaves
+    its error for the next one to ask: f and J do not take it for theirs."""
+    mech = box_mechanism(1)
+    cells = synthetic_cells(mech, 2, seed=2)
+    gpu = CampSolver(mech, 2)
+    gpu.set_rates(cells.rates)
+    assert gpu.eval_deriv(cells.state, cells.env)[0] == 0
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64.so" in line)
+    hip = ctypes.CDLL(path)
+    for call in (gpu.eval_deriv, gpu.eval_jac):
+        assert hip.hipSetDevice(99) != 0
+        assert call(cells.state, cells.env)[0] == 0
+    hip.hipGetLastError()
